@@ -450,6 +450,15 @@ int lmk_apply_rotary_qk(const lmk_tensor4* q, const lmk_tensor4* k, const lmk_te
                         const int64_t* position_ids, int64_t pos_stride_b, int B, int H, int L, int D, int dtype,
                         void* stream);
 
+/* The same for one tensor or two (x2, out2 may be NULL), with the direction as an argument.  transposed != 0: the
+ * transpose of the (linear) rotation, which its gradient takes -- the same expression with the sine table's halves
+ * swapped and negated, x*cos - rotate_half(x)*cat(sin[D/2:], sin[:D/2]), same three roundings; the table is read
+ * that way in place. */
+int lmk_rotate_qk(const lmk_tensor4* x, const lmk_tensor4* out, const lmk_tensor4* x2, const lmk_tensor4* out2,
+                  const void* cos_table, const void* sin_table, int64_t table_stride_row, int64_t n_pos,
+                  const int64_t* position_ids, int64_t pos_stride_b, int B, int H, int L, int D, int dtype,
+                  int transposed, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -174,6 +174,7 @@ struct RotaryParams {
   int64_t x2s_b, x2s_h, x2s_r, o2s_b, o2s_h, o2s_r;
   const int64_t* pos;
   int64_t pos_stride_b, n_pos;
+  int transposed;                                 // the gradient's rotation: the sine table's halves swapped and negated
   int B, H, L;
   int64_t xs_b, xs_h, xs_r, os_b, os_h, os_r, cs_r;
 };

@@ -1346,7 +1346,10 @@ __global__ __launch_bounds__(256) void lmk_rotary_kernel(RotaryParams p) {
     other2 = *(const u32x4_t*)(src2 + 16 * (j ^ (LPR / 2)));
   }
   const u32x4_t c = *(const u32x4_t*)((const char*)p.cos + 2 * (pos * p.cs_r) + 16 * j);
-  const u32x4_t s = *(const u32x4_t*)((const char*)p.sin + 2 * (pos * p.cs_r) + 16 * j);
+  u32x4_t s = *(const u32x4_t*)((const char*)p.sin + 2 * (pos * p.cs_r) + 16 * (p.transposed ? j ^ (LPR / 2) : j));
+  const uint32_t flip = p.transposed ? 0x80008000u : 0u;         // sign bits of two 16-bit values
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] ^= flip;
   float o[8];
   rotate_chunk<T>(x, other, c, s, j >= LPR / 2, o);
   const u32x4_t r = {pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};

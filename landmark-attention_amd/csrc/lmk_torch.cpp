@@ -1,0 +1,490 @@
+// Host path of the Python shim in native code: landmark_hip/_native.so, loaded by landmark_hip/_lib.py.
+//
+// A training step on a short sequence or a decode step keeps the GPU busy for 20-100 us, and the same calls made from
+// Python -- a descriptor per tensor, a conversion per argument, an autograd node that has to take the interpreter lock
+// in the engine's thread -- take as long or longer.  Here an entry point of the shim is one call: arguments are read
+// from the tensors, outputs and workspaces come from torch's allocator, the launches go through the C ABI of
+// include/lmk.h (liblandmark_hip.so) on torch's current stream, and the backward is a C++ autograd node.
+//
+// Errors keep their Python types: AssertionError for what the shim asserts, LmkError for a code of the C ABI.
+#include <Python.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+
+#include <cmath>
+#include <string>
+
+#include "../../include/lmk.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+PyObject* g_lmk_error = nullptr;                         // landmark_hip._lib.LmkError
+
+struct Failed {                                          // an error on its way to Python
+  int code;                                              // of the C ABI; 0: an AssertionError
+  std::string text;
+};
+void need(bool ok, const char* text) {
+  if (!ok) throw Failed{0, text};
+}
+void check(int code) {
+  if (code != 0) throw Failed{code, lmk_strerror(code)};
+}
+void set_python_error(const Failed& f) {                 // with the interpreter lock held
+  if (f.code == 0 || g_lmk_error == nullptr) {
+    PyErr_SetString(f.code == 0 ? PyExc_AssertionError : PyExc_RuntimeError, f.text.c_str());
+    return;
+  }
+  PyObject* e = PyObject_CallFunction(g_lmk_error, "is", f.code, f.text.c_str());
+  if (e == nullptr) return;
+  PyErr_SetObject(g_lmk_error, e);
+  Py_DECREF(e);
+}
+
+// Runs f without the interpreter lock.
+template <class F>
+auto without_gil(F&& f) {
+  struct Release {
+    PyThreadState* s = PyEval_SaveThread();
+    ~Release() { PyEval_RestoreThread(s); }
+  } release;
+  return f();
+}
+
+// ---- what the kernels take
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kBFloat16: return LMK_DTYPE_BF16;
+    case at::kHalf: return LMK_DTYPE_F16;
+    default: return -1;
+  }
+}
+lmk_tensor4 t4(const Tensor& t) {
+  const auto s = t.strides();
+  return lmk_tensor4{t.data_ptr(), s[0], s[1], s[2]};
+}
+// Tensors the kernels can read in place (unit stride along D, rows walked forwards, 16-byte aligned) as they are,
+// others as a contiguous copy.
+Tensor kernel_ready(const Tensor& t) {
+  const auto s = t.strides();
+  const bool ok = s[3] == 1 && s[2] > 0 && ((s[0] | s[1] | s[2]) & 7) == 0 &&
+                  (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+  return ok ? t : t.contiguous();
+}
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+Tensor bytes_on(const Tensor& like, size_t n) {
+  return at::empty({(int64_t)n}, like.options().dtype(at::kByte));
+}
+bool same_shape(const Tensor& a, const Tensor& b) { return a.sizes() == b.sizes(); }
+
+// ---- attention
+// How a block of tokens is stored: BLOCKS = tensors as they are, any block of 2..128 tokens; PADDED = rows of `block`
+// slots of which `block_real` hold tokens (all of them for a native block size).
+struct Shape {
+  int B, H, Lq, Lk, D, n_prefix, block, block_real, dtype;
+  bool blocks;
+  float scale;
+};
+
+Shape shape_of(const Tensor& q, const Tensor& k, int n_prefix, double scale, int block, int block_real, bool blocks) {
+  return Shape{(int)q.size(0), (int)q.size(1), (int)q.size(2), (int)k.size(2), (int)q.size(3), n_prefix, block, block_real,
+               dtype_code(q), blocks, (float)scale};
+}
+
+// (o, statistics): statistics (2, B*H, Lq) fp32, the forward's L and M.
+std::pair<Tensor, Tensor> forward(const Shape& s, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& group_scale) {
+  Tensor o = at::empty_like(q);                          // keeps q's memory layout
+  Tensor st = at::empty({2, (int64_t)s.B * s.H, s.Lq}, q.options().dtype(at::kFloat));
+  const lmk_tensor4 tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o);
+  float* L = st.data_ptr<float>();
+  float* M = L + (int64_t)s.B * s.H * s.Lq;
+  void* stream = stream_of(q);
+  if (group_scale.defined())
+    check(lmk_attn_fwd_group_scale(&tq, &tk, &tv, &to, L, M, group_scale.data_ptr<float>(), s.B, s.H, s.Lq, s.Lk, s.D, s.scale,
+                                   s.block, s.n_prefix, s.dtype, stream));
+  else if (s.blocks)
+    check(lmk_attn_fwd_blocks(&tq, &tk, &tv, &to, L, M, s.B, s.H, s.Lq, s.Lk, s.D, s.scale, s.block, s.n_prefix, s.dtype, stream));
+  else
+    check(lmk_attn_fwd_padded(&tq, &tk, &tv, &to, L, M, s.B, s.H, s.Lq, s.Lk, s.D, s.scale, s.block, s.block_real, s.n_prefix,
+                              s.dtype, stream));
+  return {o, st};
+}
+
+struct HandoverLimits {                                  // HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS of attention.py
+  int64_t max_bytes, min_keys;
+};
+
+variable_list backward(const Shape& s, const HandoverLimits& limits, const Tensor& q, const Tensor& k, const Tensor& v,
+                       const Tensor& o, const float* l, const float* m, const Tensor& dout, const Tensor& group_scale) {
+  Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);   // each in its input's layout
+  size_t nbytes;
+  if (group_scale.defined()) {
+    nbytes = lmk_attn_bwd_group_scale_workspace_bytes(s.B, s.H, s.Lq, s.Lk, s.block);
+  } else if (s.blocks) {
+    nbytes = lmk_attn_bwd_blocks_workspace_bytes(s.B, s.H, s.Lq, s.Lk, s.block);
+  } else {
+    nbytes = lmk_attn_bwd_workspace_bytes(s.B, s.H, s.Lq, s.Lk, s.block);
+    if (s.block_real == s.block) {
+      const size_t ho = lmk_attn_bwd_handover_workspace_bytes(s.B, s.H, s.Lq, s.Lk, s.block);
+      if (ho > 0 && (int64_t)ho <= limits.max_bytes && s.Lk >= limits.min_keys) nbytes = ho;   // the size picks the kernels
+    }
+  }
+  Tensor ws = bytes_on(q, nbytes);
+  const lmk_tensor4 tq = t4(q), tk = t4(k), tv = t4(v), to = t4(o), tdo = t4(dout), tdq = t4(dq), tdk = t4(dk), tdv = t4(dv);
+  void* stream = stream_of(q);
+  if (group_scale.defined())
+    check(lmk_attn_bwd_group_scale(&tq, &tk, &tv, &to, &tdo, l, m, group_scale.data_ptr<float>(), &tdq, &tdk, &tdv,
+                                   ws.data_ptr(), nbytes, s.B, s.H, s.Lq, s.Lk, s.D, s.scale, s.block, s.n_prefix, s.dtype, stream));
+  else if (s.blocks)
+    check(lmk_attn_bwd_blocks(&tq, &tk, &tv, &to, &tdo, l, m, &tdq, &tdk, &tdv, ws.data_ptr(), nbytes, s.B, s.H, s.Lq, s.Lk,
+                              s.D, s.scale, s.block, s.n_prefix, s.dtype, stream));
+  else
+    check(lmk_attn_bwd_padded(&tq, &tk, &tv, &to, &tdo, l, m, &tdq, &tdk, &tdv, ws.data_ptr(), nbytes, s.B, s.H, s.Lq, s.Lk,
+                              s.D, s.scale, s.block, s.block_real, s.n_prefix, s.dtype, stream));
+  return {dq, dk, dv};
+}
+
+// Runs a backward's body in the engine's thread; an error of ours leaves as the Python exception it stands for.
+template <class F>
+variable_list node_body(F&& f) {
+  try {
+    return f();
+  } catch (const Failed& e) {
+    PyGILState_STATE g = PyGILState_Ensure();
+    set_python_error(e);
+    python_error err;
+    err.persist();
+    PyGILState_Release(g);
+    throw err;
+  }
+}
+
+struct AttentionBackward : public torch::autograd::Node {
+  SavedVariable q, k, v, o, st, gs;
+  bool has_gs = false;
+  Shape s;
+  HandoverLimits limits;
+
+  variable_list apply(variable_list&& grads) override {
+    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    return node_body([&] {
+      need(s.Lq % s.block_real == 0 && s.Lk % s.block_real == 0, "Backward supported only for full blocks");
+      const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(getptr()), st_ = st.unpack();
+      const Tensor gs_ = has_gs ? gs.unpack() : Tensor();
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(q_.device());
+      const float* L = st_.data_ptr<float>();
+      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(grads[0]), gs_);
+    });
+  }
+  std::string name() const override { return "FusedLandmarkAttentionBackward"; }
+  void release_variables() override {
+    for (SavedVariable* x : {&q, &k, &v, &o, &st, &gs}) x->reset_data();
+  }
+};
+
+// fused_landmark_attention for landmarks at fixed stride, head dims 64 and 128.
+Tensor attention(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& gs_in, bool has_scale, double scale,
+                 int64_t block, HandoverLimits limits) {
+  need(q_in.dim() == 4 && k_in.dim() == 4 && v_in.dim() == 4, "q, k, v are (batch, heads, rows, head dim)");
+  const int64_t Lq = q_in.size(2), Lk = k_in.size(2), D = q_in.size(3);
+  need(block > 0 && (Lk - Lq) % block == 0, "the keys in front of the first query must be whole blocks");
+  need(k_in.size(0) == q_in.size(0) && k_in.size(1) == q_in.size(1) && k_in.size(3) == D && same_shape(k_in, v_in),
+       "k and v must have the same shape, and q's batch, heads and head dim");
+  need(D <= 128, "FlashAttention only support head dimensions up to 128");
+  need(q_in.scalar_type() == k_in.scalar_type() && q_in.scalar_type() == v_in.scalar_type(), "All tensors must have the same type");
+  need(q_in.is_cuda() && k_in.is_cuda() && v_in.is_cuda(), "q, k, v must be on the GPU");
+  need(dtype_code(q_in) >= 0, "HIP kernels are built for bf16 and fp16");
+  need(D == 64 || D == 128, "HIP kernels are built for head dims (64, 128)");
+  const int n_prefix = (int)((Lk - Lq) / block);
+  const bool native = block == 32 || block == 64 || block == 128, has_gs = gs_in.defined();
+  if (has_gs) {
+    need(block >= 2 && block <= 128, "group dropout: blocks of 2..128 tokens");
+    need(gs_in.dim() == 4 && gs_in.size(0) == q_in.size(0) && gs_in.size(1) == q_in.size(1) && gs_in.size(2) == Lk / block &&
+             gs_in.size(3) == Lq && gs_in.scalar_type() == at::kFloat && gs_in.device() == q_in.device(),
+         "group_scale is (B, H, Lk / block_size, Lq) fp32 on q's device");
+  }
+  if (!has_scale) scale = 1.0 / std::sqrt((double)D);
+  c10::DeviceGuard device(q_in.device());
+  Tensor q, k, v, gs;
+  std::pair<Tensor, Tensor> r;
+  const bool differentiate =
+      at::GradMode::is_enabled() && (q_in.requires_grad() || k_in.requires_grad() || v_in.requires_grad());
+  Shape s;
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    q = kernel_ready(q_in);
+    k = kernel_ready(k_in);
+    v = kernel_ready(v_in);
+    if (has_gs) gs = gs_in.contiguous();
+    s = shape_of(q, k, n_prefix, scale, (int)block, (int)block, !native);
+    r = forward(s, q, k, v, gs);
+  }
+  if (differentiate) {
+    auto node = std::shared_ptr<AttentionBackward>(new AttentionBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(q_in, k_in, v_in));
+    // a tensor that was copied into kernel layout is saved as that copy, and has no history of its own
+    node->q = SavedVariable(q, false);
+    node->k = SavedVariable(k, false);
+    node->v = SavedVariable(v, false);
+    node->st = SavedVariable(r.second, false);
+    node->has_gs = has_gs;
+    if (has_gs) node->gs = SavedVariable(gs, false);
+    node->s = s;
+    node->limits = limits;
+    torch::autograd::set_history(r.first, node);
+    node->o = SavedVariable(r.first, true);
+  }
+  return r.first;
+}
+
+// ---- rotary embedding
+struct Tables {
+  Tensor cos, sin;
+};
+// (n_pos, D) views of the tables the kernels can read: unit stride along D, 16-byte aligned rows, one row stride.
+Tables tables(const Tensor& cos_in, const Tensor& sin_in, at::ScalarType dtype) {
+  Tensor cos = cos_in.dim() == 2 ? cos_in : cos_in.reshape({-1, cos_in.size(-1)});
+  Tensor sin = sin_in.dim() == 2 ? sin_in : sin_in.reshape({-1, sin_in.size(-1)});
+  need(cos.scalar_type() == dtype && sin.scalar_type() == dtype, "rotary tables must be in the model dtype (llama_mem.py:121-124)");
+  need(same_shape(cos, sin), "the rotary tables must have one shape");
+  auto aligned = [](const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
+  if (cos.stride(1) != 1 || cos.stride(0) % 8 || !aligned(cos)) cos = cos.contiguous();
+  if (sin.stride(1) != 1 || sin.stride(0) != cos.stride(0) || !aligned(sin)) {
+    sin = sin.contiguous();
+    cos = cos.contiguous();
+  }
+  return {cos, sin};
+}
+
+// q may be undefined; `transposed`: the rotation the gradient takes.
+std::pair<Tensor, Tensor> rotate(const Tensor& q_in, const Tensor& k_in, const Tables& t, const Tensor& pos, bool transposed) {
+  const Tensor k = kernel_ready(k_in), q = q_in.defined() ? kernel_ready(q_in) : Tensor();
+  Tensor ko = at::empty_like(k), qo = q.defined() ? at::empty_like(q) : Tensor();
+  const int B = (int)k.size(0), H = (int)k.size(1), L = (int)k.size(2), D = (int)k.size(3);
+  const int64_t pos_stride = (pos.size(0) == B && B > 1) ? L : 0;
+  const lmk_tensor4 tk = t4(k), tko = t4(ko);
+  lmk_tensor4 tq = {}, tqo = {};
+  if (q.defined()) {
+    tq = t4(q);
+    tqo = t4(qo);
+  }
+  check(lmk_rotate_qk(&tk, &tko, q.defined() ? &tq : nullptr, q.defined() ? &tqo : nullptr, t.cos.data_ptr(),
+                                t.sin.data_ptr(), t.cos.stride(0), t.cos.size(0), pos.data_ptr<int64_t>(), pos_stride, B, H, L, D,
+                                dtype_code(k), transposed ? 1 : 0, stream_of(k)));
+  return {qo, ko};
+}
+
+struct RotaryBackward : public torch::autograd::Node {
+  SavedVariable cos, sin, pos;
+  bool has_q = false;
+
+  variable_list apply(variable_list&& grads) override {
+    return node_body([&]() -> variable_list {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      const Tables t = {cos.unpack(), sin.unpack()};
+      const Tensor pos_ = pos.unpack();
+      const Tensor &gk = grads[has_q ? 1 : 0], gq = has_q ? grads[0] : Tensor();
+      if (!gk.defined() && !gq.defined()) return has_q ? variable_list{Tensor(), Tensor()} : variable_list{Tensor()};
+      c10::DeviceGuard device((gk.defined() ? gk : gq).device());
+      if (!has_q) return {rotate(Tensor(), gk, t, pos_, true).second};
+      if (!gk.defined()) return {rotate(Tensor(), gq, t, pos_, true).second, Tensor()};
+      auto r = rotate(gq, gk, t, pos_, true);
+      return {r.first, r.second};
+    });
+  }
+  std::string name() const override { return "RotaryEmbeddingBackward"; }
+  void release_variables() override {
+    for (SavedVariable* x : {&cos, &sin, &pos}) x->reset_data();
+  }
+};
+
+// apply_rotary_pos_emb; q undefined or of k's shape
+std::pair<Tensor, Tensor> rotary(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const Tensor& pos_in) {
+  need(k.dim() == 4 && k.is_cuda() && dtype_code(k) >= 0, "k is (batch, heads, rows, head dim), bf16 or fp16, on the GPU");
+  need(!q.defined() || (q.scalar_type() == k.scalar_type() && q.device() == k.device()), "q and k must have one type and device");
+  need(pos_in.dim() == 2 && pos_in.size(1) == k.size(2) && (pos_in.size(0) == 1 || pos_in.size(0) == k.size(0)),
+       "position_ids is (1, rows) or (batch, rows)");
+  need(pos_in.scalar_type() == at::kLong && pos_in.device() == k.device(), "position_ids is int64 on k's device");
+  c10::DeviceGuard device(k.device());
+  const bool has_q = q.defined();
+  Tables t;
+  Tensor pos;
+  std::pair<Tensor, Tensor> r;
+  {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    t = tables(cos, sin, k.scalar_type());
+    pos = pos_in.contiguous();
+    r = rotate(q, k, t, pos, false);
+  }
+  if (at::GradMode::is_enabled() && (k.requires_grad() || (has_q && q.requires_grad()))) {
+    auto node = std::shared_ptr<RotaryBackward>(new RotaryBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(has_q ? torch::autograd::collect_next_edges(q, k) : torch::autograd::collect_next_edges(k));
+    node->cos = SavedVariable(t.cos, false);
+    node->sin = SavedVariable(t.sin, false);
+    node->pos = SavedVariable(pos, false);
+    node->has_q = has_q;
+    if (has_q) torch::autograd::set_history(r.first, node);
+    torch::autograd::set_history(r.second, node);
+  }
+  return r;
+}
+
+// ---- Python
+Tensor tensor_arg(PyObject* o) {                         // None: an undefined tensor
+  if (o == Py_None) return Tensor();
+  if (!THPVariable_Check(o)) throw Failed{0, "expected a tensor"};
+  return THPVariable_Unpack(o);
+}
+int64_t int_arg(PyObject* o) {
+  const int64_t v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+double float_arg(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+void count(Py_ssize_t n, Py_ssize_t want) { need(n == want, "wrong number of arguments"); }
+
+PyObject* tuple_of(std::initializer_list<Tensor> ts) {
+  PyObject* t = PyTuple_New((Py_ssize_t)ts.size());
+  Py_ssize_t i = 0;
+  for (const Tensor& x : ts) {
+    PyObject* o = x.defined() ? THPVariable_Wrap(x) : Py_NewRef(Py_None);
+    PyTuple_SET_ITEM(t, i++, o);
+  }
+  return t;
+}
+
+template <class F>
+PyObject* guarded(F&& f) {
+  HANDLE_TH_ERRORS
+  try {
+    return f();
+  } catch (const Failed& e) {
+    set_python_error(e);
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_set_error_class(PyObject*, PyObject* cls) {
+  Py_XDECREF(g_lmk_error);
+  g_lmk_error = Py_NewRef(cls);
+  Py_RETURN_NONE;
+}
+
+// attention(q, k, v, group_scale | None, sm_scale | None, block, handover_max_bytes, handover_min_keys) -> out
+PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 8);
+    const Tensor q = tensor_arg(a[0]), k = tensor_arg(a[1]), v = tensor_arg(a[2]), gs = tensor_arg(a[3]);
+    const bool has_scale = a[4] != Py_None;
+    const double scale = has_scale ? float_arg(a[4]) : 0.0;
+    const int64_t block = int_arg(a[5]);
+    const HandoverLimits limits = {int_arg(a[6]), int_arg(a[7])};
+    return THPVariable_Wrap(without_gil([&] { return attention(q, k, v, gs, has_scale, scale, block, limits); }));
+  });
+}
+
+// attn_fwd(q, k, v, group_scale | None, n_prefix, sm_scale, block, block_real, blocks) -> (o, L, M)
+PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 9);
+    const Tensor q = tensor_arg(a[0]), k = tensor_arg(a[1]), v = tensor_arg(a[2]), gs = tensor_arg(a[3]);
+    const Shape s = shape_of(q, k, (int)int_arg(a[4]), float_arg(a[5]), (int)int_arg(a[6]), (int)int_arg(a[7]), a[8] == Py_True);
+    Tensor L, M;
+    const Tensor o = without_gil([&] {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(q.device());
+      auto r = forward(s, q, k, v, gs);
+      L = r.second.select(0, 0);
+      M = r.second.select(0, 1);
+      return r.first;
+    });
+    return tuple_of({o, L, M});
+  });
+}
+
+// attn_bwd(q, k, v, o, do, L, M, group_scale | None, n_prefix, sm_scale, block, block_real, blocks, handover_max_bytes,
+//          handover_min_keys) -> (dq, dk, dv)
+PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 15);
+    Tensor t[8];
+    for (int i = 0; i < 8; ++i) t[i] = tensor_arg(a[i]);
+    const Shape s = shape_of(t[0], t[1], (int)int_arg(a[8]), float_arg(a[9]), (int)int_arg(a[10]), (int)int_arg(a[11]), a[12] == Py_True);
+    const HandoverLimits limits = {int_arg(a[13]), int_arg(a[14])};
+    const variable_list g = without_gil([&] {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(t[0].device());
+      return backward(s, limits, t[0], t[1], t[2], t[3], t[5].data_ptr<float>(), t[6].data_ptr<float>(), t[4], t[7]);
+    });
+    return tuple_of({g[0], g[1], g[2]});
+  });
+}
+
+// rotary(q | None, k, cos, sin, position_ids) -> (q_embed | None, k_embed)
+PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 5);
+    const Tensor q = tensor_arg(a[0]), k = tensor_arg(a[1]), cos = tensor_arg(a[2]), sin = tensor_arg(a[3]), pos = tensor_arg(a[4]);
+    const auto r = without_gil([&] { return rotary(q, k, cos, sin, pos); });
+    return tuple_of({r.first, r.second});
+  });
+}
+
+// The attention node as Python sees it: an autograd node with `saved_tensors` (q, k, v, o, L, M, and the group factors if
+// there are any), as a Python autograd Function has them.
+PyObject* py_saved_tensors(PyObject* self, void*) {
+  return guarded([&]() -> PyObject* {
+    auto node = std::static_pointer_cast<AttentionBackward>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata);
+    const Tensor q = node->q.unpack(), k = node->k.unpack(), v = node->v.unpack(), o = node->o.unpack(node), st = node->st.unpack();
+    if (!node->has_gs) return tuple_of({q, k, v, o, st.select(0, 0), st.select(0, 1)});
+    return tuple_of({q, k, v, o, st.select(0, 0), st.select(0, 1), node->gs.unpack()});
+  });
+}
+PyTypeObject g_attention_node_type;
+using namespace torch::autograd;                         // names inside the macro
+PyGetSetDef g_attention_node_properties[] = {
+    THP_FUNCTION_DEFAULT_PROPERTIES,
+    {"saved_tensors", py_saved_tensors, nullptr, nullptr, nullptr},
+    {nullptr, nullptr, nullptr, nullptr, nullptr},
+};
+
+#define LMK_FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(f)), METH_FASTCALL, nullptr
+PyMethodDef g_methods[] = {
+    {"set_error_class", py_set_error_class, METH_O, nullptr},
+    {"attention", LMK_FAST(py_attention)},
+    {"attn_fwd", LMK_FAST(py_attn_fwd)},
+    {"attn_bwd", LMK_FAST(py_attn_bwd)},
+    {"rotary", LMK_FAST(py_rotary)},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  PyTypeObject* node = torch::autograd::_initFunctionPyTypeObject(
+      g_attention_node_type, "landmark_hip.FusedLandmarkAttentionBackward", g_attention_node_properties, nullptr);
+  torch::autograd::registerCppFunction(typeid(AttentionBackward), node);
+  return PyModule_Create(&g_module);
+}

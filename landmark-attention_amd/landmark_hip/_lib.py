@@ -31,6 +31,22 @@ class Tensor4(ctypes.Structure):
 
 
 _lib = None
+_native_module = None
+
+
+def native():
+    """The shim's host path in native code (``csrc/lmk_torch.cpp``): calls the same C ABI."""
+    global _native_module
+    if _native_module is None:
+        lib()                                    # liblandmark_hip.so, which it links against
+        try:
+            from . import _native as m
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_native.so')} cannot be loaded ({e}): build it with "
+                              "`python landmark-attention_amd/build.py`; there is no fallback path") from e
+        m.set_error_class(LmkError)
+        _native_module = m
+    return _native_module
 
 
 def lib() -> ctypes.CDLL:
@@ -132,6 +148,8 @@ def lib() -> ctypes.CDLL:
         L.lmk_apply_rotary.argtypes = [T4, T4, vp, vp, i64, i64, vp, i64, i, i, i, i, i, vp]
         L.lmk_attn_fwd_rotary_q.restype = i
         L.lmk_attn_fwd_rotary_q.argtypes = [T4, T4, T4, T4, vp, vp, vp, vp, i64, i64, vp, i64, i, i, i, i, i, f, i, i, i, vp]
+        L.lmk_rotate_qk.restype = i
+        L.lmk_rotate_qk.argtypes = [T4, T4, T4, T4, vp, vp, i64, i64, vp, i64, i, i, i, i, i, i, vp]
         L.lmk_apply_rotary_qk.restype = i
         L.lmk_apply_rotary_qk.argtypes = [T4, T4, T4, T4, vp, vp, i64, i64, vp, i64, i, i, i, i, i, vp]
         _lib = L

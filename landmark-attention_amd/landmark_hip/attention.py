@@ -64,68 +64,24 @@ def _repack(x, block_size, block, unpad=False, rows=None):
 
 def _launch_fwd_blocks(q, k, v, n_prefix, sm_scale, block_tokens):
     """Forward for any block size 2..128 on the tensors as they are; L, M are indexed by token rows."""
-    B, H, Lq, D = q.shape
-    Lk = k.shape[2]
-    o = torch.empty_like(q)
-    L = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-    M = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-    rc = _lib.lib().lmk_attn_fwd_blocks(_lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o),
-                                        L.data_ptr(), M.data_ptr(), B, H, Lq, Lk, D, float(sm_scale), int(block_tokens),
-                                        int(n_prefix), _lib.DTYPE_CODES[q.dtype], _lib.current_stream(q.device))
-    _lib.check(rc)
-    return o, L, M
+    return _lib.native().attn_fwd(q, k, v, None, n_prefix, sm_scale, block_tokens, block_tokens, True)
 
 
 def _launch_bwd_blocks(q, k, v, o, do, L, M, n_prefix, sm_scale, block_tokens):
-    B, H, Lq, D = q.shape
-    Lk = k.shape[2]
-    lib = _lib.lib()
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    nbytes = lib.lmk_attn_bwd_blocks_workspace_bytes(B, H, Lq, Lk, int(block_tokens))
-    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-    rc = lib.lmk_attn_bwd_blocks(_lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o), _lib.tensor4(do),
-                                 L.data_ptr(), M.data_ptr(), _lib.tensor4(dq), _lib.tensor4(dk), _lib.tensor4(dv),
-                                 ws.data_ptr(), nbytes, B, H, Lq, Lk, D, float(sm_scale), int(block_tokens),
-                                 int(n_prefix), _lib.DTYPE_CODES[q.dtype], _lib.current_stream(q.device))
-    _lib.check(rc)
-    return dq, dk, dv
+    return _lib.native().attn_bwd(q, k, v, o, do, L, M, None, n_prefix, sm_scale, block_tokens, block_tokens, True,
+                                  HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
 
 
 def _launch_fwd(q, k, v, n_prefix, sm_scale, block, block_real=None):
-    block_real = block if block_real is None else block_real
-    B, H, Lq, D = q.shape
-    Lk = k.shape[2]
-    o = torch.empty_like(q)        # keeps q's memory layout: a (B,L,H,D)-backed q gives an output whose
-    #                                transpose(1, 2).reshape(B, L, H*D) for o_proj (llama_mem.py:484-486) is a view
-    L = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-    M = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-    rc = _lib.lib().lmk_attn_fwd_padded(_lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o),
-                                        L.data_ptr(), M.data_ptr(), B, H, Lq, Lk, D, float(sm_scale), int(block),
-                                        int(block_real), int(n_prefix), _lib.DTYPE_CODES[q.dtype],
-                                        _lib.current_stream(q.device))
-    _lib.check(rc)
-    return o, L, M
+    """o keeps q's memory layout: a (B,L,H,D)-backed q gives an output whose transpose(1, 2).reshape(B, L, H*D) for
+    o_proj (llama_mem.py:484-486) is a view."""
+    return _lib.native().attn_fwd(q, k, v, None, n_prefix, sm_scale, block, block if block_real is None else block_real,
+                                  False)
 
 
 def _launch_bwd(q, k, v, o, do, L, M, n_prefix, sm_scale, block, block_real=None):
-    block_real = block if block_real is None else block_real
-    B, H, Lq, D = q.shape
-    Lk = k.shape[2]
-    lib = _lib.lib()
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)     # each in its input's layout
-    nbytes = lib.lmk_attn_bwd_workspace_bytes(B, H, Lq, Lk, int(block))
-    if block_real == block:
-        ho = lib.lmk_attn_bwd_handover_workspace_bytes(B, H, Lq, Lk, int(block))
-        if 0 < ho <= HANDOVER_MAX_BYTES and Lk >= HANDOVER_MIN_KEYS:
-            nbytes = ho          # the library picks the hand-over kernels from the size it is handed
-    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-    rc = lib.lmk_attn_bwd_padded(_lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o),
-                                 _lib.tensor4(do), L.data_ptr(), M.data_ptr(), _lib.tensor4(dq), _lib.tensor4(dk),
-                                 _lib.tensor4(dv), ws.data_ptr(), nbytes, B, H, Lq, Lk, D, float(sm_scale),
-                                 int(block), int(block_real), int(n_prefix), _lib.DTYPE_CODES[q.dtype],
-                                 _lib.current_stream(q.device))
-    _lib.check(rc)
-    return dq, dk, dv
+    return _lib.native().attn_bwd(q, k, v, o, do, L, M, None, n_prefix, sm_scale, block,
+                                  block if block_real is None else block_real, False, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
 
 
 class FusedLandmarkAttention(torch.autograd.Function):
@@ -150,13 +106,10 @@ class FusedLandmarkAttention(torch.autograd.Function):
         ctx.N_PREFIX_Q = n_prefix_q
         ctx.BLOCK = block_size
         ctx.real_rows = (seqlen_q, seqlen_k)
-        with _lib.on_device(q.device):
-            if block == block_size:
-                o, L, m = _launch_fwd(q, k, v, n_prefix_q, sm_scale, block_size)
-            else:
-                o, L, m = _launch_fwd_blocks(q, k, v, n_prefix_q, sm_scale, block_size)
-            ctx.save_for_backward(q, k, v, o, L, m)
-            return o
+        launch = _launch_fwd if block == block_size else _launch_fwd_blocks
+        o, L, m = launch(q, k, v, n_prefix_q, sm_scale, block_size)
+        ctx.save_for_backward(q, k, v, o, L, m)
+        return o
 
     @staticmethod
     def backward(ctx, do):
@@ -167,11 +120,8 @@ class FusedLandmarkAttention(torch.autograd.Function):
         assert rows_k % BLOCK == 0, "Backward supported only for full blocks"
         block = storage_block(BLOCK)
         do = _lib.kernel_ready(do)
-        with _lib.on_device(q.device):
-            if block == BLOCK:
-                dq, dk, dv = _launch_bwd(q, k, v, o, do, l, m, ctx.N_PREFIX_Q, ctx.sm_scale, BLOCK)
-            else:
-                dq, dk, dv = _launch_bwd_blocks(q, k, v, o, do, l, m, ctx.N_PREFIX_Q, ctx.sm_scale, BLOCK)
+        launch = _launch_bwd if block == BLOCK else _launch_bwd_blocks
+        dq, dk, dv = launch(q, k, v, o, do, l, m, ctx.N_PREFIX_Q, ctx.sm_scale, BLOCK)
         return dq, dk, dv, None, None, None
 
 
@@ -191,15 +141,7 @@ class FusedLandmarkAttentionGroupScale(torch.autograd.Function):
         assert group_scale.device == q.device
         q, k, v = _lib.kernel_ready(q), _lib.kernel_ready(k), _lib.kernel_ready(v)
         group_scale = group_scale.contiguous()
-        o = torch.empty_like(q)
-        L = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-        M = torch.empty((B * H, Lq), device=q.device, dtype=torch.float32)
-        with _lib.on_device(q.device):
-            rc = _lib.lib().lmk_attn_fwd_group_scale(
-                _lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o), L.data_ptr(), M.data_ptr(),
-                group_scale.data_ptr(), B, H, Lq, Lk, D, float(sm_scale), int(block_size), int(n_prefix_q),
-                _lib.DTYPE_CODES[q.dtype], _lib.current_stream(q.device))
-        _lib.check(rc)
+        o, L, M = _lib.native().attn_fwd(q, k, v, group_scale, n_prefix_q, sm_scale, block_size, block_size, True)
         ctx.save_for_backward(q, k, v, o, L, M, group_scale)
         ctx.args = (n_prefix_q, sm_scale, block_size)
         return o
@@ -211,18 +153,8 @@ class FusedLandmarkAttentionGroupScale(torch.autograd.Function):
         B, H, Lq, D = q.shape
         Lk = k.shape[2]
         assert Lq % block_size == 0 and Lk % block_size == 0, "Backward supported only for full blocks"
-        do = _lib.kernel_ready(do)
-        lib = _lib.lib()
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        nbytes = lib.lmk_attn_bwd_group_scale_workspace_bytes(B, H, Lq, Lk, int(block_size))
-        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-        with _lib.on_device(q.device):
-            rc = lib.lmk_attn_bwd_group_scale(
-                _lib.tensor4(q), _lib.tensor4(k), _lib.tensor4(v), _lib.tensor4(o), _lib.tensor4(do), L.data_ptr(),
-                M.data_ptr(), group_scale.data_ptr(), _lib.tensor4(dq), _lib.tensor4(dk), _lib.tensor4(dv), ws.data_ptr(),
-                nbytes, B, H, Lq, Lk, D, float(sm_scale), int(block_size), int(n_prefix_q), _lib.DTYPE_CODES[q.dtype],
-                _lib.current_stream(q.device))
-        _lib.check(rc)
+        dq, dk, dv = _lib.native().attn_bwd(q, k, v, o, _lib.kernel_ready(do), L, M, group_scale, n_prefix_q, sm_scale,
+                                            block_size, block_size, True, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
         return dq, dk, dv, None, None, None, None
 
 
@@ -369,25 +301,17 @@ def fused_landmark_attention(q, k, v, is_mem, sm_scale=None, block_size=64, grou
                 sm_scale = 1.0 / math.sqrt(q.size(-1))
             return FusedLandmarkAttentionSegments.apply(q, k, v, segments, sm_scale)
 
-    n_history_kv = k.shape[-2] - q.shape[-2]
-    assert n_history_kv % block_size == 0
-    n_history_blocks = n_history_kv // block_size
-
-    if sm_scale is None:
-        sm_scale = 1.0 / math.sqrt(q.size(-1))
-
-    if group_scale is not None:
-        return FusedLandmarkAttentionGroupScale.apply(q, k, v, group_scale, n_history_blocks, sm_scale, block_size)
-
     d = q.size(-1)
-    if d in PADDED_HEAD_DIMS:
+    if d in PADDED_HEAD_DIMS and group_scale is None:
         # head dims 16 and 32 (flash_landmark_attention.py:321) run on the 64-wide kernels: zero columns add
         # nothing to a score and give zero output columns, which are dropped again; autograd differentiates
         # through the padding and the slice
-        pad = (0, 64 - d)
-        q, k, v = (torch.nn.functional.pad(t, pad) for t in (q, k, v))
-        return FusedLandmarkAttention.apply(q, k, v, n_history_blocks, sm_scale, block_size)[..., :d]
-    return FusedLandmarkAttention.apply(q, k, v, n_history_blocks, sm_scale, block_size)
+        q, k, v = (torch.nn.functional.pad(t, (0, 64 - d)) for t in (q, k, v))
+        return fused_landmark_attention(q, k, v, None, 1.0 / math.sqrt(d) if sm_scale is None else sm_scale, block_size)[..., :d]
+    if group_scale is None:
+        storage_block(block_size)               # ValueError for block sizes the kernels do not cover
+    # the same as FusedLandmarkAttention(GroupScale).apply, with a backward node that needs no interpreter
+    return _lib.native().attention(q, k, v, group_scale, sm_scale, block_size, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
 
 
 def fused_landmark_attention_rotary_q(q, k, v, cos, sin, position_ids, is_mem=None, sm_scale=None, block_size=64):
