@@ -316,6 +316,22 @@ int lmk_retrieve_and_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, con
                             int reuse_landmark_keys, void* attend_workspace, size_t attend_workspace_bytes, int B,
                             int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream);
 
+/* New rows into a cache: k and v (B,H,T,D; D a multiple of 8) are copied to k_dst and v_dst, whose ptr is where row 0
+ * of batch 0, head 0 goes -- the torch.cat of llama_mem.py:424-425 into buffers with room to spare, in one launch. */
+int lmk_cache_append(const lmk_tensor4* k, const lmk_tensor4* v, const lmk_tensor4* k_dst, const lmk_tensor4* v_dst, int B,
+                     int H, int T, int D, void* stream);
+
+/* lmk_retrieve_and_attend followed by lmk_cache_append of (k_append, v_loc) -- llama_mem.py:318-430 as one call.
+ * k_append: the new keys without rotary.  The destination rows must lie outside the S cached rows.  In decoding the
+ * rows are stored by the gather launch itself. */
+int lmk_retrieve_attend_append(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
+                               const lmk_tensor4* k_loc, const lmk_tensor4* v_loc, const lmk_tensor4* k_append,
+                               const lmk_tensor4* k_dst, const lmk_tensor4* v_dst, const void* cos_table,
+                               const void* sin_table, int64_t table_stride_row, int64_t n_pos, int64_t* idx_out,
+                               const lmk_tensor4* out, void* retrieve_workspace, size_t retrieve_workspace_bytes,
+                               int reuse_landmark_keys, void* attend_workspace, size_t attend_workspace_bytes, int B,
+                               int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream);
+
 /* ---- ring cache of blocks (lm_benchmark) -----------------------------------------------
  * Block selection of MemLMCacheStorage.retrieve_for_query
  * (lm_benchmark/models/caches/mem_cache.py:50-85): the cache is a ring buffer of `n_blocks`
@@ -458,6 +474,19 @@ int lmk_rotate_qk(const lmk_tensor4* x, const lmk_tensor4* out, const lmk_tensor
                   const void* cos_table, const void* sin_table, int64_t table_stride_row, int64_t n_pos,
                   const int64_t* position_ids, int64_t pos_stride_b, int B, int H, int L, int D, int dtype,
                   int transposed, void* stream);
+
+/* MemLMCacheStorage.store_in_cache (lm_benchmark/models/caches/mem_cache.py:111-158) in one launch: the `tail` tokens
+ * waiting in tail_k, tail_v (B,H,block,D) and the T new ones (k, v: (B,H,T,D), keys without positions) are laid out
+ * block by block into the ring -- slot ring_next first, wrapping at n_slots; with more complete blocks than slots the
+ * newest n_slots are kept -- and what is left of the last block becomes the new tail, with its marks out of is_mem
+ * (bool, row stride is_mem_stride_b, unit stride) in tail_is_mem.
+ * ring_k, ring_v: (B, n_slots, block, H, D) with element strides ring_stride_{b,slot,token,head}, unit along D.
+ * D a multiple of 8; the counters (next slot, blocks stored, new tail) are the caller's. */
+int lmk_ring_store(const lmk_tensor4* k, const lmk_tensor4* v, const void* is_mem, int64_t is_mem_stride_b,
+                   const lmk_tensor4* tail_k, const lmk_tensor4* tail_v, void* tail_is_mem, int64_t tail_is_mem_stride_b,
+                   void* ring_k, void* ring_v, int64_t ring_stride_b, int64_t ring_stride_slot, int64_t ring_stride_token,
+                   int64_t ring_stride_head, int B, int H, int T, int D, int block, int n_slots, int tail, int ring_next,
+                   void* stream);
 
 #ifdef __cplusplus
 }

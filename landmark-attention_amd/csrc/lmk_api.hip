@@ -676,6 +676,31 @@ int lmk_retrieve_topk_static(const lmk_tensor4* q, const lmk_tensor4* kcache, co
                             LMK_STATIC_SCRATCH_BYTES, B, H, T, S, D, block, top_k, dtype, stream);
 }
 
+// New tokens' rows on their way into a cache: keys without rotary and values (B,H,T,D), and where their first row goes.
+struct AppendArgs {
+  const lmk_tensor4 *k, *v, *k_dst, *v_dst;
+};
+
+static int check_append(const AppendArgs& a, int D) {
+  int rc;
+  if ((rc = check_tensor(a.k)) || (rc = check_tensor(a.v)) || (rc = check_tensor(a.k_dst)) || (rc = check_tensor(a.v_dst))) return rc;
+  return D > 0 && D % 8 == 0 ? LMK_OK : LMK_ERR_UNSUPPORTED;
+}
+
+int lmk_cache_append(const lmk_tensor4* k, const lmk_tensor4* v, const lmk_tensor4* k_dst, const lmk_tensor4* v_dst, int B,
+                     int H, int T, int D, void* stream) {
+  const AppendArgs a = {k, v, k_dst, v_dst};
+  if (int rc = check_append(a, D)) return rc;
+  if (B <= 0 || H <= 0 || T <= 0) return LMK_ERR_SHAPE;
+  lmk::CopyRowsParams p = {};
+  p.src[0] = k->ptr; p.ss_b[0] = k->stride_b; p.ss_h[0] = k->stride_h; p.ss_r[0] = k->stride_row;
+  p.src[1] = v->ptr; p.ss_b[1] = v->stride_b; p.ss_h[1] = v->stride_h; p.ss_r[1] = v->stride_row;
+  p.dst[0] = k_dst->ptr; p.ds_b[0] = k_dst->stride_b; p.ds_h[0] = k_dst->stride_h; p.ds_r[0] = k_dst->stride_row;
+  p.dst[1] = v_dst->ptr; p.ds_b[1] = v_dst->stride_b; p.ds_h[1] = v_dst->stride_h; p.ds_r[1] = v_dst->stride_row;
+  p.B = B; p.H = H; p.T = T; p.chunks = D / 8;
+  return lmk::launch_copy_rows(p, (hipStream_t)stream);
+}
+
 // `candidates`: the selection has stopped after its slice step (lmk::launch_fwd32_topk_slices) and the gather picks
 // a row's k best from what that step left, writing them to idx on the way; else idx holds the indices already.
 static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache, const int64_t* idx,
@@ -683,7 +708,9 @@ static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, c
                               const lmk_tensor4* o_loc, const float* L_loc, const float* M_loc, int64_t stat_stride,
                               const lmk_tensor4* out, int B, int H, int T, int S, int D, float sm_scale, int block,
                               int top_k, int dtype, void* stream, const lmk::RetrParams* candidates,
-                              const lmk_tensor4* k_new = nullptr, const lmk_tensor4* v_new = nullptr) {
+                              const lmk_tensor4* k_new = nullptr, const lmk_tensor4* v_new = nullptr,
+                              const AppendArgs* append = nullptr) {
+  // append (with k_new): the new tokens' rows are stored in the cache by the same launch
   // k_new, v_new: the gather kernel attends to the rows' local window itself (gather_takes_local_window) and
   // o_loc, L_loc, M_loc are not read
   const bool local = k_new != nullptr;
@@ -712,6 +739,13 @@ static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, c
     p.local_pos0 = p.local_row0;
     p.k_new = k_new->ptr; p.kns_b = k_new->stride_b; p.kns_h = k_new->stride_h; p.kns_r = k_new->stride_row;
     p.v_new = v_new->ptr; p.vns_b = v_new->stride_b; p.vns_h = v_new->stride_h; p.vns_r = v_new->stride_row;
+    if (append != nullptr) {
+      const lmk_tensor4 *ak = append->k, *av = append->v, *dk = append->k_dst, *dv = append->v_dst;
+      p.ap_k = ak->ptr; p.aks_b = ak->stride_b; p.aks_h = ak->stride_h; p.aks_r = ak->stride_row;
+      p.ap_v = av->ptr; p.avs_b = av->stride_b; p.avs_h = av->stride_h; p.avs_r = av->stride_row;
+      p.ap_kd = dk->ptr; p.akd_b = dk->stride_b; p.akd_h = dk->stride_h; p.akd_r = dk->stride_row;
+      p.ap_vd = dv->ptr; p.avd_b = dv->stride_b; p.avd_h = dv->stride_h; p.avd_r = dv->stride_row;
+    }
   } else {
     p.o_loc = o_loc->ptr; p.L_loc = L_loc; p.M_loc = M_loc; p.stat_stride = stat_stride;
     p.ols_b = o_loc->stride_b; p.ols_h = o_loc->stride_h; p.ols_r = o_loc->stride_row;
@@ -874,6 +908,38 @@ int lmk_ring_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kring, const
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   const int slots = block == 32 ? 32 : (block <= 64 ? 64 : 128);
   return lmk::launch_gather_attend(p, D, slots, dtype, (hipStream_t)stream);
+}
+
+int lmk_ring_store(const lmk_tensor4* k, const lmk_tensor4* v, const void* is_mem, int64_t is_mem_stride_b,
+                   const lmk_tensor4* tail_k, const lmk_tensor4* tail_v, void* tail_is_mem, int64_t tail_is_mem_stride_b,
+                   void* ring_k, void* ring_v, int64_t ring_stride_b, int64_t ring_stride_slot, int64_t ring_stride_token,
+                   int64_t ring_stride_head, int B, int H, int T, int D, int block, int n_slots, int tail, int ring_next,
+                   void* stream) {
+  int rc;
+  if ((rc = check_tensor(k)) || (rc = check_tensor(v)) || (rc = check_tensor(tail_k)) || (rc = check_tensor(tail_v))) return rc;
+  if (is_mem == nullptr || tail_is_mem == nullptr || ring_k == nullptr || ring_v == nullptr) return LMK_ERR_NULL;
+  if (!aligned16(ring_k) || !aligned16(ring_v) || !stride_ok(ring_stride_b) || !stride_ok(ring_stride_slot) ||
+      !stride_ok(ring_stride_token) || !stride_ok(ring_stride_head))
+    return LMK_ERR_ALIGN;
+  if (B <= 0 || H <= 0 || T <= 0 || n_slots <= 0 || block < 2 || tail < 0 || tail >= block) return LMK_ERR_SHAPE;
+  if (ring_next < 0 || ring_next >= n_slots || (int64_t)tail + T >= ((int64_t)1 << 31)) return LMK_ERR_SHAPE;
+  if (D <= 0 || D % 8 != 0) return LMK_ERR_UNSUPPORTED;
+  lmk::RingStoreParams p = {};
+  const lmk_tensor4 *src[2] = {k, v}, *tl[2] = {tail_k, tail_v};
+  for (int w = 0; w < 2; ++w) {
+    p.src[w] = src[w]->ptr; p.ss_b[w] = src[w]->stride_b; p.ss_h[w] = src[w]->stride_h; p.ss_r[w] = src[w]->stride_row;
+    p.tail[w] = tl[w]->ptr; p.ts_b[w] = tl[w]->stride_b; p.ts_h[w] = tl[w]->stride_h; p.ts_r[w] = tl[w]->stride_row;
+  }
+  p.ring[0] = ring_k; p.ring[1] = ring_v;
+  p.rs_b = ring_stride_b; p.rs_slot = ring_stride_slot; p.rs_tok = ring_stride_token; p.rs_h = ring_stride_head;
+  p.is_mem = static_cast<const unsigned char*>(is_mem); p.ims_b = is_mem_stride_b;
+  p.tail_is_mem = static_cast<unsigned char*>(tail_is_mem); p.tims_b = tail_is_mem_stride_b;
+  p.B = B; p.H = H; p.T = T; p.chunks = D / 8; p.block = block; p.n_slots = n_slots; p.n_tail = tail;
+  const int n_new = (tail + T) / block;
+  p.full = n_new * block;
+  p.dropped = n_new > n_slots ? n_new - n_slots : 0;             // the newest blocks win (mem_cache.py:134-143)
+  p.first_slot = (int)(((int64_t)ring_next + p.dropped) % n_slots);
+  return lmk::launch_ring_store(p, (hipStream_t)stream);
 }
 
 int lmk_local_window(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
@@ -1071,12 +1137,19 @@ int lmk_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor
                            M + inc, W, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream);
 }
 
-int lmk_retrieve_and_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
+static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
                             const lmk_tensor4* k_loc, const lmk_tensor4* v_loc, const void* cos_table,
                             const void* sin_table, int64_t table_stride_row, int64_t n_pos, int64_t* idx_out,
                             const lmk_tensor4* out, void* retrieve_workspace, size_t retrieve_workspace_bytes,
                             int reuse_landmark_keys, void* attend_workspace, size_t attend_workspace_bytes, int B,
-                            int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream) {
+                            int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream,
+                            const AppendArgs* append) {
+  if (append != nullptr) {
+    if (int rc = check_append(*append, D)) return rc;
+  }
+  auto append_rows = [&]() {                              // behind everything that reads the cache
+    return append == nullptr ? LMK_OK : lmk_cache_append(append->k, append->v, append->k_dst, append->v_dst, B, H, T, D, stream);
+  };
   // everything the attend step would reject is rejected here, before the selection is enqueued
   if (int rc = attend_precheck(q, kcache, vcache, idx_out, k_loc, v_loc, cos_table, sin_table, table_stride_row, n_pos,
                                out, attend_workspace, B, H, T, S, D, sm_scale, block, top_k, dtype, true))
@@ -1097,11 +1170,11 @@ int lmk_retrieve_and_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, con
       if (!reuse_landmark_keys && (rc = lmk::launch_landmark_keys(pr, D, dtype, (hipStream_t)stream))) return rc;
       if ((rc = lmk::launch_topk_slices(pr, D, dtype, (hipStream_t)stream))) return rc;
       return gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, nullptr, nullptr,
-                                nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, &pr, k_loc, v_loc);
+                                nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, &pr, k_loc, v_loc, append);
     }
     if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, reuse_landmark_keys != 0, (hipStream_t)stream))) return rc;
     return gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, nullptr, nullptr,
-                              nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr, k_loc, v_loc);
+                              nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr, k_loc, v_loc, append);
   }
   if (block == 32) {
     // The forward over the local window needs nothing from the selection and alone fills a fraction of the chip, so
@@ -1145,16 +1218,44 @@ int lmk_retrieve_and_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, con
       if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, true, (hipStream_t)stream))) return rc;   // keys are rotated already
     }
     const lmk_tensor4 o_loc = {w + l.o_win + (size_t)inc * D * 2, o_win.stride_b, o_win.stride_h, o_win.stride_row};
-    return gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc,
-                              M + inc, W, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream,
-                              by_slices ? &pr : nullptr);
+    if ((rc = gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc,
+                                 M + inc, W, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream,
+                                 by_slices ? &pr : nullptr)))
+      return rc;
+    return append_rows();
   }
   if (int rc = retrieve_topk_impl(reuse_landmark_keys != 0, q, kcache, cos_table, sin_table, table_stride_row, n_pos,
                                   idx_out, retrieve_workspace, retrieve_workspace_bytes, B, H, T, S, D, block, top_k,
                                   dtype, stream))
     return rc;
-  return lmk_attend(q, kcache, vcache, idx_out, k_loc, v_loc, cos_table, sin_table, table_stride_row, n_pos, out,
-                    attend_workspace, attend_workspace_bytes, B, H, T, S, D, sm_scale, block, top_k, dtype, stream);
+  if (int rc = lmk_attend(q, kcache, vcache, idx_out, k_loc, v_loc, cos_table, sin_table, table_stride_row, n_pos, out,
+                          attend_workspace, attend_workspace_bytes, B, H, T, S, D, sm_scale, block, top_k, dtype, stream))
+    return rc;
+  return append_rows();
+}
+
+int lmk_retrieve_and_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
+                            const lmk_tensor4* k_loc, const lmk_tensor4* v_loc, const void* cos_table,
+                            const void* sin_table, int64_t table_stride_row, int64_t n_pos, int64_t* idx_out,
+                            const lmk_tensor4* out, void* retrieve_workspace, size_t retrieve_workspace_bytes,
+                            int reuse_landmark_keys, void* attend_workspace, size_t attend_workspace_bytes, int B,
+                            int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream) {
+  return retrieve_and_attend_impl(q, kcache, vcache, k_loc, v_loc, cos_table, sin_table, table_stride_row, n_pos, idx_out, out,
+                                  retrieve_workspace, retrieve_workspace_bytes, reuse_landmark_keys, attend_workspace,
+                                  attend_workspace_bytes, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr);
+}
+
+int lmk_retrieve_attend_append(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
+                               const lmk_tensor4* k_loc, const lmk_tensor4* v_loc, const lmk_tensor4* k_append,
+                               const lmk_tensor4* k_dst, const lmk_tensor4* v_dst, const void* cos_table,
+                               const void* sin_table, int64_t table_stride_row, int64_t n_pos, int64_t* idx_out,
+                               const lmk_tensor4* out, void* retrieve_workspace, size_t retrieve_workspace_bytes,
+                               int reuse_landmark_keys, void* attend_workspace, size_t attend_workspace_bytes, int B,
+                               int H, int T, int S, int D, float sm_scale, int block, int top_k, int dtype, void* stream) {
+  const AppendArgs append = {k_append, v_loc, k_dst, v_dst};
+  return retrieve_and_attend_impl(q, kcache, vcache, k_loc, v_loc, cos_table, sin_table, table_stride_row, n_pos, idx_out, out,
+                                  retrieve_workspace, retrieve_workspace_bytes, reuse_landmark_keys, attend_workspace,
+                                  attend_workspace_bytes, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, &append);
 }
 
 }  // extern "C"

@@ -145,6 +145,10 @@ struct RetrParams {
   int local, local_inc;
   const void *k_new, *v_new;
   int64_t kns_b, kns_h, kns_r, vns_b, vns_h, vns_r, local_row0, local_pos0;
+  // with `local`, optional: the new tokens' rows (keys without rotary, values) are stored in the cache on the way
+  const void *ap_k, *ap_v;
+  void *ap_kd, *ap_vd;
+  int64_t aks_b, aks_h, aks_r, avs_b, avs_h, avs_r, akd_b, akd_h, akd_r, avd_b, avd_h, avd_r;
   int64_t qs_b, qs_h, qs_r, kcs_b, kcs_h, kcs_r, vcs_b, vcs_h, vcs_r, cs_r;
   int64_t ols_b, ols_h, ols_r, outs_b, outs_h, outs_r;
   float sqrt_hd, scale_log2;
@@ -190,6 +194,27 @@ struct PadParams {
 int launch_pad_blocks(const PadParams& p, int D, bool unpad, hipStream_t stream);
 
 int launch_rotary(const RotaryParams& p, int D, int dtype, hipStream_t stream);
+
+// copies (B, H, T) rows of `chunks` 16-byte chunks, of two tensors at once
+struct CopyRowsParams {
+  const void* src[2];
+  void* dst[2];
+  int B, H, T, chunks;
+  int64_t ss_b[2], ss_h[2], ss_r[2], ds_b[2], ds_h[2], ds_r[2];   // element strides (16-bit elements)
+};
+int launch_copy_rows(const CopyRowsParams& p, hipStream_t stream);
+
+// a chunk into the ring cache: see lmk_ring_store.  [0] keys, [1] values.
+struct RingStoreParams {
+  const void* src[2];
+  void *tail[2], *ring[2];
+  const unsigned char* is_mem;
+  unsigned char* tail_is_mem;
+  int B, H, T, chunks, block, n_slots, n_tail;
+  int full, dropped, first_slot;                  // rows of complete blocks, blocks not kept, slot of the first kept one
+  int64_t ss_b[2], ss_h[2], ss_r[2], ts_b[2], ts_h[2], ts_r[2], rs_b, rs_slot, rs_tok, rs_h, ims_b, tims_b;
+};
+int launch_ring_store(const RingStoreParams& p, hipStream_t stream);
 
 // Selection by slices, for a handful of query rows (decoding): a row's cached blocks are split into slices of 256
 // over as many workgroups of four waves, and a row's slices are merged afterwards.

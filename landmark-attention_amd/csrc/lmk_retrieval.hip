@@ -759,6 +759,15 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
     unpack8(*(const vec_t*)(qp + PB * j), qlo);
     unpack8(*(const vec_t*)(qp + D + PB * j), qhi);
   }
+  // The row's own key (without rotary) and value on their way into the cache: fetched here by one of the row's waves
+  // (lanes 0 .. D/8-1 the key, 32 .. the value), stored at the end, so that nothing waits for them.  Nobody reads the
+  // destination in this launch: it lies behind the cached rows.
+  const bool appends = LOCAL && p.ap_k != nullptr && (!SPLIT || wave == NWV - 1) && (lane & 31) < D / 8;
+  u32x4_t ap = {0, 0, 0, 0};
+  if (LOCAL && appends)
+    ap = *(const u32x4_t*)((lane < 32 ? (const char*)p.ap_k + 2 * (b * p.aks_b + hh * p.aks_h + (int64_t)t * p.aks_r)
+                                      : (const char*)p.ap_v + 2 * (b * p.avs_b + hh * p.avs_h + (int64_t)t * p.avs_r)) +
+                           16 * (lane & 31));
   const char* kc = (const char*)p.kcache + 2 * (b * p.kcs_b + hh * p.kcs_h);
   const char* vc = (const char*)p.vcache + 2 * (b * p.vcs_b + hh * p.vcs_h);
   const float c2 = p.scale_log2;
@@ -980,6 +989,10 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
     }
     blk = blk_next;
   }
+  if (LOCAL && appends)
+    *(u32x4_t*)((lane < 32 ? (char*)p.ap_kd + 2 * (b * p.akd_b + hh * p.akd_h + (int64_t)t * p.akd_r)
+                           : (char*)p.ap_vd + 2 * (b * p.avd_b + hh * p.avd_h + (int64_t)t * p.avd_r)) +
+                16 * (lane & 31)) = ap;
 #pragma unroll
   for (int e = 0; e < E; ++e) {                                   // sum over the eight key groups
     alo[e] += dpp_f<0x128>(alo[e]);
@@ -1368,6 +1381,68 @@ static int launch_rotary_t(const RotaryParams& p, hipStream_t stream) {
   const dim3 grid((unsigned)((rows + RPW - 1) / RPW));
   if (p.x2 != nullptr) hipLaunchKernelGGL((lmk_rotary_kernel<T, D, true>), grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL((lmk_rotary_kernel<T, D, false>), grid, dim3(256), 0, stream, p);
+  return (int)hipGetLastError();
+}
+
+// New rows of a cache's keys (blockIdx.y 0) and values (1), one 16-byte chunk per thread.
+__global__ __launch_bounds__(256) void lmk_copy_rows_kernel(CopyRowsParams p) {
+  const int w = blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / p.chunks;
+  const int c = (int)(i % p.chunks);
+  if (row >= (int64_t)p.B * p.H * p.T) return;
+  const int t = (int)(row % p.T), bh = (int)(row / p.T), b = bh / p.H, h = bh % p.H;
+  const char* s = (const char*)p.src[w] + 2 * (b * p.ss_b[w] + h * p.ss_h[w] + t * p.ss_r[w]) + 16 * c;
+  char* d = (char*)p.dst[w] + 2 * (b * p.ds_b[w] + h * p.ds_h[w] + t * p.ds_r[w]) + 16 * c;
+  *(u32x4_t*)d = *(const u32x4_t*)s;
+}
+
+// One 16-byte chunk per thread of the rows [tail ; new tokens] of keys (blockIdx.y 0) and values (1); blockIdx.y 2: the
+// new tail's marks, a byte per thread.  A tail row is read and overwritten in the same launch, so its thread does both:
+// row i < n_tail goes to the ring and then, if the new tail has a row i, fetches that row too.
+__global__ __launch_bounds__(256) void lmk_ring_store_kernel(RingStoreParams p) {
+  const int w = blockIdx.y, rows = p.n_tail + p.T, rest = rows - p.full;
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (w == 2) {
+    const int j = (int)(n % p.block);
+    const int64_t b = n / p.block;
+    const int src = p.full + j - p.n_tail;                        // token of the chunk behind row j of the tail; < 0: row j stays
+    if (b < p.B && j < rest && src >= 0) p.tail_is_mem[b * p.tims_b + j] = p.is_mem[b * p.ims_b + src];
+    return;
+  }
+  const int c = (int)(n % p.chunks);
+  const int64_t bhi = n / p.chunks;
+  const int i = (int)(bhi % rows);
+  const int64_t bh = bhi / rows;
+  if (bh >= (int64_t)p.B * p.H) return;
+  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+  const char* src = (const char*)p.src[w] + 2 * (b * p.ss_b[w] + h * p.ss_h[w]) + 16 * c;
+  char* tail = (char*)p.tail[w] + 2 * (b * p.ts_b[w] + h * p.ts_h[w]) + 16 * c;
+  auto chunk_row = [&](int t) { return *(const u32x4_t*)(src + 2 * t * p.ss_r[w]); };
+  auto tail_row = [&](int j) { return (u32x4_t*)(tail + 2 * j * p.ts_r[w]); };
+  if (i < p.full) {
+    const u32x4_t x = i < p.n_tail ? *tail_row(i) : chunk_row(i - p.n_tail);
+    const int blk = i / p.block - p.dropped;
+    if (blk >= 0) {
+      const int slot = (p.first_slot + blk) % p.n_slots;
+      *(u32x4_t*)((char*)p.ring[w] + 2 * (b * p.rs_b + slot * p.rs_slot + (i % p.block) * p.rs_tok + h * p.rs_h) + 16 * c) = x;
+    }
+    if (i < p.n_tail && i < rest) *tail_row(i) = chunk_row(p.full + i - p.n_tail);   // full > n_tail: a token of the chunk
+  } else {
+    const int j = i - p.full;                                     // row of the new tail
+    if (p.full > 0 ? j >= p.n_tail : i >= p.n_tail) *tail_row(j) = chunk_row(i - p.n_tail);
+  }
+}
+
+int launch_ring_store(const RingStoreParams& p, hipStream_t stream) {
+  const int64_t n = (int64_t)p.B * p.H * (p.n_tail + p.T) * p.chunks, marks = (int64_t)p.B * p.block;
+  hipLaunchKernelGGL(lmk_ring_store_kernel, dim3((unsigned)((std::max(n, marks) + 255) / 256), 3), dim3(256), 0, stream, p);
+  return (int)hipGetLastError();
+}
+
+int launch_copy_rows(const CopyRowsParams& p, hipStream_t stream) {
+  const int64_t n = (int64_t)p.B * p.H * p.T * p.chunks;
+  hipLaunchKernelGGL(lmk_copy_rows_kernel, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, stream, p);
   return (int)hipGetLastError();
 }
 

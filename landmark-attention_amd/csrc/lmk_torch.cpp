@@ -22,8 +22,10 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
+#include <vector>
 
 #include "../../include/lmk.h"
 
@@ -345,6 +347,156 @@ std::pair<Tensor, Tensor> rotary(const Tensor& q, const Tensor& k, const Tensor&
   return r;
 }
 
+// ---- the mem-cache step
+// Where a cache's new rows go: the buffers and the row of the first new token.
+struct Append {
+  Tensor k_nopos, k_buf, v_buf;
+  int64_t row;
+};
+
+// One step of the mem-cache path over the first S rows of k_cache, v_cache (GPU memory, or pinned host memory for the
+// selection per head on `landmarks` alone): (out, idx), and the append.  `shared`: one selection per head.
+std::pair<Tensor, Tensor> mem_cache_step(const Tensor& q_in, const Tensor& kc_in, const Tensor& vc_in, int64_t S,
+                                         const Tensor& kl_in, const Tensor& vl_in, const Tensor& cos, const Tensor& sin,
+                                         int block, int top_k, bool has_scale, double scale, bool shared, Tensor ws, bool reuse,
+                                         const Append* append) {
+  need(q_in.dim() == 4 && kc_in.dim() == 4 && vc_in.dim() == 4 && kl_in.dim() == 4 && vl_in.dim() == 4,
+       "queries, cache and new keys and values are (batch, heads, rows, head dim)");
+  const int B = (int)q_in.size(0), H = (int)q_in.size(1), T = (int)q_in.size(2), D = (int)q_in.size(3);
+  need(kc_in.size(0) == B && kc_in.size(1) == H && kc_in.size(3) == D && same_shape(kc_in, vc_in) &&
+           q_in.scalar_type() == kc_in.scalar_type() && q_in.scalar_type() == vc_in.scalar_type() && q_in.is_cuda() &&
+           kc_in.is_cuda() && vc_in.is_cuda(),
+       "the cache must have the queries' batch, heads, head dim, type and device");
+  need(same_shape(kl_in, q_in) && same_shape(vl_in, q_in) && kl_in.scalar_type() == q_in.scalar_type() &&
+           vl_in.scalar_type() == q_in.scalar_type() && kl_in.is_cuda() && vl_in.is_cuda(),
+       "the new keys and values must have the queries' shape, type and device");
+  const int dtype = dtype_code(q_in);
+  need(dtype >= 0, "HIP kernels are built for bf16 and fp16");
+  need(block > 0 && (S % block == 0 || T + S % block <= block), "new chunk and cached tail must fit one block (llama_mem.py:330)");
+  if (!has_scale) scale = 1.0 / std::sqrt((double)D);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  c10::DeviceGuard device(q_in.device());
+  const Tensor q = kernel_ready(q_in), kc = kernel_ready(kc_in), vc = kernel_ready(vc_in), kl = kernel_ready(kl_in),
+               vl = kernel_ready(vl_in);
+  const Tables t = tables(cos, sin, q.scalar_type());
+  const int64_t k = std::min<int64_t>(top_k, S / block), inc = S % block;
+  const size_t rbytes = lmk_retrieve_workspace_bytes(B, H, T, (int)S, D, block);
+  if (!ws.defined()) ws = bytes_on(q, rbytes);
+  need(ws.scalar_type() == at::kByte && ws.is_contiguous() && (size_t)ws.numel() >= rbytes && ws.device() == q.device(),
+       "workspace: contiguous uint8, at least lmk_retrieve_workspace_bytes long, on the queries' device");
+  Tensor idx = at::empty({B, H, shared ? 1 : T, std::max<int64_t>(k, 0)}, q.options().dtype(at::kLong));
+  const lmk_tensor4 tq = t4(q), tkc = t4(kc), tvc = t4(vc), tkl = t4(kl), tvl = t4(vl);
+  const void *pc = t.cos.data_ptr(), *ps = t.sin.data_ptr();
+  const int64_t cs = t.cos.stride(0), n_pos = t.cos.size(0);
+  void* stream = stream_of(q);
+
+  Tensor kn;
+  lmk_tensor4 tkn = {}, tkd = {}, tvd = {};
+  if (append != nullptr) {
+    need(append->k_nopos.dim() == 4 && same_shape(append->k_nopos, q_in) && append->k_nopos.scalar_type() == q.scalar_type() &&
+             append->k_nopos.is_cuda(),
+         "the keys to append must have the queries' shape, type and device");
+    need(append->row >= S && append->row + T <= append->k_buf.size(2), "no room for the new rows");
+    kn = kernel_ready(append->k_nopos);
+    tkn = t4(kn);
+    auto at_row = [&](const Tensor& buf) {
+      lmk_tensor4 d = t4(buf);
+      d.ptr = static_cast<char*>(d.ptr) + 2 * append->row * d.stride_row;
+      return d;
+    };
+    tkd = at_row(append->k_buf);
+    tvd = at_row(append->v_buf);
+  }
+
+  if (!shared) {
+    const size_t abytes = lmk_attend_workspace_bytes(B, H, T, (int)S, D, block);
+    Tensor aws = bytes_on(q, abytes), out = at::empty_like(q);
+    const lmk_tensor4 tout = t4(out);
+    if (append != nullptr)
+      check(lmk_retrieve_attend_append(&tq, &tkc, &tvc, &tkl, &tvl, &tkn, &tkd, &tvd, pc, ps, cs, n_pos, idx.data_ptr<int64_t>(),
+                                       &tout, ws.data_ptr(), rbytes, reuse ? 1 : 0, aws.data_ptr(), abytes, B, H, T, (int)S, D,
+                                       (float)scale, block, top_k, dtype, stream));
+    else
+      check(lmk_retrieve_and_attend(&tq, &tkc, &tvc, &tkl, &tvl, pc, ps, cs, n_pos, idx.data_ptr<int64_t>(), &tout, ws.data_ptr(),
+                                    rbytes, reuse ? 1 : 0, aws.data_ptr(), abytes, B, H, T, (int)S, D, (float)scale, block, top_k,
+                                    dtype, stream));
+    return {out, idx};
+  }
+  // one selection per head: the selected blocks, rotated, and the local window form one sequence for the fused forward
+  check(lmk_retrieve_topk_shared(&tq, &tkc, pc, ps, cs, n_pos, idx.data_ptr<int64_t>(), nullptr, ws.data_ptr(), rbytes, B, H, T,
+                                 (int)S, D, block, top_k, dtype, stream));
+  const int64_t rows = k * block + inc + T;
+  Tensor win = at::empty({2, B, H, rows, D}, q.options());
+  const Tensor k_win = win.select(0, 0), v_win = win.select(0, 1);
+  const Tensor q_win = inc ? at::empty({B, H, inc + T, D}, q.options()) : q;
+  const lmk_tensor4 tqw = t4(q_win), tkw = t4(k_win), tvw = t4(v_win);
+  check(lmk_gather_window(&tq, &tkc, &tvc, idx.data_ptr<int64_t>(), &tkl, &tvl, pc, ps, cs, n_pos, inc ? &tqw : nullptr, &tkw,
+                          &tvw, B, H, T, (int)S, D, block, top_k, dtype, stream));
+  Tensor o = forward(shape_of(q_win, k_win, (int)k, scale, block, block, false), q_win, k_win, v_win, Tensor()).first;
+  if (append != nullptr) check(lmk_cache_append(&tkn, &tvl, &tkd, &tvd, B, H, T, D, stream));
+  return {inc ? o.narrow(2, inc, T) : o, idx};
+}
+
+// ---- the ring cache (MemLMCacheStorage): buffers (B, slots, block, nh, hs), tail (B, nh, block, hs)
+struct Ring {
+  Tensor k, v, tail_k, tail_v;
+  int tail, filled, oldest, top_k, method;
+};
+
+// attention of a chunk over the ring and itself: (y, slots), slots undefined while the ring holds no block
+std::pair<Tensor, Tensor> ring_attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& cos,
+                                      const Tensor& sin, const Ring& r, int64_t start, bool has_scale, double scale) {
+  need(q_in.dim() == 4 && q_in.is_cuda() && q_in.scalar_type() == r.k.scalar_type() && same_shape(k_in, q_in) &&
+           same_shape(v_in, q_in) && k_in.scalar_type() == q_in.scalar_type() && v_in.scalar_type() == q_in.scalar_type() &&
+           k_in.is_cuda() && v_in.is_cuda(),
+       "q, k, v must have one shape, the cache's type, and be on the GPU");
+  const int B = (int)q_in.size(0), H = (int)q_in.size(1), T = (int)q_in.size(2), D = (int)q_in.size(3), block = (int)r.k.size(2);
+  need(B <= r.k.size(0) && H == r.k.size(3) && D == r.k.size(4), "the chunk must have the cache's heads and head dim");
+  need(start >= r.tail, "the tokens behind the last complete block need positions of their own");
+  if (!has_scale) scale = 1.0 / std::sqrt((double)D);
+  const int dtype = dtype_code(q_in);
+  need(dtype >= 0, "HIP kernels are built for bf16 and fp16");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  c10::DeviceGuard device(q_in.device());
+  const Tensor q = kernel_ready(q_in), k = kernel_ready(k_in), v = kernel_ready(v_in);
+  const Tables t = tables(cos, sin, q.scalar_type());
+  const lmk_tensor4 tq = t4(q), tk = t4(k), tv = t4(v);
+  const void *pc = t.cos.data_ptr(), *ps = t.sin.data_ptr();
+  const int64_t cs = t.cos.stride(0), n_pos = t.cos.size(0), W = r.tail + T;
+  void* stream = stream_of(q);
+  Tensor q_win = q, k_win = k, v_win = v, win;
+  if (r.tail > 0) {
+    // the tokens behind the last complete block open the chunk's first block, their keys rotated at start - tail ..,
+    // zero rows standing in for their queries
+    win = at::empty({3, B, H, W, D}, q.options());
+    q_win = win.select(0, 0);
+    k_win = win.select(0, 1);
+    v_win = win.select(0, 2);
+    const lmk_tensor4 tlk = t4(r.tail_k), tlv = t4(r.tail_v), a = t4(q_win), b = t4(k_win), c = t4(v_win);
+    check(lmk_ring_local_window(&tq, &tlk, &tlv, &tk, &tv, pc, ps, cs, n_pos, &a, &b, &c, B, H, T, r.tail, start - r.tail, D,
+                                dtype, stream));
+  }
+  auto fwd = forward(shape_of(q_win, k_win, 0, scale, block, block, true), q_win, k_win, v_win, Tensor());
+  const Tensor o_loc = r.tail > 0 ? fwd.first.narrow(2, r.tail, T) : fwd.first;
+  if (r.filled == 0 || r.top_k == 0) return {o_loc, Tensor()};
+  auto ring4 = [](const Tensor& x) { return lmk_tensor4{x.data_ptr(), x.stride(0), x.stride(3), x.stride(2)}; };
+  const lmk_tensor4 rk = ring4(r.k), rv = ring4(r.v), to = t4(o_loc);
+  std::vector<int64_t> shape = {B};
+  if (r.method != LMK_SELECT_MAX_OVER_HEADS) shape.push_back(H);
+  if (r.method != LMK_SELECT_MAX_OVER_TOKENS) shape.push_back(T);
+  shape.push_back(r.top_k);
+  Tensor slots = at::empty(shape, q.options().dtype(at::kLong));
+  const size_t nbytes = lmk_retrieve_workspace_bytes(B, H, T, r.filled * block, D, block);
+  Tensor ws = bytes_on(q, nbytes), out = at::empty_like(q);
+  check(lmk_ring_retrieve_topk(&tq, &rk, pc, ps, cs, n_pos, slots.data_ptr<int64_t>(), ws.data_ptr(), nbytes, B, H, T, r.filled, D,
+                               block, r.top_k, r.oldest, r.method, dtype, stream));
+  const float* L = fwd.second.data_ptr<float>() + r.tail;
+  const lmk_tensor4 tout = t4(out);
+  check(lmk_ring_gather_attend(&tq, &rk, &rv, slots.data_ptr<int64_t>(), pc, ps, cs, n_pos, &to, L, L + (int64_t)B * H * W, W, &tout,
+                               B, H, T, r.filled, D, (float)scale, block, r.top_k, r.oldest, r.method, dtype, stream));
+  return {out, slots};
+}
+
 // ---- Python
 Tensor tensor_arg(PyObject* o) {                         // None: an undefined tensor
   if (o == Py_None) return Tensor();
@@ -451,6 +603,100 @@ PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// mem_cache_step(q, k_cache, v_cache, cached_rows, k_loc, v_loc, cos, sin, block, top_k, sm_scale | None, shared,
+//                workspace | None, reuse_landmark_keys, k_append | None) -> (out, idx)
+// With k_append the new rows are stored behind the cached ones: k_cache and v_cache are then the cache's buffers.
+PyObject* py_mem_cache_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 15);
+    const Tensor q = tensor_arg(a[0]), kc = tensor_arg(a[1]), vc = tensor_arg(a[2]), kl = tensor_arg(a[4]), vl = tensor_arg(a[5]),
+                 cos = tensor_arg(a[6]), sin = tensor_arg(a[7]), ws = tensor_arg(a[12]), kn = tensor_arg(a[14]);
+    const int64_t S = int_arg(a[3]), block = int_arg(a[8]), top_k = int_arg(a[9]);
+    const bool has_scale = a[10] != Py_None, shared = a[11] == Py_True, reuse = a[13] == Py_True;
+    const double scale = has_scale ? float_arg(a[10]) : 0.0;
+    const auto r = without_gil([&] {
+      const Append append = {kn, kc, vc, S};
+      return mem_cache_step(q, kc, vc, S, kl, vl, cos, sin, (int)block, (int)top_k, has_scale, scale, shared, ws, reuse,
+                            kn.defined() ? &append : nullptr);
+    });
+    return tuple_of({r.first, r.second});
+  });
+}
+
+// retrieve_workspace_bytes(B, H, T, S, D, block)
+PyObject* py_retrieve_workspace_bytes(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 6);
+    return PyLong_FromSize_t(lmk_retrieve_workspace_bytes((int)int_arg(a[0]), (int)int_arg(a[1]), (int)int_arg(a[2]),
+                                                          (int)int_arg(a[3]), (int)int_arg(a[4]), (int)int_arg(a[5])));
+  });
+}
+
+// cache_append(k, v, k_buf, v_buf, row): rows of k and v (B, H, T, D) into the buffers from `row` on
+PyObject* py_cache_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 5);
+    const Tensor k_in = tensor_arg(a[0]), v_in = tensor_arg(a[1]), kb = tensor_arg(a[2]), vb = tensor_arg(a[3]);
+    const int64_t row = int_arg(a[4]);
+    without_gil([&] {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(k_in.device());
+      const Tensor k = kernel_ready(k_in), v = kernel_ready(v_in);
+      need(row >= 0 && row + k.size(2) <= kb.size(2), "no room for the new rows");
+      lmk_tensor4 tk = t4(k), tv = t4(v), tkd = t4(kb), tvd = t4(vb);
+      tkd.ptr = static_cast<char*>(tkd.ptr) + 2 * row * tkd.stride_row;
+      tvd.ptr = static_cast<char*>(tvd.ptr) + 2 * row * tvd.stride_row;
+      check(lmk_cache_append(&tk, &tv, &tkd, &tvd, (int)k.size(0), (int)k.size(1), (int)k.size(2), (int)k.size(3), stream_of(k)));
+      return 0;
+    });
+    Py_RETURN_NONE;
+  });
+}
+
+// ring_attend(q, k, v, cos, sin, ring_k, ring_v, tail_k, tail_v, tail, filled, oldest, top_k, method, start, sm_scale | None)
+//   -> (y, slots | None)
+PyObject* py_ring_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 16);
+    Tensor t[9];
+    for (int i = 0; i < 9; ++i) t[i] = tensor_arg(a[i]);
+    const Ring ring = {t[5], t[6], t[7], t[8], (int)int_arg(a[9]), (int)int_arg(a[10]), (int)int_arg(a[11]), (int)int_arg(a[12]),
+                       (int)int_arg(a[13])};
+    const int64_t start = int_arg(a[14]);
+    const bool has_scale = a[15] != Py_None;
+    const double scale = has_scale ? float_arg(a[15]) : 0.0;
+    const auto r = without_gil([&] { return ring_attend(t[0], t[1], t[2], t[3], t[4], ring, start, has_scale, scale); });
+    return tuple_of({r.first, r.second});
+  });
+}
+
+// ring_store(k, v, is_mem, tail_k, tail_v, tail_is_mem, ring_k, ring_v, tail, next_slot)
+PyObject* py_ring_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 10);
+    Tensor t[8];
+    for (int i = 0; i < 8; ++i) t[i] = tensor_arg(a[i]);
+    const int tail = (int)int_arg(a[8]), next = (int)int_arg(a[9]);
+    without_gil([&] {
+      const Tensor &rk = t[6], &rv = t[7];
+      need(t[0].dim() == 4 && same_shape(t[0], t[1]) && t[0].size(0) <= rk.size(0) && t[0].size(1) == rk.size(3) &&
+               t[0].size(3) == rk.size(4) && same_shape(rk, rv) && rk.strides() == rv.strides(),
+           "keys and values must have one shape, and the cache's heads and head dim");
+      need(t[2].dim() == 2 && t[2].size(0) == t[0].size(0) && t[2].size(1) == t[0].size(2) && t[2].scalar_type() == at::kBool,
+           "is_mem is (batch, rows), bool");
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(t[0].device());
+      const Tensor k = kernel_ready(t[0]), v = kernel_ready(t[1]), marks = t[2].stride(1) == 1 ? t[2] : t[2].contiguous();
+      const lmk_tensor4 tk = t4(k), tv = t4(v), tlk = t4(t[3]), tlv = t4(t[4]);
+      check(lmk_ring_store(&tk, &tv, marks.data_ptr(), marks.stride(0), &tlk, &tlv, t[5].data_ptr(), t[5].stride(0), rk.data_ptr(),
+                           rv.data_ptr(), rk.stride(0), rk.stride(1), rk.stride(2), rk.stride(3), (int)k.size(0), (int)k.size(1),
+                           (int)k.size(2), (int)k.size(3), (int)rk.size(2), (int)rk.size(1), tail, next, stream_of(k)));
+      return 0;
+    });
+    Py_RETURN_NONE;
+  });
+}
+
 // The attention node as Python sees it: an autograd node with `saved_tensors` (q, k, v, o, L, M, and the group factors if
 // there are any), as a Python autograd Function has them.
 PyObject* py_saved_tensors(PyObject* self, void*) {
@@ -476,6 +722,11 @@ PyMethodDef g_methods[] = {
     {"attn_fwd", LMK_FAST(py_attn_fwd)},
     {"attn_bwd", LMK_FAST(py_attn_bwd)},
     {"rotary", LMK_FAST(py_rotary)},
+    {"mem_cache_step", LMK_FAST(py_mem_cache_step)},
+    {"retrieve_workspace_bytes", LMK_FAST(py_retrieve_workspace_bytes)},
+    {"cache_append", LMK_FAST(py_cache_append)},
+    {"ring_attend", LMK_FAST(py_ring_attend)},
+    {"ring_store", LMK_FAST(py_ring_store)},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};

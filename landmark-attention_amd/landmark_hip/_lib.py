@@ -121,6 +121,13 @@ def lib() -> ctypes.CDLL:
         L.lmk_retrieve_and_attend.restype = i
         L.lmk_retrieve_and_attend.argtypes = [T4, T4, T4, T4, T4, vp, vp, i64, i64, vp, T4, vp, sz, i, vp, sz,
                                               i, i, i, i, i, f, i, i, i, vp]
+        L.lmk_cache_append.restype = i
+        L.lmk_cache_append.argtypes = [T4, T4, T4, T4, i, i, i, i, vp]
+        L.lmk_retrieve_attend_append.restype = i
+        L.lmk_retrieve_attend_append.argtypes = [T4, T4, T4, T4, T4, T4, T4, T4, vp, vp, i64, i64, vp, T4, vp, sz, i, vp, sz,
+                                                 i, i, i, i, i, f, i, i, i, vp]
+        L.lmk_ring_store.restype = i
+        L.lmk_ring_store.argtypes = [T4, T4, vp, i64, T4, T4, vp, i64, vp, vp, i64, i64, i64, i64, i, i, i, i, i, i, i, i, vp]
         L.lmk_local_window.restype = i
         L.lmk_local_window.argtypes = [T4, T4, T4, T4, T4, vp, vp, i64, i64, T4, T4, T4, i, i, i, i, i, i, i, vp]
         L.lmk_attn_fwd_segments.restype = i

@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .retrieval import attend_shared, retrieve_and_attend, retrieve_topk_from_landmarks
+from .retrieval import attend_shared, retrieve_topk_from_landmarks
 
 
 class LandmarkKVCache:
@@ -33,7 +33,7 @@ class LandmarkKVCache:
     @property
     def past_key_value(self):
         """The reference's cache tuple (``llama_mem.py:430``): views, no copy."""
-        return self._k[:, :, : self.length], self._v[:, :, : self.length]
+        return self._k.narrow(2, 0, self.length), self._v.narrow(2, 0, self.length)
 
     def _reserve(self, rows: int) -> None:
         if rows <= self.capacity:
@@ -50,9 +50,18 @@ class LandmarkKVCache:
         t = key_states_before_pos.shape[2]
         assert key_states_before_pos.shape == value_states.shape == self._k.shape[:2] + (t, self._k.shape[3])
         self._reserve(self.length + t)
-        self._k[:, :, self.length : self.length + t] = key_states_before_pos
-        self._v[:, :, self.length : self.length + t] = value_states
+        if t > 0 and self._rows_as_they_are(key_states_before_pos) and self._rows_as_they_are(value_states):
+            _lib.native().cache_append(key_states_before_pos, value_states, self._k, self._v, self.length)
+        else:
+            self._k[:, :, self.length : self.length + t] = key_states_before_pos
+            self._v[:, :, self.length : self.length + t] = value_states
         self.length += t
+
+    def _rows_as_they_are(self, x) -> bool:
+        """Rows of the buffers' own 16-bit type and device: one launch copies keys and values (torch's indexed
+        assignment takes two, and converts)."""
+        return x.is_cuda and x.dtype == self._k.dtype and x.device == self._k.device and x.dtype in _lib.DTYPE_CODES \
+            and self._k.shape[3] % 8 == 0
 
     def step(self, query_states, key_states, key_states_before_pos, value_states, cos, sin, block: int, top_k: int,
              sm_scale=None, aggregate=None):
@@ -63,20 +72,32 @@ class LandmarkKVCache:
         The landmark keys are rotated at positions that move only when a cached block completes
         (``:359-365``), and appends never touch complete blocks, so between two landmarks the rotated keys of
         the previous step are reused (per-token selection; same tables, block and top_k)."""
+        if aggregate and aggregate != "max_over_tokens":
+            raise NotImplementedError(aggregate)                        # llama_mem.py:381-382
+        native = _lib.native()
         B, H, T, D = query_states.shape
-        nbytes = _lib.lib().lmk_retrieve_workspace_bytes(B, H, T, self.length, D, int(block))
-        if self._ws is None or self._ws.numel() < nbytes or self._ws.device != query_states.device:
-            self._ws = torch.empty(max(nbytes, 2 * (self._ws.numel() if self._ws is not None else 0)),
-                                   device=query_states.device, dtype=torch.uint8)
+        length = self.length
+        nbytes = native.retrieve_workspace_bytes(B, H, T, length, D, block)
+        ws = self._ws
+        if ws is None or ws.numel() < nbytes or ws.device != query_states.device:
+            self._ws = ws = torch.empty(max(nbytes, 2 * (ws.numel() if ws is not None else 0)),
+                                        device=query_states.device, dtype=torch.uint8)
             self._ws_key = None
-        key = (self.length // block, int(block), int(top_k), cos.data_ptr(), sin.data_ptr(), self._k.data_ptr())
-        reuse = aggregate is None and key == self._ws_key
-        out, idx = retrieve_and_attend(query_states, self.past_key_value, key_states, value_states, cos, sin,
-                                       block, top_k, sm_scale, aggregate, workspace=self._ws,
-                                       reuse_landmark_keys=reuse)
-        self._ws_key = key if aggregate is None else None
-        self.append(key_states_before_pos, value_states)
-        return out, idx
+        key = (length // block, int(block), int(top_k), cos.data_ptr(), sin.data_ptr(), self._k.data_ptr())
+        fits = length + T <= self.capacity and self._rows_as_they_are(key_states_before_pos) \
+            and self._rows_as_they_are(value_states)
+        # the new rows go into the buffers in the same call where they have room; growing the buffers reads them first
+        result = native.mem_cache_step(query_states, self._k if fits else self.past_key_value[0],
+                                       self._v if fits else self.past_key_value[1], length, key_states, value_states, cos, sin,
+                                       block, top_k, sm_scale, bool(aggregate), ws,
+                                       not aggregate and key == self._ws_key,
+                                       key_states_before_pos if fits else None)
+        self._ws_key = None if aggregate else key
+        if fits:
+            self.length = length + T
+        else:
+            self.append(key_states_before_pos, value_states)
+        return result
 
 
 class OffloadedLandmarkCache:

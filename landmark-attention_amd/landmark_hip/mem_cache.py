@@ -44,6 +44,7 @@ class MemLMCacheStorage:
         self.last_incomplete_len = 0
         self.cache_iter = 0
         self.cache_size = 0
+        self._tail_regular = True           # the tail's marks continue the stream: no landmark among them
 
     # ------------------------------------------------------------------ geometry
     @property
@@ -64,11 +65,25 @@ class MemLMCacheStorage:
     def store_in_cache(self, keys, values_dict) -> None:
         """``store_in_cache`` (``:111-158``): keys (B, nh, T, hs) without positions, ``values_dict`` with
         ``'v'`` (B, nh, T, hs) and ``'is_mem'`` (B, T)."""
-        B = keys.shape[0]
+        is_mem = values_dict["is_mem"]
         n0, bs, cap = self.last_incomplete_len, self.block, self.cache_mem_k.shape[1]
+        if self._tail_regular and self._continues_the_stream(keys, values_dict["v"], is_mem, n0, bs):
+            # known to be laid out as it must (a mask tensor is compared once, not once per layer and step): one launch
+            # and no synchronisation
+            dtype, next_slot = self.cache_mem_k.dtype, self.cache_iter
+            _lib.native().ring_store(keys.to(dtype), values_dict["v"].to(dtype), is_mem, self.last_incomplete_k,
+                                     self.last_incomplete_v, self.last_incomplete_ismem, self.cache_mem_k, self.cache_mem_v,
+                                     n0, next_slot)
+            total = n0 + keys.shape[2]
+            n_new = total // bs
+            self.last_incomplete_len = total - n_new * bs
+            self.cache_iter = (next_slot + n_new) % cap
+            self.cache_size += n_new
+            return
+        B = keys.shape[0]
         k = torch.cat((self.last_incomplete_k[:B, :, :n0], keys.to(self.cache_mem_k.dtype)), dim=2)
         v = torch.cat((self.last_incomplete_v[:B, :, :n0], values_dict["v"].to(self.cache_mem_v.dtype)), dim=2)
-        is_mem = torch.cat((self.last_incomplete_ismem[:B, :n0], values_dict["is_mem"]), dim=1)
+        is_mem = torch.cat((self.last_incomplete_ismem[:B, :n0], is_mem), dim=1)
         _, nh, total, hs = k.shape
         rest = total % bs
         full = total - rest
@@ -94,6 +109,21 @@ class MemLMCacheStorage:
         self.cache_mem_v[:B, :kept - first] = vb[:, first:]
         self.cache_iter = (start + kept) % cap if start + kept >= cap else start + kept
         self.cache_size += n_new
+        self._tail_regular = rest == 0 or not bool(is_mem[:, full:].any())
+
+    def _continues_the_stream(self, keys, values, is_mem, offset, block) -> bool:
+        """Whether the chunk can be stored as it is: rows the kernel copies, marks that put a landmark at the end of
+        every block and nowhere else."""
+        if not (keys.is_cuda and values.is_cuda and is_mem.is_cuda and is_mem.dtype == torch.bool and is_mem.dim() == 2
+                and self.cache_mem_k.dtype in _lib.DTYPE_CODES and self.cache_mem_k.is_cuda and keys.shape[2] > 0
+                and self.cache_mem_k.shape[4] % 8 == 0):
+            return False
+        from .attention import _check_is_mem
+        try:
+            _check_is_mem(is_mem, block, offset=offset)
+        except AssertionError:
+            return False
+        return True
 
     # ----------------------------------------------------------------- selection
     def select_blocks(self, q, cos, sin):
@@ -148,50 +178,12 @@ class MemLMCacheStorage:
         Returns ``(y (B, nh, T, hs), slots)``: y is ``att @ v + att_prefix @ cache_v`` (``:235-240``), slots the
         picked blocks in the shape of ``select_blocks`` (None while the cache holds no block or ``cache_topk`` is 0,
         ``:48-49``).  Call ``store_in_cache`` afterwards, as the layer does (``:246-248``)."""
-        from .attention import _check_is_mem, _launch_fwd_blocks
-        import math
-        B, nh, T, hs = q.shape
+        from .attention import _check_is_mem
         block, tail = self.block, self.last_incomplete_len
-        assert q.dtype == self.cache_mem_k.dtype and q.is_cuda and k.shape == v.shape == q.shape
         # is_mem must continue the stream (a landmark closes every block); the check costs a device->host sync, paid
         # once per mask tensor state and tail length, not per call
         _check_is_mem(is_mem, block, offset=tail)
-        if sm_scale is None:
-            sm_scale = 1.0 / math.sqrt(hs)
-        cos, sin = _tables(cos, sin, q.dtype)
-        if tail:
-            # the tokens behind the last complete block open the chunk's first block (:43-46): their keys rotated at
-            # start_index - tail .., zero rows standing in for their queries -- one launch writes the three windows
-            assert start_index >= tail
-            q, k, v = (_lib.kernel_ready(t) for t in (q, k, v))
-            q_win, k_win, v_win = (torch.empty((B, nh, tail + T, hs), dtype=q.dtype, device=q.device) for _ in range(3))
-            with _lib.on_device(q.device):
-                rc = _lib.lib().lmk_ring_local_window(
-                    _lib.tensor4(q), _lib.tensor4(self.last_incomplete_k[:B]), _lib.tensor4(self.last_incomplete_v[:B]),
-                    _lib.tensor4(k), _lib.tensor4(v), cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0],
-                    _lib.tensor4(q_win), _lib.tensor4(k_win), _lib.tensor4(v_win), B, nh, T, tail,
-                    int(start_index - tail), hs, _lib.DTYPE_CODES[q.dtype], _lib.current_stream(q.device))
-            _lib.check(rc)
-        else:
-            q_win, k_win, v_win = (_lib.kernel_ready(t) for t in (q, k, v))
-        W = tail + T
-        with _lib.on_device(q.device):
-            # blocks of any size up to 128 tokens, read as they are (the benchmark's 51 run in 64 slots)
-            o_win, L, M = _launch_fwd_blocks(q_win, k_win, v_win, 0, sm_scale, block)
-            o_loc, L_loc, M_loc, stat_stride = o_win[:, :, tail:], L[:, tail:], M[:, tail:], W
-            n = self.filled
-            if n == 0 or self.cache_topk == 0:
-                return o_loc, None
-            slots = self.select_blocks(q, cos, sin)
-            q = _lib.kernel_ready(q)
-            out = torch.empty_like(q)
-            kring = self.cache_mem_k[:B, :n].flatten(1, 2).transpose(1, 2)    # (B, nh, n*block, hs) views, no copy
-            vring = self.cache_mem_v[:B, :n].flatten(1, 2).transpose(1, 2)
-            rc = _lib.lib().lmk_ring_gather_attend(
-                _lib.tensor4(q), _lib.tensor4(kring), _lib.tensor4(vring), slots.data_ptr(), cos.data_ptr(),
-                sin.data_ptr(), cos.stride(0), cos.shape[0], _lib.tensor4(o_loc), L_loc.data_ptr(), M_loc.data_ptr(),
-                stat_stride, _lib.tensor4(out), B, nh, T, n, hs, float(sm_scale), block, self.cache_topk,
-                self.oldest_slot, SELECTION_METHODS[self.cache_selection_method], _lib.DTYPE_CODES[q.dtype],
-                _lib.current_stream(q.device))
-        _lib.check(rc)
-        return out, slots
+        # blocks of any size up to 128 tokens, read as they are (the benchmark's 51 run in 64 slots)
+        return _lib.native().ring_attend(q, k, v, cos, sin, self.cache_mem_k, self.cache_mem_v, self.last_incomplete_k,
+                                         self.last_incomplete_v, tail, self.filled, self.oldest_slot, self.cache_topk,
+                                         SELECTION_METHODS[self.cache_selection_method], start_index, sm_scale)
