@@ -136,6 +136,7 @@ typedef __attribute__((address_space(3))) float* lds_f32_ptr;
 typedef __attribute__((address_space(3))) u32x2_t* lds_u32x2_ptr;
 __device__ __forceinline__ u32x4_t lds_ld128(int addr) { return *(lds_u32x4_ptr)(uintptr_t)(uint32_t)addr; }
 __device__ __forceinline__ void lds_st128(int addr, u32x4_t v) { *(lds_u32x4_ptr)(uintptr_t)(uint32_t)addr = v; }
+__device__ __forceinline__ float lds_ld32(int addr) { return *(lds_f32_ptr)(uintptr_t)(uint32_t)addr; }
 __device__ __forceinline__ void lds_st32(int addr, float v) { *(lds_f32_ptr)(uintptr_t)(uint32_t)addr = v; }
 __device__ __forceinline__ u32x2_t lds_ld_tr(int addr) {
   s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(uintptr_t)(uint32_t)addr);

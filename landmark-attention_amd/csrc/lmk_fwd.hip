@@ -491,8 +491,23 @@ static int launch_fwd_d(const FwdParams& p, int D, int BS, hipStream_t stream) {
   return LMK_ERR_UNSUPPORTED;
 }
 
+// Whether the workgroups of 64 rows whose waves split the keys (lmk_fwd_split.hip) are faster than those of 256 rows
+// that share one K/V stream.  They are wherever a launch of the latter does not fill the chip, and beyond that up to a
+// point that depends on how much a workgroup of 256 rows leaves idle: measured over head dims 64 and 128, blocks of 51,
+// 64, 100 and 128 tokens, 128 to 10000 keys (us, 256 rows -> 64 rows, at n = workgroups of 256 rows / compute unit):
+//   D128, whole blocks:       n 0.5  32.9 -> 17.3,  n 1  60 -> 52,  n 1.5  43.6 -> 42.0 (L1024), 93 -> 98 (L3072),  n 2  83 -> 92
+//   D64, whole blocks:        n 1.5  27.5 -> 24.6,  n 3  48.7 -> 46.7,  n 4  69 -> 67 (L1024), 188 -> 199 (L4096)
+//   D128, slots to tokens:    n 2.3  85 -> 68,  n 3.4  324 -> 312,  n 5.1  509 -> 518 (L4080), 146 -> 137 (L510)
+static bool few_query_rows(const FwdParams& p, int D, int BS) {
+  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 255) / 256), cus = cu_count();
+  const bool whole = p.Lq_real <= 0 && p.n_real == BS;
+  if (whole && D == 128) return 2 * n <= (p.Lk <= 2048 ? 3 : 2) * cus;
+  return n <= 3 * cus || p.Lk <= 1024;
+}
+
 int launch_fwd(const FwdParams& p, int D, int BS, int dtype, hipStream_t stream) {
   if (BS == 32) return launch_fwd32(p, D, dtype, stream);
+  if (few_query_rows(p, D, BS)) return launch_fwd_split(p, D, BS, dtype, stream);
   if (dtype == LMK_DTYPE_BF16) return launch_fwd_d<bf16_t>(p, D, BS, stream);
   if (dtype == LMK_DTYPE_F16) return launch_fwd_d<f16_t>(p, D, BS, stream);
   return LMK_ERR_UNSUPPORTED;

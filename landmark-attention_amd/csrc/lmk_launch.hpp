@@ -72,6 +72,7 @@ struct FwdParams {
 };
 
 int launch_fwd(const FwdParams& p, int D, int BS, int dtype, hipStream_t stream);
+int launch_fwd_split(const FwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // few query rows, blocks 64 and 128
 int launch_fwd32(const FwdParams& p, int D, int dtype, hipStream_t stream);   // block 32 specialisation
 
 struct BwdParams {
