@@ -15,8 +15,8 @@
 //   dkdv   key-stationary, S layout (lane = key): purely elementwise between its four
 //          products S = Q K^T, dP = dO V^T, dV^T += dO^T W, dK^T += Q^T dS
 //          (lmk_bwd_dkdv32.hip, all block sizes).
-// This file holds the pre kernel, the dQ kernel for blocks of 64 and 128 keys (block 32 has its own in
-// lmk_bwd_dq32.hip) and the dispatch.
+// This file holds the pre kernel, the dQ kernel for many query rows of whole blocks of 64 keys (block 32 has its own in
+// lmk_bwd_dq32.hip, everything else is lmk_bwd_dq_split.hip's) and the dispatch.
 //
 // All probabilities are used normalised (exp2(s*c - mhat) already divides by L), so dO is
 // consumed as is; the reference's rescaled copy dO/L (:147) is not needed.
@@ -68,17 +68,17 @@ __global__ __launch_bounds__(256) void lmk_bwd_pre_kernel(BwdParams p, int block
 }
 
 // ---------------------------------------------------------------------------
-// dq (+ per-block statistics), landmark blocks of 64 and 128 keys
+// dq (+ per-block statistics), landmark blocks of 64 keys, many query rows
 // ---------------------------------------------------------------------------
 // A workgroup is 8 waves = 256 query rows, two waves per SIMD; a wave keeps the fragments of its 32
 // rows of Q and dO and its dQ^T accumulator in registers.  One stage is one landmark block: its K and
 // V rows come into one of two LDS buffers by direct global->LDS loads (no staging registers: the kernel
 // has to stay inside 256 registers for two waves to share a SIMD), requested one stage ahead, each wave
 // fetching its share; one barrier per stage.  The block's local softmax needs all its scores before any
-// weight is final, so the S^T tiles of the whole block stay in registers; with four tiles per block the
-// dP^T tiles do not fit beside them and are computed twice (once for nD, once for dS).
-template <class T, int D, int BS>
+// weight is final, so the S^T tiles of the whole block stay in registers.
+template <class T, int D>
 struct DqCfg {
+  static constexpr int BS = 64;
   static constexpr int NT = BS / 32;                       // MFMA tiles per landmark block
   static constexpr int NW = 8;
   static constexpr int CH = D / 8;
@@ -91,7 +91,6 @@ struct DqCfg {
   static constexpr int RPD = 1024 / ROWB;                  // rows covered by one 1 KB request
   static constexpr int NREQ = 2 * BS / RPD;                // requests per stage
   static constexpr int PER_WAVE = NREQ / NW;
-  static constexpr bool KEEP_DP = NT <= 2;                 // dP^T tiles kept beside the S^T tiles
   static_assert(NREQ % NW == 0, "every wave issues the same number of requests");
 };
 
@@ -105,16 +104,10 @@ __device__ __forceinline__ void dq_dma16(const void* base_uniform, uint32_t voff
                :: "v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_off)) : "memory");
 }
 
-// VIRT: tensors in token layout (p.Lq_real > 0); a template parameter because the slot arithmetic costs the
-// slot-layout instantiations registers they do not have.
-// SEG (with VIRT): blocks of unequal length, looked up in p.seg -- a template parameter for the same reason.
-// PLAIN (without VIRT): every block has BS tokens in its BS slots -- no padding slots to mask; the masks' scalar
-// registers and the branch are what it saves the common case.
-template <class T, int D, int BS, bool VIRT, bool SEG = false, bool PLAIN = false>
+template <class T, int D>
 __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
-  static_assert(VIRT || !SEG, "the table describes tensors in token layout");
-  static_assert(!PLAIN || !VIRT, "plain: the tensors' rows are the kernel's rows");
-  using C = DqCfg<T, D, BS>;
+  using C = DqCfg<T, D>;
+  constexpr int BS = C::BS;
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -145,14 +138,6 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
   const int cblk = dt / C::NT, tsub = dt % C::NT;          // the wave's own block and its tile inside it
   const bool active = q0 < p.Lq;                           // Lq is a multiple of the block: whole tiles only
   const int qrow = q0 + ql;
-  // token layout: the tensors' rows are tokens, the kernel's rows (and the workspace's) are slots.  A slot without
-  // a token is a query row of zeros with mhat = 1e30: its gate, its weights and every term it leaves for the dK/dV
-  // kernel come out as exact zeros (a = 1e30), whatever that kernel reads for its Q and dO rows.
-  constexpr bool virt = VIRT;
-  const int nfull_k = p.n_full_k;
-  const int* seg_k = SEG ? p.seg : nullptr;
-  const int* seg_q = SEG ? p.seg + p.n_prefix : nullptr;   // the queries' first block
-  const int qtok = !active ? -1 : (virt ? slot_to_token_row<BS>(qrow, p.n_real, p.n_full_q, seg_q) : qrow);
 
   u32x4_t qf[C::KS], gf[C::KS];
 #pragma unroll
@@ -160,9 +145,9 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
     u32x4_t z = {0, 0, 0, 0};
     qf[ks] = z;
     gf[ks] = z;
-    if (qtok >= 0) {
-      qf[ks] = *(const u32x4_t*)(qp + 2 * ((int64_t)qtok * p.qs_r + 16 * ks + 8 * h));
-      gf[ks] = *(const u32x4_t*)(gp + 2 * ((int64_t)qtok * p.dos_r + 16 * ks + 8 * h));
+    if (active) {
+      qf[ks] = *(const u32x4_t*)(qp + 2 * ((int64_t)qrow * p.qs_r + 16 * ks + 8 * h));
+      gf[ks] = *(const u32x4_t*)(gp + 2 * ((int64_t)qrow * p.dos_r + 16 * ks + 8 * h));
     }
   }
   // row terms (the reference's _bwd_preprocess, flash_landmark_attention.py:125-149): delta = rowsum(O * dO)
@@ -171,21 +156,17 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
   float mhat = 0.f, delta = 0.f;
   if (active) {
     float sum = 0.f;
-    mhat = 1e30f;
-    if (qtok >= 0) {
-      const char* orow = (const char*)p.o + 2 * (b * p.os_b + hh * p.os_h + (int64_t)qtok * p.os_r);
+    const char* orow = (const char*)p.o + 2 * (b * p.os_b + hh * p.os_h + (int64_t)qrow * p.os_r);
 #pragma unroll
-      for (int ks = 0; ks < C::KS; ++ks) {
-        const u32x4_t o4 = *(const u32x4_t*)(orow + 2 * (16 * ks + 8 * h));
+    for (int ks = 0; ks < C::KS; ++ks) {
+      const u32x4_t o4 = *(const u32x4_t*)(orow + 2 * (16 * ks + 8 * h));
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          sum += unpack_lo<T>(o4[i]) * unpack_lo<T>(gf[ks][i]) + unpack_hi<T>(o4[i]) * unpack_hi<T>(gf[ks][i]);
-      }
-      const int64_t li = (int64_t)bh * (virt ? p.Lq_real : p.Lq) + qtok;   // L, M follow the tensors' layout
-      mhat = p.M[li] * kLog2e + fast_log2(p.L[li]);
+      for (int i = 0; i < 4; ++i)
+        sum += unpack_lo<T>(o4[i]) * unpack_lo<T>(gf[ks][i]) + unpack_hi<T>(o4[i]) * unpack_hi<T>(gf[ks][i]);
     }
     delta = pair_sum(sum);
     const int64_t ri = (int64_t)bh * p.Lq + qrow;
+    mhat = p.M[ri] * kLog2e + fast_log2(p.L[ri]);
     if (h == 0) {
       p.delta[ri] = delta;
       p.mhat[ri] = mhat;
@@ -210,24 +191,15 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
     src[i] = (uint32_t)(2 * ((int64_t)row * (is_v ? p.vs_r : p.ks_r) + 8 * (cp ^ f)));
   }
   const uint32_t step_k = (uint32_t)(2 * (int64_t)BS * p.ks_r), step_v = (uint32_t)(2 * (int64_t)BS * p.vs_r);
-  int blk_req = 0;                                         // block the next request fetches
   auto request = [&](int buf) __attribute__((always_inline)) {   // next block in key order -> buffer buf
 #pragma unroll
     for (int i = 0; i < C::PER_WAVE; ++i) {
       const int r = wave * C::PER_WAVE + i;
       const bool is_v = r >= n_k;                          // wave-uniform
       const int dst = buf * C::STAGE_BYTES + (is_v ? C::TILE_BYTES : 0) + C::RPD * (r % n_k) * C::ROWB;
-      if (virt) {                                          // the slot's token row, worked out per request
-        const int row = C::RPD * (r % n_k) + lane / C::CH, cp = lane % C::CH;
-        const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
-        const int tok = slot_to_token_row_clamped<BS>(blk_req * BS + row, p.n_real, nfull_k, seg_k);
-        dq_dma16(is_v ? vp : kp, (uint32_t)(2 * ((int64_t)tok * (is_v ? p.vs_r : p.ks_r) + 8 * (cp ^ f))), dst);
-      } else {
-        dq_dma16(is_v ? vp : kp, src[i], dst);
-        src[i] += is_v ? step_v : step_k;
-      }
+      dq_dma16(is_v ? vp : kp, src[i], dst);
+      src[i] += is_v ? step_v : step_k;
     }
-    ++blk_req;
   };
 
   f32x16_t acc[C::DC];
@@ -236,11 +208,6 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dc][r] = 0.f;
   const float c2 = p.scale_log2;
-  // A block narrower than BS tokens is stored with its n_norm normal keys in front, its landmark in the
-  // last slot and padding in between: slots n_norm .. BS-2 hold no key and no query may see them.
-  // With blocks of unequal length n_norm is the stage's block's (uniform over the workgroup).
-  const int n_norm_all = p.n_real - 1;
-  const bool padded = !PLAIN && (n_norm_all < BS - 1 || seg_k != nullptr);   // uniform over the launch
 
   // LDS byte offsets of this lane's operand fragments inside a 32-row tile: the swizzle repeats every 16
   // rows, so a tile at row 32u is the same offsets plus 32u rows -- an immediate of the LDS instruction
@@ -348,26 +315,12 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
   const uint32_t stat_row = 4u * (uint32_t)qrow;
   // ---------------- earlier block s at LDS byte addresses kb (K rows) / vb (V rows)
   auto earlier_block = [&](const int kb, const int vb, const int s) __attribute__((always_inline)) {
-    int n_norm = n_norm_all;
-    if constexpr (SEG) n_norm = block_normal_keys<BS>(s, p.n_real, nfull_k, seg_k);
-    float gscale = 1.f;                                    // group dropout: this block's factor for this query row
-    if constexpr (VIRT)
-      if (p.group_scale != nullptr && qtok >= 0) gscale = p.group_scale[(int64_t)bh * p.gs_bh + (int64_t)s * p.gs_blk + qtok];
-    f32x16_t sc[C::NT], dp[C::KEEP_DP ? C::NT : 1];
+    f32x16_t sc[C::NT], dp[C::NT];
     row_tiles(kb, qf, sc, std::integral_constant<int, C::NT>{});
-    if (padded) {                                          // padding slots leave the local softmax
-#pragma unroll
-      for (int u = 0; u < C::NT; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kl = 32 * u + 8 * (r >> 2) + 4 * h + (r & 3);
-          if (kl >= n_norm && kl < BS - 1) sc[u][r] = -INFINITY;
-        }
-    }
     const float s_last = sc[C::NT - 1][15];
     float mx = (h == 0) ? s_last : -INFINITY;
     float t_lm = 0.f, mloc = 0.f, den = 0.f, spd = 0.f;
-    if constexpr (C::KEEP_DP) {
+    {
       // dP^T does not depend on S^T: at head dim 64 its MFMAs carry the local softmax of the scores, a slice behind
       // each -- first the maximum (one slice per tile), then the exponentials and their sum.  (At head dim 128 the
       // same placement measured 7 % slower than the softmax behind the MFMAs, in the compiler's order.)
@@ -418,27 +371,6 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
       for (int u = 0; u < C::NT; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) spd = __builtin_fmaf(sc[u][r], dp[u][r], spd);
-    } else {
-#pragma unroll
-      for (int u = 0; u < C::NT; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (!(u == C::NT - 1 && r == 15)) mx = fmaxf(mx, sc[u][r]);
-      mx = pair_max(mx);
-      t_lm = pair_hi(s_last) * c2;
-      mloc = mx * c2;
-#pragma unroll
-      for (int u = 0; u < C::NT; ++u) {
-        row_tiles(vb + 32 * u * C::ROWB, gf, dp, std::integral_constant<int, 1>{});
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float e = fast_exp2(__builtin_fmaf(sc[u][r], c2, -mloc));
-          if (u == C::NT - 1 && r == 15) e = (h == 0) ? e : 0.f;
-          sc[u][r] = e;
-          den += e;
-          spd = __builtin_fmaf(e, dp[0][r], spd);
-        }
-      }
     }
     den = pair_sum(den);
     spd = pair_sum(spd);
@@ -446,24 +378,15 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
     const float nD = spd * invden;
     const float glog = t_lm - mhat;                        // log2 of the normalised gate
     const float g = fast_exp2(glog);
-    // out_i = .. + gscale * g * (P V): the weights carry the factor, the landmark's dS sees it through nD
-    const float f = g * invden * gscale;
-    const float dslm = g * (gscale * nD - delta);          // dS at the block's landmark key
+    const float f = g * invden;
+    const float dslm = g * (nD - delta);                   // dS at the block's landmark key
     if (h == 0) {                                          // a scalar base per (head, block) plus the row's 32-bit offset
       const int64_t sb = 4 * ((int64_t)bh * p.n_blocks + s) * p.Lq;
-      *(float*)((char*)p.stat_a + sb + stat_row) = gscale > 0.f ? mloc + fast_log2(den) - glog - fast_log2(gscale) : 1e30f;
+      *(float*)((char*)p.stat_a + sb + stat_row) = mloc + fast_log2(den) - glog;
       *(float*)((char*)p.stat_n + sb + stat_row) = nD;
       *(float*)((char*)p.stat_l + sb + stat_row) = dslm;
     }
-    if constexpr (C::KEEP_DP) {
-      dq_tiles(kb, 0, sc, dp, 1, f, nD, dslm, std::integral_constant<int, C::NT>{});
-    } else {
-#pragma unroll
-      for (int u = 0; u < C::NT; ++u) {
-        row_tiles(vb + 32 * u * C::ROWB, gf, dp, std::integral_constant<int, 1>{});
-        dq_tiles(kb + 32 * u * C::ROWB, u, sc + u, dp, 0, f, nD, dslm, std::integral_constant<int, 1>{});
-      }
-    }
+    dq_tiles(kb, 0, sc, dp, 1, f, nD, dslm, std::integral_constant<int, C::NT>{});
   };
 
   // Stages in front of the workgroup's first query block are earlier blocks for every wave: they run two at a
@@ -494,8 +417,6 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
     if (s < cblk) {
       earlier_block(kb, vb, s);
     } else if (s == cblk) {
-      int n_norm = n_norm_all;
-      if constexpr (SEG) n_norm = block_normal_keys<BS>(s, p.n_real, nfull_k, seg_k);
       const int lim = ql - ((tsub == C::NT - 1 && ql == 31) ? 1 : 0);
 #pragma unroll
       for (int u = 0; u < C::NT; ++u) {
@@ -506,9 +427,7 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int key = 8 * (r >> 2) + 4 * h + (r & 3);
-            const int kl = 32 * u + key;
-            const bool pad = padded && kl >= n_norm && kl < BS - 1;   // only the landmark query could reach one
-            const float pr = ((u < tsub || key <= lim) && !pad) ? fast_exp2(__builtin_fmaf(sc[r], c2, -mhat)) : 0.f;
+            const float pr = (u < tsub || key <= lim) ? fast_exp2(__builtin_fmaf(sc[r], c2, -mhat)) : 0.f;
             ds[r] = pr * (d[r] - delta);
           }
           dq_tile(kb + 32 * u * C::ROWB, ds);
@@ -522,10 +441,9 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
   if (active) {
     static_assert(C::STAGE_BYTES / C::NW >= 2048, "32 rows x 32 columns of 16 bits per wave");
     const int free_buf = (n_stages & 1) * C::STAGE_BYTES;  // the last stage sits in buffer (n_stages - 1) & 1
-    store_tile_rows<T, C::DC>(acc, p.scale, free_buf + wave * (C::STAGE_BYTES / C::NW),
+    store_tile_rows<T, C::DC, false>(acc, p.scale, free_buf + wave * (C::STAGE_BYTES / C::NW),
                               [&](int r) __attribute__((always_inline)) -> char* {
-      const int tok = virt ? slot_to_token_row<BS>(q0 + r, p.n_real, p.n_full_q, seg_q) : q0 + r;
-      return tok < 0 ? nullptr : dqp + 2 * ((int64_t)tok * p.dqs_r);
+      return dqp + 2 * ((int64_t)(q0 + r) * p.dqs_r);
     });
   }
 }
@@ -533,6 +451,17 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+// Whether workgroups of 256 rows (lmk_bwd_dq_kernel) are faster than those of 64 rows whose waves split the keys
+// (lmk_bwd_dq_split.hip): only with whole blocks of 64 keys and more long rows than fill the chip twice.  Measured (us, 256
+// rows -> 64 rows, D128, at n = workgroups of 256 rows / compute unit): n 0.5 79 -> 30 (L2048), n 1 34.2 -> 29.6 (L512),
+// n 1.5 141 -> 134 (L3072), n 2 125.5 -> 124.5 (L2048), n 3 121 -> 117 (L960), n 4 134 -> 127 (L512) but 449 -> 469 (L4096),
+// n 8 551 -> 661 (L2048); D64 n 4 286 -> 293 (L4096), 72 -> 69 (L512).  With tokens in slots or blocks of 128 the 64-row
+// kernel was 1 % behind at worst and 30-60 % ahead at block 128 (no room for a block's dP tiles in the other).
+static bool many_query_rows(const BwdParams& p) {
+  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 255) / 256);
+  return p.Lq_real <= 0 && p.n_real == 64 && p.Lk > 1024 && n > 2 * cu_count();
+}
+
 template <class T, int D, int BS>
 static int launch_bwd_t(const BwdParams& p, int phases, hipStream_t stream) {
   int rc;
@@ -546,30 +475,14 @@ static int launch_bwd_t(const BwdParams& p, int phases, hipStream_t stream) {
   if (phases & 2) {
     if constexpr (BS == 32) {
       if ((rc = launch_bwd_dq32(p, D, std::is_same<T, bf16_t>::value ? LMK_DTYPE_BF16 : LMK_DTYPE_F16, stream))) return rc;
+    } else if (BS == 128 || !many_query_rows(p)) {
+      if ((rc = launch_bwd_dq_split(p, D, BS, std::is_same<T, bf16_t>::value ? LMK_DTYPE_BF16 : LMK_DTYPE_F16, stream))) return rc;
     } else {
-      using C = DqCfg<T, D, BS>;
-      const dim3 grid(((p.Lq + 255) / 256) * p.B * p.H);
-      if (p.Lq_real > 0 && p.seg != nullptr) {
-        auto kern = lmk_bwd_dq_kernel<T, D, BS, true, true>;
-        static std::atomic<uint64_t> lds_ok{0};
-        if ((rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok))) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(64 * C::NW), C::LDS_BYTES, stream, p);
-      } else if (p.Lq_real > 0) {
-        auto kern = lmk_bwd_dq_kernel<T, D, BS, true>;
-        static std::atomic<uint64_t> lds_ok{0};
-        if ((rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok))) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(64 * C::NW), C::LDS_BYTES, stream, p);
-      } else if (p.n_real == BS) {
-        auto kern = lmk_bwd_dq_kernel<T, D, BS, false, false, true>;
-        static std::atomic<uint64_t> lds_ok{0};
-        if ((rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok))) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(64 * C::NW), C::LDS_BYTES, stream, p);
-      } else {
-        auto kern = lmk_bwd_dq_kernel<T, D, BS, false>;
-        static std::atomic<uint64_t> lds_ok{0};
-        if ((rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok))) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(64 * C::NW), C::LDS_BYTES, stream, p);
-      }
+      using C = DqCfg<T, D>;
+      auto kern = lmk_bwd_dq_kernel<T, D>;
+      static std::atomic<uint64_t> lds_ok{0};
+      if ((rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok))) return rc;
+      hipLaunchKernelGGL(kern, dim3(((p.Lq + 255) / 256) * p.B * p.H), dim3(64 * C::NW), C::LDS_BYTES, stream, p);
       if ((rc = (int)hipGetLastError())) return rc;
     }
   }

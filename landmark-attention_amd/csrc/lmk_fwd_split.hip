@@ -15,6 +15,7 @@
 
 #include "lmk_common.hpp"
 #include "lmk_launch.hpp"
+#include "lmk_split.hpp"
 
 namespace lmk {
 
@@ -47,19 +48,6 @@ struct FwdSplitCfg {
   static_assert(QT * DC * (KP - 1) * 4096 <= (KP > 2 ? LM_BASE : V_BASE), "the parts' accumulators fit the stage");
 };
 
-// One 1 KB direct global->LDS request of a wave: lane i's 16 bytes land at lds_off + 16*i (lds_off wave-uniform, in M0).
-__device__ __forceinline__ void split_dma16(const void* base_uniform, uint32_t voff, uint32_t lds_off) {
-  const uint64_t b = (uint64_t)base_uniform;
-  const uint64_t base = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) |
-                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_off)) : "memory");
-}
-
-// How the tensors' rows make up the kernel's slots: PLAIN: every block has BS tokens in BS slots; TOKENS: blocks of
-// n_real tokens, rows = tokens or rows = slots (FwdParams::Lq_real); FACTORS: the same with group dropout factors;
-// TABLE: blocks of unequal length, looked up in FwdParams::seg.
-enum { PLAIN, TOKENS, FACTORS, TABLE };
 template <class T, int D, int BS, int KP, int LAYOUT>
 __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p) {
   constexpr bool plain = LAYOUT == PLAIN, GS = LAYOUT == FACTORS, SEG = LAYOUT == TABLE;
@@ -71,9 +59,8 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
   const int part = wave % KP, tq = wave / KP;
   const int ql = lane & 31, h = lane >> 5;
 
-  // ---- workgroup -> head, batch, 64-row query tile (heavy tiles first): with a multiple of 8 heads all of a head's
-  // workgroups land on one XCD, and there is nothing to divide
-  const int hh = blockIdx.x, b = blockIdx.y, qt = gridDim.z - 1 - blockIdx.z;
+  // ---- workgroup -> head, batch, 64-row query tile (launch_rows64)
+  const int hh = blockIdx.x, b = p.b0 + blockIdx.y, qt = p.qt_top - blockIdx.z;
   const int bh = b * p.H + hh;
   const char* qp = (const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h);
   const char* kp = (const char*)p.k + 2 * (b * p.ks_b + hh * p.ks_h);
@@ -138,7 +125,6 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
       }
     }
   };
-  auto wait_all = [&]() __attribute__((always_inline)) { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
 
   u32x4_t qf[C::KS];                                    // Q fragments (B operand): query qrow, head dims 16*ks + 8h .. +7
   const float c2 = p.scale_log2;
@@ -169,10 +155,6 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
       }
     }
   }
-  auto zero16 = [](f32x16_t& x) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) x[r] = 0.f;
-  };
   f32x16_t acc[C::DC];
 #pragma unroll
   for (int dc = 0; dc < C::DC; ++dc) zero16(acc[dc]);
@@ -205,7 +187,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
         __builtin_amdgcn_s_waitcnt(0x0f70 | C::PER_WAVE);
       } else {
         if (base == 0) request(false, 0);
-        wait_all();
+        wait_vm0();
       }
       __syncthreads();
       if (base == 0) {
@@ -374,8 +356,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
       const int blk = min(st * (KP / C::NH) + part / C::NH, cblk - 1);
       if (blk >= 0) {
         const float* src = p.group_scale + (int64_t)bh * p.gs_bh + (int64_t)blk * p.gs_blk + max(qtok, 0);
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-                     :: "v"(src), "s"(__builtin_amdgcn_readfirstlane(C::GS_BASE + wave * 256)) : "memory");
+        split_dma4(src, C::GS_BASE + wave * 256);
       }
     }
   };
@@ -383,11 +364,11 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
   // ---- stages of earlier blocks only
   const int last = cblk * C::NH / KP, own = cblk * C::NH % KP;   // the stage of the own block, and the own block's first part
   for (int st = 0; st < last; ++st) {
-    wait_all();
+    wait_vm0();
     __syncthreads();                                    // K of the stage is there; V of the one before has been read
     request_v(st);
     earlier_scores(st);
-    wait_all();
+    wait_vm0();
     __syncthreads();                                    // V is there; K has been read
     request(false, st + 1);
     earlier_product();
@@ -395,7 +376,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
   // ---- the own block's stage: parts in front of it have an earlier block, the others take its causal tiles
   float Mrun = R;
   {
-    wait_all();
+    wait_vm0();
     __syncthreads();
     request_v(last);
     const int np = KP - own;                            // tile u of the own block goes to part own + u % np
@@ -443,7 +424,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
           for (int r = 0; r < 16; ++r) acc[dc][r] *= alpha;
       }
     }
-    wait_all();
+    wait_vm0();
     __syncthreads();
     if (earlier) {
       earlier_product();
@@ -516,9 +497,7 @@ static int launch_fwd_split_t(const FwdParams& p, hipStream_t stream) {
   using C = FwdSplitCfg<T, D, BS, KP>;
   auto kern = lmk_fwd_split_kernel<T, D, BS, KP, LAYOUT>;
   static std::atomic<uint64_t> lds_ok{0};
-  if (int rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok)) return rc;
-  hipLaunchKernelGGL(kern, dim3(p.H, p.B, (p.Lq + 63) / 64), dim3(64 * C::NW), C::LDS_BYTES, stream, p);
-  return (int)hipGetLastError();
+  return launch_rows64(kern, p, 64 * C::NW, C::LDS_BYTES, lds_ok, stream);
 }
 
 template <class T, int D, int BS, int KP>
@@ -536,13 +515,9 @@ static int launch_fwd_split_d(const FwdParams& p, int BS, int kparts, hipStream_
   return LMK_ERR_UNSUPPORTED;
 }
 
-// Two parts leave room for two workgroups on a compute unit.  Four parts put two waves on every SIMD when each
-// compute unit has one workgroup (B2 H8 L1024 block 64: 16.8 -> 15.1 us), and still pay with two if the walk is long
-// (B1 H12 L2500: 34.6 -> 32.2; at B1 H32 L1024 they lose, 17.3 -> 19.6).
 int launch_fwd_split(const FwdParams& p, int D, int BS, int dtype, hipStream_t stream) {
   if (p.seg != nullptr && p.group_scale != nullptr) return LMK_ERR_UNSUPPORTED;
-  const int64_t n = (int64_t)p.B * p.H * ((p.Lq + 63) / 64), cus = cu_count();
-  const int kparts = n <= cus || (n <= 2 * cus && p.Lk >= 2048) ? 4 : 2;
+  const int kparts = key_parts(p.B, p.H, p.Lq, p.Lk);
   if (dtype == LMK_DTYPE_BF16) {
     if (D == 128) return launch_fwd_split_d<bf16_t, 128>(p, BS, kparts, stream);
     if (D == 64) return launch_fwd_split_d<bf16_t, 64>(p, BS, kparts, stream);

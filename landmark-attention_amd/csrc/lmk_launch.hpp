@@ -40,6 +40,15 @@ inline int cu_count() {
   return v;
 }
 
+// Key parts of the kernels with 64 query rows per workgroup (lmk_fwd_split.hip, lmk_bwd_dq_split.hip).  Two leave room for
+// two workgroups on a compute unit.  Four put two waves on every SIMD when each compute unit has one workgroup (B2 H8
+// L1024 block 64: forward 16.8 -> 15.1 us, dQ 20.7 -> 18.3), and still pay with two workgroups if the walk is long (B1 H8
+// L4096: dQ 75.8 -> 65.7; at B1 H32 L1024 they lose, 25.3 -> 26.9).
+inline int key_parts(int B, int H, int Lq, int Lk) {
+  const int64_t n = (int64_t)B * H * ((Lq + 63) / 64), cus = cu_count();
+  return n <= cus || (n <= 2 * cus && Lk >= 2048) ? 4 : 2;
+}
+
 struct FwdParams {
   const void *q, *k, *v;
   void* o;
@@ -69,6 +78,7 @@ struct FwdParams {
   int64_t rope_pos_stride_b, rope_cs_r, rope_n_pos;
   int64_t qs_b, qs_h, qs_r, ks_b, ks_h, ks_r, vs_b, vs_h, vs_r, os_b, os_h, os_r;  // element strides
   float scale_log2;  // sm_scale * log2(e)
+  int b0, qt_top;    // of a launch with 64 query rows per workgroup: first batch, last row tile (launch_rows64)
 };
 
 int launch_fwd(const FwdParams& p, int D, int BS, int dtype, hipStream_t stream);
@@ -98,11 +108,13 @@ struct BwdParams {
   int64_t qs_b, qs_h, qs_r, ks_b, ks_h, ks_r, vs_b, vs_h, vs_r, os_b, os_h, os_r, dos_b, dos_h, dos_r;
   int64_t dqs_b, dqs_h, dqs_r, dks_b, dks_h, dks_r, dvs_b, dvs_h, dvs_r;
   float scale, scale_log2;
+  int b0, qt_top;                // as in FwdParams
 };
 
 // phases: bit 0 = pre, bit 1 = dq, bit 2 = dkdv
 int launch_bwd(const BwdParams& p, int D, int BS, int dtype, int phases, hipStream_t stream);
 int launch_bwd_dq32(const BwdParams& p, int D, int dtype, hipStream_t stream);     // block 32 specialisation
+int launch_bwd_dq_split(const BwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // blocks 64 and 128, 64 rows a workgroup
 int launch_bwd_dkdv32(const BwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // two-role kernel, all block sizes
 int launch_bwd_dkdv32_handover(const BwdParams& p, int D, int dtype, hipStream_t stream);  // block 32, dS read from p.ds_tiles
 
