@@ -462,6 +462,21 @@ static bool many_query_rows(const BwdParams& p) {
   return p.Lq_real <= 0 && p.n_real == 64 && p.Lk > 1024 && n > 2 * cu_count();
 }
 
+// Whether the dK/dV kernel with 128 keys per workgroup and roles (lmk_bwd_dkdv32.hip) is faster than the one with 64 keys
+// (lmk_bwd_dkdv_split.hip).  At head dim 128 it is when its workgroups come in whole rounds of the compute units, from two
+// 64-key workgroups per compute unit on.  Measured (us, 128 keys -> 64 keys): filled, B4 H32 L512 32.6 -> 38.6, B2 H32 L2048
+// 142 -> 155, B32 H32 L512 272 -> 299; not filled, B3 H32 L1024 (288 workgroups) 93 -> 72, B16 H12 L448 (384) 49 -> 44, B2 H32
+// L2040 block 51 (320) all of the backward 516 -> 415; few workgroups, B2 H8 L1024 32.4 -> 22.7, B1 H8 L4096 108 -> 82.  At
+// head dim 64 three 64-key workgroups share a compute unit, and they lose only where long walks meet few workgroups:
+// B3 H32 L1024 65 -> 44, B2 H32 L2048 93 -> 93, B32 H32 L512 161 -> 149, but B1 H12 L4096 81 -> 86, B1 H8 L16384 618 -> 649.
+static bool dkdv_fills_the_chip(const BwdParams& p, int D) {
+  const int64_t heads = (int64_t)p.B * p.H, cus = cu_count(), n64 = heads * ((p.Lk + 63) / 64);
+  if (n64 <= 2 * cus) return false;
+  const int64_t wgs = heads * dkdv32_groups(p), rounds = (wgs + cus - 1) / cus;
+  const bool filled = 10 * wgs >= 9 * rounds * cus;
+  return D == 128 ? filled : p.Lk >= 2048 && (n64 <= 3 * cus || (filled && p.Lk > 8192));
+}
+
 template <class T, int D, int BS>
 static int launch_bwd_t(const BwdParams& p, int phases, hipStream_t stream) {
   int rc;
@@ -491,6 +506,8 @@ static int launch_bwd_t(const BwdParams& p, int phases, hipStream_t stream) {
       if (BS != 32) return LMK_ERR_UNSUPPORTED;
       return launch_bwd_dkdv32_handover(p, D, std::is_same<T, bf16_t>::value ? LMK_DTYPE_BF16 : LMK_DTYPE_F16, stream);
     }
+    if (BS != 32 && !dkdv_fills_the_chip(p, D))
+      return launch_bwd_dkdv_split(p, D, BS, std::is_same<T, bf16_t>::value ? LMK_DTYPE_BF16 : LMK_DTYPE_F16, stream);
     return launch_bwd_dkdv32(p, D, BS, std::is_same<T, bf16_t>::value ? LMK_DTYPE_BF16 : LMK_DTYPE_F16, stream);
   }
   return 0;

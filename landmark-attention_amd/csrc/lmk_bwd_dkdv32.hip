@@ -586,12 +586,7 @@ static int launch_dkdv32_t(const BwdParams& p, hipStream_t stream) {
   auto kern = lmk_bwd_dkdv32_kernel<T, D, BS, VIRT, SEG>;
   static std::atomic<uint64_t> lds_ok{0};
   if (int rc = allow_dynamic_lds(kern, C::LDS_BYTES, lds_ok)) return rc;
-  // workgroups per head: enough for about one workgroup per CU, at most four 128-key tiles each
-  const int64_t items = (int64_t)p.n_kvtiles * p.B * p.H;
-  int per_wg = (int)(items / cu_count());
-  per_wg = per_wg < 1 ? 1 : (per_wg > 4 ? 4 : per_wg);
-  const int groups = (p.n_kvtiles + per_wg - 1) / per_wg;
-  hipLaunchKernelGGL(kern, dim3(groups * p.B * p.H), dim3(C::NTHR), C::LDS_BYTES, stream, p);
+  hipLaunchKernelGGL(kern, dim3(dkdv32_groups(p) * p.B * p.H), dim3(C::NTHR), C::LDS_BYTES, stream, p);
   return (int)hipGetLastError();
 }
 

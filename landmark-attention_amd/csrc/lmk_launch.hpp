@@ -108,7 +108,7 @@ struct BwdParams {
   int64_t qs_b, qs_h, qs_r, ks_b, ks_h, ks_r, vs_b, vs_h, vs_r, os_b, os_h, os_r, dos_b, dos_h, dos_r;
   int64_t dqs_b, dqs_h, dqs_r, dks_b, dks_h, dks_r, dvs_b, dvs_h, dvs_r;
   float scale, scale_log2;
-  int b0, qt_top;                // as in FwdParams
+  int b0, qt_top, kt0;           // as in FwdParams; kt0: first unit of keys of a launch with 64 keys per workgroup
 };
 
 // phases: bit 0 = pre, bit 1 = dq, bit 2 = dkdv
@@ -116,7 +116,16 @@ int launch_bwd(const BwdParams& p, int D, int BS, int dtype, int phases, hipStre
 int launch_bwd_dq32(const BwdParams& p, int D, int dtype, hipStream_t stream);     // block 32 specialisation
 int launch_bwd_dq_split(const BwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // blocks 64 and 128, 64 rows a workgroup
 int launch_bwd_dkdv32(const BwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // two-role kernel, all block sizes
+int launch_bwd_dkdv_split(const BwdParams& p, int D, int BS, int dtype, hipStream_t stream);   // blocks 64 and 128, 64 keys a workgroup
 int launch_bwd_dkdv32_handover(const BwdParams& p, int D, int dtype, hipStream_t stream);  // block 32, dS read from p.ds_tiles
+
+// workgroups per head of lmk_bwd_dkdv32_kernel: enough for about one per CU, at most four 128-key tiles each
+inline int dkdv32_groups(const BwdParams& p) {
+  const int64_t items = (int64_t)p.n_kvtiles * p.B * p.H;
+  int per_wg = (int)(items / cu_count());
+  per_wg = per_wg < 1 ? 1 : (per_wg > 4 ? 4 : per_wg);
+  return (p.n_kvtiles + per_wg - 1) / per_wg;
+}
 
 // dS tiles (2 KB each) one (batch, head) leaves behind in the hand-over: query tile j sees key blocks 0 .. n_prefix + j
 __host__ __device__ inline int64_t handover_tiles_per_head(int64_t n_qtiles32, int64_t n_prefix) {

@@ -1,5 +1,5 @@
-"""The forward and dQ kernels whose waves split the keys of 64 query rows (blocks of 64 and 128 slots): both numbers of parts and the
-256-row kernel on the other side of the dispatch, at the edges of tiles, stages and blocks, against the fp32 oracle on
+"""The forward, dQ and dK/dV kernels with 64 rows per workgroup (blocks of 64 and 128 slots): both numbers of parts and the
+kernels on the other side of the dispatch, at the edges of tiles, stages and blocks, against the fp32 oracle on
 the same 16-bit inputs.  Heads are independent, so the first and the last stand for the rest.
 """
 import pytest
@@ -33,12 +33,14 @@ def test_forward_matches_the_oracle_on_every_side_of_the_dispatch(B, H, Lq, Lk, 
         assert (out[s] - want).abs().max() <= TOL
 
 
-# the backward's dQ kernels: the same two numbers of parts, and (last two) whole blocks of 64 with many long rows
+# the backward's kernels: the same two numbers of parts, and (last two) whole blocks of 64 with many long rows
 GRAD_CASES = [(1, 2, n * block, n * block, D, block) for D, block in ((128, 64), (64, 64), (128, 128), (64, 128), (128, 51), (64, 100))
               for n in (1, 2, 5)]
 GRAD_CASES += [(1, 2, 128, 128 + 3 * 64, 128, 64), (1, 1, 200, 1200, 64, 100)]
 GRAD_CASES += [(6, 50, 128, 128, 128, 64), (6, 50, 128, 256, 64, 128), (6, 50, 153, 153, 128, 51), (5, 60, 300, 300, 64, 100)]
 GRAD_CASES += [(2, 52, 1088, 1088, 128, 64), (2, 52, 1088, 1152, 64, 64)]
+# dK/dV with 128 keys per workgroup: whole rounds of compute units, long walks of few workgroups; a history of several blocks
+GRAD_CASES += [(4, 32, 512, 512, 128, 64), (1, 12, 4096, 4096, 64, 64), (1, 3, 256, 640, 128, 128)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
