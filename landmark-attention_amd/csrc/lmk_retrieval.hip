@@ -20,6 +20,7 @@
 //           their gather positions (:386-388, :408-410), local softmax per block gated by its
 //           landmark, and merge with the attention over the local chunk (computed by the fused
 //           forward kernel) through the shared global softmax bucket.
+#include <algorithm>
 #include "lmk_common.hpp"
 #include "lmk_landmark_keys.hpp"
 #include "lmk_launch.hpp"
@@ -712,6 +713,9 @@ __device__ __forceinline__ float sum8(float d) {                  // sum over th
 // The picked blocks of a row are read at p.idx[b * idx_sb + h * idx_sh + t * idx_st + 0 .. k-1] (selections shared
 // by the heads or by the queries have a zero stride there); a block counts among the k newest, whose keys sit one
 // block further on, by its age in the ring (p.ring_start = slot of the oldest block, 0 for a flat cache).
+// Most waves that share a row's blocks out beside its window's: with a block per wave no wave walks two of them one after
+// the other; blocks of 128 need the registers of fewer waves.
+constexpr int gather_waves(int BS) { return BS <= 64 ? 8 : 4; }
 template <int E> struct PieceVec;
 template <> struct PieceVec<8> { using type = u32x4_t; };
 template <> struct PieceVec<4> { using type = u32x2_t; };
@@ -723,17 +727,19 @@ template <> struct PieceVec<4> { using type = u32x2_t; };
 // softmax, instead of coming in as (o_loc, L_loc, M_loc) from a forward launch over a window another launch built:
 // a decode step is then the selection and this kernel.  Its keys join the global bucket directly (own-block rule:
 // causal, the landmark token does not see itself; flash_landmark_attention.py:78-100).
-// With SPLIT the window has a fifth wave of its own (blocks of 128 keep four waves, whose registers the kernel needs:
-// there the window goes to the wave next in turn behind the blocks).
+// With SPLIT the window has a wave of its own and every picked block, up to gather_waves(), as well (32 sequences of 32
+// heads, five blocks of 64 each: 71 -> 61 us for the step together with the chunks of 32 keys, whose registers leave
+// room for three waves per SIMD).
 template <class T, int D, int BS, bool SPLIT, bool PADDED, bool MERGE = false, bool LOCAL = false>
-__global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_gather_attend_kernel(RetrParams p) {
-  constexpr int NWV = (SPLIT && LOCAL && BS <= 64) ? 5 : 4;      // waves of a workgroup
+__global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256) void lmk_gather_attend_kernel(RetrParams p) {
+  const int nblk = SPLIT ? (int)(blockDim.x >> 6) - (LOCAL ? 1 : 0) : 1;   // waves that share the row's blocks out
+  constexpr int NWV = SPLIT ? (LOCAL ? gather_waves(BS) + 1 : 4) : 1;
   static_assert((D == 128 || D == 64) && (BS == 32 || BS % 64 == 0), "8 lanes x 2 pieces per row; whole chunks of keys");
   static_assert(!LOCAL || !PADDED, "the local window sits in a block of BS tokens");
   constexpr int E = D / 16;                                       // head dims per lane and rotary half: 8 or 4
   constexpr int PB = 2 * E;                                       // bytes of one piece
   using vec_t = typename PieceVec<E>::type;                       // one piece: E 16-bit values
-  constexpr int CK = BS < 64 ? BS : 64;                           // keys per chunk
+  constexpr int CK = BS == 32 || (BS == 64 && D == 128) ? 32 : 64;  // keys per chunk
   constexpr int KPG = CK / 8;                                     // keys per 8-lane group and chunk
   constexpr int NC = BS / CK;                                     // chunks per block
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -742,7 +748,7 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
   // selected blocks the four waves share out (block js goes to wave js % 4) and merge at the end
   const int64_t row = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
   if (row >= (int64_t)p.B * p.H * p.T) return;                    // SPLIT: the whole workgroup leaves
-  const int js0 = SPLIT ? (wave < 4 ? wave : p.k) : 0, jstep = SPLIT ? 4 : 1;   // (the window's wave takes no block)
+  const int js0 = SPLIT ? (wave < nblk ? wave : p.k) : 0, jstep = nblk;   // (the window's wave takes no block)
   const int bh = (int)(row / p.T), t = (int)(row % p.T);
   const int b = bh / p.H, hh = bh % p.H;
 
@@ -762,7 +768,7 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
   // The row's own key (without rotary) and value on their way into the cache: fetched here by one of the row's waves
   // (lanes 0 .. D/8-1 the key, 32 .. the value), stored at the end, so that nothing waits for them.  Nobody reads the
   // destination in this launch: it lies behind the cached rows.
-  const bool appends = LOCAL && p.ap_k != nullptr && (!SPLIT || wave == NWV - 1) && (lane & 31) < D / 8;
+  const bool appends = LOCAL && p.ap_k != nullptr && (!SPLIT || wave == nblk) && (lane & 31) < D / 8;
   u32x4_t ap = {0, 0, 0, 0};
   if (LOCAL && appends)
     ap = *(const u32x4_t*)((lane < 32 ? (const char*)p.ap_k + 2 * (b * p.aks_b + hh * p.aks_h + (int64_t)t * p.aks_r)
@@ -823,7 +829,7 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
     }
   };
   if constexpr (LOCAL) {
-    if (!SPLIT || wave == (NWV == 5 ? 4 : (p.k & 3))) {
+    if (!SPLIT || wave == nblk) {
       const int inc = p.local_inc, own = inc + t;                 // window rows: inc of the cache, then the new tokens
       const char* kn = (const char*)p.k_new + 2 * (b * p.kns_b + hh * p.kns_h);
       const char* vn = (const char*)p.v_new + 2 * (b * p.vns_b + hh * p.vns_h);
@@ -1018,17 +1024,16 @@ __global__ __launch_bounds__((SPLIT && LOCAL && BS <= 64) ? 320 : 256) void lmk_
     }
     __syncthreads();
     if (wave != 0) return;
+    const int nw = nblk + (LOCAL ? 1 : 0);
     float Mall = part_ml[0][0];                                   // wave 0 always has a block (k >= 1)
-#pragma unroll
-    for (int w = 1; w < NWV; ++w) Mall = fmaxf(Mall, part_ml[w][0]);
+    for (int w = 1; w < nw; ++w) Mall = fmaxf(Mall, part_ml[w][0]);
     lrun = 0.f;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       alo[e] = 0.f;
       ahi[e] = 0.f;
     }
-#pragma unroll
-    for (int w = 0; w < NWV; ++w) {
+    for (int w = 0; w < nw; ++w) {
       const float sw = fast_exp2(part_ml[w][0] - Mall);           // 0 for a wave without blocks (M = -inf)
       lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
 #pragma unroll
@@ -1220,10 +1225,10 @@ static int launch_gather_b(const RetrParams& p, hipStream_t stream) {
       const bool split = rows <= 1024 && p.k > 1;
       const dim3 grid((unsigned)(split ? rows : (rows + 3) / 4));
       if (p.merge_slices > 0) {
-        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, true, true>), grid, dim3(BS <= 64 ? 320 : 256), 0, stream, p);
+        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, true, true>), grid, dim3(64 * (std::min(p.k, gather_waves(BS)) + 1)), 0, stream, p);
         else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, true, true>), grid, dim3(256), 0, stream, p);
       } else {
-        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, false, true>), grid, dim3(BS <= 64 ? 320 : 256), 0, stream, p);
+        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, false, true>), grid, dim3(64 * (std::min(p.k, gather_waves(BS)) + 1)), 0, stream, p);
         else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, false, true>), grid, dim3(256), 0, stream, p);
       }
       return (int)hipGetLastError();
