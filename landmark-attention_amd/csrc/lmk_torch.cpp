@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <cmath>
@@ -67,6 +68,10 @@ auto without_gil(F&& f) {
   } release;
   return f();
 }
+
+// Calls that torch has to see as one operation: torch.jit.trace would record no more of what is done here than the
+// allocation of the outputs.  Such a call is left to an autograd Function, in Python.
+bool left_to_a_function() { return torch::jit::tracer::isTracing(); }
 
 // ---- what the kernels take
 int dtype_code(const Tensor& t) {
@@ -316,30 +321,37 @@ struct RotaryBackward : public torch::autograd::Node {
   }
 };
 
-// apply_rotary_pos_emb; q undefined or of k's shape
-std::pair<Tensor, Tensor> rotary(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const Tensor& pos_in) {
-  need(k.dim() == 4 && k.is_cuda() && dtype_code(k) >= 0, "k is (batch, heads, rows, head dim), bf16 or fp16, on the GPU");
-  need(!q.defined() || (q.scalar_type() == k.scalar_type() && q.device() == k.device()), "q and k must have one type and device");
-  need(pos_in.dim() == 2 && pos_in.size(1) == k.size(2) && (pos_in.size(0) == 1 || pos_in.size(0) == k.size(0)),
-       "position_ids is (1, rows) or (batch, rows)");
-  need(pos_in.scalar_type() == at::kLong && pos_in.device() == k.device(), "position_ids is int64 on k's device");
-  c10::DeviceGuard device(k.device());
-  const bool has_q = q.defined();
+struct RotaryArgs {
   Tables t;
   Tensor pos;
+};
+// What rotate() takes besides the rows x, checked and laid out as the kernel reads it.
+RotaryArgs rotary_args(const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& pos) {
+  need(x.dim() == 4 && x.is_cuda() && dtype_code(x) >= 0, "k is (batch, heads, rows, head dim), bf16 or fp16, on the GPU");
+  need(pos.dim() == 2 && pos.size(1) == x.size(2) && (pos.size(0) == 1 || pos.size(0) == x.size(0)),
+       "position_ids is (1, rows) or (batch, rows)");
+  need(pos.scalar_type() == at::kLong && pos.device() == x.device(), "position_ids is int64 on k's device");
+  return {tables(cos, sin, x.scalar_type()), pos.contiguous()};
+}
+
+// apply_rotary_pos_emb; q undefined or of k's shape
+std::pair<Tensor, Tensor> rotary(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, const Tensor& pos) {
+  need(!q.defined() || (q.scalar_type() == k.scalar_type() && q.device() == k.device()), "q and k must have one type and device");
+  c10::DeviceGuard device(k.device());
+  const bool has_q = q.defined();
+  RotaryArgs a;
   std::pair<Tensor, Tensor> r;
   {
     at::AutoDispatchBelowADInplaceOrView guard;
-    t = tables(cos, sin, k.scalar_type());
-    pos = pos_in.contiguous();
-    r = rotate(q, k, t, pos, false);
+    a = rotary_args(k, cos, sin, pos);
+    r = rotate(q, k, a.t, a.pos, false);
   }
   if (at::GradMode::is_enabled() && (k.requires_grad() || (has_q && q.requires_grad()))) {
     auto node = std::shared_ptr<RotaryBackward>(new RotaryBackward(), torch::autograd::deleteNode);
     node->set_next_edges(has_q ? torch::autograd::collect_next_edges(q, k) : torch::autograd::collect_next_edges(k));
-    node->cos = SavedVariable(t.cos, false);
-    node->sin = SavedVariable(t.sin, false);
-    node->pos = SavedVariable(pos, false);
+    node->cos = SavedVariable(a.t.cos, false);
+    node->sin = SavedVariable(a.t.sin, false);
+    node->pos = SavedVariable(a.pos, false);
     node->has_q = has_q;
     if (has_q) torch::autograd::set_history(r.first, node);
     torch::autograd::set_history(r.second, node);
@@ -543,7 +555,8 @@ PyObject* py_set_error_class(PyObject*, PyObject* cls) {
   Py_RETURN_NONE;
 }
 
-// attention(q, k, v, group_scale | None, sm_scale | None, block, handover_max_bytes, handover_min_keys) -> out
+// attention(q, k, v, group_scale | None, sm_scale | None, block, handover_max_bytes, handover_min_keys) -> out, or None for
+// a call that an autograd Function has to make
 PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     count(n, 8);
@@ -552,6 +565,7 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const double scale = has_scale ? float_arg(a[4]) : 0.0;
     const int64_t block = int_arg(a[5]);
     const HandoverLimits limits = {int_arg(a[6]), int_arg(a[7])};
+    if (left_to_a_function()) Py_RETURN_NONE;
     return THPVariable_Wrap(without_gil([&] { return attention(q, k, v, gs, has_scale, scale, block, limits); }));
   });
 }
@@ -593,13 +607,29 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// rotary(q | None, k, cos, sin, position_ids) -> (q_embed | None, k_embed)
+// rotary(q | None, k, cos, sin, position_ids) -> (q_embed | None, k_embed), or None for a call that an autograd Function
+// has to make
 PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     count(n, 5);
     const Tensor q = tensor_arg(a[0]), k = tensor_arg(a[1]), cos = tensor_arg(a[2]), sin = tensor_arg(a[3]), pos = tensor_arg(a[4]);
+    if (left_to_a_function()) Py_RETURN_NONE;
     const auto r = without_gil([&] { return rotary(q, k, cos, sin, pos); });
     return tuple_of({r.first, r.second});
+  });
+}
+
+// rotate(x, cos, sin, position_ids) -> x_embed: the launch alone, without autograd
+PyObject* py_rotate(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    count(n, 4);
+    const Tensor x = tensor_arg(a[0]), cos = tensor_arg(a[1]), sin = tensor_arg(a[2]), pos = tensor_arg(a[3]);
+    return THPVariable_Wrap(without_gil([&] {
+      at::AutoDispatchBelowADInplaceOrView guard;
+      c10::DeviceGuard device(x.device());
+      const RotaryArgs r = rotary_args(x, cos, sin, pos);
+      return rotate(Tensor(), x, r.t, r.pos, false).second;
+    }));
   });
 }
 
@@ -722,6 +752,7 @@ PyMethodDef g_methods[] = {
     {"attn_fwd", LMK_FAST(py_attn_fwd)},
     {"attn_bwd", LMK_FAST(py_attn_bwd)},
     {"rotary", LMK_FAST(py_rotary)},
+    {"rotate", LMK_FAST(py_rotate)},
     {"mem_cache_step", LMK_FAST(py_mem_cache_step)},
     {"retrieve_workspace_bytes", LMK_FAST(py_retrieve_workspace_bytes)},
     {"cache_append", LMK_FAST(py_cache_append)},

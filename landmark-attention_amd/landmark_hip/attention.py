@@ -311,7 +311,17 @@ def fused_landmark_attention(q, k, v, is_mem, sm_scale=None, block_size=64, grou
     if group_scale is None:
         storage_block(block_size)               # ValueError for block sizes the kernels do not cover
     # the same as FusedLandmarkAttention(GroupScale).apply, with a backward node that needs no interpreter
-    return _lib.native().attention(q, k, v, group_scale, sm_scale, block_size, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
+    out = _lib.native().attention(q, k, v, group_scale, sm_scale, block_size, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
+    if out is not None:
+        return out
+    # under torch.jit.trace: the Function, which the tracer records as an operation
+    n_history = k.shape[-2] - q.shape[-2]
+    assert n_history % block_size == 0
+    if sm_scale is None:
+        sm_scale = 1.0 / math.sqrt(d)
+    if group_scale is None:
+        return FusedLandmarkAttention.apply(q, k, v, n_history // block_size, sm_scale, block_size)
+    return FusedLandmarkAttentionGroupScale.apply(q, k, v, group_scale, n_history // block_size, sm_scale, block_size)
 
 
 def fused_landmark_attention_rotary_q(q, k, v, cos, sin, position_ids, is_mem=None, sm_scale=None, block_size=64):

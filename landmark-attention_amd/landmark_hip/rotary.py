@@ -24,12 +24,29 @@ def _transposed_sin(sin):
     return (-torch.cat((sin[..., h:], sin[..., :h]), dim=-1)).contiguous()
 
 
+class _Rotary(torch.autograd.Function):
+    """The rotation of one tensor as an operation torch can record; the backward is the transposed rotation."""
+
+    @staticmethod
+    def forward(ctx, x, cos, sin, position_ids):
+        ctx.save_for_backward(cos, sin, position_ids)
+        return _lib.native().rotate(x, cos, sin, position_ids)
+
+    @staticmethod
+    def backward(ctx, dy):
+        cos, sin, position_ids = ctx.saved_tensors
+        return _lib.native().rotate(dy, cos, _transposed_sin(sin), position_ids), None, None, None
+
+
 def apply_rotary_pos_emb(q, k, cos, sin, position_ids):
     """``(q_embed, k_embed)`` as ``llama_mem.py:134-149`` returns them; ``q_embed`` is ``None`` when
     ``q`` is.  q, k: ``(B, nh, L, hd)`` bf16/fp16 on the GPU with hd 64 or 128.  Differentiable in q and k,
     as the reference's expression is (the tables and positions get no gradient): the backward is the transposed
     rotation (``_transposed_sin``), for which the kernel reads the sine table in place."""
-    rotary = _lib.native().rotary
     if q is not None and q.shape != k.shape:    # e.g. fewer key heads: one launch per tensor
-        return rotary(None, q, cos, sin, position_ids)[1], rotary(None, k, cos, sin, position_ids)[1]
-    return rotary(q, k, cos, sin, position_ids)
+        return tuple(apply_rotary_pos_emb(None, x, cos, sin, position_ids)[1] for x in (q, k))
+    rotated = _lib.native().rotary(q, k, cos, sin, position_ids)
+    if rotated is not None:
+        return rotated
+    # under torch.jit.trace: a Function per tensor, which the tracer records as an operation
+    return None if q is None else _Rotary.apply(q, cos, sin, position_ids), _Rotary.apply(k, cos, sin, position_ids)

@@ -1,0 +1,65 @@
+"""The shim's native host path under the parts of torch that have to see a call as one operation of its own: what an
+autograd Function is given (a tracer's record, a refusal of forward-mode gradients, zeros for outputs without a
+gradient, saved tensors as they were) holds for the C++ nodes too."""
+import pytest
+import torch
+
+from oracle import rotary as orot
+from tests.util import make_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+def _attention_args(B, H, Lq, Lk, D, block, seed, dropout=False):
+    q, k, v = (t.cuda() for t in make_qkv(B, H, Lq, Lk, D, seed=seed))
+    g = torch.Generator().manual_seed(seed)
+    factors = (torch.rand(B, H, Lk // block, Lq, generator=g) >= 0.5).float().mul(2.0).cuda() if dropout else None
+    return q, k, v, factors
+
+
+def _rotary_args(B, H, L, D, seed):
+    q, k, _ = (t.cuda() for t in make_qkv(B, H, L, L, D, seed=seed))
+    cos, sin = (t.cuda() for t in orot.rotary_tables(2 * L, D, torch.bfloat16))
+    return q, k, cos, sin, torch.arange(3, 3 + L, device="cuda")[None]
+
+
+@pytest.mark.parametrize("D,block,dropout", [(128, 32, False), (64, 51, False), (32, 64, False), (64, 51, True)])
+def test_a_traced_attention_computes_on_the_inputs_of_each_call(D, block, dropout):
+    from ltriton.flash_landmark_attention import fused_landmark_attention
+    print(f"case trace attention D{D} bs{block} dropout{dropout}", flush=True)
+    f = (lambda q, k, v, gs: fused_landmark_attention(q, k, v, None, block_size=block, group_scale=gs)) if dropout else \
+        (lambda q, k, v: fused_landmark_attention(q, k, v, None, block_size=block))
+    args = [[t for t in _attention_args(1, 2, L, L + n * block, D, block, seed, dropout) if t is not None]
+            for seed, (L, n) in enumerate([(4 * block, 0), (4 * block, 0), (2 * block, 3)])]       # other lengths, a history
+    traced = torch.jit.trace(f, args[0])
+    for a in args:
+        leaves = [t.detach().requires_grad_(i < 3) for i, t in enumerate(a)]
+        want, got = f(*leaves), traced(*leaves)
+        assert torch.equal(got, want)
+        do = torch.ones_like(want)
+        for x, y in zip(torch.autograd.grad(got, leaves[:3], do), torch.autograd.grad(want, leaves[:3], do)):
+            assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("shapes", ["q and k", "k alone", "fewer key heads"])
+def test_a_traced_rotary_computes_on_the_inputs_of_each_call(shapes):
+    from landmark_hip.rotary import apply_rotary_pos_emb
+    print(f"case trace rotary {shapes}", flush=True)
+
+    def f(q, k, cos, sin, pos):
+        q_embed, k_embed = apply_rotary_pos_emb(None if shapes == "k alone" else q, k, cos, sin, pos)
+        return k_embed if q_embed is None else (q_embed, k_embed)
+
+    args = [list(_rotary_args(2, 4, L, 64, seed)) for seed, L in enumerate([40, 40, 23])]
+    for a in args:
+        a[1] = a[1][:, :2].contiguous() if shapes == "fewer key heads" else a[1]
+    traced = torch.jit.trace(f, args[0])
+    for a in args:
+        leaves = [t.detach().requires_grad_(i < 2) for i, t in enumerate(a)]
+        used = leaves[1:2] if shapes == "k alone" else leaves[:2]
+        outs = [f(*leaves), traced(*leaves)]
+        grads = []
+        for out in outs:
+            out = out if isinstance(out, tuple) else (out,)
+            grads.append(torch.autograd.grad(out, used, [torch.sin(o.detach().float()).bfloat16() for o in out]) + out)
+        assert all(torch.equal(x, y) for x, y in zip(*grads))
