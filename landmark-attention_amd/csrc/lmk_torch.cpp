@@ -70,8 +70,14 @@ auto without_gil(F&& f) {
 }
 
 // Calls that torch has to see as one operation: torch.jit.trace would record no more of what is done here than the
-// allocation of the outputs.  Such a call is left to an autograd Function, in Python.
-bool left_to_a_function() { return torch::jit::tracer::isTracing(); }
+// allocation of the outputs, and a forward-mode gradient of an input would be lost where a Function without a jvp refuses
+// it.  Such a call is left to an autograd Function, in Python.
+bool left_to_a_function(std::initializer_list<Tensor> inputs) {
+  if (torch::jit::tracer::isTracing()) return true;
+  for (const Tensor& t : inputs)
+    if (t.defined() && t._fw_grad(/*level=*/0).defined()) return true;
+  return false;
+}
 
 // ---- what the kernels take
 int dtype_code(const Tensor& t) {
@@ -565,7 +571,7 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const double scale = has_scale ? float_arg(a[4]) : 0.0;
     const int64_t block = int_arg(a[5]);
     const HandoverLimits limits = {int_arg(a[6]), int_arg(a[7])};
-    if (left_to_a_function()) Py_RETURN_NONE;
+    if (left_to_a_function({q, k, v, gs})) Py_RETURN_NONE;
     return THPVariable_Wrap(without_gil([&] { return attention(q, k, v, gs, has_scale, scale, block, limits); }));
   });
 }
@@ -613,7 +619,7 @@ PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     count(n, 5);
     const Tensor q = tensor_arg(a[0]), k = tensor_arg(a[1]), cos = tensor_arg(a[2]), sin = tensor_arg(a[3]), pos = tensor_arg(a[4]);
-    if (left_to_a_function()) Py_RETURN_NONE;
+    if (left_to_a_function({q, k, cos, sin})) Py_RETURN_NONE;
     const auto r = without_gil([&] { return rotary(q, k, cos, sin, pos); });
     return tuple_of({r.first, r.second});
   });

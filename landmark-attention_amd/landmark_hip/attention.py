@@ -314,7 +314,7 @@ def fused_landmark_attention(q, k, v, is_mem, sm_scale=None, block_size=64, grou
     out = _lib.native().attention(q, k, v, group_scale, sm_scale, block_size, HANDOVER_MAX_BYTES, HANDOVER_MIN_KEYS)
     if out is not None:
         return out
-    # under torch.jit.trace: the Function, which the tracer records as an operation
+    # under torch.jit.trace, which records the Function as an operation, or with a forward-mode gradient, which it refuses
     n_history = k.shape[-2] - q.shape[-2]
     assert n_history % block_size == 0
     if sm_scale is None:

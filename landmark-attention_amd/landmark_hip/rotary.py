@@ -48,5 +48,6 @@ def apply_rotary_pos_emb(q, k, cos, sin, position_ids):
     rotated = _lib.native().rotary(q, k, cos, sin, position_ids)
     if rotated is not None:
         return rotated
-    # under torch.jit.trace: a Function per tensor, which the tracer records as an operation
+    # under torch.jit.trace, which records a Function (one per tensor) as an operation, or with forward-mode gradients, which
+    # it refuses
     return None if q is None else _Rotary.apply(q, cos, sin, position_ids), _Rotary.apply(k, cos, sin, position_ids)

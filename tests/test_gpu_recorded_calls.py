@@ -63,3 +63,37 @@ def test_a_traced_rotary_computes_on_the_inputs_of_each_call(shapes):
             out = out if isinstance(out, tuple) else (out,)
             grads.append(torch.autograd.grad(out, used, [torch.sin(o.detach().float()).bfloat16() for o in out]) + out)
         assert all(torch.equal(x, y) for x, y in zip(*grads))
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "group factors", "none"])
+def test_attention_refuses_forward_mode_gradients(which):
+    import torch.autograd.forward_ad as fw
+    from ltriton.flash_landmark_attention import fused_landmark_attention
+    args = dict(zip(["q", "k", "v", "group factors"], _attention_args(1, 2, 96, 96, 64, 32, 5, dropout=which == "group factors")))
+    call = lambda: fused_landmark_attention(args["q"], args["k"], args["v"], None, block_size=32, group_scale=args["group factors"])
+    want = call()
+    with fw.dual_level():
+        if which == "none":                                   # a dual level by itself changes nothing
+            assert torch.equal(call(), want)
+            return
+        args[which] = fw.make_dual(args[which], torch.ones_like(args[which]))
+        with pytest.raises(NotImplementedError):
+            call()
+
+
+@pytest.mark.parametrize("which", [0, 1, 2, 3, None])
+def test_rotary_refuses_forward_mode_gradients(which):
+    import torch.autograd.forward_ad as fw
+    from landmark_hip.rotary import apply_rotary_pos_emb
+    args = list(_rotary_args(1, 2, 33, 64, 6))
+    want = apply_rotary_pos_emb(*args)
+    with fw.dual_level():
+        if which is None:
+            assert all(torch.equal(a, b) for a, b in zip(apply_rotary_pos_emb(*args), want))
+            return
+        args[which] = fw.make_dual(args[which], torch.ones_like(args[which]))
+        with pytest.raises(NotImplementedError):
+            apply_rotary_pos_emb(*args)
+        if which == 1:
+            with pytest.raises(NotImplementedError):
+                apply_rotary_pos_emb(None, *args[1:])
