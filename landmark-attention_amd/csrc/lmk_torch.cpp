@@ -715,6 +715,9 @@ PyObject* py_ring_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int tail = (int)int_arg(a[8]), next = (int)int_arg(a[9]);
     without_gil([&] {
       const Tensor &rk = t[6], &rv = t[7];
+      for (const Tensor& x : t)                          // one kernel reads and writes them all
+        need(x.defined() && x.device() == rk.device(), "keys, values and is_mem must be on the cache's device");
+      need(rk.is_cuda(), "the cache must be on the GPU");
       need(t[0].dim() == 4 && same_shape(t[0], t[1]) && t[0].size(0) <= rk.size(0) && t[0].size(1) == rk.size(3) &&
                t[0].size(3) == rk.size(4) && same_shape(rk, rv) && rk.strides() == rv.strides(),
            "keys and values must have one shape, and the cache's heads and head dim");

@@ -112,11 +112,11 @@ class MemLMCacheStorage:
         self._tail_regular = rest == 0 or not bool(is_mem[:, full:].any())
 
     def _continues_the_stream(self, keys, values, is_mem, offset, block) -> bool:
-        """Whether the chunk can be stored as it is: rows the kernel copies, marks that put a landmark at the end of
-        every block and nowhere else."""
-        if not (keys.is_cuda and values.is_cuda and is_mem.is_cuda and is_mem.dtype == torch.bool and is_mem.dim() == 2
-                and self.cache_mem_k.dtype in _lib.DTYPE_CODES and self.cache_mem_k.is_cuda and keys.shape[2] > 0
-                and self.cache_mem_k.shape[4] % 8 == 0):
+        """Whether the chunk can be stored as it is: rows on the cache's GPU, which the kernel copies, marks that put a
+        landmark at the end of every block and nowhere else."""
+        ring = self.cache_mem_k
+        if not (ring.is_cuda and keys.device == values.device == is_mem.device == ring.device and is_mem.dtype == torch.bool
+                and is_mem.dim() == 2 and ring.dtype in _lib.DTYPE_CODES and keys.shape[2] > 0 and ring.shape[4] % 8 == 0):
             return False
         from .attention import _check_is_mem
         try:
