@@ -87,6 +87,8 @@ class MemLMCacheStorage:
         _, nh, total, hs = k.shape
         rest = total % bs
         full = total - rest
+        # the new tail's own state: it is there also when the blocks in front of it are refused below
+        self._tail_regular = rest == 0 or not bool(is_mem[:, full:].any())
         self.last_incomplete_k[:B, :, :rest] = k[:, :, full:]
         self.last_incomplete_v[:B, :, :rest] = v[:, :, full:]
         self.last_incomplete_ismem[:B, :rest] = is_mem[:, full:]
@@ -109,7 +111,6 @@ class MemLMCacheStorage:
         self.cache_mem_v[:B, :kept - first] = vb[:, first:]
         self.cache_iter = (start + kept) % cap if start + kept >= cap else start + kept
         self.cache_size += n_new
-        self._tail_regular = rest == 0 or not bool(is_mem[:, full:].any())
 
     def _continues_the_stream(self, keys, values, is_mem, offset, block) -> bool:
         """Whether the chunk can be stored as it is: rows on the cache's GPU, which the kernel copies, marks that put a

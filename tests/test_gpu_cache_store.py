@@ -62,3 +62,14 @@ def test_append_by_kernel_equals_slices(D):
         cache.append(k, v)
     pk, pv = cache.past_key_value
     assert torch.equal(pk, torch.cat(ks, 2)) and torch.equal(pv, torch.cat(vs, 2))
+
+
+def test_a_store_behind_a_refused_one_looks_at_the_tail_it_left():
+    from landmark_hip.mem_cache import MemLMCacheStorage
+    s = MemLMCacheStorage(1, 4, 3, 2, 64, dtype=torch.float16, device="cuda")
+    x = torch.zeros(1, 2, 6, 64, dtype=torch.float16, device="cuda")
+    marks = torch.tensor([[False, True, False, True, True, False]], device="cuda")       # the tail opens with a landmark
+    with pytest.raises(AssertionError):
+        s.store_in_cache(x, {"v": x, "is_mem": marks})
+    with pytest.raises(AssertionError):
+        s.store_in_cache(x[:, :, :2], {"v": x[:, :, :2], "is_mem": torch.tensor([[False, True]], device="cuda")})

@@ -39,3 +39,17 @@ def test_the_native_store_refuses_tensors_of_several_devices(elsewhere):
         _lib.native().ring_store(*args, 0, 0)
     with pytest.raises(AssertionError, match="GPU"):                               # one device, but the CPU
         _lib.native().ring_store(*(t.to("cpu") if t.is_cpu else torch.zeros(t.shape, dtype=t.dtype) for t in args), 0, 0)
+
+
+def test_a_refused_store_does_not_leave_its_tail_to_the_path_that_does_not_look_at_it(monkeypatch):
+    from landmark_hip import _lib
+    s = _storage()
+    x = torch.zeros(1, 2, 6, 8, dtype=torch.bfloat16)
+    marks = torch.tensor([[False, True, False, True, True, False]])       # a landmark too many; then the tail opens with one
+    with pytest.raises(AssertionError):
+        s.store_in_cache(x, {"v": x, "is_mem": marks})
+    # the chunk by itself continues the stream, as _check_is_mem would find on the GPU
+    monkeypatch.setattr(s, "_continues_the_stream", lambda *a: True)
+    monkeypatch.setattr(_lib, "native", lambda: pytest.fail("stored without a look at the tail"))
+    with pytest.raises(AssertionError, match="every block"):
+        s.store_in_cache(x[:, :, :2], {"v": x[:, :, :2], "is_mem": torch.tensor([[False, True]])})
