@@ -194,15 +194,16 @@ struct AttentionBackward : public torch::autograd::Node {
   HandoverLimits limits;
 
   variable_list apply(variable_list&& grads) override {
-    if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
     return node_body([&] {
+      // an output that no gradient reaches: zeros, as an autograd Function is given
+      const Tensor dout = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
       need(s.Lq % s.block_real == 0 && s.Lk % s.block_real == 0, "Backward supported only for full blocks");
       const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(getptr()), st_ = st.unpack();
       const Tensor gs_ = has_gs ? gs.unpack() : Tensor();
       at::AutoDispatchBelowADInplaceOrView guard;
       c10::DeviceGuard device(q_.device());
       const float* L = st_.data_ptr<float>();
-      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(grads[0]), gs_);
+      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(dout), gs_);
     });
   }
   std::string name() const override { return "FusedLandmarkAttentionBackward"; }

@@ -97,3 +97,26 @@ def test_rotary_refuses_forward_mode_gradients(which):
         if which == 1:
             with pytest.raises(NotImplementedError):
                 apply_rotary_pos_emb(None, *args[1:])
+
+
+class _NoGradient(torch.autograd.Function):
+    """Hands its input on and no gradient back."""
+
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, dy):
+        return None
+
+
+@pytest.mark.parametrize("D,block,dropout", [(128, 32, False), (64, 51, True)])
+def test_an_output_that_no_gradient_reaches_gives_zero_gradients(D, block, dropout):
+    # as the reference's Function does, whose backward is handed zeros (flash_landmark_attention.py:356-389)
+    from ltriton.flash_landmark_attention import fused_landmark_attention
+    q, k, v, factors = _attention_args(1, 2, 2 * block, 4 * block, D, block, 7, dropout)
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    out = fused_landmark_attention(*leaves, None, block_size=block, group_scale=factors)
+    for x, g in zip(leaves, torch.autograd.grad(_NoGradient.apply(out).float().sum(), leaves)):
+        assert g.shape == x.shape and g.dtype == x.dtype and not g.any()
