@@ -89,6 +89,7 @@ int dtype_code(const Tensor& t) {
 }
 lmk_tensor4 t4(const Tensor& t) {
   const auto s = t.strides();
+  need(s.size() == 4 && s[3] == 1, "a tensor of four dimensions, the last one dense");
   return lmk_tensor4{t.data_ptr(), s[0], s[1], s[2]};
 }
 // Tensors the kernels can read in place (unit stride along D, rows walked forwards, 16-byte aligned) as they are,
@@ -187,8 +188,26 @@ variable_list node_body(F&& f) {
   }
 }
 
+// A tensor saved for the backward.  Saved-tensor hooks may hand back any other in its place: one that is not what was saved
+// is refused before a kernel is given its address.
+struct Saved {
+  SavedVariable x;
+  at::DimVector shape;
+  at::ScalarType type = at::kFloat;
+  at::Device device = at::kCPU;
+
+  Saved() = default;
+  Saved(const Tensor& t, bool is_output) : x(t, is_output), shape(t.sizes()), type(t.scalar_type()), device(t.device()) {}
+  Tensor unpack(std::shared_ptr<torch::autograd::Node> saved_for = nullptr) const {
+    Tensor t = x.unpack(std::move(saved_for));
+    need(t.defined() && t.sizes() == shape && t.scalar_type() == type && t.device() == device,
+         "saved-tensor hooks must hand back the shape, type and device that were saved");
+    return t;
+  }
+};
+
 struct AttentionBackward : public torch::autograd::Node {
-  SavedVariable q, k, v, o, st, gs;
+  Saved q, k, v, o, st, gs;
   bool has_gs = false;
   Shape s;
   HandoverLimits limits;
@@ -202,13 +221,14 @@ struct AttentionBackward : public torch::autograd::Node {
       const Tensor gs_ = has_gs ? gs.unpack() : Tensor();
       at::AutoDispatchBelowADInplaceOrView guard;
       c10::DeviceGuard device(q_.device());
-      const float* L = st_.data_ptr<float>();
-      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(dout), gs_);
+      const Tensor stats = st_.contiguous();
+      const float* L = stats.data_ptr<float>();
+      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(dout), has_gs ? gs_.contiguous() : gs_);
     });
   }
   std::string name() const override { return "FusedLandmarkAttentionBackward"; }
   void release_variables() override {
-    for (SavedVariable* x : {&q, &k, &v, &o, &st, &gs}) x->reset_data();
+    for (Saved* s : {&q, &k, &v, &o, &st, &gs}) s->x.reset_data();
   }
 };
 
@@ -253,16 +273,16 @@ Tensor attention(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, con
     auto node = std::shared_ptr<AttentionBackward>(new AttentionBackward(), torch::autograd::deleteNode);
     node->set_next_edges(torch::autograd::collect_next_edges(q_in, k_in, v_in));
     // a tensor that was copied into kernel layout is saved as that copy, and has no history of its own
-    node->q = SavedVariable(q, false);
-    node->k = SavedVariable(k, false);
-    node->v = SavedVariable(v, false);
-    node->st = SavedVariable(r.second, false);
+    node->q = Saved(q, false);
+    node->k = Saved(k, false);
+    node->v = Saved(v, false);
+    node->st = Saved(r.second, false);
     node->has_gs = has_gs;
-    if (has_gs) node->gs = SavedVariable(gs, false);
+    if (has_gs) node->gs = Saved(gs, false);
     node->s = s;
     node->limits = limits;
     torch::autograd::set_history(r.first, node);
-    node->o = SavedVariable(r.first, true);
+    node->o = Saved(r.first, true);
   }
   return r.first;
 }
@@ -304,34 +324,34 @@ std::pair<Tensor, Tensor> rotate(const Tensor& q_in, const Tensor& k_in, const T
   return {qo, ko};
 }
 
+struct RotaryArgs {
+  Tables t;
+  Tensor pos;
+};
 struct RotaryBackward : public torch::autograd::Node {
-  SavedVariable cos, sin, pos;
+  Saved cos, sin, pos;
   bool has_q = false;
 
   variable_list apply(variable_list&& grads) override {
     return node_body([&]() -> variable_list {
+      const Tensor cos_ = cos.unpack(), sin_ = sin.unpack(), pos_ = pos.unpack();
       at::AutoDispatchBelowADInplaceOrView guard;
-      const Tables t = {cos.unpack(), sin.unpack()};
-      const Tensor pos_ = pos.unpack();
+      const RotaryArgs args = {tables(cos_, sin_, cos_.scalar_type()), pos_.contiguous()};
       const Tensor &gk = grads[has_q ? 1 : 0], gq = has_q ? grads[0] : Tensor();
       if (!gk.defined() && !gq.defined()) return has_q ? variable_list{Tensor(), Tensor()} : variable_list{Tensor()};
       c10::DeviceGuard device((gk.defined() ? gk : gq).device());
-      if (!has_q) return {rotate(Tensor(), gk, t, pos_, true).second};
-      if (!gk.defined()) return {rotate(Tensor(), gq, t, pos_, true).second, Tensor()};
-      auto r = rotate(gq, gk, t, pos_, true);
+      if (!has_q) return {rotate(Tensor(), gk, args.t, args.pos, true).second};
+      if (!gk.defined()) return {rotate(Tensor(), gq, args.t, args.pos, true).second, Tensor()};
+      auto r = rotate(gq, gk, args.t, args.pos, true);
       return {r.first, r.second};
     });
   }
   std::string name() const override { return "RotaryEmbeddingBackward"; }
   void release_variables() override {
-    for (SavedVariable* x : {&cos, &sin, &pos}) x->reset_data();
+    for (Saved* s : {&cos, &sin, &pos}) s->x.reset_data();
   }
 };
 
-struct RotaryArgs {
-  Tables t;
-  Tensor pos;
-};
 // What rotate() takes besides the rows x, checked and laid out as the kernel reads it.
 RotaryArgs rotary_args(const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& pos) {
   need(x.dim() == 4 && x.is_cuda() && dtype_code(x) >= 0, "k is (batch, heads, rows, head dim), bf16 or fp16, on the GPU");
@@ -356,9 +376,9 @@ std::pair<Tensor, Tensor> rotary(const Tensor& q, const Tensor& k, const Tensor&
   if (at::GradMode::is_enabled() && (k.requires_grad() || (has_q && q.requires_grad()))) {
     auto node = std::shared_ptr<RotaryBackward>(new RotaryBackward(), torch::autograd::deleteNode);
     node->set_next_edges(has_q ? torch::autograd::collect_next_edges(q, k) : torch::autograd::collect_next_edges(k));
-    node->cos = SavedVariable(a.t.cos, false);
-    node->sin = SavedVariable(a.t.sin, false);
-    node->pos = SavedVariable(a.pos, false);
+    node->cos = Saved(a.t.cos, false);
+    node->sin = Saved(a.t.sin, false);
+    node->pos = Saved(a.pos, false);
     node->has_q = has_q;
     if (has_q) torch::autograd::set_history(r.first, node);
     torch::autograd::set_history(r.second, node);

@@ -120,3 +120,49 @@ def test_an_output_that_no_gradient_reaches_gives_zero_gradients(D, block, dropo
     out = fused_landmark_attention(*leaves, None, block_size=block, group_scale=factors)
     for x, g in zip(leaves, torch.autograd.grad(_NoGradient.apply(out).float().sum(), leaves)):
         assert g.shape == x.shape and g.dtype == x.dtype and not g.any()
+
+
+def _unpacked_as(change):
+    return torch.autograd.graph.saved_tensors_hooks(lambda t: t, change)
+
+
+_LAYOUTS = {
+    "contiguous copies": lambda t: t.clone(memory_format=torch.contiguous_format),
+    "rows apart": lambda t: torch.cat((t, t), dim=-1)[..., : t.shape[-1]],
+    "through the host": lambda t: t.cpu().cuda(),
+}
+_NOT_AS_SAVED = {
+    "another type": lambda t: t.half(),
+    "wider": lambda t: t.float(),
+    "last dim not dense": lambda t: torch.stack((t, t), dim=-1)[..., 0],
+    "fewer rows": lambda t: t[..., : t.shape[-2] - 1, :],
+    "on the host": lambda t: t.cpu(),
+}
+
+
+@pytest.mark.parametrize("how", [*_LAYOUTS, *_NOT_AS_SAVED])
+@pytest.mark.parametrize("what", ["attention", "attention with factors", "rotary"])
+def test_what_saved_tensor_hooks_hand_back_is_used_or_refused(what, how):
+    # the kernels take a pointer, a type and strides: a hook's tensor is used when it is what was saved, in any layout they
+    # read, and refused on the host otherwise
+    from landmark_hip.rotary import apply_rotary_pos_emb
+    from ltriton.flash_landmark_attention import fused_landmark_attention
+    print(f"case hooks {what}: {how}", flush=True)
+    if what == "rotary":
+        q, k, *tables = _rotary_args(2, 3, 40, 64, 8)
+        leaves = [t.requires_grad_(True) for t in (q, k)]
+        call = lambda: torch.stack(apply_rotary_pos_emb(*leaves, *tables))
+    else:
+        q, k, v, factors = _attention_args(2, 2, 102, 153, 64, 51, 8, what != "attention")
+        leaves = [t.transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(True) for t in (q, k, v)]
+        call = lambda: fused_landmark_attention(*leaves, None, block_size=51, group_scale=factors)
+    do = torch.randn(call().shape, generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    want = torch.autograd.grad(call(), leaves, do)
+    with _unpacked_as((_LAYOUTS | _NOT_AS_SAVED)[how]):
+        out = call()
+    if how in _LAYOUTS:
+        for x, y in zip(torch.autograd.grad(out, leaves, do), want):
+            assert torch.equal(x, y)
+    elif not (what == "rotary" and how == "last dim not dense"):          # tables and positions are laid out anew
+        with pytest.raises(AssertionError):
+            torch.autograd.grad(out, leaves, do)
