@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -212,22 +213,32 @@ struct AttentionBackward : public torch::autograd::Node {
   Shape s;
   HandoverLimits limits;
 
+  // The tensors the backward works on: unpacked and released by one thread at a time, as torch's generated nodes do it.
+  // (Hooks may run meanwhile, so no thread may wait here with the interpreter lock held.)
+  struct Unpacked {
+    Tensor q, k, v, o, st, gs;
+  };
+  Unpacked unpack(std::shared_ptr<Node> self) {
+    std::lock_guard<std::mutex> lock(mutex_);
+    return {q.unpack(), k.unpack(), v.unpack(), o.unpack(std::move(self)), st.unpack(), has_gs ? gs.unpack() : Tensor()};
+  }
+
   variable_list apply(variable_list&& grads) override {
     return node_body([&] {
       // an output that no gradient reaches: zeros, as an autograd Function is given
       const Tensor dout = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
       need(s.Lq % s.block_real == 0 && s.Lk % s.block_real == 0, "Backward supported only for full blocks");
-      const Tensor q_ = q.unpack(), k_ = k.unpack(), v_ = v.unpack(), o_ = o.unpack(getptr()), st_ = st.unpack();
-      const Tensor gs_ = has_gs ? gs.unpack() : Tensor();
+      const Unpacked t = unpack(getptr());
       at::AutoDispatchBelowADInplaceOrView guard;
-      c10::DeviceGuard device(q_.device());
-      const Tensor stats = st_.contiguous();
+      c10::DeviceGuard device(t.q.device());
+      const Tensor stats = t.st.contiguous(), factors = has_gs ? t.gs.contiguous() : Tensor();
       const float* L = stats.data_ptr<float>();
-      return backward(s, limits, q_, k_, v_, o_, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(dout), has_gs ? gs_.contiguous() : gs_);
+      return backward(s, limits, t.q, t.k, t.v, t.o, L, L + (int64_t)s.B * s.H * s.Lq, kernel_ready(dout), factors);
     });
   }
   std::string name() const override { return "FusedLandmarkAttentionBackward"; }
   void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
     for (Saved* s : {&q, &k, &v, &o, &st, &gs}) s->x.reset_data();
   }
 };
@@ -334,7 +345,13 @@ struct RotaryBackward : public torch::autograd::Node {
 
   variable_list apply(variable_list&& grads) override {
     return node_body([&]() -> variable_list {
-      const Tensor cos_ = cos.unpack(), sin_ = sin.unpack(), pos_ = pos.unpack();
+      Tensor cos_, sin_, pos_;
+      {
+        std::lock_guard<std::mutex> lock(mutex_);          // against release_variables in another thread
+        cos_ = cos.unpack();
+        sin_ = sin.unpack();
+        pos_ = pos.unpack();
+      }
       at::AutoDispatchBelowADInplaceOrView guard;
       const RotaryArgs args = {tables(cos_, sin_, cos_.scalar_type()), pos_.contiguous()};
       const Tensor &gk = grads[has_q ? 1 : 0], gq = has_q ? grads[0] : Tensor();
@@ -348,6 +365,7 @@ struct RotaryBackward : public torch::autograd::Node {
   }
   std::string name() const override { return "RotaryEmbeddingBackward"; }
   void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
     for (Saved* s : {&cos, &sin, &pos}) s->x.reset_data();
   }
 };
@@ -762,9 +780,9 @@ PyObject* py_ring_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_saved_tensors(PyObject* self, void*) {
   return guarded([&]() -> PyObject* {
     auto node = std::static_pointer_cast<AttentionBackward>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata);
-    const Tensor q = node->q.unpack(), k = node->k.unpack(), v = node->v.unpack(), o = node->o.unpack(node), st = node->st.unpack();
-    if (!node->has_gs) return tuple_of({q, k, v, o, st.select(0, 0), st.select(0, 1)});
-    return tuple_of({q, k, v, o, st.select(0, 0), st.select(0, 1), node->gs.unpack()});
+    const auto t = without_gil([&] { return node->unpack(node); });
+    if (!node->has_gs) return tuple_of({t.q, t.k, t.v, t.o, t.st.select(0, 0), t.st.select(0, 1)});
+    return tuple_of({t.q, t.k, t.v, t.o, t.st.select(0, 0), t.st.select(0, 1), t.gs});
   });
 }
 PyTypeObject g_attention_node_type;

@@ -166,3 +166,52 @@ def test_what_saved_tensor_hooks_hand_back_is_used_or_refused(what, how):
     elif not (what == "rotary" and how == "last dim not dense"):          # tables and positions are laid out anew
         with pytest.raises(AssertionError):
             torch.autograd.grad(out, leaves, do)
+
+
+@pytest.mark.parametrize("what,other", [("attention", "backward"), ("attention", "saved_tensors"), ("rotary", "backward")])
+def test_threads_use_a_shared_node_one_after_the_other(what, other):
+    # a backward pass unpacks and releases a node's saved tensors in the engine's thread, another thread looks at them
+    # through the node's `saved_tensors`: they belong to one of them at a time
+    import threading
+    from landmark_hip.rotary import apply_rotary_pos_emb
+    from ltriton.flash_landmark_attention import fused_landmark_attention
+    inside, peak, changed = 0, 0, threading.Condition()
+
+    def unpack(t):                                            # stays a moment for the other thread to come in
+        nonlocal inside, peak
+        with changed:
+            inside += 1
+            peak = max(peak, inside)
+            changed.notify_all()
+            changed.wait_for(lambda: peak > 1, timeout=0.1)
+            inside -= 1
+        return t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        if what == "attention":
+            q, k, v, _ = _attention_args(1, 2, 64, 64, 64, 32, 9)
+            leaves = [t.requires_grad_(True) for t in (q, k, v)]
+            out = fused_landmark_attention(*leaves, None, block_size=32)
+        else:
+            _, k, *tables = _rotary_args(1, 2, 40, 64, 9)
+            leaves = [k.requires_grad_(True)]
+            out = apply_rotary_pos_emb(None, k, *tables)[1]
+    loss = out.float().sum()
+    start, errors = threading.Barrier(2), []
+
+    def use(kind):
+        try:
+            start.wait(timeout=20)
+            if kind == "backward":
+                torch.autograd.grad(loss, leaves, retain_graph=True)
+            else:
+                assert torch.equal(out.grad_fn.saved_tensors[3], out)
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=use, args=(kind,)) for kind in ("backward", other)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=30)
+    assert not errors and not any(t.is_alive() for t in threads) and peak == 1
