@@ -739,7 +739,10 @@ __global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256)
   constexpr int E = D / 16;                                       // head dims per lane and rotary half: 8 or 4
   constexpr int PB = 2 * E;                                       // bytes of one piece
   using vec_t = typename PieceVec<E>::type;                       // one piece: E 16-bit values
-  constexpr int CK = BS == 32 || (BS == 64 && D == 128) ? 32 : 64;  // keys per chunk
+  // keys per chunk: with the window inside, chunks of 32 leave room for three waves per SIMD at blocks of 64 and head dim
+  // 128; without it two run whichever is taken, and 64 keys keep more loads in flight (a chunk step at block 64: 256 queries of
+  // 32 heads, top 4, 186.5 -> 184.0 us; 64 queries, top 5, 86.6 -> 83.5)
+  constexpr int CK = BS == 32 || (LOCAL && BS == 64 && D == 128) ? 32 : 64;
   constexpr int KPG = CK / 8;                                     // keys per 8-lane group and chunk
   constexpr int NC = BS / CK;                                     // chunks per block
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
