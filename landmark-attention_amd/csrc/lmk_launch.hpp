@@ -165,6 +165,7 @@ struct RetrParams {
   // gather step with the rows' local window inside (local != 0): the new tokens' keys and values (rotated by the
   // caller), the number of cached tokens behind the last complete block, their first row in the cache and its position
   int local, local_inc;
+  int block_waves, window_wave;                   // of a row's waves: those that share its blocks out, the one with its window
   const void *k_new, *v_new;
   int64_t kns_b, kns_h, kns_r, vns_b, vns_h, vns_r, local_row0, local_pos0;
   // with `local`, optional: the new tokens' rows (keys without rotary, values) are stored in the cache on the way

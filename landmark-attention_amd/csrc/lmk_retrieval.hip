@@ -713,9 +713,18 @@ __device__ __forceinline__ float sum8(float d) {                  // sum over th
 // The picked blocks of a row are read at p.idx[b * idx_sb + h * idx_sh + t * idx_st + 0 .. k-1] (selections shared
 // by the heads or by the queries have a zero stride there); a block counts among the k newest, whose keys sit one
 // block further on, by its age in the ring (p.ring_start = slot of the oldest block, 0 for a flat cache).
-// Most waves that share a row's blocks out beside its window's: with a block per wave no wave walks two of them one after
-// the other; blocks of 128 need the registers of fewer waves.
-constexpr int gather_waves(int BS) { return BS <= 64 ? 8 : 4; }
+// Keys per chunk: with the window inside, chunks of 32 leave room for three waves per SIMD at blocks of 64 and head dim
+// 128; without it two run whichever is taken, and 64 keys keep more loads in flight (a chunk step at block 64: 256 queries of
+// 32 heads, top 4, 186.5 -> 184.0 us; 64 queries, top 5, 86.6 -> 83.5).
+constexpr int gather_chunk(int BS, int D, bool LOCAL) { return BS == 32 || (LOCAL && BS == 64 && D == 128) ? 32 : 64; }
+// Most waves that share out a row's blocks when its window is attended to here as well.  A wave per block keeps no wave
+// walking two of them one after the other while the others are done; beyond six, waves of two blocks each are level again
+// and their partial sums cheaper to merge (1024 rows, block 32, top 8: 72.4 with eight waves, 66.6 us with four).  Blocks of
+// 128 hold 237 registers (head dim 64) or 307 (128): a fifth wave of blocks would halve the waves a CU takes.
+constexpr int gather_waves(int BS, int D, int CK) { return BS == 128 ? 4 : BS == 64 && D == 128 ? (CK == 64 ? 4 : 8) : 6; }
+// The same with a wave for the window alone, which blocks of 128 at head dim 128 have no room for: the workgroup's registers
+// would be halved to 256, 90 of them spilled (128 rows, top 7: 43.2 against 31.9 us; 512 rows, top 4: 64.8 against 58.3).
+constexpr int gather_max_waves(int BS, int D, int CK) { return gather_waves(BS, D, CK) + (BS == 128 && D == 128 ? 0 : 1); }
 template <int E> struct PieceVec;
 template <> struct PieceVec<8> { using type = u32x4_t; };
 template <> struct PieceVec<4> { using type = u32x2_t; };
@@ -727,31 +736,31 @@ template <> struct PieceVec<4> { using type = u32x2_t; };
 // softmax, instead of coming in as (o_loc, L_loc, M_loc) from a forward launch over a window another launch built:
 // a decode step is then the selection and this kernel.  Its keys join the global bucket directly (own-block rule:
 // causal, the landmark token does not see itself; flash_landmark_attention.py:78-100).
-// With SPLIT the window has a wave of its own and every picked block, up to gather_waves(), as well (32 sequences of 32
-// heads, five blocks of 64 each: 71 -> 61 us for the step together with the chunks of 32 keys, whose registers leave
-// room for three waves per SIMD).
-template <class T, int D, int BS, bool SPLIT, bool PADDED, bool MERGE = false, bool LOCAL = false>
-__global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256) void lmk_gather_attend_kernel(RetrParams p) {
-  const int nblk = SPLIT ? (int)(blockDim.x >> 6) - (LOCAL ? 1 : 0) : 1;   // waves that share the row's blocks out
-  constexpr int NWV = SPLIT ? (LOCAL ? gather_waves(BS) + 1 : 4) : 1;
+// With SPLIT a row has a workgroup, in which p.block_waves waves share its blocks out and wave p.window_wave takes its window
+// (32 sequences of 32 heads over 4096 tokens, new inputs on every pass: five blocks of 64 each 78.4 with four waves for the
+// blocks and chunks of 64, 73.8 us as it is; three blocks 62.3 and 45.7).
+template <class T, int D, int BS, bool SPLIT, bool PADDED, bool MERGE = false, bool LOCAL = false,
+          int CK = gather_chunk(BS, D, LOCAL)>
+__global__ __launch_bounds__(SPLIT && LOCAL ? 64 * gather_max_waves(BS, D, CK) : 256,
+                             SPLIT && LOCAL && gather_waves(BS, D, CK) > 4 ? 3 : 1)
+void lmk_gather_attend_kernel(RetrParams p) {
+  const int nblk = SPLIT ? (LOCAL ? p.block_waves : 4) : 1;       // waves that share the row's blocks out
+  constexpr int NWV = SPLIT ? (LOCAL ? gather_max_waves(BS, D, CK) : 4) : 1;
   static_assert((D == 128 || D == 64) && (BS == 32 || BS % 64 == 0), "8 lanes x 2 pieces per row; whole chunks of keys");
   static_assert(!LOCAL || !PADDED, "the local window sits in a block of BS tokens");
   constexpr int E = D / 16;                                       // head dims per lane and rotary half: 8 or 4
   constexpr int PB = 2 * E;                                       // bytes of one piece
   using vec_t = typename PieceVec<E>::type;                       // one piece: E 16-bit values
-  // keys per chunk: with the window inside, chunks of 32 leave room for three waves per SIMD at blocks of 64 and head dim
-  // 128; without it two run whichever is taken, and 64 keys keep more loads in flight (a chunk step at block 64: 256 queries of
-  // 32 heads, top 4, 186.5 -> 184.0 us; 64 queries, top 5, 86.6 -> 83.5)
-  constexpr int CK = BS == 32 || (LOCAL && BS == 64 && D == 128) ? 32 : 64;
   constexpr int KPG = CK / 8;                                     // keys per 8-lane group and chunk
   constexpr int NC = BS / CK;                                     // chunks per block
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 7, g = lane >> 3;                           // head-dim chunk pair, key group
   // (bh, t): a wave's own row, or -- SPLIT, for launches with few rows -- the workgroup's row, whose
-  // selected blocks the four waves share out (block js goes to wave js % 4) and merge at the end
+  // selected blocks its waves share out (block js goes to wave js % nblk) and merge at the end
   const int64_t row = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
   if (row >= (int64_t)p.B * p.H * p.T) return;                    // SPLIT: the whole workgroup leaves
-  const int js0 = SPLIT ? (wave < nblk ? wave : p.k) : 0, jstep = nblk;   // (the window's wave takes no block)
+  const int js0 = SPLIT ? (wave < nblk ? wave : p.k) : 0, jstep = nblk;   // (a wave of the window's own takes no block)
+  const bool windows = LOCAL && (!SPLIT || wave == p.window_wave);
   const int bh = (int)(row / p.T), t = (int)(row % p.T);
   const int b = bh / p.H, hh = bh % p.H;
 
@@ -771,7 +780,7 @@ __global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256)
   // The row's own key (without rotary) and value on their way into the cache: fetched here by one of the row's waves
   // (lanes 0 .. D/8-1 the key, 32 .. the value), stored at the end, so that nothing waits for them.  Nobody reads the
   // destination in this launch: it lies behind the cached rows.
-  const bool appends = LOCAL && p.ap_k != nullptr && (!SPLIT || wave == nblk) && (lane & 31) < D / 8;
+  const bool appends = windows && p.ap_k != nullptr && (lane & 31) < D / 8;
   u32x4_t ap = {0, 0, 0, 0};
   if (LOCAL && appends)
     ap = *(const u32x4_t*)((lane < 32 ? (const char*)p.ap_k + 2 * (b * p.aks_b + hh * p.aks_h + (int64_t)t * p.aks_r)
@@ -832,7 +841,7 @@ __global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256)
     }
   };
   if constexpr (LOCAL) {
-    if (!SPLIT || wave == nblk) {
+    if (windows) {
       const int inc = p.local_inc, own = inc + t;                 // window rows: inc of the cache, then the new tokens
       const char* kn = (const char*)p.k_new + 2 * (b * p.kns_b + hh * p.kns_h);
       const char* vn = (const char*)p.v_new + 2 * (b * p.vns_b + hh * p.vns_h);
@@ -1011,7 +1020,7 @@ __global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256)
     alo[e] += __shfl_xor(alo[e], 32, 64);
     ahi[e] += __shfl_xor(ahi[e], 32, 64);
   }
-  if constexpr (SPLIT) {                                          // the four waves' partial (M, l, acc) -> wave 0
+  if constexpr (SPLIT) {                                          // the waves' partial (M, l, acc) -> wave 0
     __shared__ float part_acc[NWV][D];
     __shared__ float part_ml[NWV][2];
     if (g == 0) {
@@ -1027,22 +1036,30 @@ __global__ __launch_bounds__(SPLIT && LOCAL ? 64 * (gather_waves(BS) + 1) : 256)
     }
     __syncthreads();
     if (wave != 0) return;
-    const int nw = nblk + (LOCAL ? 1 : 0);
-    float Mall = part_ml[0][0];                                   // wave 0 always has a block (k >= 1)
-    for (int w = 1; w < nw; ++w) Mall = fmaxf(Mall, part_ml[w][0]);
+    const int nw = LOCAL ? max(p.block_waves, p.window_wave + 1) : NWV;   // of NWV; unrolled, the loads are in flight together
+    float mw[NWV], Mall = part_ml[0][0];                          // wave 0 always has a block (k >= 1)
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      mw[w] = part_ml[w][0];
+      mw[w] = w < nw ? mw[w] : -INFINITY;
+      Mall = fmaxf(Mall, mw[w]);
+    }
     lrun = 0.f;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       alo[e] = 0.f;
       ahi[e] = 0.f;
     }
-    for (int w = 0; w < nw; ++w) {
-      const float sw = fast_exp2(part_ml[w][0] - Mall);           // 0 for a wave without blocks (M = -inf)
-      lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        alo[e] = __builtin_fmaf(part_acc[w][E * j + e], sw, alo[e]);
-        ahi[e] = __builtin_fmaf(part_acc[w][D / 2 + E * j + e], sw, ahi[e]);
+    for (int w = 0; w < NWV; ++w) {
+      if (w < nw) {
+        const float sw = fast_exp2(mw[w] - Mall);                 // 0 for a wave without blocks (M = -inf)
+        lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          alo[e] = __builtin_fmaf(part_acc[w][E * j + e], sw, alo[e]);
+          ahi[e] = __builtin_fmaf(part_acc[w][D / 2 + E * j + e], sw, ahi[e]);
+        }
       }
     }
     Mrun = Mall;
@@ -1220,20 +1237,44 @@ int launch_retrieve_topk(const RetrParams& p, int D, int dtype, bool reuse_landm
   return LMK_ERR_UNSUPPORTED;
 }
 
+// The gather with the rows' window inside, a workgroup per row.
+template <class T, int D, int BS, int CK>
+static int launch_gather_split(RetrParams p, int64_t rows, hipStream_t stream) {
+  constexpr int most = gather_waves(BS, D, CK);
+  int own = 1;                                                    // the window has a wave of its own
+  if (BS == 128) {
+    // at head dim 64 while every row's five waves find a CU of their own (32 rows, top 4: 18.5 -> 16.6 us; 256 rows, top 8: 32.7 ->
+    // 28.5): a CU takes eight waves, so two workgroups of four and only one of five (512 rows, top 4: 28.0 against 32.5)
+    own = D == 64 && rows <= 256 ? 1 : 0;
+    p.block_waves = own ? std::min(p.k, most) : most;
+  } else {
+    const int per = (p.k + most - 1) / most;                      // blocks a wave walks one after the other
+    p.block_waves = (p.k + per - 1) / per;
+  }
+  p.window_wave = own ? p.block_waves : p.k % p.block_waves;
+  const dim3 grid((unsigned)rows), wg(64 * (p.block_waves + own));
+  if (p.merge_slices > 0) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, false, true, true, CK>), grid, wg, 0, stream, p);
+  else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, false, false, true, CK>), grid, wg, 0, stream, p);
+  return (int)hipGetLastError();
+}
+
 template <class T, int D, int BS, bool PADDED>
 static int launch_gather_b(const RetrParams& p, hipStream_t stream) {
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   if (p.local) {                          // with the row's local window: blocks as they are only
     if constexpr (!PADDED) {
-      const bool split = rows <= 1024 && p.k > 1;
-      const dim3 grid((unsigned)(split ? rows : (rows + 3) / 4));
-      if (p.merge_slices > 0) {
-        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, true, true>), grid, dim3(64 * (std::min(p.k, gather_waves(BS)) + 1)), 0, stream, p);
-        else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, true, true>), grid, dim3(256), 0, stream, p);
-      } else {
-        if (split) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, PADDED, false, true>), grid, dim3(64 * (std::min(p.k, gather_waves(BS)) + 1)), 0, stream, p);
-        else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, false, true>), grid, dim3(256), 0, stream, p);
+      constexpr int CK = gather_chunk(BS, D, true);
+      if (rows <= 1024 && p.k > 1) {
+        // from seven blocks on at most four waves, in chunks of 64 keys, where the rows fill the chip (1024 rows, top 7: 88.0 us
+        // against 97.0 in chunks of 32 and 89.7 with a wave per block; 256 rows, top 8: 29.7, 30.9 and 30.1) and not with few
+        // of them (128 rows, top 7: 24.3 against 22.2 with a wave per block)
+        if constexpr (BS == 64 && D == 128)
+          if (p.k > 6 && rows > 128) return launch_gather_split<T, D, BS, 64>(p, rows, stream);
+        return launch_gather_split<T, D, BS, CK>(p, rows, stream);
       }
+      const dim3 grid((unsigned)((rows + 3) / 4));
+      if (p.merge_slices > 0) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, true, true>), grid, dim3(256), 0, stream, p);
+      else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, false, true>), grid, dim3(256), 0, stream, p);
       return (int)hipGetLastError();
     } else {
       return LMK_ERR_UNSUPPORTED;

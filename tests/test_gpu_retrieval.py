@@ -177,11 +177,14 @@ def test_incomplete_cached_block(n_mems, inc, T, block, top_k, D):
     # a wave per picked block, up to eight (four at block 128), beside the window's own
     (12, 33, 1, 5, 2, 3, 128, torch.bfloat16, 64),     # six waves
     (12, 60, 4, 8, 2, 3, 128, torch.float16, 64),      # nine: every one there is
-    (15, 33, 2, 11, 1, 2, 128, torch.bfloat16, 64),    # three waves take a second block
-    (300, 41, 1, 9, 1, 4, 128, torch.bfloat16, 64),    # one does, behind two slices to merge
+    (15, 33, 2, 11, 1, 2, 128, torch.bfloat16, 64),    # six waves of one or two blocks
+    (300, 41, 1, 9, 1, 4, 128, torch.bfloat16, 64),    # five, behind two slices to merge
+    (12, 33, 1, 7, 5, 32, 128, torch.bfloat16, 64),    # more rows: four waves of two blocks in chunks of 64 keys
+    (12, 0, 2, 8, 3, 32, 128, torch.float16, 64),
     (20, 30, 2, 9, 1, 2, 64, torch.bfloat16, 32),
-    (9, 125, 3, 6, 1, 2, 128, torch.bfloat16, 128),    # block 128: two of four waves take a second block
-    (9, 40, 2, 7, 1, 2, 64, torch.float16, 128),
+    (9, 125, 3, 6, 1, 2, 128, torch.bfloat16, 128),    # block 128: the window goes to a wave that has a block
+    (9, 40, 2, 7, 1, 2, 64, torch.float16, 128),       # and at head dim 64 to one of its own
+    (9, 40, 1, 4, 9, 32, 64, torch.bfloat16, 128),     # but not with many rows
     (12, 33, 3, 5, 12, 32, 128, torch.bfloat16, 64),   # a wave per row in chunks of 32 keys
 ])
 def test_decode_rows_attend_to_their_local_window_inside_the_gather(n_mems, inc, T, top_k, B, H, D, dtype, block):
