@@ -14,7 +14,7 @@
 //          block's landmark key.
 //   dkdv   key-stationary, S layout (lane = key): purely elementwise between its four
 //          products S = Q K^T, dP = dO V^T, dV^T += dO^T W, dK^T += Q^T dS
-//          (lmk_bwd_dkdv32.hip, all block sizes).
+//          (lmk_bwd_dkdv_split.hip with 64 keys a workgroup, lmk_bwd_dkdv32.hip with 128).
 // This file holds the pre kernel, the dQ kernel for many query rows of whole blocks of 64 keys (block 32 has its own in
 // lmk_bwd_dq32.hip, everything else is lmk_bwd_dq_split.hip's) and the dispatch.
 //

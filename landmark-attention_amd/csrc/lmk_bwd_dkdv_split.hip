@@ -253,8 +253,8 @@ __global__ __launch_bounds__(256 * QP, 2) void lmk_bwd_dkdv_split_kernel(BwdPara
     });
     f32x4 y[4];
     row_tile(C::HALF, vf, dp, [&](int n) __attribute__((always_inline)) {   // W under dP's MFMAs
-      constexpr int G0 = C::KS > 4 ? 2 : 0, EV = C::KS > 4 ? 1 : 1;
-      if (n >= G0 && (n - G0) % EV == 0 && (n - G0) / EV < 4) weigh((n - G0) / EV);
+      constexpr int G0 = C::KS > 4 ? 2 : 0;
+      if (n >= G0 && n - G0 < 4) weigh(n - G0);
       if (more && n % 2 == 0) request_piece(st + 1, (C::KS + n) / 2);
       if (more && n == 1) request_piece(st + 1, PIECES - 1);
       if (n == C::KS - 1) {

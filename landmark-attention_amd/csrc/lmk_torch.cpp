@@ -411,8 +411,8 @@ struct Append {
   int64_t row;
 };
 
-// One step of the mem-cache path over the first S rows of k_cache, v_cache (GPU memory, or pinned host memory for the
-// selection per head on `landmarks` alone): (out, idx), and the append.  `shared`: one selection per head.
+// One step of the mem-cache path over the first S rows of k_cache, v_cache: (out, idx), and the append.  `shared`: one
+// selection per head.
 std::pair<Tensor, Tensor> mem_cache_step(const Tensor& q_in, const Tensor& kc_in, const Tensor& vc_in, int64_t S,
                                          const Tensor& kl_in, const Tensor& vl_in, const Tensor& cos, const Tensor& sin,
                                          int block, int top_k, bool has_scale, double scale, bool shared, Tensor ws, bool reuse,
@@ -423,10 +423,10 @@ std::pair<Tensor, Tensor> mem_cache_step(const Tensor& q_in, const Tensor& kc_in
   need(kc_in.size(0) == B && kc_in.size(1) == H && kc_in.size(3) == D && same_shape(kc_in, vc_in) &&
            q_in.scalar_type() == kc_in.scalar_type() && q_in.scalar_type() == vc_in.scalar_type() && q_in.is_cuda() &&
            kc_in.is_cuda() && vc_in.is_cuda(),
-       "the cache must have the queries' batch, heads, head dim, type and device");
+       "the cache must have the queries' batch, heads, head dim and type, and be on the GPU");
   need(same_shape(kl_in, q_in) && same_shape(vl_in, q_in) && kl_in.scalar_type() == q_in.scalar_type() &&
            vl_in.scalar_type() == q_in.scalar_type() && kl_in.is_cuda() && vl_in.is_cuda(),
-       "the new keys and values must have the queries' shape, type and device");
+       "the new keys and values must have the queries' shape and type, and be on the GPU");
   const int dtype = dtype_code(q_in);
   need(dtype >= 0, "HIP kernels are built for bf16 and fp16");
   need(block > 0 && (S % block == 0 || T + S % block <= block), "new chunk and cached tail must fit one block (llama_mem.py:330)");
@@ -452,7 +452,7 @@ std::pair<Tensor, Tensor> mem_cache_step(const Tensor& q_in, const Tensor& kc_in
   if (append != nullptr) {
     need(append->k_nopos.dim() == 4 && same_shape(append->k_nopos, q_in) && append->k_nopos.scalar_type() == q.scalar_type() &&
              append->k_nopos.is_cuda(),
-         "the keys to append must have the queries' shape, type and device");
+         "the keys to append must have the queries' shape and type, and be on the GPU");
     need(append->row >= S && append->row + T <= append->k_buf.size(2), "no room for the new rows");
     kn = kernel_ready(append->k_nopos);
     tkn = t4(kn);
