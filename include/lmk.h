@@ -285,6 +285,14 @@ int lmk_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk
                       const lmk_tensor4* out, int B, int H, int T, int S, int D, float sm_scale, int block, int top_k,
                       int dtype, void* stream);
 
+/* Scratch of a gather by block: (row, picked block) pairs of a step in which a block is picked by several rows are worked on
+ * block by block, on the matrix cores, and what each pair contributes is kept in fp32 until its row's are summed.  0 where the
+ * gather by row serves.  n_blocks: complete blocks of the cache; shared: the queries of a head share one selection.
+ * lmk_attend and lmk_retrieve_and_attend work by block when their attend workspace is this much larger than
+ * lmk_attend_workspace_bytes, lmk_ring_gather_attend_blocks when its workspace holds it; the results are the same
+ * attention, summed in another order. */
+size_t lmk_gather_blocks_workspace_bytes(int B, int H, int T, int n_blocks, int D, int block, int top_k, int shared);
+
 /* The attend step in one call: lmk_local_window (when S % block > 0), lmk_attn_fwd on the local
  * window and lmk_gather_attend, enqueued back to back with the window, its output and its statistics
  * in `workspace` (at least lmk_attend_workspace_bytes(...) bytes, 16-byte aligned).  Same result as
@@ -377,6 +385,13 @@ int lmk_ring_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kring, const
                            const lmk_tensor4* o_loc, const float* L_loc, const float* M_loc, int64_t stat_stride,
                            const lmk_tensor4* out, int B, int H, int T, int n_blocks, int D, float sm_scale, int block,
                            int top_k, int ring_start, int method, int dtype, void* stream);
+/* The same with scratch (16-byte aligned; may be null) for a gather by block. */
+int lmk_ring_gather_attend_blocks(const lmk_tensor4* q, const lmk_tensor4* kring, const lmk_tensor4* vring, const int64_t* idx,
+                                  const void* cos_table, const void* sin_table, int64_t table_stride_row, int64_t n_pos,
+                                  const lmk_tensor4* o_loc, const float* L_loc, const float* M_loc, int64_t stat_stride,
+                                  const lmk_tensor4* out, void* workspace, size_t workspace_bytes, int B, int H, int T,
+                                  int n_blocks, int D, float sm_scale, int block, int top_k, int ring_start, int method,
+                                  int dtype, void* stream);
 
 /* Local window of the attend step when the cache ends in an incomplete block of
  * inc = S % block tokens (llama_mem.py:329-342; needs inc > 0 and T + inc <= block, the

@@ -1,5 +1,6 @@
 // C ABI of liblandmark_hip.so: argument validation on the host, then dispatch
 // to the kernel launchers.  Declarations and the contract live in include/lmk.h.
+#include <algorithm>
 #include <cmath>
 
 #include <mutex>
@@ -701,6 +702,24 @@ int lmk_cache_append(const lmk_tensor4* k, const lmk_tensor4* v, const lmk_tenso
   return lmk::launch_copy_rows(p, (hipStream_t)stream);
 }
 
+// The workspace of a gather by block, or an empty one where the gather by row serves or `bytes` at `ptr` do not suffice.
+struct BlocksWorkspace {
+  void* ptr = nullptr;
+  int rows = 0;                                             // of a (batch, head) at a time
+};
+static BlocksWorkspace blocks_workspace(void* ptr, size_t bytes, int B, int H, int T, int n_blocks, int D, int block, int k,
+                                        bool shared, const lmk_tensor4* kcache, const lmk_tensor4* vcache, int64_t table_stride_row) {
+  const int rows = lmk::gather_blocks_rows(B, H, T, n_blocks, D, block, k, shared);
+  if (rows == 0 || ptr == nullptr || bytes < lmk_gather_blocks_workspace_bytes(B, H, T, n_blocks, D, block, k, shared)) return {};
+  for (int64_t stride : {kcache->stride_row, vcache->stride_row, table_stride_row})   // rows of a block are addressed with 32 bits
+    if (stride < 0 || stride * 2 * 128 >= ((int64_t)1 << 31)) return {};
+  return {ptr, rows};
+}
+static void set_blocks_workspace(lmk::RetrParams& p, const BlocksWorkspace& w, int D) {
+  p.part = static_cast<float*>(w.ptr);
+  p.part_score = p.part + (int64_t)p.B * p.H * w.rows * p.k * D;
+}
+
 // `candidates`: the selection has stopped after its slice step (lmk::launch_fwd32_topk_slices) and the gather picks
 // a row's k best from what that step left, writing them to idx on the way; else idx holds the indices already.
 static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache, const int64_t* idx,
@@ -709,7 +728,7 @@ static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, c
                               const lmk_tensor4* out, int B, int H, int T, int S, int D, float sm_scale, int block,
                               int top_k, int dtype, void* stream, const lmk::RetrParams* candidates,
                               const lmk_tensor4* k_new = nullptr, const lmk_tensor4* v_new = nullptr,
-                              const AppendArgs* append = nullptr) {
+                              const AppendArgs* append = nullptr, const BlocksWorkspace& blocks = {}) {
   // append (with k_new): the new tokens' rows are stored in the cache by the same launch
   // k_new, v_new: the gather kernel attends to the rows' local window itself (gather_takes_local_window) and
   // o_loc, L_loc, M_loc are not read
@@ -761,7 +780,18 @@ static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, c
     p.approx = candidates->approx;
     p.exact = candidates->exact;
   }
+  if (blocks.rows > 0 && !local && candidates == nullptr) {
+    set_blocks_workspace(p, blocks, D);
+    return lmk::launch_gather_blocks(p, D, block, blocks.rows, dtype, (hipStream_t)stream);
+  }
   return lmk::launch_gather_attend(p, D, block, dtype, (hipStream_t)stream);
+}
+
+size_t lmk_gather_blocks_workspace_bytes(int B, int H, int T, int n_blocks, int D, int block, int top_k, int shared) {
+  if (B <= 0 || H <= 0 || T <= 0 || n_blocks <= 0 || D <= 0 || top_k <= 0) return 0;
+  const int k = top_k < n_blocks ? top_k : n_blocks;
+  const int64_t rows = lmk::gather_blocks_rows(B, H, T, n_blocks, D, block, k, shared != 0);
+  return align256((size_t)((int64_t)B * H * rows * k * lmk::gather_blocks_pick_bytes(D)));
 }
 
 int lmk_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache, const int64_t* idx,
@@ -871,6 +901,17 @@ int lmk_ring_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kring, const
                            const lmk_tensor4* o_loc, const float* L_loc, const float* M_loc, int64_t stat_stride,
                            const lmk_tensor4* out, int B, int H, int T, int n_blocks, int D, float sm_scale, int block,
                            int top_k, int ring_start, int method, int dtype, void* stream) {
+  return lmk_ring_gather_attend_blocks(q, kring, vring, idx, cos_table, sin_table, table_stride_row, n_pos, o_loc, L_loc, M_loc,
+                                       stat_stride, out, nullptr, 0, B, H, T, n_blocks, D, sm_scale, block, top_k, ring_start,
+                                       method, dtype, stream);
+}
+
+int lmk_ring_gather_attend_blocks(const lmk_tensor4* q, const lmk_tensor4* kring, const lmk_tensor4* vring, const int64_t* idx,
+                                  const void* cos_table, const void* sin_table, int64_t table_stride_row, int64_t n_pos,
+                                  const lmk_tensor4* o_loc, const float* L_loc, const float* M_loc, int64_t stat_stride,
+                                  const lmk_tensor4* out, void* workspace, size_t workspace_bytes, int B, int H, int T,
+                                  int n_blocks, int D, float sm_scale, int block, int top_k, int ring_start, int method,
+                                  int dtype, void* stream) {
   int rc;
   if ((rc = check_tensor(q)) || (rc = check_tensor(kring)) || (rc = check_tensor(vring)) || (rc = check_tensor(o_loc)) ||
       (rc = check_tensor(out)))
@@ -907,6 +948,13 @@ int lmk_ring_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kring, const
   p.cs_r = table_stride_row;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   const int slots = block == 32 ? 32 : (block <= 64 ? 64 : 128);
+  if (workspace != nullptr && !aligned16(workspace)) return LMK_ERR_ALIGN;
+  const BlocksWorkspace blocks = blocks_workspace(workspace, workspace_bytes, B, H, T, n_blocks, D, block, top_k,
+                                                  method == LMK_SELECT_MAX_OVER_TOKENS, kring, vring, table_stride_row);
+  if (blocks.rows > 0) {
+    set_blocks_workspace(p, blocks, D);
+    return lmk::launch_gather_blocks(p, D, slots, blocks.rows, dtype, (hipStream_t)stream);
+  }
   return lmk::launch_gather_attend(p, D, slots, dtype, (hipStream_t)stream);
 }
 
@@ -1133,8 +1181,10 @@ int lmk_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor
   }
   // the window's last T rows, read in place
   const lmk_tensor4 o_loc = {w + l.o_win + (size_t)inc * D * 2, o_win.stride_b, o_win.stride_h, o_win.stride_row};
-  return lmk_gather_attend(q, kcache, vcache, idx, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc,
-                           M + inc, W, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream);
+  const BlocksWorkspace blocks = blocks_workspace(w + l.total, workspace_bytes - l.total, B, H, T, S / block, D, block,
+                                                  std::min(top_k, S / block), false, kcache, vcache, table_stride_row);
+  return gather_attend_impl(q, kcache, vcache, idx, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc, M + inc, W,
+                            out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr, nullptr, nullptr, nullptr, blocks);
 }
 
 static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor4* vcache,
@@ -1208,9 +1258,12 @@ static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kca
       return rc;
     }
     const bool by_slices = lmk::topk_slices(pr) > 0;
+    const BlocksWorkspace blocks = blocks_workspace(w + l.total, attend_workspace_bytes - l.total, B, H, T, S / block, D, block,
+                                                    pr.k, false, kcache, vcache, table_stride_row);
     if (by_slices) {
       if (!reuse_landmark_keys && (rc = lmk::launch_landmark_keys(pr, D, dtype, (hipStream_t)stream))) return rc;
       if ((rc = lmk::launch_fwd32_topk_slices(pf, pr, D, dtype, (hipStream_t)stream))) return rc;
+      if (blocks.rows > 0 && (rc = lmk::launch_topk_slice_merge(pr, (hipStream_t)stream))) return rc;
     } else {
       if (reuse_landmark_keys) rc = lmk::launch_fwd(pf, D, block, dtype, (hipStream_t)stream);
       else rc = lmk::launch_fwd32_landmark_keys(pf, pr, D, dtype, (hipStream_t)stream);
@@ -1220,7 +1273,7 @@ static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kca
     const lmk_tensor4 o_loc = {w + l.o_win + (size_t)inc * D * 2, o_win.stride_b, o_win.stride_h, o_win.stride_row};
     if ((rc = gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc,
                                  M + inc, W, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream,
-                                 by_slices ? &pr : nullptr)))
+                                 by_slices && blocks.rows == 0 ? &pr : nullptr, nullptr, nullptr, nullptr, blocks)))
       return rc;
     return append_rows();
   }

@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "../../include/lmk.h"
 
@@ -145,6 +147,7 @@ struct RetrParams {
   const void *q, *kcache, *vcache, *cos, *sin;   // q rotated; caches un-rotated; tables (n_pos, D)
   const void* o_loc;                              // attention over the local chunk (gather step)
   const float *L_loc, *M_loc;
+  float *part, *part_score;                       // gather by block: what a pick contributes, and its landmark's score (null: row by row)
   int64_t stat_stride;                            // floats between consecutive (batch, head) rows of L_loc, M_loc
   void* out;
   int64_t* idx;                                   // (B, H, T, k) ascending block indices
@@ -263,6 +266,7 @@ int launch_fwd32_landmark_keys(const FwdParams& pf, const RetrParams& pr, int D,
 int launch_fwd32_topk_slices(const FwdParams& pf, const RetrParams& pr, int D, int dtype, hipStream_t stream);
 int launch_landmark_keys(const RetrParams& p, int D, int dtype, hipStream_t stream);   // the rotation alone
 int launch_topk_slices(const RetrParams& p, int D, int dtype, hipStream_t stream);     // the selection's slice step alone
+int launch_topk_slice_merge(const RetrParams& p, hipStream_t stream);                  // behind it: the rows' indices
 // rows whose local window the gather kernel attends to itself: window inside one block, a handful of new tokens
 constexpr int kLocalMaxT = 4;
 inline bool gather_takes_local_window(int T, int S, int block) {
@@ -270,5 +274,24 @@ inline bool gather_takes_local_window(int T, int S, int block) {
 }
 // BS: slots per block (32, 64 or 128); p.block <= BS tokens per block in the cache
 int launch_gather_attend(const RetrParams& p, int D, int BS, int dtype, hipStream_t stream);
+
+// Gather by block (lmk_gather_blocks.hip): the rows of a (batch, head) whose picks the workspace holds at a time, or 0 where
+// the gather by row serves.  A rotation of a block's keys serves the picks of one rank, and a block is picked at about
+// sqrt(k) ranks, so what decides is picks per block and rank, times the block (a pick costs 1 KB of workspace traffic at head
+// dim 128 whatever its block); and the rows' reads must outweigh the second launch.  Whole steps by row and by block, us, 32
+// heads, 256 queries, top 4, D128: block 32, 8 picks a block 90.1 / 80.3, 4 picks 100.3 / 106.9; block 64, 8 picks 156 / 112,
+// 4 picks 172 / 159; block 128, 4 picks 400 / 292, top 1 of 256 blocks, 1 pick 153 / 199.  Fewer rows: 8 heads, 128 queries,
+// block 64, 8 picks, 134 MB 44.1 / 41.2; at D64, 67 MB 32.4 / 33.1; block 128 at D64, 134 MB 42.8 / 44.9 and 268 MB 67.4 / 62.3.
+constexpr int64_t kGatherBlocksBytes = (int64_t)256 << 20;        // of workspace, at most
+inline int64_t gather_blocks_pick_bytes(int D) { return 4 * ((int64_t)D + 1); }
+inline int gather_blocks_rows(int B, int H, int T, int num_mems, int D, int block, int k, bool shared) {
+  if (block < 2 || block > 128 || k < 1 || k > 64 || num_mems < 1 || num_mems > 65535) return 0;
+  const int64_t heads = (int64_t)B * H, rows = std::min<int64_t>(T, kGatherBlocksBytes / (heads * k * gather_blocks_pick_bytes(D)));
+  if (heads * rows * k * block * 4 * D < (int64_t)(block > 64 && D == 64 ? 256 : 128) << 20) return 0;
+  // one selection for all rows of a head: k blocks, each at one rank
+  const double picks = shared ? (double)rows : (double)rows * k / num_mems / std::sqrt((double)k);
+  return picks * block >= 192 ? (int)rows : 0;
+}
+int launch_gather_blocks(const RetrParams& p, int D, int BS, int rows, int dtype, hipStream_t stream);
 
 }  // namespace lmk

@@ -1107,6 +1107,12 @@ void lmk_gather_attend_kernel(RetrParams p) {
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+int launch_topk_slice_merge(const RetrParams& p, hipStream_t stream) {
+  const int64_t rows = (int64_t)p.B * p.H * p.T;
+  hipLaunchKernelGGL(lmk_topk_slice_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, topk_slices(p));
+  return (int)hipGetLastError();
+}
+
 template <class T, int D>
 static int launch_topk_t(const RetrParams& p, bool reuse_landmark_keys, hipStream_t stream) {
   constexpr int RPW = 256 / (D / 8);
@@ -1121,8 +1127,7 @@ static int launch_topk_t(const RetrParams& p, bool reuse_landmark_keys, hipStrea
   if (n_slices > 0) {                                               // a handful of rows: every score exact, slices over the chip
     hipLaunchKernelGGL((lmk_topk_slice_kernel<T, D>), dim3((unsigned)(rows * n_slices)), dim3(64 * kSliceWaves), 0, stream, p, n_slices);
     if ((rc = (int)hipGetLastError())) return rc;
-    hipLaunchKernelGGL(lmk_topk_slice_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, n_slices);
-    return (int)hipGetLastError();
+    return launch_topk_slice_merge(p, stream);
   }
   constexpr int lds_max = (kFusedRows * (kFusedMaxMems + 8) + kFusedRows * D) * 4 + kFusedRows * kFusedList * 2 + kFusedRows * (2 * D + 16);
   static_assert(lds_max <= 160 * 1024, "the score tile, the query rows and the lists fill the LDS of a compute unit");

@@ -466,7 +466,8 @@ std::pair<Tensor, Tensor> mem_cache_step(const Tensor& q_in, const Tensor& kc_in
   }
 
   if (!shared) {
-    const size_t abytes = lmk_attend_workspace_bytes(B, H, T, (int)S, D, block);
+    const size_t abytes = lmk_attend_workspace_bytes(B, H, T, (int)S, D, block) +
+                          lmk_gather_blocks_workspace_bytes(B, H, T, (int)(S / block), D, block, top_k, 0);
     Tensor aws = bytes_on(q, abytes), out = at::empty_like(q);
     const lmk_tensor4 tout = t4(out);
     if (append != nullptr)
@@ -544,13 +545,15 @@ std::pair<Tensor, Tensor> ring_attend(const Tensor& q_in, const Tensor& k_in, co
   shape.push_back(r.top_k);
   Tensor slots = at::empty(shape, q.options().dtype(at::kLong));
   const size_t nbytes = lmk_retrieve_workspace_bytes(B, H, T, r.filled * block, D, block);
-  Tensor ws = bytes_on(q, nbytes), out = at::empty_like(q);
+  const size_t pbytes = lmk_gather_blocks_workspace_bytes(B, H, T, r.filled, D, block, r.top_k, r.method == LMK_SELECT_MAX_OVER_TOKENS);
+  Tensor ws = bytes_on(q, nbytes), picks = bytes_on(q, pbytes), out = at::empty_like(q);
   check(lmk_ring_retrieve_topk(&tq, &rk, pc, ps, cs, n_pos, slots.data_ptr<int64_t>(), ws.data_ptr(), nbytes, B, H, T, r.filled, D,
                                block, r.top_k, r.oldest, r.method, dtype, stream));
   const float* L = fwd.second.data_ptr<float>() + r.tail;
   const lmk_tensor4 tout = t4(out);
-  check(lmk_ring_gather_attend(&tq, &rk, &rv, slots.data_ptr<int64_t>(), pc, ps, cs, n_pos, &to, L, L + (int64_t)B * H * W, W, &tout,
-                               B, H, T, r.filled, D, (float)scale, block, r.top_k, r.oldest, r.method, dtype, stream));
+  check(lmk_ring_gather_attend_blocks(&tq, &rk, &rv, slots.data_ptr<int64_t>(), pc, ps, cs, n_pos, &to, L, L + (int64_t)B * H * W, W,
+                                      &tout, pbytes ? picks.data_ptr() : nullptr, pbytes, B, H, T, r.filled, D, (float)scale, block,
+                                      r.top_k, r.oldest, r.method, dtype, stream));
   return {out, slots};
 }
 

@@ -115,6 +115,8 @@ def lib() -> ctypes.CDLL:
                                         i, i, i, i, i, f, i, i, i, vp]
         L.lmk_attend_workspace_bytes.restype = sz
         L.lmk_attend_workspace_bytes.argtypes = [i, i, i, i, i, i]
+        L.lmk_gather_blocks_workspace_bytes.restype = sz
+        L.lmk_gather_blocks_workspace_bytes.argtypes = [i, i, i, i, i, i, i, i]
         L.lmk_attend.restype = i
         L.lmk_attend.argtypes = [T4, T4, T4, vp, T4, T4, vp, vp, i64, i64, T4, vp, sz,
                                  i, i, i, i, i, f, i, i, i, vp]
@@ -145,6 +147,9 @@ def lib() -> ctypes.CDLL:
         L.lmk_retrieve_topk_shared_landmarks.argtypes = L.lmk_retrieve_topk_shared.argtypes
         L.lmk_ring_retrieve_topk.restype = i
         L.lmk_ring_retrieve_topk.argtypes = [T4, T4, vp, vp, i64, i64, vp, vp, sz, i, i, i, i, i, i, i, i, i, i, vp]
+        L.lmk_ring_gather_attend_blocks.restype = i
+        L.lmk_ring_gather_attend_blocks.argtypes = [T4, T4, T4, vp, vp, vp, i64, i64, T4, vp, vp, i64, T4, vp, sz,
+                                                    i, i, i, i, i, f, i, i, i, i, i, vp]
         L.lmk_ring_gather_attend.restype = i
         L.lmk_ring_gather_attend.argtypes = [T4, T4, T4, vp, vp, vp, i64, i64, T4, vp, vp, i64, T4,
                                              i, i, i, i, i, f, i, i, i, i, i, vp]

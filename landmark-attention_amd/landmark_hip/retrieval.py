@@ -134,6 +134,7 @@ def _attend(q, k_cache, v_cache, idx, k_loc, v_loc, cos, sin, block, top_k, sm_s
     assert S % block == 0 or T + S % block <= block, "new chunk and cached tail must fit one block (llama_mem.py:330)"
     lib = _lib.lib()
     nbytes = lib.lmk_attend_workspace_bytes(B, H, T, S, D, int(block))
+    nbytes += lib.lmk_gather_blocks_workspace_bytes(B, H, T, S // int(block), D, int(block), int(top_k), 0)
     with _lib.on_device(q.device):
         ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
         out = torch.empty_like(q)

@@ -1,0 +1,85 @@
+"""Gather + attend by block against float64 and against the gather by row, through the C ABI: groups of one and of several
+picks of a rank, more picks than one search holds, more rows than the workspace holds, blocks of every slot count, a ring
+that has wrapped, shared selections, indices outside the cache.
+"""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# B, H, T, n_blocks, block, k, D, ring_start, method (0 a selection per row, 1 shared by the heads, 2 by the queries), dtype
+CASES = [
+    (1, 32, 65, 8, 64, 4, 128, 0, 0, torch.bfloat16),
+    (1, 32, 130, 9, 32, 4, 128, 5, 0, torch.bfloat16),
+    (2, 12, 255, 40, 51, 4, 64, 13, 0, torch.float16),
+    (1, 8, 140, 5, 128, 5, 128, 0, 0, torch.float16),          # every block picked by every row
+    (1, 8, 500, 7, 100, 3, 64, 6, 0, torch.bfloat16),
+    (1, 16, 65, 64, 33, 64, 64, 1, 0, torch.bfloat16),         # the most ranks there are
+    (1, 32, 600, 70, 32, 4, 64, 0, 0, torch.bfloat16),         # more picks than one search holds
+    (1, 33, 1000, 24, 64, 16, 128, 0, 0, torch.bfloat16),      # more rows than the workspace holds
+    (2, 12, 255, 40, 51, 4, 64, 39, 1, torch.bfloat16),
+    (2, 12, 255, 40, 51, 4, 64, 39, 2, torch.bfloat16),
+    (1, 40, 257, 6, 128, 1, 64, 2, 2, torch.float16),
+    (1, 16, 512, 3, 2, 3, 128, 0, 0, torch.bfloat16),          # too little to read for a second launch: by row
+]
+
+
+def _float64(q, k, v, idx, cos, sin, o_loc, L, M, block, start, heads):
+    """What the rows of `heads` attend to: the picked blocks in float64, merged with the local window."""
+    n, D = k.shape[2] // block, k.shape[-1]
+    top_k = idx.shape[-1]
+    out = torch.empty(len(heads), q.shape[2], D, dtype=torch.float64, device=q.device)
+    tok = torch.arange(block, device=q.device)
+    for i, (b, h) in enumerate(heads):
+        rows = idx[b, h].clamp(0, n - 1)                                             # (T, k)
+        newest = ((rows - start) % n) >= n - top_k
+        pos = (torch.arange(top_k, device=q.device)[None] + newest)[..., None] * block + tok        # (T, k, block)
+        kb, vb = (x[b, h].double().view(n, block, D)[rows] for x in (k, v))          # (T, k, block, D)
+        half = torch.cat((-kb[..., D // 2:], kb[..., :D // 2]), -1)
+        kb = kb * cos.double()[pos] + half * sin.double()[pos]
+        s = (kb @ q[b, h].double()[:, None, :, None])[..., 0] / math.sqrt(D)         # (T, k, block)
+        inner = (s[..., :-1].softmax(-1)[..., None] * vb[..., :-1, :]).sum(-2)       # (T, k, D)
+        w = torch.cat((s[..., -1], (M[b, h] + L[b, h].log()).double()[:, None]), -1).softmax(-1)
+        out[i] = (w[:, :-1, None] * inner).sum(1) + w[:, -1:] * o_loc[b, h].double()
+    return out
+
+
+@pytest.mark.parametrize("B,H,T,n,block,k,D,start,method,dtype", CASES)
+def test_gather_by_block_is_as_exact_as_the_gather_by_row(B, H, T, n, block, k, D, start, method, dtype):
+    from landmark_hip import _lib
+    print(f"case {B} {H} {T} {n} {block} {k} D{D} start {start} method {method} {dtype}", flush=True)
+    lib, dev = _lib.lib(), torch.device("cuda")
+    g = torch.Generator(device=dev).manual_seed(T + n)
+    make = lambda *shape: torch.randn(*shape, device=dev, generator=g).mul_(0.7).to(dtype)
+    q, o_loc = make(B, H, T, D), make(B, H, T, D)
+    kc, vc = make(B, H, n * block, D), make(B, H, n * block, D)
+    M = torch.randn(B, H, T, device=dev, generator=g)
+    L = torch.rand(B, H, T, device=dev, generator=g) * 20 + 1
+    angle = torch.outer(torch.arange((k + 1) * block, device=dev).float(), 1e4 ** (-torch.arange(0, D, 2, device=dev).float() / D))
+    cos, sin = (torch.cat((x, x), -1).to(dtype) for x in (angle.cos(), angle.sin()))
+    shape = ((B, H, T), (B, T), (B, H))[method]
+    idx = torch.rand(*shape, n, device=dev, generator=g).argsort(-1)[..., :k].sort(-1).values.contiguous()
+    idx.view(-1)[0], idx.view(-1)[-1] = -3, n + 5                                    # read as the first and the last block
+    out = [torch.empty_like(q) for _ in range(2)]
+    need = lib.lmk_gather_blocks_workspace_bytes(B, H, T, n, D, block, k, int(method == 2))
+    assert (need == 0) == (block == 2)
+    if need:
+        assert need <= (256 << 20) + 256 and (need < B * H * T * k * (D + 1) * 4) == (T == 1000)
+    ws = torch.empty(max(need, 16), device=dev, dtype=torch.uint8)
+    for i, nbytes in enumerate((0, need)):
+        _lib.check(lib.lmk_ring_gather_attend_blocks(
+            _lib.tensor4(q), _lib.tensor4(kc), _lib.tensor4(vc), idx.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.stride(0),
+            cos.shape[0], _lib.tensor4(o_loc), L.data_ptr(), M.data_ptr(), T, _lib.tensor4(out[i]), ws.data_ptr(), nbytes, B, H, T, n,
+            D, 1 / math.sqrt(D), block, k, start, method, _lib.DTYPE_CODES[dtype], _lib.current_stream(dev)))
+    rows = (idx, idx[:, None], idx[:, :, None])[method].expand(B, H, T, k)
+    heads = sorted({(0, 0), (B - 1, H - 1)})
+    want = _float64(q, kc, vc, rows, cos, sin, o_loc, L, M, block, start, heads)
+    by_row, by_block = ((torch.stack([o[b, h] for b, h in heads]).double() - want) for o in out)
+    # both round the weights and the output to 16 bits: 2^-9 (2^-12) of values up to about 3
+    bound = 2e-2 if dtype == torch.bfloat16 else 2.5e-3
+    assert by_block.abs().max() <= bound
+    # the rotated keys' 16 bits and more are far below those roundings
+    assert by_block.norm() <= 1.01 * by_row.norm()
+    print("error by row / by block", (by_row.norm() / want.norm()).item(), (by_block.norm() / want.norm()).item(), flush=True)
