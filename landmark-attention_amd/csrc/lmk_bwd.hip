@@ -187,7 +187,7 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq_kernel(BwdParams p) {
     const int r = wave * C::PER_WAVE + i;
     const bool is_v = r >= n_k;
     const int row = C::RPD * (r % n_k) + lane / C::CH, cp = lane % C::CH;
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     src[i] = (uint32_t)(2 * ((int64_t)row * (is_v ? p.vs_r : p.ks_r) + 8 * (cp ^ f)));
   }
   const uint32_t step_k = (uint32_t)(2 * (int64_t)BS * p.ks_r), step_v = (uint32_t)(2 * (int64_t)BS * p.vs_r);

@@ -148,8 +148,8 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dkdv32_ho_kernel(BwdParams p) 
   if (!role_k) {
     const int chp = lane % C::CH;
     const int row0 = C::RPD * (tile * C::NDMA) + lane / C::CH, row1 = row0 + C::RPD;
-    const int f0 = (((row0 & 3) << 2) | ((row0 >> 2) & 3)) & (C::CH - 1);
-    const int f1 = (((row1 & 3) << 2) | ((row1 >> 2) & 3)) & (C::CH - 1);
+    const int f0 = tile_swizzle<D>(row0);
+    const int f1 = tile_swizzle<D>(row1);
     q_vo0 = (uint32_t)(2 * (row0 * p.qs_r + 8 * (chp ^ f0)));      // the chunk that belongs at LDS position chp
     g_vo0 = (uint32_t)(2 * (row0 * p.dos_r + 8 * (chp ^ f0)));
     if (C::NDMA > 1) {

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256 * QP, 2) void lmk_bwd_dkdv_split_kernel(BwdPara
   // ---- direct loads: a wave fetches 16 rows of each tensor's 64; the LDS swizzle is applied on the source side
   const int r_lane = lane / C::CH, cp = lane % C::CH;
   auto swz = [&](int row) __attribute__((always_inline)) {
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     return 16 * (cp ^ f);
   };
   const int w4 = wave & 3;

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq32_kernel(BwdParams p) {
     const int part = n % per;
     r_isv[d] = n >= per;
     const int row = C::RPD * part + lane / C::CH, chp = lane % C::CH;
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     const int64_t rs = r_isv[d] ? p.vs_r : p.ks_r;
     r_vo[d] = (uint32_t)(2 * (row * rs + 8 * (chp ^ f)));
     r_lds[d] = (r_isv[d] ? C::BLK_BYTES : 0) + part * 1024;
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(512, 2) void lmk_bwd_dq32_kernel(BwdParams p) {
 #pragma unroll
     for (int n = 0; n < 32 / C::RPD; ++n) {
       const int row = C::RPD * n + lane / C::CH, chp = lane % C::CH;
-      const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+      const int f = tile_swizzle<D>(row);
       dq_dma16(gt, (uint32_t)(2 * (row * p.dos_r + 8 * (chp ^ f))), goff + n * 1024);
     }
   }

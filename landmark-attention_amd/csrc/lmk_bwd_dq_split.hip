@@ -87,7 +87,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_bwd_dq_split_kernel(BwdParams
   // ---- direct loads, as in lmk_fwd_split.hip
   const int r_lane = lane / C::CH, cp = lane % C::CH;
   auto swz = [&](int row) __attribute__((always_inline)) {
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     return 16 * (cp ^ f);
   };
   auto first_row = [&](int blk) __attribute__((always_inline)) { return SEG ? p.seg[blk] : blk * n_tok; };

@@ -103,18 +103,24 @@ __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_lo
 
 // ---- LDS tile addressing ---------------------------------------------------
 // Tiles are stored row-major, 2*D bytes per row, in 16-byte chunks whose index is
-// XOR-swizzled with f(row) = ((row & 3) << 2) | ((row >> 2) & 3).  One layout serves
-// both ways a tile is read:
+// XOR-swizzled with f(row).  One layout serves both ways a tile is read (the banks are 256 bytes wide):
 //   * as an MFMA operand with the head dim along k: lane -> (row l%32, one 16-byte chunk);
-//     f is a bijection on 16 consecutive rows, so 16 lanes cover all 16 chunk columns;
-//   * transposed, with ds_read_b64_tr_b16: a 16-lane group touches 4 consecutive rows x
-//     32 bytes; the (row & 3) << 2 term sends the four rows to four different 64-byte
-//     column groups.
+//     16 consecutive rows must cover all 16 chunks of the banks;
+//   * transposed, with ds_read_b64_tr_b16: 32 lanes touch 4 consecutive rows x 64 bytes, which
+//     must be four different quarters of the banks.
+// Head dim 128: a row is the banks' width; f(row) = ((row & 3) << 2) | ((row >> 2) & 3) is a bijection on 16 rows, and
+// its upper term parts the 4 rows.  Head dim 64: two rows share the banks' width, even rows one half and odd rows the
+// other; f(row) = ((row & 2) << 1) | ((row >> 2) & 3) is a bijection on the 8 rows of a half, and its upper term parts the
+// 2 of a half.  (The lower three bits of the other f send rows r and r + 2 to the same chunks, two accesses for every read;
+// with this one dK/dV of B4 H32 L512 block 64 takes 19.8 us for 20.9, of B2 H8 L1024 15.4 for 16.2, of B1 H8 L1024 block
+// 32 22.7 for 23.4; the other kernels wait for less of LDS and gain 0-1 %.)
+template <int D>
+__device__ __forceinline__ int tile_swizzle(int row) {
+  return (D == 64 ? (row & 2) << 1 : (row & 3) << 2) | ((row >> 2) & 3);
+}
 template <int D>
 __device__ __forceinline__ int tile_off(int row, int chunk) {
-  constexpr int CH = D / 8;
-  const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (CH - 1);
-  return row * (2 * D) + ((chunk ^ f) << 4);
+  return row * (2 * D) + ((chunk ^ tile_swizzle<D>(row)) << 4);
 }
 
 typedef __attribute__((address_space(3))) s16x4_t* lds_s16x4_ptr;

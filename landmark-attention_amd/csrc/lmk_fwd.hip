@@ -131,7 +131,7 @@ __global__ __launch_bounds__(512, 2) void lmk_fwd_kernel(FwdParams p) {
     const int r = wave * C::PER_WAVE + i;
     const bool is_v = r >= n_k;
     const int row = C::RPD * (r % n_k) + lane / C::CH, cp = lane % C::CH;
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     const int64_t rs = is_v ? p.vs_r : p.ks_r;
     src[i] = (uint32_t)(2 * ((int64_t)row * rs + 8 * (cp ^ f)));
     const int row_last = min((n_kstages - 1) * C::SK + row, p.Lk - 1);
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(512, 2) void lmk_fwd_kernel(FwdParams p) {
       const int dst = buf * C::STAGE_BYTES + (is_v ? C::TILE_BYTES : 0) + C::RPD * (r % n_k) * C::ROWB;
       if (virt) {                                       // the slot's token row, worked out per request
         const int row = C::RPD * (r % n_k) + lane / C::CH, cp = lane % C::CH;
-        const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+        const int f = tile_swizzle<D>(row);
         const int tok = slot_to_token_row_clamped<BS>(min(blk_req * C::SK + row, p.Lk - 1), p.n_real, nfull_k, seg_k);
         fwd_dma16(is_v ? vp : kp, (uint32_t)(2 * ((int64_t)tok * (is_v ? p.vs_r : p.ks_r) + 8 * (cp ^ f))), dst);
       } else {
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(512, 2) void lmk_fwd_kernel(FwdParams p) {
       for (int i = 0; i < LM_PER_WAVE; ++i) {
         const int r = wave * LM_PER_WAVE + i;
         const int row = C::RPD * r + lane / C::CH, cp = lane % C::CH;
-        const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+        const int f = tile_swizzle<D>(row);
         const int slot = min(base + row, wg_cblk - 1) * BS + BS - 1;     // an earlier block: complete, inside the table
         const int tok = virt ? slot_to_token_row_clamped<BS>(slot, p.n_real, nfull_k, seg_k) : slot;
         fwd_dma16(kp, (uint32_t)(2 * ((int64_t)tok * p.ks_r + 8 * (cp ^ f))), C::LM_BASE + C::RPD * r * C::ROWB);

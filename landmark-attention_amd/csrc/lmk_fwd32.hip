@@ -166,7 +166,7 @@ __device__ __forceinline__ void fwd32_body(const FwdParams& p, const int bid_) {
     const int part = n % per;
     r_isv[d] = n >= per;
     const int row = C::RPD * part + lane / C::CH, chp = lane % C::CH;
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     const int64_t rs = r_isv[d] ? p.vs_r : p.ks_r;
     r_vo[d] = (uint32_t)(2 * (row * rs + 8 * (chp ^ f)));
     r_vo_last[d] = (uint32_t)(2 * (min(row, last_rows - 1) * rs + 8 * (chp ^ f)));
@@ -195,7 +195,7 @@ __device__ __forceinline__ void fwd32_body(const FwdParams& p, const int bid_) {
     for (int i = 0; i < C::LM_REQ; ++i) {
       const int part = (wave * C::LM_REQ + i) % per;
       const int row = C::RPD * part + lane / C::CH, chp = lane % C::CH;
-      const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+      const int f = tile_swizzle<D>(row);
       const int blk = min(32 * lt + row, max(n_lm - 1, 0));
       const uint32_t vo = (uint32_t)(2 * (((int64_t)blk * 32 + 31) * p.ks_r + 8 * (chp ^ f)));
       fw_dma16(kp, vo, C::LM_OFF + (lt & 1) * C::BLK_BYTES + part * 1024);

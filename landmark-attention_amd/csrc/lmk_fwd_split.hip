@@ -84,7 +84,7 @@ __global__ __launch_bounds__(128 * KP, 2) void lmk_fwd_split_kernel(FwdParams p)
   // position i%CH, so it fetches the chunk tile_off() stores there.
   const int r_lane = lane / C::CH, cp = lane % C::CH;
   auto swz = [&](int row) __attribute__((always_inline)) {
-    const int f = (((row & 3) << 2) | ((row >> 2) & 3)) & (C::CH - 1);
+    const int f = tile_swizzle<D>(row);
     return 16 * (cp ^ f);
   };
   // A block of n tokens holds them in its first slots, the last one (of a complete block: its landmark) in slot BS-1;

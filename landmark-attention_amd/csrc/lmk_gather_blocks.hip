@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256, 2) void lmk_gather_blocks_kernel(RetrParams p,
         const uint32_t stride = (uint32_t)(2 * (v ? p.vcs_r : p.kcs_r));
 #pragma unroll
         for (int i = 0; i < C::PER_WAVE; ++i) {
-          const int r = row + C::RPD * i, f = (((r & 3) << 2) | ((r >> 2) & 3)) & (C::CH - 1);
+          const int r = row + C::RPD * i, f = tile_swizzle<D>(r);
           split_dma16(src, (uint32_t)token_of(r) * stride + 16 * ((lane % C::CH) ^ f), (2 * g + v) * C::TILE + 1024 * (wave * C::PER_WAVE + i));
         }
       }
