@@ -7,6 +7,24 @@
 
 namespace lmk {
 
+// Chunk j (8 head dims) of the landmark key of block m, what its rotation takes: the chunk, the one D / 2 away, the table rows.
+struct LandmarkChunk {
+  u32x4_t x, other, c, s;
+};
+template <int D>
+__device__ __forceinline__ LandmarkChunk load_landmark_chunk(const RetrParams& p, int b, int hh, int m, int j) {
+  int age = m - p.ring_start;                              // ring caches: slot ring_start holds the oldest block
+  age += age < 0 ? p.num_mems : 0;
+  const int slot = (age < p.num_mems - p.k) ? 0 : age - (p.num_mems - p.k) + 1;
+  const int64_t pos = (int64_t)slot * p.block + (p.block - 1) + p.prefix_len;
+  // the landmark is the last row of block m of the cache -- or row m of an array that holds the landmark keys alone
+  const int64_t lm_row = p.lm_dense ? (int64_t)m : (int64_t)m * p.block + p.block - 1;
+  const char* src = (const char*)p.kcache + 2 * (b * p.kcs_b + hh * p.kcs_h + lm_row * p.kcs_r);
+  return {*(const u32x4_t*)(src + 16 * j), *(const u32x4_t*)(src + 16 * (j ^ (D / 16))),
+          *(const u32x4_t*)((const char*)p.cos + 2 * (pos * p.cs_r) + 16 * j),
+          *(const u32x4_t*)((const char*)p.sin + 2 * (pos * p.cs_r) + 16 * j)};
+}
+
 // One workgroup of NTHR threads rotates R * NTHR / (D / 8) landmark keys, R per thread with the loads of all R in
 // flight together; `wg` is its index among the workgroups that do so (the kernel of lmk_retrieval.hip runs nothing
 // else; the one of lmk_fwd32.hip runs them beside a forward, whose registers and LDS leave room for few workgroups
@@ -18,29 +36,18 @@ __device__ __forceinline__ void landmark_keys_body(const RetrParams& p, int wg) 
   const int tid = threadIdx.x, j = tid % LPR;
   const int64_t total = (int64_t)p.B * p.H * p.num_mems;
   int64_t row[R];
-  u32x4_t x[R], other[R], c[R], s[R];
+  LandmarkChunk k[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     row[i] = ((int64_t)wg * R + i) * RPW + tid / LPR;      // (bh, m)
     const int64_t rr = row[i] < total ? row[i] : total - 1;   // past the end: a re-read that is never stored
     const int bh = (int)(rr / p.num_mems), m = (int)(rr % p.num_mems);
-    const int b = bh / p.H, hh = bh % p.H;
-    int age = m - p.ring_start;                            // ring caches: slot ring_start holds the oldest block
-    age += age < 0 ? p.num_mems : 0;
-    const int slot = (age < p.num_mems - p.k) ? 0 : age - (p.num_mems - p.k) + 1;
-    const int64_t pos = (int64_t)slot * p.block + (p.block - 1) + p.prefix_len;
-    // the landmark is the last row of block m of the cache -- or row m of an array that holds the landmark keys alone
-    const int64_t lm_row = p.lm_dense ? (int64_t)m : (int64_t)m * p.block + p.block - 1;
-    const char* src = (const char*)p.kcache + 2 * (b * p.kcs_b + hh * p.kcs_h + lm_row * p.kcs_r);
-    x[i] = *(const u32x4_t*)(src + 16 * j);
-    other[i] = *(const u32x4_t*)(src + 16 * (j ^ (LPR / 2)));
-    c[i] = *(const u32x4_t*)((const char*)p.cos + 2 * (pos * p.cs_r) + 16 * j);
-    s[i] = *(const u32x4_t*)((const char*)p.sin + 2 * (pos * p.cs_r) + 16 * j);
+    k[i] = load_landmark_chunk<D>(p, bh / p.H, bh % p.H, m, j);
   }
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     float r[8];
-    rotate_chunk<T>(x[i], other[i], c[i], s[i], j >= LPR / 2, r);
+    rotate_chunk<T>(k[i].x, k[i].other, k[i].c, k[i].s, j >= LPR / 2, r);
     const bool ok = row[i] < total;
     u32x4_t o = {pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
     if (ok) {

@@ -82,70 +82,143 @@ __device__ __forceinline__ uint32_t prob_bits<f16_t>(float x) { return pack2<f16
 
 // Scores of every query against every landmark key, in the contract's order, into p.approx (B*H*T, num_mems).
 // The contract's dot product is a chain of fp32 fmas over d ascending, and v_mfma_f32_32x32x1_2b_f32 is 2 x 32 x 32 of
-// exactly that step: C[i][j] = fma(A[i], B[j], C[i][j]).  A wave takes 64 query rows (a lane holds its row, packed) and
-// 64 keys (lanes 0..31 hold keys 0..31, lanes 32..63 keys 32..63, packed, 16 bytes per lane and chunk straight from the
-// tiles of the rotated keys); per dimension one unpack each and two MFMAs -- the 64 rows as two blocks of 32 against
-// the keys of the first 32 lanes (BLGP 1), then against those of the other 32 (BLGP 2) -- 4 matrix-pipe cycles per
-// score.  (On the vector unit a score is 128 fmas plus whatever brings the key's value to every lane -- an unpack per
+// exactly that step: C[i][j] = fma(A[i], B[j], C[i][j]).  A wave takes 64 query rows (a lane holds its row, packed) and 32
+// keys (both halves of the wave hold them); per dimension one unpack each and one MFMA of 64 cycles.  (On the vector unit a
+// score is 128 fmas plus whatever brings the key's value to every lane -- an unpack per
 // fma with a key per lane, scalar loads of 8 bytes per score with the key in scalar registers, 16 times the LDS
 // traffic with every lane reading the value, fmas that take the value from the lane that holds it (row_newbcast) --
 // and every such kernel took 50-60 us at config 4's shapes.)
-constexpr int kScoreRows = 64, kScoreKeys = 64;                   // per wave
+// A workgroup's four waves are QW groups of query rows x 4 / QW groups of keys; it rotates its keys itself, into LDS.
+// A chain of 128 dependent MFMAs is 4 us, and what lies around it -- first loads, rotation, 32 quotients, stores -- 6 more: with
+// tiles of 64 keys and the rotation in a launch of its own, 32 heads, 256 queries, 256 blocks took 3.9 + 19.6 us (D64 3.5 + 16.4),
+// as it is 13.8 (11.0); 64 heads, 512 queries, 1024 blocks 12.1 + 103.8 and 106 (7.3 + 67.1 and 61).
+constexpr int kScoreRows = 64, kScoreKeys = 32;                   // per wave
 
-template <class T, int D>
-__global__ __launch_bounds__(256) void lmk_block_score_kernel(RetrParams p) {
+template <class T, int D, int QW>
+__global__ __launch_bounds__(256) void lmk_block_score_kernel(RetrParams p, int n_qs, int n_kc, int64_t agg_words, int agg_per_wg) {
   constexpr int CPR = D / 8;                                      // 16-byte chunks per row of 16-bit values
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int KEYS = kScoreKeys * 4 / QW;                       // of the workgroup
+  constexpr int ROWB = 2 * D + 16;                                // 16 lanes reading 16 B of 16 rows hit every bank once
+  constexpr int NI = KEYS * CPR / 256;
+  static_assert(KEYS * CPR % 256 == 0, "whole chunks per thread");
+  constexpr int QROWB = 80;                                       // a row's four chunks in the query tile: likewise
+  __shared__ __align__(16) unsigned char keys[KEYS * ROWB], rows[4][64 * QROWB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NM = p.num_mems;
-  const int n_qg = (p.T + kScoreRows - 1) / kScoreRows, n_kc = (NM + kScoreKeys - 1) / kScoreKeys;
-  // wave -> (query group, keys, head), query group first: the waves that run side by side read the same keys
-  const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
-  {
-    // the vectors the next kernel takes its maxima into start at zero: every wave of this one clears its share
-    const int64_t words = (int64_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H) * NM, n_waves = (int64_t)gridDim.x * 4;
-    const int64_t per = (words + n_waves - 1) / n_waves, end = min(words, (wid + 1) * per);
-    for (int64_t i = wid * per + lane; i < end; i += 64) p.agg[i] = 0u;
-  }
-  const int qg = (int)(wid % n_qg), kc = (int)((wid / n_qg) % n_kc);
-  const int64_t bh64 = wid / n_qg / n_kc;
-  if (bh64 >= (int64_t)p.B * p.H) return;                         // no workgroup-wide barrier in this kernel
-  const int bh = (int)bh64;
+  // workgroup -> (queries, keys, head), queries first: the workgroups that run side by side read the same keys
+  const uint32_t at = blockIdx.x / (uint32_t)n_qs;
+  const int qg = (int)(blockIdx.x - at * n_qs) * QW + wave % QW;
+  const int bh = (int)(at / (uint32_t)n_kc), m0 = (int)(at - (uint32_t)bh * n_kc) * KEYS;
   const int b = bh / p.H, hh = bh % p.H;
-  const int m0 = kc * kScoreKeys;
-  u32x4_t qp[CPR], kp[CPR];                                       // this lane's query row and key, packed
-  {
-    const int t = min(qg * kScoreRows + lane, p.T - 1);           // rows behind the last one: a re-read, never stored
-    const char* src = (const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h + (int64_t)t * p.qs_r);
+  // the keys of this thread, two at a time: four would cost head dim 128 its third wave per SIMD
+  constexpr int NB = NI < 2 ? NI : 2;
+  LandmarkChunk raw[NB];
+  auto load_raw = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
-    for (int c = 0; c < CPR; ++c) qp[c] = *(const u32x4_t*)(src + 16 * c);
-    const int m = min(m0 + lane, (int)(32 * lk_tiles(NM)) - 1);   // keys behind the last tile: likewise
-    const char* lk = (const char*)p.lk_rot + (int64_t)bh * lk_tiles(NM) * lk_tile_bytes(D) + lk_key_offset(m, D);
-#pragma unroll
-    for (int c = 0; c < CPR; ++c) kp[c] = *(const u32x4_t*)(lk + 512 * c);
-  }
-  f32x32_t lo, hi;                                                // scores against keys m0 .. +31 and m0 + 32 .. + 63
-#pragma unroll
-  for (int r = 0; r < 32; ++r) lo[r] = hi[r] = 0.f;
-#pragma unroll
-  for (int c = 0; c < CPR; ++c)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {                                 // dimension 8 c + i
-      const float qv = (i & 1) ? unpack_hi<T>(qp[c][i >> 1]) : unpack_lo<T>(qp[c][i >> 1]);
-      const float kv = (i & 1) ? unpack_hi<T>(kp[c][i >> 1]) : unpack_lo<T>(kp[c][i >> 1]);
-      lo = __builtin_amdgcn_mfma_f32_32x32x1f32(qv, kv, lo, 0, 0, 1);
-      hi = __builtin_amdgcn_mfma_f32_32x32x1f32(qv, kv, hi, 0, 0, 2);
+    for (int i = 0; i < NB; ++i) {
+      const int it = tid + 256 * (first + i);
+      raw[i] = load_landmark_chunk<D>(p, b, hh, min(m0 + it / CPR, NM - 1), it % CPR);   // keys behind the last one: a re-read, never stored
     }
-  // register 16 blk + r of lane l: row 32 blk + 8 (r / 4) + 4 (l / 32) + r % 4, key l % 32 of the accumulator's 32
-  const int key = lane & 31, rsub = 4 * (lane >> 5);
-  const int64_t row0 = (int64_t)bh * p.T;
+  };
+  load_raw(0);
+  // the wave's 64 query rows, 64 bytes of 16 rows per load; they change lanes through LDS
+  u32x4_t qp[CPR];                                                // this lane's query row, packed
+#pragma unroll
+  for (int c = 0; c < CPR; ++c) {
+    const int t = min(qg * kScoreRows + 16 * (c & 3) + (lane >> 2), p.T - 1);   // rows behind the last one: likewise
+    qp[c] = *(const u32x4_t*)((const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h + (int64_t)t * p.qs_r) + 64 * (c >> 2) + 16 * (lane & 3));
+  }
+  // the vectors the next kernel takes its maxima into start at zero: every workgroup of this one clears its share
+  for (int i = tid; i < agg_per_wg; i += 256) {
+    const int64_t w = (int64_t)blockIdx.x * agg_per_wg + i;
+    if (w < agg_words) p.agg[w] = 0u;
+  }
+#pragma unroll
+  for (int first = 0; first < NI; first += NB) {
+    if (first > 0) load_raw(first);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int it = tid + 256 * (first + i), j = it % CPR;
+      float r[8];
+      rotate_chunk<T>(raw[i].x, raw[i].other, raw[i].c, raw[i].s, j >= CPR / 2, r);
+      *(u32x4_t*)(keys + it / CPR * ROWB + 16 * j) = u32x4_t{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int c = 0; c < CPR; c += 4) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();                              // the chunks before have been read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(u32x4_t*)(rows[wave] + (16 * i + (lane >> 2)) * QROWB + 16 * (lane & 3)) = qp[c + i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qp[c + i] = *(const u32x4_t*)(rows[wave] + lane * QROWB + 16 * i);
+  }
+  __syncthreads();
+  const int k0 = wave / QW * kScoreKeys, key = lane & 31;
+  if (qg * kScoreRows >= p.T || m0 + k0 >= NM) return;            // no barrier below
+  // its key, two chunks at a time: as a whole it would cost a third of the waves a SIMD takes
+  u32x4_t kp[2];
+  auto load_key = [&](int c) __attribute__((always_inline)) { kp[c & 1] = *(const u32x4_t*)(keys + (k0 + key) * ROWB + 16 * c); };
+  load_key(0);
+  load_key(1);
+  f32x32_t acc;
+#pragma unroll
+  for (int r = 0; r < 32; ++r) acc[r] = 0.f;
+  // dimensions 8 c + i.  A chunk's operands are unpacked together, under the MFMAs of the chunk before: an unpack that writes
+  // the operand of an MFMA in flight waits for its end
+  float qv[2][8], kv[2][8];
+  auto unpack = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      qv[c & 1][i] = (i & 1) ? unpack_hi<T>(qp[c][i >> 1]) : unpack_lo<T>(qp[c][i >> 1]);
+      kv[c & 1][i] = (i & 1) ? unpack_hi<T>(kp[c & 1][i >> 1]) : unpack_lo<T>(kp[c & 1][i >> 1]);
+      asm volatile("" : "+v"(qv[c & 1][i]), "+v"(kv[c & 1][i]));
+    }
+    if (c + 2 < CPR) load_key(c + 2);
+  };
+  unpack(0);
+#pragma unroll
+  for (int c = 0; c < CPR; ++c) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x1f32(qv[c & 1][i], kv[c & 1][i], acc, 0, 0, 0);
+      if (i == 3 && c + 1 < CPR) unpack(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 32; ++r) acc[r] = contract<T>(acc[r], p.sqrt_hd);
+  // register 16 blk + r of lane l: row 32 blk + 8 (r / 4) + 4 (l / 32) + r % 4, key l % 32
+  if (m0 + k0 + key >= NM) return;
+  const int t0 = qg * kScoreRows + 4 * (lane >> 5);
+  float* dst = p.approx + ((int64_t)bh * p.T + t0) * NM + m0 + k0 + key;
+  const bool whole = (qg + 1) * kScoreRows <= p.T;                // uniform
 #pragma unroll
   for (int r = 0; r < 32; ++r) {
-    const int t = qg * kScoreRows + 32 * (r >> 4) + 8 * ((r & 15) >> 2) + rsub + (r & 3);
-    if (t >= p.T) continue;
-    float* dst = p.approx + (row0 + t) * NM + m0 + key;
-    if (m0 + key < NM) dst[0] = contract<T>(lo[r], p.sqrt_hd);
-    if (m0 + 32 + key < NM) dst[32] = contract<T>(hi[r], p.sqrt_hd);
+    const int t = 32 * (r >> 4) + 8 * ((r & 15) >> 2) + (r & 3);
+    if (whole || t0 + t < p.T) dst[(int64_t)t * NM] = acc[r];
   }
+}
+
+template <class T, int D>
+static int launch_scores(const RetrParams& p, hipStream_t stream) {
+  // A workgroup's waves share its keys as far as there are query rows for them and at most a quarter of the waves is left
+  // without (5 groups of rows, 24 heads of 512 blocks, D128: a step takes 73.6 us with four waves along the rows, 72.9 with two)
+  const int groups = (p.T + kScoreRows - 1) / kScoreRows;
+  int qw = 4;
+  while (qw > 1 && 3 * ((groups + qw - 1) / qw * qw) > 4 * groups) qw >>= 1;
+  const int keys = kScoreKeys * 4 / qw, n_qs = (groups + qw - 1) / qw, n_kc = (p.num_mems + keys - 1) / keys;
+  const int64_t wgs = (int64_t)p.B * p.H * n_qs * n_kc, words = (int64_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H) * p.num_mems;
+  const int per_wg = (int)((words + wgs - 1) / wgs);
+  const dim3 grid((unsigned)wgs);
+  if (qw == 4) hipLaunchKernelGGL((lmk_block_score_kernel<T, D, 4>), grid, dim3(256), 0, stream, p, n_qs, n_kc, words, per_wg);
+  else if (qw == 2) hipLaunchKernelGGL((lmk_block_score_kernel<T, D, 2>), grid, dim3(256), 0, stream, p, n_qs, n_kc, words, per_wg);
+  else hipLaunchKernelGGL((lmk_block_score_kernel<T, D, 1>), grid, dim3(256), 0, stream, p, n_qs, n_kc, words, per_wg);
+  return (int)hipGetLastError();
 }
 
 // The rows' scores (p.approx) -> softmax -> 16-bit probabilities -> maximum per block into agg, which holds zeros on
@@ -1150,15 +1223,9 @@ static int launch_topk_t(const RetrParams& p, bool reuse_landmark_keys, hipStrea
 
 template <class T, int D>
 static int launch_topk_shared_t(const RetrParams& p, hipStream_t stream) {
-  constexpr int RPW = 256 / (D / 8);
-  const int64_t lkrows = (int64_t)p.B * p.H * p.num_mems;
   int rc;
-  hipLaunchKernelGGL((lmk_landmark_keys_kernel<T, D>), dim3((unsigned)((lkrows + RPW - 1) / RPW)), dim3(256), 0, stream, p);
-  if ((rc = (int)hipGetLastError())) return rc;
   const int64_t sel_rows = p.agg_over_heads ? (int64_t)p.B * p.T : (int64_t)p.B * p.H;   // vectors to pick from
-  const int64_t score_waves = (int64_t)p.B * p.H * ((p.T + kScoreRows - 1) / kScoreRows) * ((p.num_mems + kScoreKeys - 1) / kScoreKeys);
-  hipLaunchKernelGGL((lmk_block_score_kernel<T, D>), dim3((unsigned)((score_waves + 3) / 4)), dim3(256), 0, stream, p);
-  if ((rc = (int)hipGetLastError())) return rc;
+  if ((rc = launch_scores<T, D>(p, stream))) return rc;
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   const int is_bf16 = std::is_same<T, bf16_t>::value ? 1 : 0;
   if (p.num_mems <= 64 * 32) {

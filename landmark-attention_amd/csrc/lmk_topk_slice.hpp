@@ -12,9 +12,15 @@ namespace lmk {
 // ---------------------------------------------------------------------------
 // helpers of the selection: the rounding contract and a wave-wide arg-best
 // ---------------------------------------------------------------------------
+// round(x / s) for a 16-bit value x and s = sqrt(64) or sqrt(128), without a division's ten dependent steps: q = x y with y
+// the nearest to 1 / s, then one step with the exact remainder (Markstein), which rounds to what IEEE division rounds to for
+// all 65536 values of either type (tests/test_score_contract.py goes through them).  An exact q, infinities and NaN have no
+// step to take.
 template <class T>
 __device__ __forceinline__ float contract(float dot, float sqrt_hd) {
-  return round_to<T>(__fdiv_rn(round_to<T>(dot), sqrt_hd));
+  const float x = round_to<T>(dot), y = 1.0f / sqrt_hd, q = x * y;
+  const float r = __builtin_fmaf(-q, sqrt_hd, x);
+  return round_to<T>(fabsf(r) > 0.f ? __builtin_fmaf(r, y, q) : q);
 }
 
 // wave-wide arg-best under (value desc, index asc); every lane gets the winner.  Inside a row of 16
