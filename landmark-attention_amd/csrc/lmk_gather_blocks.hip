@@ -280,12 +280,13 @@ __global__ __launch_bounds__(256, 2) void lmk_gather_blocks_kernel(RetrParams p,
 template <class T, int D>
 __global__ __launch_bounds__(256) void lmk_gather_combine_kernel(RetrParams p, int t_first, int t_rows) {
   constexpr int LPR = D / 4;
-  const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
-  if (row >= (int64_t)p.B * p.H * t_rows) return;
+  const uint32_t row = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;   // 32-bit as every launch's threads are
   const int j = threadIdx.x % LPR, k = p.k;
-  const int bh = (int)(row / t_rows), t = t_first + (int)(row % t_rows), b = bh / p.H, hh = bh % p.H;
-  const float* sc = p.part_score + row * k;
-  const float* part = p.part + row * k * D + 4 * j;
+  const int bh = (int)(row / (uint32_t)t_rows), t = t_first + (int)(row - (uint32_t)bh * t_rows);
+  if (bh >= p.B * p.H) return;
+  const int b = (int)((uint32_t)bh / (uint32_t)p.H), hh = bh - b * p.H;
+  const float* sc = p.part_score + (int64_t)row * k;
+  const float* part = p.part + (int64_t)row * k * D + 4 * j;
   const int64_t srow = (int64_t)bh * p.stat_stride + t;
   const float Ml = p.M_loc[srow] * kLog2e, Ll = p.L_loc[srow];
   const u32x2_t ol = *(const u32x2_t*)((const char*)p.o_loc + 2 * (b * p.ols_b + hh * p.ols_h + (int64_t)t * p.ols_r) + 8 * j);

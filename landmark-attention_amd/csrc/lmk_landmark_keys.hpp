@@ -34,15 +34,19 @@ __device__ __forceinline__ void landmark_keys_body(const RetrParams& p, int wg) 
   constexpr int LPR = D / 8;
   constexpr int RPW = NTHR / LPR;
   const int tid = threadIdx.x, j = tid % LPR;
-  const int64_t total = (int64_t)p.B * p.H * p.num_mems;
-  int64_t row[R];
+  // indices of threads and of what they work on stay below 2^32, the launch's own limit: a 64-bit division is 100 instructions
+  const uint32_t total = (uint32_t)(p.B * p.H) * (uint32_t)p.num_mems;
+  uint32_t row[R];
+  int bh[R], m[R];
   LandmarkChunk k[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    row[i] = ((int64_t)wg * R + i) * RPW + tid / LPR;      // (bh, m)
-    const int64_t rr = row[i] < total ? row[i] : total - 1;   // past the end: a re-read that is never stored
-    const int bh = (int)(rr / p.num_mems), m = (int)(rr % p.num_mems);
-    k[i] = load_landmark_chunk<D>(p, bh / p.H, bh % p.H, m, j);
+    row[i] = ((uint32_t)wg * R + i) * RPW + tid / LPR;     // (bh, m)
+    const uint32_t rr = min(row[i], total - 1);            // past the end: a re-read that is never stored
+    bh[i] = (int)(rr / (uint32_t)p.num_mems);
+    m[i] = (int)(rr - (uint32_t)bh[i] * p.num_mems);
+    const int b = (int)((uint32_t)bh[i] / (uint32_t)p.H);
+    k[i] = load_landmark_chunk<D>(p, b, bh[i] - b * p.H, m[i], j);
   }
 #pragma unroll
   for (int i = 0; i < R; ++i) {
@@ -50,11 +54,7 @@ __device__ __forceinline__ void landmark_keys_body(const RetrParams& p, int wg) 
     rotate_chunk<T>(k[i].x, k[i].other, k[i].c, k[i].s, j >= LPR / 2, r);
     const bool ok = row[i] < total;
     u32x4_t o = {pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
-    if (ok) {
-      const int64_t bh = row[i] / p.num_mems;
-      const int m = (int)(row[i] % p.num_mems);
-      *(u32x4_t*)((char*)p.lk_rot + bh * lk_tiles(p.num_mems) * lk_tile_bytes(D) + lk_key_offset(m, D) + 512 * j) = o;
-    }
+    if (ok) *(u32x4_t*)((char*)p.lk_rot + bh[i] * lk_tiles(p.num_mems) * lk_tile_bytes(D) + lk_key_offset(m[i], D) + 512 * j) = o;
     float nrm = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) nrm += r[e] * r[e];

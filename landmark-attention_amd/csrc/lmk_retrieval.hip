@@ -230,21 +230,22 @@ static int launch_scores(const RetrParams& p, hipStream_t stream) {
 // patterns order like the values.
 template <int NPL>
 __global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int model_is_bf16, int rows_per_wave) {
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int NM = p.num_mems;
   // rows that share a vector: the T queries of a (batch, head), or the H heads of a (batch, query)
   const int group = p.agg_over_heads ? p.H : p.T;
   const int per_group = (group + rows_per_wave - 1) / rows_per_wave;
-  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= (int64_t)per_group * (p.agg_over_heads ? p.B * p.T : p.B * p.H)) return;
-  const int64_t vec = w / per_group;                              // (batch, query) or (batch, head)
-  const int first = (int)(w % per_group) * rows_per_wave, last = min(first + rows_per_wave, group);
+  const uint32_t w = blockIdx.x * 4 + wave;                       // scalar, and 32-bit as every launch's waves are
+  const uint32_t vec = w / (uint32_t)per_group;                   // (batch, query) or (batch, head)
+  if (vec >= (uint32_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H)) return;
+  const int first = (int)(w - vec * per_group) * rows_per_wave, last = min(first + rows_per_wave, group);
+  const uint32_t vec_b = vec / (uint32_t)p.T, vec_t = vec - vec_b * p.T;   // (with agg_over_heads)
   uint32_t best[NPL];
 #pragma unroll
   for (int i = 0; i < NPL; ++i) best[i] = 0u;
   for (int g = first; g < last; ++g) {
     // over heads: vec = b T + t, row (b H + g) T + t; over queries: vec = b H + h, row vec T + g
-    const int64_t row = p.agg_over_heads ? ((vec / p.T) * p.H + g) * p.T + vec % p.T : vec * p.T + g;
+    const int64_t row = p.agg_over_heads ? ((int64_t)vec_b * p.H + g) * p.T + vec_t : (int64_t)vec * p.T + g;
     const float* sc = p.approx + row * NM;
     float x[NPL];
 #pragma unroll
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int m
       }
     }
   }
-  uint32_t* agg = p.agg + vec * NM;
+  uint32_t* agg = p.agg + (int64_t)vec * NM;
 #pragma unroll
   for (int i = 0; i < NPL; ++i)
     if (lane + 64 * i < NM) atomicMax(agg + lane + 64 * i, best[i]);
@@ -826,16 +827,17 @@ void lmk_gather_attend_kernel(RetrParams p) {
   using vec_t = typename PieceVec<E>::type;                       // one piece: E 16-bit values
   constexpr int KPG = CK / 8;                                     // keys per 8-lane group and chunk
   constexpr int NC = BS / CK;                                     // chunks per block
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = SPLIT ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);   // (what SPLIT makes of it overflows the scalar registers)
   const int j = lane & 7, g = lane >> 3;                           // head-dim chunk pair, key group
   // (bh, t): a wave's own row, or -- SPLIT, for launches with few rows -- the workgroup's row, whose
   // selected blocks its waves share out (block js goes to wave js % nblk) and merge at the end
-  const int64_t row = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
-  if (row >= (int64_t)p.B * p.H * p.T) return;                    // SPLIT: the whole workgroup leaves
+  const uint32_t row = SPLIT ? blockIdx.x : blockIdx.x * 4 + wave;   // scalar, and 32-bit as every launch's waves are
+  if (row >= (uint32_t)(p.B * p.H) * (uint32_t)p.T) return;       // SPLIT: the whole workgroup leaves
   const int js0 = SPLIT ? (wave < nblk ? wave : p.k) : 0, jstep = nblk;   // (a wave of the window's own takes no block)
   const bool windows = LOCAL && (!SPLIT || wave == p.window_wave);
-  const int bh = (int)(row / p.T), t = (int)(row % p.T);
-  const int b = bh / p.H, hh = bh % p.H;
+  const int bh = (int)(row / (uint32_t)p.T), t = (int)(row - (uint32_t)bh * p.T);
+  const int b = (int)((uint32_t)bh / (uint32_t)p.H), hh = bh - b * p.H;
 
   auto unpack8 = [](const vec_t u, float* o) {
 #pragma unroll
@@ -1404,15 +1406,15 @@ __global__ __launch_bounds__(256) void lmk_local_window_kernel(WindowParams p) {
   constexpr int RPW = 256 / LPR;
   const int tid = threadIdx.x, j = tid % LPR;
   const int W = p.n_sel + p.inc + p.T;
-  const int64_t row = (int64_t)blockIdx.x * RPW + tid / LPR;      // (bh, r)
-  if (row >= (int64_t)p.B * p.H * W) return;
-  const int bh = (int)(row / W), r = (int)(row % W);
-  const int b = bh / p.H, hh = bh % p.H;
+  const uint32_t row = blockIdx.x * RPW + tid / LPR;              // (bh, r); 32-bit as every launch's threads are
+  const int bh = (int)(row / (uint32_t)W), r = (int)(row - (uint32_t)bh * W);
+  if (bh >= p.B * p.H) return;
+  const int b = (int)((uint32_t)bh / (uint32_t)p.H), hh = bh - b * p.H;
   u32x4_t qo = {0, 0, 0, 0}, ko, vo;
   if (r < p.n_sel + p.inc) {
     int64_t src_row, pos;
     if (r < p.n_sel) {
-      const int slot = r / p.block, tok = r % p.block;
+      const int slot = (int)((uint32_t)r / (uint32_t)p.block), tok = r - slot * p.block;
       int64_t blk = p.idx[(int64_t)bh * p.k + slot];
       blk = blk < 0 ? 0 : (blk >= p.num_mems ? p.num_mems - 1 : blk);   // never read outside the cache
       src_row = blk * p.block + tok;
@@ -1453,66 +1455,79 @@ static int launch_window_t(const WindowParams& p, hipStream_t stream) {
 // ---------------------------------------------------------------------------
 // rotary embedding of a whole (B, H, L, D) tensor at per-(batch, token) positions
 // (apply_rotary_pos_emb, llama_mem.py:134-149): x*cos + rotate_half(x)*sin with the model dtype's
-// rounding after each of the three elementwise operations.  One 16-byte chunk per thread; a row's
-// chunks sit in one wave and every lane loads before any lane stores, so out may be x itself.
+// rounding after each of the three elementwise operations.  A thread takes the 16-byte chunk j of a row's first half and
+// its partner of the second, so that every value is read once, and reads both before it stores either: out may be x itself.
 // PAIR: a second tensor of the same shape (the layer's q and k, :298) is rotated by the same thread with the
 // same table rows, in the same launch.
+// Rows that lie side by side in memory -- the heads of a token in (B, L, H, D)-backed views -- are taken side by side.
+// Bound by memory: 2 x 128 heads of 512 rows of 128 (67 MB) take 13.2 us, 5.1 TB/s; with 64-bit row indices, 73 wide multiplies
+// a thread, and every row read twice 14.7.
 // ---------------------------------------------------------------------------
 template <class T, int D, bool PAIR>
-__global__ __launch_bounds__(256) void lmk_rotary_kernel(RotaryParams p) {
-  constexpr int LPR = D / 8;
+__global__ __launch_bounds__(256) void lmk_rotary_kernel(RotaryParams p, int heads_inner) {
+  constexpr int LPR = D / 16;
   constexpr int RPW = 256 / LPR;
   const int tid = threadIdx.x, j = tid % LPR;
-  const int64_t row = (int64_t)blockIdx.x * RPW + tid / LPR;      // (b, h, l)
-  if (row >= (int64_t)p.B * p.H * p.L) return;
-  const int l = (int)(row % p.L);
-  const int bh = (int)(row / p.L);
-  const int b = bh / p.H, hh = bh % p.H;
+  const uint32_t n = blockIdx.x * RPW + tid / LPR;                // row of the batch's L H
+  const uint32_t inner = heads_inner ? p.H : p.L;
+  const int q = (int)(n / inner), r = (int)(n - (uint32_t)q * inner);
+  const int l = heads_inner ? q : r, hh = heads_inner ? r : q, b = p.b0 + blockIdx.y;
+  if (q >= (heads_inner ? p.L : p.H)) return;
   int64_t pos = p.pos[(int64_t)b * p.pos_stride_b + l];
   pos = pos < 0 ? 0 : (pos >= p.n_pos ? p.n_pos - 1 : pos);      // never read outside the tables
-  const char* src = (const char*)p.x + 2 * (b * p.xs_b + hh * p.xs_h + (int64_t)l * p.xs_r);
-  const u32x4_t x = *(const u32x4_t*)(src + 16 * j);
-  const u32x4_t other = *(const u32x4_t*)(src + 16 * (j ^ (LPR / 2)));
-  u32x4_t x2 = {0, 0, 0, 0}, other2 = {0, 0, 0, 0};
+  const char* src = (const char*)p.x + 2 * (b * p.xs_b + hh * p.xs_h + (int64_t)l * p.xs_r) + 16 * j;
+  const u32x4_t lo = *(const u32x4_t*)src, hi = *(const u32x4_t*)(src + D);
+  u32x4_t lo2 = {0, 0, 0, 0}, hi2 = {0, 0, 0, 0};
   if (PAIR) {                                                     // the second tensor's row at the same (b, h, l)
-    const char* src2 = (const char*)p.x2 + 2 * (b * p.x2s_b + hh * p.x2s_h + (int64_t)l * p.x2s_r);
-    x2 = *(const u32x4_t*)(src2 + 16 * j);
-    other2 = *(const u32x4_t*)(src2 + 16 * (j ^ (LPR / 2)));
+    const char* src2 = (const char*)p.x2 + 2 * (b * p.x2s_b + hh * p.x2s_h + (int64_t)l * p.x2s_r) + 16 * j;
+    lo2 = *(const u32x4_t*)src2;
+    hi2 = *(const u32x4_t*)(src2 + D);
   }
-  const u32x4_t c = *(const u32x4_t*)((const char*)p.cos + 2 * (pos * p.cs_r) + 16 * j);
-  u32x4_t s = *(const u32x4_t*)((const char*)p.sin + 2 * (pos * p.cs_r) + 16 * (p.transposed ? j ^ (LPR / 2) : j));
+  const char *cr = (const char*)p.cos + 2 * (pos * p.cs_r) + 16 * j, *sr = (const char*)p.sin + 2 * (pos * p.cs_r) + 16 * j;
+  const u32x4_t cl = *(const u32x4_t*)cr, ch = *(const u32x4_t*)(cr + D);
+  u32x4_t sl = *(const u32x4_t*)(sr + (p.transposed ? D : 0)), sh = *(const u32x4_t*)(sr + (p.transposed ? 0 : D));
   const uint32_t flip = p.transposed ? 0x80008000u : 0u;         // sign bits of two 16-bit values
 #pragma unroll
-  for (int i = 0; i < 4; ++i) s[i] ^= flip;
-  float o[8];
-  rotate_chunk<T>(x, other, c, s, j >= LPR / 2, o);
-  const u32x4_t r = {pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};
-  *(u32x4_t*)((char*)p.out + 2 * (b * p.os_b + hh * p.os_h + (int64_t)l * p.os_r) + 16 * j) = r;
-  if (PAIR) {
-    rotate_chunk<T>(x2, other2, c, s, j >= LPR / 2, o);
-    const u32x4_t r2 = {pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};
-    *(u32x4_t*)((char*)p.out2 + 2 * (b * p.o2s_b + hh * p.o2s_h + (int64_t)l * p.o2s_r) + 16 * j) = r2;
+  for (int i = 0; i < 4; ++i) {
+    sl[i] ^= flip;
+    sh[i] ^= flip;
   }
+  auto rotate = [&](const u32x4_t& a, const u32x4_t& z, char* dst) __attribute__((always_inline)) {
+    float o[8];
+    rotate_chunk<T>(a, z, cl, sl, false, o);
+    const u32x4_t x = {pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};
+    rotate_chunk<T>(z, a, ch, sh, true, o);
+    const u32x4_t y = {pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])};
+    *(u32x4_t*)dst = x;
+    *(u32x4_t*)(dst + D) = y;
+  };
+  rotate(lo, hi, (char*)p.out + 2 * (b * p.os_b + hh * p.os_h + (int64_t)l * p.os_r) + 16 * j);
+  if (PAIR) rotate(lo2, hi2, (char*)p.out2 + 2 * (b * p.o2s_b + hh * p.o2s_h + (int64_t)l * p.o2s_r) + 16 * j);
 }
 
 template <class T, int D>
 static int launch_rotary_t(const RotaryParams& p, hipStream_t stream) {
-  constexpr int RPW = 256 / (D / 8);
-  const int64_t rows = (int64_t)p.B * p.H * p.L;
-  const dim3 grid((unsigned)((rows + RPW - 1) / RPW));
-  if (p.x2 != nullptr) hipLaunchKernelGGL((lmk_rotary_kernel<T, D, true>), grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((lmk_rotary_kernel<T, D, false>), grid, dim3(256), 0, stream, p);
+  constexpr int RPW = 256 / (D / 16), kMax = 65535;               // the grid's y is 16 bits
+  const int64_t rows = (int64_t)p.H * p.L;
+  const int heads_inner = p.xs_h < p.xs_r ? 1 : 0;
+  RotaryParams c = p;
+  for (c.b0 = 0; c.b0 < p.B; c.b0 += kMax) {
+    const dim3 grid((unsigned)((rows + RPW - 1) / RPW), std::min(p.B - c.b0, kMax));
+    if (p.x2 != nullptr) hipLaunchKernelGGL((lmk_rotary_kernel<T, D, true>), grid, dim3(256), 0, stream, c, heads_inner);
+    else hipLaunchKernelGGL((lmk_rotary_kernel<T, D, false>), grid, dim3(256), 0, stream, c, heads_inner);
+  }
   return (int)hipGetLastError();
 }
 
 // New rows of a cache's keys (blockIdx.y 0) and values (1), one 16-byte chunk per thread.
 __global__ __launch_bounds__(256) void lmk_copy_rows_kernel(CopyRowsParams p) {
   const int w = blockIdx.y;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = i / p.chunks;
-  const int c = (int)(i % p.chunks);
-  if (row >= (int64_t)p.B * p.H * p.T) return;
-  const int t = (int)(row % p.T), bh = (int)(row / p.T), b = bh / p.H, h = bh % p.H;
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;              // 32-bit as every launch's threads are
+  const uint32_t row = i / (uint32_t)p.chunks;
+  const int c = (int)(i - row * p.chunks);
+  const int bh = (int)(row / (uint32_t)p.T), t = (int)(row - (uint32_t)bh * p.T);
+  if (bh >= p.B * p.H) return;
+  const int b = (int)((uint32_t)bh / (uint32_t)p.H), h = bh - b * p.H;
   const char* s = (const char*)p.src[w] + 2 * (b * p.ss_b[w] + h * p.ss_h[w] + t * p.ss_r[w]) + 16 * c;
   char* d = (char*)p.dst[w] + 2 * (b * p.ds_b[w] + h * p.ds_h[w] + t * p.ds_r[w]) + 16 * c;
   *(u32x4_t*)d = *(const u32x4_t*)s;
@@ -1523,30 +1538,28 @@ __global__ __launch_bounds__(256) void lmk_copy_rows_kernel(CopyRowsParams p) {
 // row i < n_tail goes to the ring and then, if the new tail has a row i, fetches that row too.
 __global__ __launch_bounds__(256) void lmk_ring_store_kernel(RingStoreParams p) {
   const int w = blockIdx.y, rows = p.n_tail + p.T, rest = rows - p.full;
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t n = blockIdx.x * 256 + threadIdx.x;              // 32-bit as every launch's threads are
   if (w == 2) {
-    const int j = (int)(n % p.block);
-    const int64_t b = n / p.block;
+    const int b = (int)(n / (uint32_t)p.block), j = (int)(n - (uint32_t)b * p.block);
     const int src = p.full + j - p.n_tail;                        // token of the chunk behind row j of the tail; < 0: row j stays
     if (b < p.B && j < rest && src >= 0) p.tail_is_mem[b * p.tims_b + j] = p.is_mem[b * p.ims_b + src];
     return;
   }
-  const int c = (int)(n % p.chunks);
-  const int64_t bhi = n / p.chunks;
-  const int i = (int)(bhi % rows);
-  const int64_t bh = bhi / rows;
-  if (bh >= (int64_t)p.B * p.H) return;
-  const int b = (int)(bh / p.H), h = (int)(bh % p.H);
+  const uint32_t bhi = n / (uint32_t)p.chunks;
+  const int c = (int)(n - bhi * p.chunks);
+  const int bh = (int)(bhi / (uint32_t)rows), i = (int)(bhi - (uint32_t)bh * rows);
+  if (bh >= p.B * p.H) return;
+  const int b = (int)((uint32_t)bh / (uint32_t)p.H), h = bh - b * p.H;
   const char* src = (const char*)p.src[w] + 2 * (b * p.ss_b[w] + h * p.ss_h[w]) + 16 * c;
   char* tail = (char*)p.tail[w] + 2 * (b * p.ts_b[w] + h * p.ts_h[w]) + 16 * c;
   auto chunk_row = [&](int t) { return *(const u32x4_t*)(src + 2 * t * p.ss_r[w]); };
   auto tail_row = [&](int j) { return (u32x4_t*)(tail + 2 * j * p.ts_r[w]); };
   if (i < p.full) {
     const u32x4_t x = i < p.n_tail ? *tail_row(i) : chunk_row(i - p.n_tail);
-    const int blk = i / p.block - p.dropped;
+    const int whole = (int)((uint32_t)i / (uint32_t)p.block), blk = whole - p.dropped;
     if (blk >= 0) {
-      const int slot = (p.first_slot + blk) % p.n_slots;
-      *(u32x4_t*)((char*)p.ring[w] + 2 * (b * p.rs_b + slot * p.rs_slot + (i % p.block) * p.rs_tok + h * p.rs_h) + 16 * c) = x;
+      const int slot = (int)((uint32_t)(p.first_slot + blk) % (uint32_t)p.n_slots);
+      *(u32x4_t*)((char*)p.ring[w] + 2 * (b * p.rs_b + slot * p.rs_slot + (i - whole * p.block) * p.rs_tok + h * p.rs_h) + 16 * c) = x;
     }
     if (i < p.n_tail && i < rest) *tail_row(i) = chunk_row(p.full + i - p.n_tail);   // full > n_tail: a token of the chunk
   } else {
