@@ -168,7 +168,7 @@ struct RetrParams {
   // gather step with the rows' local window inside (local != 0): the new tokens' keys and values (rotated by the
   // caller), the number of cached tokens behind the last complete block, their first row in the cache and its position
   int local, local_inc;
-  int block_waves, window_wave;                   // of a row's waves: those that share its blocks out, the one with its window
+  int block_waves;                                // of a row's waves: those that share its blocks out
   const void *k_new, *v_new;
   int64_t kns_b, kns_h, kns_r, vns_b, vns_h, vns_r, local_row0, local_pos0;
   // with `local`, optional: the new tokens' rows (keys without rotary, values) are stored in the cache on the way
@@ -274,6 +274,7 @@ inline bool gather_takes_local_window(int T, int S, int block) {
 }
 // BS: slots per block (32, 64 or 128); p.block <= BS tokens per block in the cache
 int launch_gather_attend(const RetrParams& p, int D, int BS, int dtype, hipStream_t stream);
+int launch_gather_decode(const RetrParams& p, int D, int dtype, hipStream_t stream);   // p.local: blocks of 32, 64 and 128 as they are
 
 // Gather by block (lmk_gather_blocks.hip): the rows of a (batch, head) whose picks the workspace holds at a time, or 0 where
 // the gather by row serves.  A rotation of a block's keys serves the picks of one rank, and a block is picked at about

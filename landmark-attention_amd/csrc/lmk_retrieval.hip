@@ -791,14 +791,6 @@ __device__ __forceinline__ float sum8(float d) {                  // sum over th
 // 128; without it two run whichever is taken, and 64 keys keep more loads in flight (a chunk step at block 64: 256 queries of
 // 32 heads, top 4, 186.5 -> 184.0 us; 64 queries, top 5, 86.6 -> 83.5).
 constexpr int gather_chunk(int BS, int D, bool LOCAL) { return BS == 32 || (LOCAL && BS == 64 && D == 128) ? 32 : 64; }
-// Most waves that share out a row's blocks when its window is attended to here as well.  A wave per block keeps no wave
-// walking two of them one after the other while the others are done; beyond six, waves of two blocks each are level again
-// and their partial sums cheaper to merge (1024 rows, block 32, top 8: 72.4 with eight waves, 66.6 us with four).  Blocks of
-// 128 hold 237 registers (head dim 64) or 307 (128): a fifth wave of blocks would halve the waves a CU takes.
-constexpr int gather_waves(int BS, int D, int CK) { return BS == 128 ? 4 : BS == 64 && D == 128 ? (CK == 64 ? 4 : 8) : 6; }
-// The same with a wave for the window alone, which blocks of 128 at head dim 128 have no room for: the workgroup's registers
-// would be halved to 256, 90 of them spilled (128 rows, top 7: 43.2 against 31.9 us; 512 rows, top 4: 64.8 against 58.3).
-constexpr int gather_max_waves(int BS, int D, int CK) { return gather_waves(BS, D, CK) + (BS == 128 && D == 128 ? 0 : 1); }
 template <int E> struct PieceVec;
 template <> struct PieceVec<8> { using type = u32x4_t; };
 template <> struct PieceVec<4> { using type = u32x2_t; };
@@ -810,32 +802,26 @@ template <> struct PieceVec<4> { using type = u32x2_t; };
 // softmax, instead of coming in as (o_loc, L_loc, M_loc) from a forward launch over a window another launch built:
 // a decode step is then the selection and this kernel.  Its keys join the global bucket directly (own-block rule:
 // causal, the landmark token does not see itself; flash_landmark_attention.py:78-100).
-// With SPLIT a row has a workgroup, in which p.block_waves waves share its blocks out and wave p.window_wave takes its window
-// (32 sequences of 32 heads over 4096 tokens, new inputs on every pass: five blocks of 64 each 78.4 with four waves for the
-// blocks and chunks of 64, 73.8 us as it is; three blocks 62.3 and 45.7).
+// (Decode steps of more rows than lmk_gather_decode_kernel is the better one for.)
 template <class T, int D, int BS, bool SPLIT, bool PADDED, bool MERGE = false, bool LOCAL = false,
           int CK = gather_chunk(BS, D, LOCAL)>
-__global__ __launch_bounds__(SPLIT && LOCAL ? 64 * gather_max_waves(BS, D, CK) : 256,
-                             SPLIT && LOCAL && gather_waves(BS, D, CK) > 4 ? 3 : 1)
-void lmk_gather_attend_kernel(RetrParams p) {
-  const int nblk = SPLIT ? (LOCAL ? p.block_waves : 4) : 1;       // waves that share the row's blocks out
-  constexpr int NWV = SPLIT ? (LOCAL ? gather_max_waves(BS, D, CK) : 4) : 1;
+__global__ __launch_bounds__(256) void lmk_gather_attend_kernel(RetrParams p) {
+  constexpr int NWV = SPLIT ? 4 : 1;                              // waves that share the row's blocks out
   static_assert((D == 128 || D == 64) && (BS == 32 || BS % 64 == 0), "8 lanes x 2 pieces per row; whole chunks of keys");
-  static_assert(!LOCAL || !PADDED, "the local window sits in a block of BS tokens");
+  static_assert(!LOCAL || (!PADDED && !SPLIT), "the local window sits in a block of BS tokens; a wave per row");
   constexpr int E = D / 16;                                       // head dims per lane and rotary half: 8 or 4
   constexpr int PB = 2 * E;                                       // bytes of one piece
   using vec_t = typename PieceVec<E>::type;                       // one piece: E 16-bit values
   constexpr int KPG = CK / 8;                                     // keys per 8-lane group and chunk
   constexpr int NC = BS / CK;                                     // chunks per block
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = SPLIT ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);   // (what SPLIT makes of it overflows the scalar registers)
+  const int wave = SPLIT || LOCAL ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);   // (what they make of it overflows the scalar registers)
   const int j = lane & 7, g = lane >> 3;                           // head-dim chunk pair, key group
   // (bh, t): a wave's own row, or -- SPLIT, for launches with few rows -- the workgroup's row, whose
-  // selected blocks its waves share out (block js goes to wave js % nblk) and merge at the end
+  // selected blocks its waves share out (block js goes to wave js % 4) and merge at the end
   const uint32_t row = SPLIT ? blockIdx.x : blockIdx.x * 4 + wave;   // scalar, and 32-bit as every launch's waves are
   if (row >= (uint32_t)(p.B * p.H) * (uint32_t)p.T) return;       // SPLIT: the whole workgroup leaves
-  const int js0 = SPLIT ? (wave < nblk ? wave : p.k) : 0, jstep = nblk;   // (a wave of the window's own takes no block)
-  const bool windows = LOCAL && (!SPLIT || wave == p.window_wave);
+  const int js0 = SPLIT ? wave : 0, jstep = NWV;
   const int bh = (int)(row / (uint32_t)p.T), t = (int)(row - (uint32_t)bh * p.T);
   const int b = (int)((uint32_t)bh / (uint32_t)p.H), hh = bh - b * p.H;
 
@@ -852,10 +838,10 @@ void lmk_gather_attend_kernel(RetrParams p) {
     unpack8(*(const vec_t*)(qp + PB * j), qlo);
     unpack8(*(const vec_t*)(qp + D + PB * j), qhi);
   }
-  // The row's own key (without rotary) and value on their way into the cache: fetched here by one of the row's waves
+  // The row's own key (without rotary) and value on their way into the cache: fetched here
   // (lanes 0 .. D/8-1 the key, 32 .. the value), stored at the end, so that nothing waits for them.  Nobody reads the
   // destination in this launch: it lies behind the cached rows.
-  const bool appends = windows && p.ap_k != nullptr && (lane & 31) < D / 8;
+  const bool appends = LOCAL && p.ap_k != nullptr && (lane & 31) < D / 8;
   u32x4_t ap = {0, 0, 0, 0};
   if (LOCAL && appends)
     ap = *(const u32x4_t*)((lane < 32 ? (const char*)p.ap_k + 2 * (b * p.aks_b + hh * p.aks_h + (int64_t)t * p.aks_r)
@@ -916,80 +902,78 @@ void lmk_gather_attend_kernel(RetrParams p) {
     }
   };
   if constexpr (LOCAL) {
-    if (windows) {
-      const int inc = p.local_inc, own = inc + t;                 // window rows: inc of the cache, then the new tokens
-      const char* kn = (const char*)p.k_new + 2 * (b * p.kns_b + hh * p.kns_h);
-      const char* vn = (const char*)p.v_new + 2 * (b * p.vns_b + hh * p.vns_h);
-      float s_loc[KPG * NC];
+    const int inc = p.local_inc, own = inc + t;                 // window rows: inc of the cache, then the new tokens
+    const char* kn = (const char*)p.k_new + 2 * (b * p.kns_b + hh * p.kns_h);
+    const char* vn = (const char*)p.v_new + 2 * (b * p.vns_b + hh * p.vns_h);
+    float s_loc[KPG * NC];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        if (CK * c > own) {                                       // a chunk behind the row's own token (wave-uniform)
+    for (int c = 0; c < NC; ++c) {
+      if (CK * c > own) {                                       // a chunk behind the row's own token (wave-uniform)
 #pragma unroll
-          for (int i = 0; i < KPG; ++i) s_loc[KPG * c + i] = -INFINITY;
-          continue;
-        }
-#pragma unroll
-        for (int i = 0; i < KPG; ++i) {
-          const int r = CK * c + g + 8 * i;
-          const bool visible = r <= own && !(r == BS - 1 && own == BS - 1);
-          const int rc = min(r, own);                             // rows behind the row's own are never read
-          const bool cached = rc < inc;
-          const char* kr = (cached ? kc + 2 * ((p.local_row0 + rc) * p.kcs_r) : kn + 2 * ((int64_t)(rc - inc) * p.kns_r)) + PB * j;
-          const int64_t pos = inc > 0 ? p.local_pos0 + min(rc, inc - 1) : 0;   // a position the tables hold, used by cached rows only
-          const char* cr = (const char*)p.cos + 2 * (pos * p.cs_r) + PB * j;
-          const char* sr = (const char*)p.sin + 2 * (pos * p.cs_r) + PB * j;
-          float kl[E], kh[E], cl[E], ch[E], sl[E], sh[E];
-          unpack8(*(const vec_t*)(kr), kl);
-          unpack8(*(const vec_t*)(kr + D), kh);
-          unpack8(*(const vec_t*)(cr), cl);
-          unpack8(*(const vec_t*)(cr + D), ch);
-          unpack8(*(const vec_t*)(sr), sl);
-          unpack8(*(const vec_t*)(sr + D), sh);
-          float d = 0.f;
-#pragma unroll
-          for (int e = 0; e < E; ++e) {                           // cached keys are rotated in the model dtype, as the cache's
-            const float rl = cached ? round_to<T>(__builtin_fmaf(kl[e], cl[e], -kh[e] * sl[e])) : kl[e];   // window is (llama_mem.py:336-338)
-            const float rh = cached ? round_to<T>(__builtin_fmaf(kh[e], ch[e], kl[e] * sh[e])) : kh[e];
-            d = __builtin_fmaf(qlo[e], rl, d);
-            d = __builtin_fmaf(qhi[e], rh, d);
-          }
-          s_loc[KPG * c + i] = visible ? sum8(d) * c2 : -INFINITY;
-        }
+        for (int i = 0; i < KPG; ++i) s_loc[KPG * c + i] = -INFINITY;
+        continue;
       }
-      float mx = s_loc[0];                                        // row 0 is always visible
 #pragma unroll
-      for (int i = 1; i < KPG * NC; ++i) mx = fmaxf(mx, s_loc[i]);
-      mx = fmaxf(mx, dpp_f<0x128>(mx));
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      float den = 0.f;
+      for (int i = 0; i < KPG; ++i) {
+        const int r = CK * c + g + 8 * i;
+        const bool visible = r <= own && !(r == BS - 1 && own == BS - 1);
+        const int rc = min(r, own);                             // rows behind the row's own are never read
+        const bool cached = rc < inc;
+        const char* kr = (cached ? kc + 2 * ((p.local_row0 + rc) * p.kcs_r) : kn + 2 * ((int64_t)(rc - inc) * p.kns_r)) + PB * j;
+        const int64_t pos = inc > 0 ? p.local_pos0 + min(rc, inc - 1) : 0;   // a position the tables hold, used by cached rows only
+        const char* cr = (const char*)p.cos + 2 * (pos * p.cs_r) + PB * j;
+        const char* sr = (const char*)p.sin + 2 * (pos * p.cs_r) + PB * j;
+        float kl[E], kh[E], cl[E], ch[E], sl[E], sh[E];
+        unpack8(*(const vec_t*)(kr), kl);
+        unpack8(*(const vec_t*)(kr + D), kh);
+        unpack8(*(const vec_t*)(cr), cl);
+        unpack8(*(const vec_t*)(cr + D), ch);
+        unpack8(*(const vec_t*)(sr), sl);
+        unpack8(*(const vec_t*)(sr + D), sh);
+        float d = 0.f;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        if (CK * c > own) continue;
-#pragma unroll
-        for (int i = 0; i < KPG; ++i) {
-          const int rc = min(CK * c + g + 8 * i, own);
-          const bool cached = rc < inc;
-          const char* vr = (cached ? vc + 2 * ((p.local_row0 + rc) * p.vcs_r) : vn + 2 * ((int64_t)(rc - inc) * p.vns_r)) + PB * j;
-          const vec_t vlo = *(const vec_t*)(vr), vhi = *(const vec_t*)(vr + D);
-          const float e = fast_exp2(s_loc[KPG * c + i] - mx);
-          den += e;
-          const float w = round_to<T>(e);                         // weights enter PV in the model dtype
-#pragma unroll
-          for (int e2 = 0; e2 < E / 2; ++e2) {
-            alo[2 * e2] = __builtin_fmaf(w, unpack_lo<T>(vlo[e2]), alo[2 * e2]);
-            alo[2 * e2 + 1] = __builtin_fmaf(w, unpack_hi<T>(vlo[e2]), alo[2 * e2 + 1]);
-            ahi[2 * e2] = __builtin_fmaf(w, unpack_lo<T>(vhi[e2]), ahi[2 * e2]);
-            ahi[2 * e2 + 1] = __builtin_fmaf(w, unpack_hi<T>(vhi[e2]), ahi[2 * e2 + 1]);
-          }
+        for (int e = 0; e < E; ++e) {                           // cached keys are rotated in the model dtype, as the cache's
+          const float rl = cached ? round_to<T>(__builtin_fmaf(kl[e], cl[e], -kh[e] * sl[e])) : kl[e];   // window is (llama_mem.py:336-338)
+          const float rh = cached ? round_to<T>(__builtin_fmaf(kh[e], ch[e], kl[e] * sh[e])) : kh[e];
+          d = __builtin_fmaf(qlo[e], rl, d);
+          d = __builtin_fmaf(qhi[e], rh, d);
         }
+        s_loc[KPG * c + i] = visible ? sum8(d) * c2 : -INFINITY;
       }
-      den += dpp_f<0x128>(den);
-      den += __shfl_xor(den, 16, 64);
-      den += __shfl_xor(den, 32, 64);
-      Mrun = mx;
-      lrun = den;
     }
+    float mx = s_loc[0];                                        // row 0 is always visible
+#pragma unroll
+    for (int i = 1; i < KPG * NC; ++i) mx = fmaxf(mx, s_loc[i]);
+    mx = fmaxf(mx, dpp_f<0x128>(mx));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float den = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      if (CK * c > own) continue;
+#pragma unroll
+      for (int i = 0; i < KPG; ++i) {
+        const int rc = min(CK * c + g + 8 * i, own);
+        const bool cached = rc < inc;
+        const char* vr = (cached ? vc + 2 * ((p.local_row0 + rc) * p.vcs_r) : vn + 2 * ((int64_t)(rc - inc) * p.vns_r)) + PB * j;
+        const vec_t vlo = *(const vec_t*)(vr), vhi = *(const vec_t*)(vr + D);
+        const float e = fast_exp2(s_loc[KPG * c + i] - mx);
+        den += e;
+        const float w = round_to<T>(e);                         // weights enter PV in the model dtype
+#pragma unroll
+        for (int e2 = 0; e2 < E / 2; ++e2) {
+          alo[2 * e2] = __builtin_fmaf(w, unpack_lo<T>(vlo[e2]), alo[2 * e2]);
+          alo[2 * e2 + 1] = __builtin_fmaf(w, unpack_hi<T>(vlo[e2]), alo[2 * e2 + 1]);
+          ahi[2 * e2] = __builtin_fmaf(w, unpack_lo<T>(vhi[e2]), ahi[2 * e2]);
+          ahi[2 * e2 + 1] = __builtin_fmaf(w, unpack_hi<T>(vhi[e2]), ahi[2 * e2 + 1]);
+        }
+      }
+    }
+    den += dpp_f<0x128>(den);
+    den += __shfl_xor(den, 16, 64);
+    den += __shfl_xor(den, 32, 64);
+    Mrun = mx;
+    lrun = den;
   }
   int blk = 0;
   if (js0 < p.k) {
@@ -1111,12 +1095,10 @@ void lmk_gather_attend_kernel(RetrParams p) {
     }
     __syncthreads();
     if (wave != 0) return;
-    const int nw = LOCAL ? max(p.block_waves, p.window_wave + 1) : NWV;   // of NWV; unrolled, the loads are in flight together
     float mw[NWV], Mall = part_ml[0][0];                          // wave 0 always has a block (k >= 1)
 #pragma unroll
     for (int w = 0; w < NWV; ++w) {
       mw[w] = part_ml[w][0];
-      mw[w] = w < nw ? mw[w] : -INFINITY;
       Mall = fmaxf(Mall, mw[w]);
     }
     lrun = 0.f;
@@ -1127,14 +1109,12 @@ void lmk_gather_attend_kernel(RetrParams p) {
     }
 #pragma unroll
     for (int w = 0; w < NWV; ++w) {
-      if (w < nw) {
-        const float sw = fast_exp2(mw[w] - Mall);                 // 0 for a wave without blocks (M = -inf)
-        lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
+      const float sw = fast_exp2(mw[w] - Mall);                   // 0 for a wave without blocks (M = -inf)
+      lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          alo[e] = __builtin_fmaf(part_acc[w][E * j + e], sw, alo[e]);
-          ahi[e] = __builtin_fmaf(part_acc[w][D / 2 + E * j + e], sw, ahi[e]);
-        }
+      for (int e = 0; e < E; ++e) {
+        alo[e] = __builtin_fmaf(part_acc[w][E * j + e], sw, alo[e]);
+        ahi[e] = __builtin_fmaf(part_acc[w][D / 2 + E * j + e], sw, ahi[e]);
       }
     }
     Mrun = Mall;
@@ -1311,41 +1291,11 @@ int launch_retrieve_topk(const RetrParams& p, int D, int dtype, bool reuse_landm
   return LMK_ERR_UNSUPPORTED;
 }
 
-// The gather with the rows' window inside, a workgroup per row.
-template <class T, int D, int BS, int CK>
-static int launch_gather_split(RetrParams p, int64_t rows, hipStream_t stream) {
-  constexpr int most = gather_waves(BS, D, CK);
-  int own = 1;                                                    // the window has a wave of its own
-  if (BS == 128) {
-    // at head dim 64 while every row's five waves find a CU of their own (32 rows, top 4: 18.5 -> 16.6 us; 256 rows, top 8: 32.7 ->
-    // 28.5): a CU takes eight waves, so two workgroups of four and only one of five (512 rows, top 4: 28.0 against 32.5)
-    own = D == 64 && rows <= 256 ? 1 : 0;
-    p.block_waves = own ? std::min(p.k, most) : most;
-  } else {
-    const int per = (p.k + most - 1) / most;                      // blocks a wave walks one after the other
-    p.block_waves = (p.k + per - 1) / per;
-  }
-  p.window_wave = own ? p.block_waves : p.k % p.block_waves;
-  const dim3 grid((unsigned)rows), wg(64 * (p.block_waves + own));
-  if (p.merge_slices > 0) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, false, true, true, CK>), grid, wg, 0, stream, p);
-  else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, true, false, false, true, CK>), grid, wg, 0, stream, p);
-  return (int)hipGetLastError();
-}
-
 template <class T, int D, int BS, bool PADDED>
 static int launch_gather_b(const RetrParams& p, hipStream_t stream) {
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   if (p.local) {                          // with the row's local window: blocks as they are only
-    if constexpr (!PADDED) {
-      constexpr int CK = gather_chunk(BS, D, true);
-      if (rows <= 1024 && p.k > 1) {
-        // from seven blocks on at most four waves, in chunks of 64 keys, where the rows fill the chip (1024 rows, top 7: 88.0 us
-        // against 97.0 in chunks of 32 and 89.7 with a wave per block; 256 rows, top 8: 29.7, 30.9 and 30.1) and not with few
-        // of them (128 rows, top 7: 24.3 against 22.2 with a wave per block)
-        if constexpr (BS == 64 && D == 128)
-          if (p.k > 6 && rows > 128) return launch_gather_split<T, D, BS, 64>(p, rows, stream);
-        return launch_gather_split<T, D, BS, CK>(p, rows, stream);
-      }
+    if constexpr (!PADDED && D == 128 && BS <= 64) {
       const dim3 grid((unsigned)((rows + 3) / 4));
       if (p.merge_slices > 0) hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, true, true>), grid, dim3(256), 0, stream, p);
       else hipLaunchKernelGGL((lmk_gather_attend_kernel<T, D, BS, false, PADDED, false, true>), grid, dim3(256), 0, stream, p);
@@ -1603,6 +1553,9 @@ int launch_local_window(const WindowParams& p, int D, int dtype, hipStream_t str
 }
 
 int launch_gather_attend(const RetrParams& p, int D, int BS, int dtype, hipStream_t stream) {
+  // A decode step of so many rows that waves of 16 KB each fill the chip whichever way: a wave per row is as fast and has no
+  // waves for windows (2048 rows, block 64, top 6, D128: 92.2 us against 94.5; 1024 rows: 80.7 against 57.6)
+  if (p.local && !(D == 128 && BS <= 64 && (int64_t)p.B * p.H * p.T > 4 * cu_count())) return launch_gather_decode(p, D, dtype, stream);
   if (dtype == LMK_DTYPE_BF16) {
     if (D == 128) return launch_gather_t<bf16_t, 128>(p, BS, stream);
     if (D == 64) return launch_gather_t<bf16_t, 64>(p, BS, stream);

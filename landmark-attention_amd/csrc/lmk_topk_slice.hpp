@@ -98,7 +98,7 @@ __device__ __forceinline__ int rank_ascending(int& mine, int lane, int k, int nu
   age += age < 0 ? num_mems : 0;
   int rank = 0;
   for (int j = 0; j < k; ++j) {
-    const int o = __shfl(age, j, 64);
+    const int o = __builtin_amdgcn_readlane(age, j);
     rank += (o < age || (o == age && j < lane)) ? 1 : 0;
   }
   return rank;
@@ -243,6 +243,7 @@ __device__ __forceinline__ int merge_slices_row(const RetrParams& p, int n_slice
       cv = p.approx[row * p.num_mems + lane];
       ci = ((const int*)p.exact)[row * p.num_mems + lane];
     }
+    if (n_slices == 1) return ci;                                   // one slice: its candidates are the row's, best first
     int mine = 0x7fffffff;
     for (int j = 0; j < p.k; ++j) {
       float bv;
