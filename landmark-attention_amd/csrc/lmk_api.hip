@@ -609,6 +609,8 @@ static int retrieve_topk_check(const lmk_tensor4* q, const lmk_tensor4* kcache, 
   return check_retrieval(B, H, T, S, D, block, top_k, dtype, n_pos);
 }
 
+static lmk::LandmarkKeys landmark_keys(bool reuse) { return reuse ? lmk::LandmarkKeys::kRotated : lmk::LandmarkKeys::kRotate; }
+
 static int retrieve_topk_impl(bool reuse_landmark_keys, const lmk_tensor4* q, const lmk_tensor4* kcache,
                               const void* cos_table, const void* sin_table, int64_t table_stride_row, int64_t n_pos,
                               int64_t* idx_out, void* workspace, size_t workspace_bytes, int B, int H, int T, int S,
@@ -636,7 +638,7 @@ static int retrieve_topk_impl(bool reuse_landmark_keys, const lmk_tensor4* q, co
     *params_out = p;
     return LMK_OK;
   }
-  return lmk::launch_retrieve_topk(p, D, dtype, reuse_landmark_keys, (hipStream_t)stream);
+  return lmk::launch_retrieve_topk(p, D, dtype, landmark_keys(reuse_landmark_keys), (hipStream_t)stream);
 }
 
 int lmk_retrieve_topk(const lmk_tensor4* q, const lmk_tensor4* kcache, const void* cos_table, const void* sin_table,
@@ -889,7 +891,8 @@ int lmk_ring_retrieve_topk(const lmk_tensor4* q, const lmk_tensor4* kring, const
   p.qs_b = q->stride_b; p.qs_h = q->stride_h; p.qs_r = q->stride_row;
   p.kcs_b = kring->stride_b; p.kcs_h = kring->stride_h; p.kcs_r = kring->stride_row;
   p.cs_r = table_stride_row;
-  if (method == LMK_SELECT_PER_TOKEN_AND_HEAD) return lmk::launch_retrieve_topk(p, D, dtype, false, (hipStream_t)stream);
+  if (method == LMK_SELECT_PER_TOKEN_AND_HEAD)
+    return lmk::launch_retrieve_topk(p, D, dtype, lmk::LandmarkKeys::kTransient, (hipStream_t)stream);
   p.agg = reinterpret_cast<uint32_t*>(w + l.exact);                          // B*T or B*H vectors of n_blocks words: fits
   p.agg_over_heads = method == LMK_SELECT_MAX_OVER_HEADS;
   p.prob32 = 1;                                                              // softmax output stays fp32 under autocast
@@ -1222,7 +1225,7 @@ static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kca
       return gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, nullptr, nullptr,
                                 nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, &pr, k_loc, v_loc, append);
     }
-    if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, reuse_landmark_keys != 0, (hipStream_t)stream))) return rc;
+    if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, landmark_keys(reuse_landmark_keys != 0), (hipStream_t)stream))) return rc;
     return gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, nullptr, nullptr,
                               nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr, k_loc, v_loc, append);
   }
@@ -1268,7 +1271,7 @@ static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kca
       if (reuse_landmark_keys) rc = lmk::launch_fwd(pf, D, block, dtype, (hipStream_t)stream);
       else rc = lmk::launch_fwd32_landmark_keys(pf, pr, D, dtype, (hipStream_t)stream);
       if (rc) return rc;
-      if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, true, (hipStream_t)stream))) return rc;   // keys are rotated already
+      if ((rc = lmk::launch_retrieve_topk(pr, D, dtype, lmk::LandmarkKeys::kRotated, (hipStream_t)stream))) return rc;
     }
     const lmk_tensor4 o_loc = {w + l.o_win + (size_t)inc * D * 2, o_win.stride_b, o_win.stride_h, o_win.stride_row};
     if ((rc = gather_attend_impl(q, kcache, vcache, idx_out, cos_table, sin_table, table_stride_row, n_pos, &o_loc, L + inc,

@@ -256,7 +256,9 @@ inline int topk_slices(const RetrParams& p) {
   const bool few = rows <= kSliceMaxRows || (p.T <= kSliceMaxRowsPerHead && rows * n_slices < ((int64_t)1 << 30));
   return (few && (int64_t)n_slices * p.k <= kSliceMaxCand) ? n_slices : 0;
 }
-int launch_retrieve_topk(const RetrParams& p, int D, int dtype, bool reuse_landmark_keys, hipStream_t stream);
+// rotated landmark keys in p.lk_rot: to be written (a later call may reuse them), there already, or of no use to the caller
+enum class LandmarkKeys { kRotate, kRotated, kTransient };
+int launch_retrieve_topk(const RetrParams& p, int D, int dtype, LandmarkKeys keys, hipStream_t stream);
 int launch_retrieve_topk_shared(const RetrParams& p, int D, int dtype, hipStream_t stream);   // one selection per head
 int launch_local_window(const WindowParams& p, int D, int dtype, hipStream_t stream);
 // block-32 forward (pf) and the rotation of the landmark keys (pr: what launch_retrieve_topk would do first) in one launch

@@ -87,7 +87,7 @@ __device__ __forceinline__ uint32_t prob_bits<f16_t>(float x) { return pack2<f16
 // score is 128 fmas plus whatever brings the key's value to every lane -- an unpack per
 // fma with a key per lane, scalar loads of 8 bytes per score with the key in scalar registers, 16 times the LDS
 // traffic with every lane reading the value, fmas that take the value from the lane that holds it (row_newbcast) --
-// and every such kernel took 50-60 us at config 4's shapes.)
+// and every such kernel took 50-60 us at the shapes below.)
 // A workgroup's four waves are QW groups of query rows x 4 / QW groups of keys; it rotates its keys itself, into LDS.
 // A chain of 128 dependent MFMAs is 4 us, and what lies around it -- first loads, rotation, 32 quotients, stores -- 6 more: with
 // tiles of 64 keys and the rotation in a launch of its own, 32 heads, 256 queries, 256 blocks took 3.9 + 19.6 us (D64 3.5 + 16.4),
@@ -350,6 +350,133 @@ __global__ __launch_bounds__(256) void lmk_block_select_kernel(RetrParams p) {
     if (lane == j) mine = bi;
   }
   write_ascending(p.idx + (int64_t)bh * p.k, mine, lane, p.k, p.num_mems, p.ring_start);
+}
+
+// ---------------------------------------------------------------------------
+// score + select where a lane can hold a block: caches of at most 64 blocks
+// ---------------------------------------------------------------------------
+// The bracket of the fused kernel below saves exact dot products where a row has a thousand scores to rank; a row with 64
+// pays for its steps (score tile, bracket, list, evaluation, each behind a barrier or an LDS round trip) and gets little.  Here
+// lane m keeps block m's rotated key in registers, every score is the contract's dot product, and a wave takes kDirectRows rows
+// at a time, whose chains of dependent fmas fill each other's latency.  A row's values reach the fmas as scalar operands.
+// What bounds it is latency: one round trip for the keys, D * kDirectRows fmas, k picks.  40 blocks, 6120 rows, D64: 14.4 us
+// and 3.3 us of key rotation before, 8.5 us with OWN_KEYS; 136 rows over 16 blocks of 128, D128, which went by slices and their
+// merge, 9.1 -> 6.9 us.  (Left to itself the compiler sinks each row's fmas into the branch of the lanes that hold a block, one
+// row behind the other, with the loads of its values in front: 10.7 us.)
+// OWN_KEYS: the keys are rotated here, by the workgroup into LDS, once for its 4 * kDirectRows rows -- for a caller that keeps
+// no rotated keys (the ring cache).  Otherwise they are read from p.lk_rot.
+constexpr int kDirectRows = 4;
+
+template <class T, int D, bool OWN_KEYS>
+__global__ __launch_bounds__(256) void lmk_topk_direct_kernel(RetrParams p) {
+  constexpr int CH = D / 8;                                       // 16-byte chunks of a key
+  constexpr int KEYB = 2 * D + 16;                                // 16 lanes reading 16 B of 16 keys hit every bank once
+  __shared__ __align__(16) unsigned char keys[OWN_KEYS ? 64 * KEYB : 16];
+  const int tid = threadIdx.x, lane = tid & 63, NM = p.num_mems;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t groups = (uint32_t)(p.T + 4 * kDirectRows - 1) / (4 * kDirectRows);
+  const uint32_t bh = blockIdx.x / groups;
+  const int b = (int)(bh / (uint32_t)p.H), hh = (int)bh - b * p.H;
+  const int t0 = (int)(blockIdx.x - bh * groups) * 4 * kDirectRows + kDirectRows * wave;
+  // The rows come through the scalar cache (nothing in this launch writes them), 16 dims of each at a time; the next 16 are
+  // asked for when these are here, since scalar loads return in any order.  Rows past the end: the last one again.
+  typedef uint32_t u32x8_t __attribute__((ext_vector_type(8), aligned(16)));
+  typedef const __attribute__((address_space(4))) char* scalar_row_t;
+  const int rows = min(p.T - t0, kDirectRows);                    // wave-uniform; below 1: the wave only rotates keys
+  scalar_row_t q[kDirectRows];
+  u32x8_t now[kDirectRows];
+#pragma unroll
+  for (int r = 0; r < kDirectRows; ++r) {
+    q[r] = (scalar_row_t)(uintptr_t)((const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h + (int64_t)min(t0 + r, p.T - 1) * p.qs_r));
+    now[r] = *(const __attribute__((address_space(4))) u32x8_t*)q[r];
+  }
+  u32x4_t kk[CH];
+  if constexpr (OWN_KEYS) {
+    constexpr int N = 64 * CH / 256;                              // chunks per thread, all requested together
+    LandmarkChunk c[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) c[i] = load_landmark_chunk<D>(p, b, hh, min(tid / CH + 256 / CH * i, NM - 1), tid % CH);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float r[8];
+      rotate_chunk<T>(c[i].x, c[i].other, c[i].c, c[i].s, tid % CH >= CH / 2, r);
+      const u32x4_t o = {pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
+      *(u32x4_t*)(keys + (tid / CH + 256 / CH * i) * KEYB + 16 * (tid % CH)) = o;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c8 = 0; c8 < CH; ++c8) kk[c8] = *(const u32x4_t*)(keys + lane * KEYB + 16 * c8);
+  } else {
+    const char* lk = (const char*)p.lk_rot + (int64_t)bh * lk_tiles(NM) * lk_tile_bytes(D) + lk_key_offset(min(lane, NM - 1), D);
+#pragma unroll
+    for (int c8 = 0; c8 < CH; ++c8) kk[c8] = *(const u32x4_t*)(lk + 512 * c8);
+  }
+  if (rows < 1) return;                                           // behind the only barrier
+  float v[kDirectRows];
+#pragma unroll
+  for (int r = 0; r < kDirectRows; ++r) v[r] = 0.f;
+  static_assert(kDirectRows == 4, "the operands of the two empty statements below");
+#pragma unroll
+  for (int st = 0; st < D / 16; ++st) {
+    u32x8_t next[kDirectRows];
+    if (st + 1 < D / 16) {
+      int off = 32 * (st + 1);
+      asm volatile("" : "+s"(off) : "s"(now[0][0]), "s"(now[1][0]), "s"(now[2][0]), "s"(now[3][0]));
+#pragma unroll
+      for (int r = 0; r < kDirectRows; ++r) next[r] = *(const __attribute__((address_space(4))) u32x8_t*)(q[r] + off);
+      __builtin_amdgcn_sched_barrier(0);                          // left alone they sink below the fmas they are to hide behind
+    }
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {                                 // the sequential dot product of the contract, d ascending
+      const uint32_t ku = kk[2 * st + w / 4][w % 4];
+      const float k0 = unpack_lo<T>(ku), k1 = unpack_hi<T>(ku);
+#pragma unroll
+      for (int r = 0; r < kDirectRows; ++r) v[r] = __builtin_fmaf(unpack_lo<T>(now[r][w]), k0, v[r]);
+#pragma unroll
+      for (int r = 0; r < kDirectRows; ++r) v[r] = __builtin_fmaf(unpack_hi<T>(now[r][w]), k1, v[r]);
+    }
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));   // by all lanes and all rows, step by step
+#pragma unroll
+    for (int r = 0; r < kDirectRows; ++r) now[r] = next[r];
+  }
+  // k best of every row: the lowest lane among those that hold the maximum is the lowest block among the best.  No lane holds
+  // it (NaN in all that are left): the slot keeps an index past the end, clamped below.
+  uint64_t open[kDirectRows];                                     // blocks not picked yet
+  int age[kDirectRows], mine[kDirectRows], rank[kDirectRows];     // lane j: the j-th pick, and its place in the order of age
+#pragma unroll
+  for (int r = 0; r < kDirectRows; ++r) {
+    const float x = contract<T>(v[r], p.sqrt_hd);
+    v[r] = lane < NM ? x : -INFINITY;
+    open[r] = ~0ull >> (64 - NM);
+    mine[r] = 0x7fffffff;
+  }
+  for (int j = 0; j < p.k; ++j)
+#pragma unroll
+    for (int r = 0; r < kDirectRows; ++r) {
+      const float best = wave_max(v[r]);
+      const uint64_t eq = __ballot(v[r] == best) & open[r];
+      const int win = eq ? __builtin_ctzll(eq) : 0x7fffffff;
+      open[r] &= ~(eq & (0 - eq));
+      v[r] = lane == win ? -INFINITY : v[r];
+      mine[r] = lane == j ? win : mine[r];
+    }
+#pragma unroll
+  for (int r = 0; r < kDirectRows; ++r) {                         // as rank_ascending does, the rows side by side
+    mine[r] = min(mine[r], NM - 1);
+    age[r] = mine[r] - p.ring_start;
+    age[r] += age[r] < 0 ? NM : 0;
+    rank[r] = 0;
+  }
+  for (int j = 0; j < p.k; ++j)
+#pragma unroll
+    for (int r = 0; r < kDirectRows; ++r) {
+      const int o = __builtin_amdgcn_readlane(age[r], j);
+      rank[r] += (o < age[r] || (o == age[r] && j < lane)) ? 1 : 0;
+    }
+  int64_t* out = p.idx + ((int64_t)bh * p.T + t0) * p.k;
+#pragma unroll
+  for (int r = 0; r < kDirectRows; ++r)
+    if (r < rows && lane < p.k) out[r * p.k + rank[r]] = (int64_t)mine[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -1169,13 +1296,23 @@ int launch_topk_slice_merge(const RetrParams& p, hipStream_t stream) {
 }
 
 template <class T, int D>
-static int launch_topk_t(const RetrParams& p, bool reuse_landmark_keys, hipStream_t stream) {
+static int launch_topk_t(const RetrParams& p, LandmarkKeys keys, hipStream_t stream) {
   constexpr int RPW = 256 / (D / 8);
   const int64_t lkrows = (int64_t)p.B * p.H * p.num_mems;
+  const bool direct = p.num_mems <= 64;                             // a lane per block
+  const dim3 direct_grid((unsigned)p.B * p.H * (unsigned)((p.T + 4 * kDirectRows - 1) / (4 * kDirectRows)));
   int rc;
-  if (!reuse_landmark_keys) {
+  if (direct && keys == LandmarkKeys::kTransient) {
+    hipLaunchKernelGGL((lmk_topk_direct_kernel<T, D, true>), direct_grid, dim3(256), 0, stream, p);
+    return (int)hipGetLastError();
+  }
+  if (keys != LandmarkKeys::kRotated) {
     hipLaunchKernelGGL((lmk_landmark_keys_kernel<T, D>), dim3((unsigned)((lkrows + RPW - 1) / RPW)), dim3(256), 0, stream, p);
     if ((rc = (int)hipGetLastError())) return rc;
+  }
+  if (direct) {
+    hipLaunchKernelGGL((lmk_topk_direct_kernel<T, D, false>), direct_grid, dim3(256), 0, stream, p);
+    return (int)hipGetLastError();
   }
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   const int n_slices = topk_slices(p);
@@ -1280,13 +1417,13 @@ int launch_landmark_keys(const RetrParams& p, int D, int dtype, hipStream_t stre
   return LMK_ERR_UNSUPPORTED;
 }
 
-int launch_retrieve_topk(const RetrParams& p, int D, int dtype, bool reuse_landmark_keys, hipStream_t stream) {
+int launch_retrieve_topk(const RetrParams& p, int D, int dtype, LandmarkKeys keys, hipStream_t stream) {
   if (dtype == LMK_DTYPE_BF16) {
-    if (D == 128) return launch_topk_t<bf16_t, 128>(p, reuse_landmark_keys, stream);
-    if (D == 64) return launch_topk_t<bf16_t, 64>(p, reuse_landmark_keys, stream);
+    if (D == 128) return launch_topk_t<bf16_t, 128>(p, keys, stream);
+    if (D == 64) return launch_topk_t<bf16_t, 64>(p, keys, stream);
   } else if (dtype == LMK_DTYPE_F16) {
-    if (D == 128) return launch_topk_t<f16_t, 128>(p, reuse_landmark_keys, stream);
-    if (D == 64) return launch_topk_t<f16_t, 64>(p, reuse_landmark_keys, stream);
+    if (D == 128) return launch_topk_t<f16_t, 128>(p, keys, stream);
+    if (D == 64) return launch_topk_t<f16_t, 64>(p, keys, stream);
   }
   return LMK_ERR_UNSUPPORTED;
 }

@@ -1,0 +1,60 @@
+"""The selection over caches of at most 64 blocks: caches of one block, of 64 and of 65 (the other path), every remainder of the
+rows a wave takes, equal scores, rows that pick all blocks -- against the oracle's scores, and the ring's order of age likewise."""
+import pytest
+import torch
+
+from oracle import mem_cache as omc
+from oracle import retrieval as oret
+from oracle import rotary as orot
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n,T,k", [(1, 17, 1), (2, 513, 2), (40, 530, 4), (63, 515, 63), (64, 516, 5), (64, 37, 64), (65, 514, 5)])
+def test_picks_match_the_oracle(n, T, k, D, dtype):
+    from landmark_hip.retrieval import retrieve_topk
+    print(f"case {n} blocks T{T} top {k} D{D} {dtype}", flush=True)
+    B, H, block = 1, 2, 32
+    g = torch.Generator().manual_seed(n + T)
+    q = (torch.randn(B, H, T, D, generator=g) * 0.5).to(dtype)
+    kc = (torch.randn(B, H, n * block, D, generator=g) * 0.5).to(dtype)
+    cos, sin = orot.rotary_tables((n + k + 2) * block, D, dtype)
+    idx = retrieve_topk(q.cuda(), kc.cuda(), cos.cuda(), sin.cuda(), block, k).cpu()
+    want = oret.select_topk(oret.landmark_scores(q, kc, cos, sin, block, k), k)
+    assert torch.equal(idx, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_equal_scores_go_to_the_lowest_block(dtype):
+    from landmark_hip.retrieval import retrieve_topk
+    q = torch.zeros(1, 1, 21, 64, dtype=dtype)                  # every score is zero
+    kc = torch.randn(1, 1, 50 * 32, 64).to(dtype)
+    cos, sin = orot.rotary_tables(52 * 32, 64, dtype)
+    idx = retrieve_topk(q.cuda(), kc.cuda(), cos.cuda(), sin.cuda(), 32, 6).cpu()
+    assert torch.equal(idx, torch.arange(6).expand_as(idx))
+
+
+@pytest.mark.parametrize("n,oldest,T,k,block,D", [(1, 0, 3, 1, 32, 64), (40, 0, 255, 4, 51, 64), (64, 63, 130, 4, 51, 128),
+                                                  (64, 17, 33, 64, 32, 64), (65, 17, 33, 4, 32, 64), (7, 3, 18, 7, 64, 128)])
+def test_ring_picks_match_the_oracle(n, oldest, T, k, block, D):
+    from landmark_hip import _lib
+    print(f"case ring {n} blocks, oldest {oldest}, T{T} top {k} block {block} D{D}", flush=True)
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(n + T)
+    q = (torch.randn(B, H, T, D, generator=g) * 0.5).bfloat16()
+    ring = (torch.randn(B, n, block, H, D, generator=g) * 0.5).bfloat16()
+    cos, sin = orot.rotary_tables((k + 2) * block, D, torch.bfloat16)
+    want = omc.select_blocks(omc.ring_scores(q, ring, n, oldest, k, cos, sin), oldest, k, "per_token_and_head")
+    q, ring, cos, sin = (t.cuda() for t in (q, ring, cos, sin))
+    kring = ring.flatten(1, 2).transpose(1, 2)
+    lib = _lib.lib()
+    nbytes = lib.lmk_retrieve_workspace_bytes(B, H, T, n * block, D, block)
+    idx = torch.empty(B, H, T, k, device="cuda", dtype=torch.int64)
+    ws = torch.empty(nbytes, device="cuda", dtype=torch.uint8)
+    rc = lib.lmk_ring_retrieve_topk(_lib.tensor4(q), _lib.tensor4(kring), cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0],
+                                    idx.data_ptr(), ws.data_ptr(), nbytes, B, H, T, n, D, block, k, oldest, 0, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(idx.cpu(), want)
