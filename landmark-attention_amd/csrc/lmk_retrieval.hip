@@ -6,8 +6,8 @@
 // Selection must be reproducible bit for bit, so the score of (query, landmark) is defined
 // as: fp32 dot product accumulated sequentially over the head dim with one fma per element,
 // rounded to the model dtype, divided in fp32 by sqrt(hd), rounded again (the two roundings of
-// `matmul(...) / math.sqrt(head_dim)`, :367).  Evaluating that for every pair on the vector
-// ALU would dominate the step, so the work is split:
+// `matmul(...) / math.sqrt(head_dim)`, :367).  Up to 256 blocks every pair is evaluated that way (a block
+// per lane, or matrix-core tiles of the same chain); with more that would dominate the step, so the work is split:
 //   lk      rotate every cached landmark key at its slot position (:359-366), exactly as the
 //           model dtype would round it, into a dense side array, with its 2-norm
 //   score   MFMA product q . lk^T -> approximate fp32 scores
@@ -477,6 +477,179 @@ __global__ __launch_bounds__(256) void lmk_topk_direct_kernel(RetrParams p) {
 #pragma unroll
   for (int r = 0; r < kDirectRows; ++r)
     if (r < rows && lane < p.k) out[r * p.k + rank[r]] = (int64_t)mine[r];
+}
+
+// ---------------------------------------------------------------------------
+// score + select, every score exact, for caches of 65 to 256 blocks
+// ---------------------------------------------------------------------------
+// v_mfma_f32_16x16x1_4b_f32 is 4 x 16 x 16 steps of the contract's chain of fmas (see lmk_block_score_kernel): a wave takes 16
+// rows and 64 landmarks, one per lane, and per dimension unpacks one value of each and multiplies for 32 cycles.  A workgroup of
+// eight waves is TW waves along the landmarks times 8 / TW groups of 16 rows:
+//   score    the rows' values come from LDS, the keys from L2 four chunks ahead; a score, rounded, divided and rounded again, is
+//            a 16-bit pattern, and LDS keeps it as a number in the scores' order
+//   select   a wave takes four rows at a time, 16 lanes each: a lane holds the scores of landmarks l, l + 16, ... above
+//            65535 - landmark, so that one unsigned maximum finds the best score at the lowest landmark, and the next pick is the
+//            largest number below it
+// What bounds it is the chain of a tile (64 or 128 dependent steps, 1 or 2 us) and the select step's vector instructions; the
+// bracket's kernel also keeps a whole compute unit per 32 rows, so that its time goes in steps of 256 of them.  Selection in us,
+// bracket / exact: 96 blocks, 8192 rows, D64 12.7 / 7.6, D128 14.5 / 9.6; 128 blocks, 32000 rows 46.0 / 12.2, 54.0 / 18.2, 1600
+// rows 12.3 / 7.5, 14.4 / 10.0; a chunk's whole step over 256 blocks, 8320 rows 117.9 / 106.4, 189.5 / 177.7.  1024 blocks, 8192 rows, D128, by this design
+// with eight waves along the landmarks: 22 / 31, the quotients and the select step as long as the 13.7 us of matrix cores.
+constexpr int kExactMems = 256;                                   // landmarks, at most
+constexpr int kExactRows = 16;                                    // per wave
+constexpr int kExactTopK = 16;                                    // a lane per pick
+
+template <class T>
+struct ScoreOrder;                                                // 16-bit patterns with the sign bit flipped, or all bits of a
+template <>                                                       // negative value: [-inf, +inf] in order, NaN outside
+struct ScoreOrder<bf16_t> {
+  static constexpr uint32_t lo = 0x007f, hi = 0xff80;
+};
+template <>
+struct ScoreOrder<f16_t> {
+  static constexpr uint32_t lo = 0x03ff, hi = 0xfc00;
+};
+
+// maximum over the 16 lanes of a DPP row, every lane of the row gets it
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));
+}
+
+// TW: waves along the landmarks, one tile of 64 each
+template <class T, int D, int TW>
+__global__ __launch_bounds__(512, 4) void lmk_topk_exact_kernel(RetrParams p) {
+  constexpr int CPR = D / 8;                                      // 16-byte chunks per row of 16-bit values
+  constexpr int QROWB = 2 * D + 16;                               // 16 lanes reading 16 B of 16 rows hit every bank once
+  constexpr int G = 8 / TW, ROWS = G * kExactRows;                // row groups and rows of the workgroup
+  constexpr int KEYB = 2 * kExactRows + 8;                        // a landmark's 16 scores: 16 lanes reading 4 rows hit no bank twice
+  constexpr int PW = ROWS / 4 / 8;                                // passes of four rows per wave
+  constexpr int NS = 4 * TW;                                      // landmarks per lane of a pass
+  __shared__ __align__(16) unsigned char q_lds[ROWS * QROWB];
+  __shared__ __align__(16) unsigned char sc[G * TW * 64 * KEYB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int NM = p.num_mems;
+  const int n_qt = (p.T + ROWS - 1) / ROWS;
+  // Workgroups go to the eight XCDs in turn; the ones that read the same head's landmark keys are put on
+  // one XCD, so the keys come out of HBM once rather than once per L2.
+  const uint32_t wg = (gridDim.x & 7) ? blockIdx.x : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int bh = (int)(wg / (uint32_t)n_qt), t0 = (int)(wg - (uint32_t)bh * n_qt) * ROWS;
+  const int b = bh / p.H, hh = bh - b * p.H;
+  const char* qp = (const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h);
+  const char* lk = (const char*)p.lk_rot + (int64_t)bh * lk_tiles(NM) * lk_tile_bytes(D);
+
+  const int tile = wave % TW, group = wave / TW;
+  constexpr int NQ = (ROWS * CPR + 511) / 512;
+  u32x4_t rows[NQ], kc[4];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {                                  // rows past the end: the last one again, never picked for
+    const int c = min(tid + 512 * i, ROWS * CPR - 1), t = min(t0 + c / CPR, p.T - 1);
+    rows[i] = *(const u32x4_t*)(qp + 2 * ((int64_t)t * p.qs_r + 8 * (c % CPR)));
+  }
+  const char* key = lk + lk_key_offset(min(64 * tile + lane, NM - 1), D);   // past the end: a re-read, never picked
+#pragma unroll
+  for (int c = 0; c < 4; ++c) kc[c] = *(const u32x4_t*)(key + 512 * c);
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int c = min(tid + 512 * i, ROWS * CPR - 1);             // past the last chunk: that one again
+    *(u32x4_t*)(q_lds + c / CPR * QROWB + 16 * (c % CPR)) = rows[i];
+  }
+  __syncthreads();
+  if (64 * tile < NM) {                                           // wave-uniform
+    const unsigned char* qr = q_lds + (group * kExactRows + (lane & 15)) * QROWB;
+    u32x4_t qc = *(const u32x4_t*)qr;
+    // a chunk's operands are unpacked together, under the MFMAs of the chunk before: an unpack that writes the operand of an
+    // MFMA in flight waits for its end
+    float qv[2][8], kv[2][8];
+    f32x16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    auto unpack = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        qv[c & 1][i] = (i & 1) ? unpack_hi<T>(qc[i >> 1]) : unpack_lo<T>(qc[i >> 1]);
+        kv[c & 1][i] = (i & 1) ? unpack_hi<T>(kc[c & 3][i >> 1]) : unpack_lo<T>(kc[c & 3][i >> 1]);
+        asm volatile("" : "+v"(qv[c & 1][i]), "+v"(kv[c & 1][i]));
+      }
+      if (c + 1 < CPR) qc = *(const u32x4_t*)(qr + 16 * (c + 1));
+      if (c + 4 < CPR) kc[c & 3] = *(const u32x4_t*)(key + 512 * (c + 4));
+    };
+    unpack(0);
+#pragma unroll
+    for (int c = 0; c < CPR; ++c) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[c & 1][i], kv[c & 1][i], acc, 0, 0, 0);
+        if (i == 3 && c + 1 < CPR) unpack(c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // register 4 blk + r of lane l: row 4 (l / 16) + r, landmark 16 blk + l % 16 of the tile
+    unsigned char* dst = sc + ((group * TW + tile) * 64 + (lane & 15)) * KEYB + 8 * (lane >> 4);
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      uint32_t o[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {                               // + 0.0: -0 equals +0, and goes to the lower landmark
+        typedef short s16x2_t __attribute__((ext_vector_type(2)));
+        const uint32_t u = pack2<T>(contract<T>(acc[4 * blk + 2 * i], p.sqrt_hd) + 0.0f,
+                                    contract<T>(acc[4 * blk + 2 * i + 1], p.sqrt_hd) + 0.0f);
+        const s16x2_t sign = __builtin_bit_cast(s16x2_t, u) >> 15;
+        o[i] = u ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u);
+      }
+      *(u32x2_t*)(dst + 16 * blk * KEYB) = u32x2_t{o[0], o[1]};
+    }
+  }
+  __syncthreads();
+
+  const int l16 = lane & 15;
+  uint32_t x[PW][NS], best[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int row = 4 * (PW * wave + i) + (lane >> 4);            // of the workgroup
+    const unsigned char* src = sc + (row / kExactRows * TW * 64 + l16) * KEYB + 2 * (row % kExactRows);
+    best[i] = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const uint32_t v = *(const uint16_t*)(src + 16 * s * KEYB), m = 16 * s + l16;
+      x[i][s] = ((int)m < NM && v - ScoreOrder<T>::lo <= ScoreOrder<T>::hi - ScoreOrder<T>::lo) ? v << 16 | (0xffffu - m) : 0u;
+      best[i] = max(best[i], x[i][s]);
+    }
+  }
+  int mine[PW], age[PW], rank[PW];                                // lane l: pick l of its row, then its place in the order of age
+#pragma unroll
+  for (int i = 0; i < PW; ++i) mine[i] = 0;
+  for (int j = 0; j < p.k; ++j)
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const uint32_t win = row_max_u32(best[i]);                  // 0: nothing left (NaN)
+      mine[i] = l16 == j ? (int)win : mine[i];
+      uint32_t below = 0u - win;                                  // the largest below `win`, seen from there: 0 stands for none
+#pragma unroll
+      for (int s = 0; s < NS; ++s) below = max(below, x[i][s] - win);
+      best[i] = win ? below + win : 0u;
+    }
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {                                  // as rank_ascending does
+    mine[i] = mine[i] ? 0xffff - (mine[i] & 0xffff) : NM - 1;
+    age[i] = mine[i] - p.ring_start;
+    age[i] += age[i] < 0 ? NM : 0;
+    rank[i] = 0;
+  }
+  for (int j = 0; j < p.k; ++j)
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int o = __shfl(age[i], (lane & 48) + j, 64);
+      rank[i] += (o < age[i] || (o == age[i] && j < l16)) ? 1 : 0;
+    }
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int t = t0 + 4 * (PW * wave + i) + (lane >> 4);
+    if (t < p.T && l16 < p.k) p.idx[((int64_t)bh * p.T + t) * p.k + rank[i]] = (int64_t)mine[i];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1320,6 +1493,15 @@ static int launch_topk_t(const RetrParams& p, LandmarkKeys keys, hipStream_t str
     hipLaunchKernelGGL((lmk_topk_slice_kernel<T, D>), dim3((unsigned)(rows * n_slices)), dim3(64 * kSliceWaves), 0, stream, p, n_slices);
     if ((rc = (int)hipGetLastError())) return rc;
     return launch_topk_slice_merge(p, stream);
+  }
+  if (p.num_mems <= kExactMems && p.k <= kExactTopK) {
+    auto launch = [&](auto kern, int rows_per_wg) {
+      const int64_t wgs = (int64_t)p.B * p.H * ((p.T + rows_per_wg - 1) / rows_per_wg);
+      hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(512), 0, stream, p);
+    };
+    if (p.num_mems <= 128) launch(lmk_topk_exact_kernel<T, D, 2>, 4 * kExactRows);
+    else launch(lmk_topk_exact_kernel<T, D, 4>, 2 * kExactRows);
+    return (int)hipGetLastError();
   }
   constexpr int lds_max = (kFusedRows * (kFusedMaxMems + 8) + kFusedRows * D) * 4 + kFusedRows * kFusedList * 2 + kFusedRows * (2 * D + 16);
   static_assert(lds_max <= 160 * 1024, "the score tile, the query rows and the lists fill the LDS of a compute unit");
