@@ -93,6 +93,7 @@ __device__ __forceinline__ uint32_t prob_bits<f16_t>(float x) { return pack2<f16
 // tiles of 64 keys and the rotation in a launch of its own, 32 heads, 256 queries, 256 blocks took 3.9 + 19.6 us (D64 3.5 + 16.4),
 // as it is 13.8 (11.0); 64 heads, 512 queries, 1024 blocks 12.1 + 103.8 and 106 (7.3 + 67.1 and 61).
 constexpr int kScoreRows = 64, kScoreKeys = 32;                   // per wave
+constexpr int kProbMems = 64 * 32;                                // vectors of more blocks take their maxima in memory, from zero
 
 template <class T, int D, int QW>
 __global__ __launch_bounds__(256) void lmk_block_score_kernel(RetrParams p, int n_qs, int n_kc, int64_t agg_words, int agg_per_wg) {
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256) void lmk_block_score_kernel(RetrParams p, int 
     const int t = min(qg * kScoreRows + 16 * (c & 3) + (lane >> 2), p.T - 1);   // rows behind the last one: likewise
     qp[c] = *(const u32x4_t*)((const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h + (int64_t)t * p.qs_r) + 64 * (c >> 2) + 16 * (lane & 3));
   }
-  // the vectors the next kernel takes its maxima into start at zero: every workgroup of this one clears its share
+  // the vectors the next kernel may take its maxima into start at zero: every workgroup of this one clears its share
   for (int i = tid; i < agg_per_wg; i += 256) {
     const int64_t w = (int64_t)blockIdx.x * agg_per_wg + i;
     if (w < agg_words) p.agg[w] = 0u;
@@ -212,7 +213,7 @@ static int launch_scores(const RetrParams& p, hipStream_t stream) {
   int qw = 4;
   while (qw > 1 && 3 * ((groups + qw - 1) / qw * qw) > 4 * groups) qw >>= 1;
   const int keys = kScoreKeys * 4 / qw, n_qs = (groups + qw - 1) / qw, n_kc = (p.num_mems + keys - 1) / keys;
-  const int64_t wgs = (int64_t)p.B * p.H * n_qs * n_kc, words = (int64_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H) * p.num_mems;
+  const int64_t wgs = (int64_t)p.B * p.H * n_qs * n_kc, words = p.num_mems <= kProbMems ? 0 : (int64_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H) * p.num_mems;
   const int per_wg = (int)((words + wgs - 1) / wgs);
   const dim3 grid((unsigned)wgs);
   if (qw == 4) hipLaunchKernelGGL((lmk_block_score_kernel<T, D, 4>), grid, dim3(256), 0, stream, p, n_qs, n_kc, words, per_wg);
@@ -224,37 +225,95 @@ static int launch_scores(const RetrParams& p, hipStream_t stream) {
 // The rows' scores (p.approx) -> softmax -> 16-bit probabilities -> maximum per block into agg, which holds zeros on
 // entry: one vector per (batch, head), maxima over the queries -- or per (batch, query), maxima over the heads.
 // A lane owns the blocks m = lane, lane + 64, ...; a row's sum is each lane's running sum in that order, folded
-// across lanes by halves.  A wave takes `rows_per_wave` rows that share a vector one after the other with the row in
-// registers (NPL values per lane: num_mems <= 64 NPL) and the running maxima too, so a row is read once, nothing is
-// written back and the vector sees one atomic per block and wave.  fp32 probabilities are positive, so their bit
-// patterns order like the values.
+// across lanes by halves.  A wave takes rows that share a vector one after the other with the row in registers (NPL values
+// per lane: num_mems <= 64 NPL), the next one on its way, and the running maxima too; a workgroup's four waves fold theirs in
+// LDS.  Where the vector's rows fit one workgroup (n_parts == 1) its first wave picks from it there and then; otherwise every
+// workgroup leaves its part of the maxima, and lmk_block_select_kernel folds and picks.  32 heads, 256 queries, 256 blocks, top 5:
+// 5.4 + 4.0 us; with an atomic maximum in memory per block and wave, and picks by a wave over the vector in LDS, 7.4 + 7.5.
+// Probabilities are not negative, so their bit patterns order like the values.
+
+// maximum over the 16 lanes of a DPP row, every lane of the row gets it
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));
+}
+
+// The k best of a vector of 64 NPL words, lane l holding words l, l + 64, ...: 0 = no block, larger = better, equal words in
+// ascending order.  Lane j gets the j-th.  One wave.
 template <int NPL>
-__global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int model_is_bf16, int rows_per_wave) {
+__device__ __forceinline__ int pick_blocks(uint32_t (&x)[NPL], int k, int lane) {
+  int mine = 0x7fffffff;
+  for (int j = 0; j < k; ++j) {
+    uint32_t bv = 0;
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < NPL; ++i)
+      if (x[i] > bv) {                                            // ascending i = ascending index: strict > keeps the first
+        bv = x[i];
+        bi = 64 * i + lane;
+      }
+    uint32_t best = row_max_u32(bv);
+    best = max(max((uint32_t)__builtin_amdgcn_readlane((int)best, 0), (uint32_t)__builtin_amdgcn_readlane((int)best, 16)),
+               max((uint32_t)__builtin_amdgcn_readlane((int)best, 32), (uint32_t)__builtin_amdgcn_readlane((int)best, 48)));
+    if (best == 0) break;                                         // nothing left (wave-uniform)
+    const uint64_t eq = __ballot(bv == best);
+    int win;
+    if (__popcll(eq) == 1) win = __builtin_amdgcn_readlane(bi, __builtin_ctzll(eq));
+    else win = wave_min(bv == best ? bi : 0x7fffffff);
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) x[i] = (64 * i + lane == win) ? 0u : x[i];
+    if (lane == j) mine = win;
+  }
+  return mine;
+}
+
+// The words of a finished vector -> picks, and the copy the caller may have asked for.  One wave.
+template <int NPL>
+__device__ __forceinline__ void select_blocks(const RetrParams& p, int vec, uint32_t (&x)[NPL], int lane) {
+  const int NM = p.num_mems;
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) {
+    const int m = 64 * i + lane;
+    if (m < NM && p.agg_out != nullptr) p.agg_out[(int64_t)vec * NM + m] = (uint16_t)x[i];   // the vector itself, in the model dtype
+    // a zero probability is a block still; an fp32 NaN is never picked, a 16-bit one first
+    x[i] = (m < NM && !(p.prob32 && x[i] > 0x7f800000u)) ? x[i] + 1 : 0u;
+  }
+  write_ascending(p.idx + (int64_t)vec * p.k, pick_blocks<NPL>(x, p.k, lane), lane, p.k, NM, p.ring_start);
+}
+
+template <int NPL>
+__global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int model_is_bf16, int rows_per_wave, int n_parts) {
+  __shared__ uint32_t part[3][64 * NPL];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int NM = p.num_mems;
   // rows that share a vector: the T queries of a (batch, head), or the H heads of a (batch, query)
   const int group = p.agg_over_heads ? p.H : p.T;
-  const int per_group = (group + rows_per_wave - 1) / rows_per_wave;
-  const uint32_t w = blockIdx.x * 4 + wave;                       // scalar, and 32-bit as every launch's waves are
-  const uint32_t vec = w / (uint32_t)per_group;                   // (batch, query) or (batch, head)
-  if (vec >= (uint32_t)(p.agg_over_heads ? p.B * p.T : p.B * p.H)) return;
-  const int first = (int)(w - vec * per_group) * rows_per_wave, last = min(first + rows_per_wave, group);
+  const uint32_t vec = blockIdx.x / (uint32_t)n_parts;            // (batch, query) or (batch, head)
+  const int first = ((int)(blockIdx.x - vec * n_parts) * 4 + wave) * rows_per_wave, last = min(first + rows_per_wave, group);
   const uint32_t vec_b = vec / (uint32_t)p.T, vec_t = vec - vec_b * p.T;   // (with agg_over_heads)
   uint32_t best[NPL];
 #pragma unroll
   for (int i = 0; i < NPL; ++i) best[i] = 0u;
-  for (int g = first; g < last; ++g) {
+  float next[NPL];
+  auto load = [&](int g) __attribute__((always_inline)) {
     // over heads: vec = b T + t, row (b H + g) T + t; over queries: vec = b H + h, row vec T + g
     const int64_t row = p.agg_over_heads ? ((int64_t)vec_b * p.H + g) * p.T + vec_t : (int64_t)vec * p.T + g;
     const float* sc = p.approx + row * NM;
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) next[i] = (lane + 64 * i < NM) ? sc[lane + 64 * i] : -INFINITY;
+  };
+  if (first < last) load(first);
+  for (int g = first; g < last; ++g) {
     float x[NPL];
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) x[i] = (lane + 64 * i < NM) ? sc[lane + 64 * i] : -INFINITY;
+    for (int i = 0; i < NPL; ++i) x[i] = next[i];
+    if (g + 1 < last) load(g + 1);
     float mx = x[0];
 #pragma unroll
     for (int i = 1; i < NPL; ++i) mx = fmaxf(mx, x[i]);
-#pragma unroll
-    for (int msk = 32; msk >= 1; msk >>= 1) mx = fmaxf(mx, __shfl_xor(mx, msk, 64));
+    mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
@@ -276,10 +335,54 @@ __global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int m
       }
     }
   }
-  uint32_t* agg = p.agg + (int64_t)vec * NM;
+  if (wave > 0)
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) part[wave - 1][64 * i + lane] = best[i];
+  __syncthreads();
+  if (wave > 0) return;
 #pragma unroll
   for (int i = 0; i < NPL; ++i)
-    if (lane + 64 * i < NM) atomicMax(agg + lane + 64 * i, best[i]);
+    best[i] = max(max(best[i], part[0][64 * i + lane]), max(part[1][64 * i + lane], part[2][64 * i + lane]));
+  if (n_parts == 1) {
+    select_blocks<NPL>(p, (int)vec, best, lane);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < NPL; ++i)
+    if (lane + 64 * i < NM) p.agg[(int64_t)blockIdx.x * NM + lane + 64 * i] = best[i];
+}
+
+// A vector's parts, split over four waves -> its picks.
+template <int NPL>
+__global__ __launch_bounds__(256) void lmk_block_select_kernel(RetrParams p, int n_parts) {
+  __shared__ uint32_t part[3][64 * NPL];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), NM = p.num_mems;
+  uint32_t best[NPL];
+#pragma unroll
+  for (int i = 0; i < NPL; ++i) best[i] = 0u;
+  constexpr int U = NPL <= 4 ? 8 : (NPL <= 16 ? 2 : 1);           // parts in flight
+  for (int s = wave; s < n_parts; s += 4 * U) {
+    uint32_t v[U][NPL];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t* src = p.agg + ((int64_t)blockIdx.x * n_parts + min(s + 4 * u, n_parts - 1)) * NM;   // past the end: the last again
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) v[u][i] = (lane + 64 * i < NM) ? src[lane + 64 * i] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) best[i] = max(best[i], v[u][i]);
+  }
+  if (wave > 0)
+#pragma unroll
+    for (int i = 0; i < NPL; ++i) part[wave - 1][64 * i + lane] = best[i];
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int i = 0; i < NPL; ++i)
+    best[i] = max(max(best[i], part[0][64 * i + lane]), max(part[1][64 * i + lane], part[2][64 * i + lane]));
+  select_blocks<NPL>(p, (int)blockIdx.x, best, lane);
 }
 
 // The same for vectors of any length: one wave per row, the row's exponentials written back over its scores.
@@ -312,12 +415,12 @@ __global__ __launch_bounds__(256) void lmk_block_prob_long_kernel(RetrParams p, 
   }
 }
 
-// One workgroup per (batch, head): the k best blocks of agg under (value desc, index asc), ascending.
+// Behind it, one workgroup per vector: the k best blocks of agg under (value desc, index asc), ascending.
 // Four waves bring the head's vector into LDS (and write the copy the caller may have asked for); the
 // first wave then picks k times over it.  Vectors too long for the LDS buffer are read in place.
 constexpr int kSelectLds = 8192;                                  // words of the LDS copy
 
-__global__ __launch_bounds__(256) void lmk_block_select_kernel(RetrParams p) {
+__global__ __launch_bounds__(256) void lmk_block_select_long_kernel(RetrParams p) {
   __shared__ uint32_t cached[kSelectLds];
   const int tid = threadIdx.x, lane = tid & 63, bh = blockIdx.x, NM = p.num_mems;
   const uint32_t* agg = p.agg + (int64_t)bh * NM;
@@ -509,14 +612,6 @@ template <>
 struct ScoreOrder<f16_t> {
   static constexpr uint32_t lo = 0x03ff, hi = 0xfc00;
 };
-
-// maximum over the 16 lanes of a DPP row, every lane of the row gets it
-__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));
-  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));
-}
 
 // TW: waves along the landmarks, one tile of 64 each
 template <class T, int D, int TW>
@@ -1529,21 +1624,27 @@ static int launch_topk_shared_t(const RetrParams& p, hipStream_t stream) {
   if ((rc = launch_scores<T, D>(p, stream))) return rc;
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   const int is_bf16 = std::is_same<T, bf16_t>::value ? 1 : 0;
-  if (p.num_mems <= 64 * 32) {
-    // rows per wave: as many as leave the chip a few thousand waves, at most 8
+  if (p.num_mems <= kProbMems) {
+    // rows per wave: a vector's rows in one workgroup where that is at most 8 each (the launch saved outweighs the rows in a
+    // row: 255 tokens over 40 blocks, maxima over 12 heads, 44.6 -> 42.1 us a step), else as many as leave the chip a few
+    // thousand waves
     const int group = p.agg_over_heads ? p.H : p.T;
-    const int rpw = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(8, group), rows / 4096));
-    const int64_t waves = (int64_t)((group + rpw - 1) / rpw) * sel_rows;
-    const dim3 grid((unsigned)((waves + 3) / 4));
-    if (p.num_mems <= 64) hipLaunchKernelGGL(lmk_block_prob_kernel<1>, grid, dim3(256), 0, stream, p, is_bf16, rpw);
-    else if (p.num_mems <= 64 * 4) hipLaunchKernelGGL(lmk_block_prob_kernel<4>, grid, dim3(256), 0, stream, p, is_bf16, rpw);
-    else if (p.num_mems <= 64 * 16) hipLaunchKernelGGL(lmk_block_prob_kernel<16>, grid, dim3(256), 0, stream, p, is_bf16, rpw);
-    else hipLaunchKernelGGL(lmk_block_prob_kernel<32>, grid, dim3(256), 0, stream, p, is_bf16, rpw);
-  } else {
-    hipLaunchKernelGGL(lmk_block_prob_long_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, is_bf16);
+    const int rpw = group <= 32 ? (group + 3) / 4 : (int)std::max<int64_t>(1, std::min<int64_t>(8, rows / 4096));
+    const int n_parts = (group + 4 * rpw - 1) / (4 * rpw);
+    const dim3 grid((unsigned)(sel_rows * n_parts));
+    auto launch = [&](auto prob, auto select) {
+      hipLaunchKernelGGL(prob, grid, dim3(256), 0, stream, p, is_bf16, rpw, n_parts);
+      if (n_parts > 1) hipLaunchKernelGGL(select, dim3((unsigned)sel_rows), dim3(256), 0, stream, p, n_parts);
+    };
+    if (p.num_mems <= 64) launch(lmk_block_prob_kernel<1>, lmk_block_select_kernel<1>);
+    else if (p.num_mems <= 64 * 4) launch(lmk_block_prob_kernel<4>, lmk_block_select_kernel<4>);
+    else if (p.num_mems <= 64 * 16) launch(lmk_block_prob_kernel<16>, lmk_block_select_kernel<16>);
+    else launch(lmk_block_prob_kernel<32>, lmk_block_select_kernel<32>);
+    return (int)hipGetLastError();
   }
+  hipLaunchKernelGGL(lmk_block_prob_long_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p, is_bf16);
   if ((rc = (int)hipGetLastError())) return rc;
-  hipLaunchKernelGGL(lmk_block_select_kernel, dim3((unsigned)sel_rows), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(lmk_block_select_long_kernel, dim3((unsigned)sel_rows), dim3(256), 0, stream, p);
   return (int)hipGetLastError();
 }
 
