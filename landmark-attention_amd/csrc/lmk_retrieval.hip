@@ -70,6 +70,17 @@ __device__ __forceinline__ float exp2_contract(float t) {
   return __builtin_ldexpf(pl, (int)n);
 }
 
+// Sum over the wave, folded by halves (lanes 32 apart, 16 apart, ... 1 apart), every lane gets it.  Behind the fold by 8 a lane's
+// value depends on its low three bits alone, so that a rotation by 4 within the row is the exchange of lanes 4 apart.
+__device__ __forceinline__ float wave_sum_halves(float v) {
+  v = v + __shfl_xor(v, 32, 64);
+  v = v + __shfl_xor(v, 16, 64);
+  v = v + dpp_f<0x128>(v);                                        // row_ror 8
+  v = v + dpp_f<0x124>(v);                                        // row_ror 4
+  v = v + dpp_f<0x4E>(v);                                         // quad_perm [2,3,0,1]
+  return v + dpp_f<0xB1>(v);                                      // quad_perm [1,0,3,2]
+}
+
 template <class T>
 __device__ __forceinline__ uint32_t prob_bits(float x);   // non-negative fp32 -> 16-bit pattern (RNE); monotone
 template <>
@@ -324,8 +335,7 @@ __global__ __launch_bounds__(256) void lmk_block_prob_kernel(RetrParams p, int m
         sum += x[i];
       }
     }
-#pragma unroll
-    for (int msk = 32; msk >= 1; msk >>= 1) sum = sum + __shfl_xor(sum, msk, 64);
+    sum = wave_sum_halves(sum);
 #pragma unroll
     for (int i = 0; i < NPL; ++i) {
       if (lane + 64 * i < NM) {
@@ -385,6 +395,177 @@ __global__ __launch_bounds__(256) void lmk_block_select_kernel(RetrParams p, int
   select_blocks<NPL>(p, (int)blockIdx.x, best, lane);
 }
 
+// Scores, probabilities and maxima in one launch, for one selection per head over at most 256 blocks: the scores of 16 (8 / TW)
+// query rows never leave the compute unit.  The scores are tiles of 16 rows x 64 landmarks by v_mfma_f32_16x16x1_4b_f32, the step
+// of the contract's chain that lmk_block_score_kernel takes 32 x 32 at a time: half as long a chain, twice as many waves to
+// overlap.  A workgroup rotates the head's landmark keys itself; TW of its eight waves share them out, the others' rows reuse them.
+// LDS: the rotated keys, then the scores and the waves' maxima in their place; the query rows.  What bounds it is a workgroup's
+// own chain (load, rotation, products, quotients, softmax, each behind a barrier); it saves the score plane's way to memory and
+// back and a launch -- with one part, two: there the picks are made here too.
+template <int D, int TW>
+struct ScoreProb {
+  static constexpr int G = 8 / TW, ROWS = G * 16;                 // 128 / TW rows
+  static constexpr int ROWB = 2 * D + 16;                         // 16 lanes reading 16 B of 16 rows hit every bank once
+  static constexpr int KEYB = 40;                                 // a landmark's 16 scores, 8 bytes apart from a multiple of 32
+  static constexpr int SC = G * TW * 64 * KEYB, PART = 8 * TW * 64 * 4;
+  static constexpr int KEYS = TW * 64 * ROWB > SC + PART ? TW * 64 * ROWB : SC + PART;
+  static constexpr int LDS = KEYS + ROWS * ROWB;
+};
+
+template <class T, int D, int TW>
+__global__ __launch_bounds__(512) void lmk_block_score_prob_kernel(RetrParams p, int model_is_bf16, int n_parts) {
+  using C = ScoreProb<D, TW>;
+  constexpr int CPR = D / 8, ROWB = C::ROWB, KEYB = C::KEYB;
+  extern __shared__ __align__(16) unsigned char smem[];
+  unsigned char *keys = smem, *sc = smem, *q_lds = smem + C::KEYS;
+  uint32_t* part = (uint32_t*)(smem + C::SC);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int NM = p.num_mems;
+  const int bh = (int)(blockIdx.x / (uint32_t)n_parts), t0 = (int)(blockIdx.x - (uint32_t)bh * n_parts) * C::ROWS;
+  const int b = bh / p.H, hh = bh - b * p.H;
+  const int tile = wave % TW, group = wave / TW;
+  {
+    constexpr int NQ = (C::ROWS * CPR + 511) / 512, NI = TW * 64 * CPR / 512, NB = NI < 4 ? NI : 4;
+    LandmarkChunk raw[NB];
+    auto load_raw = [&](int i) __attribute__((always_inline)) {   // keys behind the last one: a re-read
+      const int it = tid + 512 * i;
+      raw[i % NB] = load_landmark_chunk<D>(p, b, hh, min(it / CPR, NM - 1), it % CPR);
+    };
+    u32x4_t rows[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {                                // rows behind the last one: likewise
+      const int c = min(tid + 512 * i, C::ROWS * CPR - 1), t = min(t0 + c / CPR, p.T - 1);
+      rows[i] = *(const u32x4_t*)((const char*)p.q + 2 * (b * p.qs_b + hh * p.qs_h + (int64_t)t * p.qs_r + 8 * (c % CPR)));
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) load_raw(i);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int c = min(tid + 512 * i, C::ROWS * CPR - 1);
+      *(u32x4_t*)(q_lds + c / CPR * ROWB + 16 * (c % CPR)) = rows[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int it = tid + 512 * i, j = it % CPR;
+      const LandmarkChunk& k = raw[i % NB];
+      float r[8];
+      rotate_chunk<T>(k.x, k.other, k.c, k.s, j >= CPR / 2, r);
+      *(u32x4_t*)(keys + it / CPR * ROWB + 16 * j) = u32x4_t{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3]), pack2<T>(r[4], r[5]), pack2<T>(r[6], r[7])};
+      if (i + NB < NI) load_raw(i + NB);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();
+  f32x16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const bool busy = 64 * tile < NM && t0 + 16 * group < p.T;      // wave-uniform
+  if (busy) {
+    const unsigned char* qr = q_lds + (16 * group + (lane & 15)) * ROWB;
+    const unsigned char* key = keys + (64 * tile + lane) * ROWB;
+    // a chunk's operands are unpacked together, under the MFMAs of the chunk before: an unpack that writes the operand of an
+    // MFMA in flight waits for its end
+    float qv[2][8], kv[2][8];
+    u32x4_t qc = *(const u32x4_t*)qr, kc = *(const u32x4_t*)key;
+    auto unpack = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        qv[c & 1][i] = (i & 1) ? unpack_hi<T>(qc[i >> 1]) : unpack_lo<T>(qc[i >> 1]);
+        kv[c & 1][i] = (i & 1) ? unpack_hi<T>(kc[i >> 1]) : unpack_lo<T>(kc[i >> 1]);
+        asm volatile("" : "+v"(qv[c & 1][i]), "+v"(kv[c & 1][i]));
+      }
+      if (c + 1 < CPR) {
+        qc = *(const u32x4_t*)(qr + 16 * (c + 1));
+        kc = *(const u32x4_t*)(key + 16 * (c + 1));
+      }
+    };
+    unpack(0);
+#pragma unroll
+    for (int c = 0; c < CPR; ++c) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(qv[c & 1][i], kv[c & 1][i], acc, 0, 0, 0);
+        if (i == 3 && c + 1 < CPR) unpack(c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __syncthreads();                                                // the keys have been read
+  if (busy) {
+    // register 4 blk + r of lane l: row 4 (l / 16) + r, landmark 16 blk + l % 16 of the tile
+    unsigned char* dst = sc + ((group * TW + tile) * 64 + (lane & 15)) * KEYB + 8 * (lane >> 4);
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = contract<T>(acc[4 * blk + i], p.sqrt_hd);
+      *(u32x2_t*)(dst + 16 * blk * KEYB) = u32x2_t{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};   // exact: rounded already
+    }
+  }
+  __syncthreads();
+  // softmax and maxima as in lmk_block_prob_kernel, the rows from LDS
+  uint32_t best[TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i) best[i] = 0u;
+  constexpr int RU = 4;                                           // rows side by side: a row is a chain of reductions
+  for (int r0 = wave; r0 < C::ROWS && t0 + r0 < p.T; r0 += 8 * RU) {
+    float x[RU][TW], mx[RU], sum[RU];
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int r = min(r0 + 8 * u, p.T - 1 - t0);                // rows behind the last one: that one again
+      const unsigned char* src = sc + (r / 16 * TW * 64 + lane) * KEYB + 2 * (r % 16);
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+        x[u][i] = (lane + 64 * i < NM) ? unpack_lo<T>((uint32_t)*(const uint16_t*)(src + 64 * i * KEYB)) : -INFINITY;
+    }
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      mx[u] = x[u][0];
+#pragma unroll
+      for (int i = 1; i < TW; ++i) mx[u] = fmaxf(mx[u], x[u][i]);
+      mx[u] = wave_max(mx[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      sum[u] = 0.f;
+#pragma unroll
+      for (int i = 0; i < TW; ++i) {
+        float d = x[u][i] - mx[u];
+        asm volatile("" : "+v"(d));                               // the product below stays a product
+        x[u][i] = exp2_contract(d * kLog2e);
+        sum[u] += lane + 64 * i < NM ? x[u][i] : 0.f;             // + 0 changes nothing
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < RU; ++u) sum[u] = wave_sum_halves(sum[u]);
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+#pragma unroll
+      for (int i = 0; i < TW; ++i) {
+        const float pr = __fdiv_rn(x[u][i], sum[u]);
+        const uint32_t bits = p.prob32 ? __float_as_uint(pr) : (model_is_bf16 ? prob_bits<bf16_t>(pr) : prob_bits<f16_t>(pr));
+        best[i] = max(best[i], bits);
+      }
+  }
+  if (wave > 0)
+#pragma unroll
+    for (int i = 0; i < TW; ++i) part[(wave * TW + i) * 64 + lane] = best[i];
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 1; w < 8; ++w)
+#pragma unroll
+    for (int i = 0; i < TW; ++i) best[i] = max(best[i], part[(w * TW + i) * 64 + lane]);
+  if (n_parts == 1) {
+    select_blocks<TW>(p, bh, best, lane);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TW; ++i)
+    if (lane + 64 * i < NM) p.agg[(int64_t)blockIdx.x * NM + lane + 64 * i] = best[i];
+}
+
 // The same for vectors of any length: one wave per row, the row's exponentials written back over its scores.
 __global__ __launch_bounds__(256) void lmk_block_prob_long_kernel(RetrParams p, int model_is_bf16) {
   const int lane = threadIdx.x & 63;
@@ -405,8 +586,7 @@ __global__ __launch_bounds__(256) void lmk_block_prob_long_kernel(RetrParams p, 
     sc[m] = e;
     sum += e;
   }
-#pragma unroll
-  for (int msk = 32; msk >= 1; msk >>= 1) sum = sum + __shfl_xor(sum, msk, 64);
+  sum = wave_sum_halves(sum);
   uint32_t* agg = p.agg + (int64_t)(p.agg_over_heads ? b * p.T + t : bh) * NM;
   for (int m = lane; m < NM; m += 64) {
     const float pr = __fdiv_rn(sc[m], sum);
@@ -1621,9 +1801,26 @@ template <class T, int D>
 static int launch_topk_shared_t(const RetrParams& p, hipStream_t stream) {
   int rc;
   const int64_t sel_rows = p.agg_over_heads ? (int64_t)p.B * p.T : (int64_t)p.B * p.H;   // vectors to pick from
+  const int is_bf16 = std::is_same<T, bf16_t>::value ? 1 : 0;
+  // Scores and maxima in one launch, but for more than 128 blocks at head dim 128 where a head's rows take several workgroups:
+  // each rotates 64 KB of keys.  Steps in us, two launches / one: 256 queries, 256 blocks, D64 35.2 / 28.9; 2 x 512 queries, 128
+  // blocks, D64 46.0 / 39.9, D128 59.8 / 54.7; 64 blocks, 512 queries, D128 43.4 / 41.0; 16 queries over 8 blocks 25.0 / 17.6.
+  // 256 blocks, D128: 16 queries 33.6 / 29.6, 256 queries 38.2 / 37.7, 512 queries 52.3 / 53.8, 2 x 400 queries 68.7 / 75.8.
+  const int tw = p.num_mems <= 64 ? 1 : (p.num_mems <= 128 ? 2 : 4), prob_parts = (p.T + 128 / tw - 1) / (128 / tw);
+  if (!p.agg_over_heads && p.num_mems <= 256 && (D == 64 || tw < 4 || prob_parts == 1)) {
+    static std::atomic<uint64_t> lds_ok[3];
+    auto launch = [&](auto kern, int lds, std::atomic<uint64_t>& ok, auto select) {
+      if (int e = allow_dynamic_lds(kern, lds, ok)) return e;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(sel_rows * prob_parts)), dim3(512), lds, stream, p, is_bf16, prob_parts);
+      if (prob_parts > 1) hipLaunchKernelGGL(select, dim3((unsigned)sel_rows), dim3(256), 0, stream, p, prob_parts);
+      return (int)hipGetLastError();
+    };
+    if (tw == 1) return launch(lmk_block_score_prob_kernel<T, D, 1>, ScoreProb<D, 1>::LDS, lds_ok[0], lmk_block_select_kernel<1>);
+    if (tw == 2) return launch(lmk_block_score_prob_kernel<T, D, 2>, ScoreProb<D, 2>::LDS, lds_ok[1], lmk_block_select_kernel<2>);
+    return launch(lmk_block_score_prob_kernel<T, D, 4>, ScoreProb<D, 4>::LDS, lds_ok[2], lmk_block_select_kernel<4>);
+  }
   if ((rc = launch_scores<T, D>(p, stream))) return rc;
   const int64_t rows = (int64_t)p.B * p.H * p.T;
-  const int is_bf16 = std::is_same<T, bf16_t>::value ? 1 : 0;
   if (p.num_mems <= kProbMems) {
     // rows per wave: a vector's rows in one workgroup where that is at most 8 each (the launch saved outweighs the rows in a
     // row: 255 tokens over 40 blocks, maxima over 12 heads, 44.6 -> 42.1 us a step), else as many as leave the chip a few
