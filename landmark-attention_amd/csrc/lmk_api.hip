@@ -745,7 +745,8 @@ static int gather_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kcache, c
   if ((rc = check_retrieval(B, H, T, S, D, block, top_k, dtype, n_pos))) return rc;
   if (!(block == 32 || block == 64 || block == 128)) return LMK_ERR_UNSUPPORTED;
   if (!local && stat_stride < T) return LMK_ERR_SHAPE;
-  if (local && !lmk::gather_takes_local_window(T, S, block)) return LMK_ERR_UNSUPPORTED;
+  if (local && !lmk::gather_takes_local_window(T, S, block, kcache->stride_row, vcache->stride_row, table_stride_row))
+    return LMK_ERR_UNSUPPORTED;
   if (!std::isfinite(sm_scale) || !(sm_scale > 0.f)) return LMK_ERR_SCALE;
   lmk::RetrParams p = {};
   fill_retr_common(p, B, H, T, S, D, block, top_k);
@@ -1163,7 +1164,8 @@ int lmk_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk_tensor
   const int inc = S % block;
   const AttendLayout l = attend_layout(B, H, T, S, D, block);
   if (workspace_bytes < l.total) return LMK_ERR_WORKSPACE;
-  if (lmk::gather_takes_local_window(T, S, block))             // a handful of new tokens: one launch, nothing staged
+  if (lmk::gather_takes_local_window(T, S, block, kcache->stride_row, vcache->stride_row, table_stride_row))
+    // a handful of new tokens: one launch, nothing staged
     return gather_attend_impl(q, kcache, vcache, idx, cos_table, sin_table, table_stride_row, n_pos, nullptr, nullptr,
                               nullptr, 0, out, B, H, T, S, D, sm_scale, block, top_k, dtype, stream, nullptr, k_loc, v_loc);
   char* w = static_cast<char*>(workspace);
@@ -1211,7 +1213,7 @@ static int retrieve_and_attend_impl(const lmk_tensor4* q, const lmk_tensor4* kca
   if (retrieve_workspace == nullptr) return LMK_ERR_NULL;
   if (!aligned16(retrieve_workspace)) return LMK_ERR_ALIGN;
   if (retrieve_workspace_bytes < retr_layout(B, H, T, S, D, block).total) return LMK_ERR_WORKSPACE;
-  if (lmk::gather_takes_local_window(T, S, block)) {
+  if (lmk::gather_takes_local_window(T, S, block, kcache->stride_row, vcache->stride_row, table_stride_row)) {
     // decode: the selection (slice step where it serves, else the fused top-k), then a gather that merges the
     // slices' candidates and attends to the local window itself -- no window, no forward launch
     int rc;

@@ -134,7 +134,8 @@ __global__ __launch_bounds__(64 * (kDecodeWaves + 1), 3) void lmk_gather_decode_
       const char* vb = vc + 2 * ((int64_t)blk * BS * p.vcs_r);
       const char *cb = (const char*)p.cos + 2 * (pos0 * p.cs_r), *sb = (const char*)p.sin + 2 * (pos0 * p.cs_r);
       __builtin_amdgcn_s_waitcnt(0xc07f);               // the block before: its keys have been read
-      // What the addresses have in common per lane; formed here, or the loop would keep forty sums of it.
+      // What the addresses have in common per lane, in 32 bits (gather_takes_local_window); formed here, or the loop would keep
+      // forty sums of it.
       int ln = lane;
       asm volatile("" : "+v"(ln));
       {

@@ -269,10 +269,14 @@ int launch_fwd32_topk_slices(const FwdParams& pf, const RetrParams& pr, int D, i
 int launch_landmark_keys(const RetrParams& p, int D, int dtype, hipStream_t stream);   // the rotation alone
 int launch_topk_slices(const RetrParams& p, int D, int dtype, hipStream_t stream);     // the selection's slice step alone
 int launch_topk_slice_merge(const RetrParams& p, hipStream_t stream);                  // behind it: the rows' indices
-// rows whose local window the gather kernel attends to itself: window inside one block, a handful of new tokens
+// rows whose local window the gather kernel attends to itself: window inside one block, a handful of new tokens, and row
+// strides of the cache and the tables that let eight rows be addressed from the first with 32 bits (a table may be handed over
+// back to front, with a negative stride; such calls take the launches of longer chunks, which form every address with 64)
 constexpr int kLocalMaxT = 4;
-inline bool gather_takes_local_window(int T, int S, int block) {
-  return (block == 32 || block == 64 || block == 128) && T <= kLocalMaxT && S % block + T <= block;
+inline bool decode_stride(int64_t elements) { return elements >= 0 && elements < ((int64_t)1 << 28); }
+inline bool gather_takes_local_window(int T, int S, int block, int64_t kcs_r, int64_t vcs_r, int64_t cs_r) {
+  return (block == 32 || block == 64 || block == 128) && T <= kLocalMaxT && S % block + T <= block && decode_stride(kcs_r) &&
+         decode_stride(vcs_r) && decode_stride(cs_r);
 }
 // BS: slots per block (32, 64 or 128); p.block <= BS tokens per block in the cache
 int launch_gather_attend(const RetrParams& p, int D, int BS, int dtype, hipStream_t stream);
