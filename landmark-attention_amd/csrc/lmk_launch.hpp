@@ -205,7 +205,7 @@ struct RotaryParams {
   const int64_t* pos;
   int64_t pos_stride_b, n_pos;
   int transposed;                                 // the gradient's rotation: the sine table's halves swapped and negated
-  int B, H, L, b0;                                // b0: first batch of the launch
+  int B, H, L, b0;                                // b0: first batch of a launch, which ends at B
   int64_t xs_b, xs_h, xs_r, os_b, os_h, os_r, cs_r;
 };
 

@@ -39,6 +39,24 @@ def test_rotary_bit_exact_against_oracle_and_torch_arithmetic(B, H, L, D, dtype)
     assert none_q is None and torch.equal(gk1.cpu(), orot.apply_rotary(k, cos, sin, row[:, None, :]))
 
 
+@pytest.mark.parametrize("B,H,L,D", [(517, 1, 1, 64), (131, 3, 1, 128), (41, 5, 3, 64), (9, 7, 5, 128)])
+@pytest.mark.parametrize("tokens_first", [False, True])
+def test_rotary_of_many_short_sequences(B, H, L, D, tokens_first):
+    # a workgroup's 32 or 64 rows are of several batches, its last ones of none; in place, each row once
+    from landmark_hip import _lib
+    print(f"case B{B} H{H} L{L} D{D} {tokens_first}", flush=True)
+    q, k, cos, sin, n_pos, g = _case(B, H, L, D, torch.bfloat16, seed=B)
+    pos = torch.randint(0, n_pos, (B, L), generator=g)
+    want = [orot.apply_rotary(x, cos, sin, pos[:, None, :]) for x in (q, k)]
+    q, k = ((x.transpose(1, 2).contiguous().cuda().transpose(1, 2) if tokens_first else x.cuda()) for x in (q, k))
+    cos, sin, pos = cos.cuda(), sin.cuda(), pos.cuda()
+    for x in (q, k):
+        _lib.check(_lib.lib().lmk_apply_rotary(_lib.tensor4(x), _lib.tensor4(x), cos.data_ptr(), sin.data_ptr(), cos.stride(0),
+                                               cos.shape[0], pos.data_ptr(), L, B, H, L, D, 0, _lib.current_stream(x.device)))
+    torch.cuda.synchronize()
+    assert torch.equal(q.cpu(), want[0]) and torch.equal(k.cpu(), want[1])
+
+
 def test_rotary_on_projection_layout_and_in_place():
     # (B, L, H, D) memory viewed as (B, H, L, D), as the projections leave it (llama_mem.py:287-289)
     from landmark_hip import _lib
