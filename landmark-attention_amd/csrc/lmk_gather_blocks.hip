@@ -9,10 +9,11 @@
 // A pick is (row, rank), and a block's keys sit at positions that depend on the pick's rank in its row: a wave takes 32
 // picks of one rank, rotates the keys for that rank as it reads them -- fragment ks of a lane holds its key's head dims
 // 16 ks + 8 h .. + 7, whose rotary partners are fragment ks + KS / 2 of the same lane -- and multiplies the rotated key as
-// the sum of two 16-bit numbers, hi + lo, so that it keeps 16 (bf16) or 22 (fp16) bits.  The local softmax and the sum
-// over the values are those of the forward kernels (a lane owns a row).  (Rotating by the whole workgroup into LDS, with picks
+// the sum of three 16-bit numbers, which keeps every bit of the fp32 rotation (KeyParts; with two, scores in the thousands
+// came out up to 1.6 times as far from float64 as row by row; the third costs the step 1 to 3 %).  The local softmax and the
+// sum over the values are those of the forward kernels (a lane owns a row).  (Rotating by the whole workgroup into LDS, with picks
 // of all ranks side by side in one product, has two barriers and a round trip to the tables per rank: block 128, head dim 128,
-// 32 heads, 256 queries, top 4 of 64 blocks 194 us a step against 123.)  What bounds it is the vector work of a rotation, ~9
+// 32 heads, 256 queries, top 4 of 64 blocks 194 us a step against 123.)  What bounds it is the vector work of a rotation, ~12
 // instructions per key and head dim, and the chain of loads in front of it: picks, queries, table rows.
 // What a pick contributes -- the landmark's score and the normalised sum over the block, fp32 -- goes to a workspace, and
 // lmk_gather_combine_kernel puts each row's picks and its local window together.
@@ -43,9 +44,44 @@ struct GatherBlocksCfg {
   static_assert(PER_WAVE * RPD * 4 == BS, "every wave issues the same number of requests");
 };
 
-template <class T> __device__ __forceinline__ float largest();
-template <> __device__ __forceinline__ float largest<bf16_t>() { return 3.3895313892515355e38f; }
-template <> __device__ __forceinline__ float largest<f16_t>() { return 65504.f; }
+// Rotated keys a, b (fp32) -> the operands hi, mid, lo of 16 bits each whose sum they are:
+//   key = up (hi + step (mid + lo)),  score = up (q . hi + step (q . mid + q . lo))
+// bf16: up = step = 1, three times eight bits by truncation: exact.  fp16: eleven bits and eleven of the rest, scaled by 1 / step
+// to lie in fp16's range whatever the key, and what is left; up keeps rotated keys of fp16's largest values in range.
+// The rest is formed from the clamped key, so that it stays finite where the key is infinite or NaN, which hi alone carries.
+template <class T>
+struct KeyParts;
+template <>
+struct KeyParts<bf16_t> {
+  static constexpr float up = 1.f, step = 1.f;
+  static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    constexpr float most = 3.4028234663852886e38f;
+    auto top = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+    auto tops = [](float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); };
+    const float ca = __builtin_amdgcn_fmed3f(a, -most, most), cb = __builtin_amdgcn_fmed3f(b, -most, most);
+    const float ma = ca - top(ca), mb = cb - top(cb);
+    hi = tops(a, b);
+    mid = tops(ma, mb);
+    lo = tops(ma - top(ma), mb - top(mb));
+  }
+};
+template <>
+struct KeyParts<f16_t> {
+  static constexpr float up = 16.f, step = 1.f / 2048.f;
+  static __device__ __forceinline__ uint32_t trunc2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+  }
+  static __device__ __forceinline__ void split(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    constexpr float most = 65504.f;
+    const float xa = a * (1.f / up), xb = b * (1.f / up);
+    const float ca = __builtin_amdgcn_fmed3f(xa, -most, most), cb = __builtin_amdgcn_fmed3f(xb, -most, most);
+    const uint32_t h = trunc2(ca, cb);
+    const float ma = (ca - unpack_lo<f16_t>(h)) * (1.f / step), mb = (cb - unpack_hi<f16_t>(h)) * (1.f / step);
+    hi = trunc2(xa, xb);
+    mid = trunc2(ma, mb);
+    lo = trunc2(ma - unpack_lo<f16_t>(mid), mb - unpack_hi<f16_t>(mid));
+  }
+};
 
 // Rows t_first .. t_first + t_rows - 1 of every (batch, head); the workspace holds these rows' picks.
 template <class T, int D, int BS, bool PADDED>
@@ -106,7 +142,8 @@ __global__ __launch_bounds__(256, 2) void lmk_gather_blocks_kernel(RetrParams p,
   int koff[C::KS];                                      // the operands' places in the first tile
 #pragma unroll
   for (int ks = 0; ks < C::KS; ++ks) koff[ks] = tile_off<D>(ql, 2 * ks + h);
-  const float c2 = p.scale_log2;
+  using P = KeyParts<T>;
+  const float c2 = p.scale_log2 * P::up;
 
   for (int seg = 0; seg < picks; seg += kPickSegment) {
     if (seg > 0) {
@@ -187,13 +224,13 @@ __global__ __launch_bounds__(256, 2) void lmk_gather_blocks_kernel(RetrParams p,
       };
 #pragma unroll
       for (int n = 0; n < PF; ++n) fetch_tables(n);
-      f32x16_t s[C::NT];
+      f32x16_t s[C::NT], rest;
 #pragma unroll
       for (int n = 0; n < NX; ++n) {
         const int nt = n / (C::KS / 2), ks = n % (C::KS / 2);
         const u32x4_t klo = lds_ld128(ktile + 32 * nt * C::ROWB + koff[ks]), khi = lds_ld128(ktile + 32 * nt * C::ROWB + koff[ks + C::KS / 2]);
         const u32x4_t *x = tab[n % PF];
-        u32x4_t hi[2], lo[2];                           // of both halves
+        u32x4_t hi[2], mid[2], lo[2];                   // of both halves
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           float y[2][2];                                // half, element
@@ -206,19 +243,29 @@ __global__ __launch_bounds__(256, 2) void lmk_gather_blocks_kernel(RetrParams p,
           rot(unpack_hi<T>(klo[d]), unpack_hi<T>(khi[d]), unpack_hi<T>(x[0][d]), unpack_hi<T>(x[1][d]), unpack_hi<T>(x[2][d]),
               unpack_hi<T>(x[3][d]), 1);
 #pragma unroll
-          for (int hf = 0; hf < 2; ++hf) {              // hi stays finite, so that lo of an infinite key is not a NaN
-            hi[hf][d] = pack2<T>(__builtin_amdgcn_fmed3f(y[hf][0], -largest<T>(), largest<T>()),
-                                 __builtin_amdgcn_fmed3f(y[hf][1], -largest<T>(), largest<T>()));
-            lo[hf][d] = pack2<T>(y[hf][0] - unpack_lo<T>(hi[hf][d]), y[hf][1] - unpack_hi<T>(hi[hf][d]));
+          for (int hf = 0; hf < 2; ++hf) {
+            uint32_t a, b, c;
+            P::split(y[hf][0], y[hf][1], a, b, c);
+            hi[hf][d] = a;
+            mid[hf][d] = b;
+            lo[hf][d] = c;
           }
         }
         if (n + PF < NX) fetch_tables(n + PF);
-        if (ks == 0) zero16(s[nt]);
+        if (ks == 0) {
+          zero16(s[nt]);
+          if (P::step != 1.f) zero16(rest);
+        }
+        f32x16_t& low = P::step == 1.f ? s[nt] : rest;
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
           s[nt] = mfma32<T>(hi[hf], qf[ks + hf * (C::KS / 2)], s[nt]);
-          s[nt] = mfma32<T>(lo[hf], qf[ks + hf * (C::KS / 2)], s[nt]);
+          low = mfma32<T>(mid[hf], qf[ks + hf * (C::KS / 2)], low);
+          low = mfma32<T>(lo[hf], qf[ks + hf * (C::KS / 2)], low);
         }
+        if (P::step != 1.f && ks + 1 == C::KS / 2)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[nt][i] = __builtin_fmaf(rest[i], P::step, s[nt][i]);
         __builtin_amdgcn_sched_barrier(0);
       }
       // ---- softmax over the block's normal keys, the landmark's score as it is (last slot: last tile, register 15, h = 1)
