@@ -31,6 +31,8 @@ struct bf16_t {};  // element tags
 struct f16_t {};
 
 constexpr float kLog2e = 1.4426950408889634f;
+// Running maximum in front of the first score: finite, so that a first score of -infinity takes its weight to 0 and not to NaN.
+constexpr float kNoScore = -3.0e38f;
 constexpr float kLn2 = 0.6931471805599453f;
 
 // ---- MFMA ---------------------------------------------------------------

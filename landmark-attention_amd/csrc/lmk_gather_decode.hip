@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * (kDecodeWaves + 1), 3) void lmk_gather_decode_
     unpack(*(const vec_t*)qp, qlo);
     unpack(*(const vec_t*)(qp + D), qhi);
   }
-  float Mrun = -INFINITY, lrun = 0.f;                   // global bucket: maximum (log2 domain), sum
+  float Mrun = kNoScore, lrun = 0.f;                    // global bucket: maximum (log2 domain), sum
   float alo[E], ahi[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) alo[i] = ahi[i] = 0.f;

@@ -1451,7 +1451,7 @@ __global__ __launch_bounds__(256) void lmk_gather_attend_kernel(RetrParams p) {
     return age >= p.num_mems - p.k;
   };
 
-  float Mrun = -INFINITY, lrun = 0.f;
+  float Mrun = kNoScore, lrun = 0.f;
   float alo[E], ahi[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) {
@@ -1684,7 +1684,7 @@ __global__ __launch_bounds__(256) void lmk_gather_attend_kernel(RetrParams p) {
     }
 #pragma unroll
     for (int w = 0; w < NWV; ++w) {
-      const float sw = fast_exp2(mw[w] - Mall);                   // 0 for a wave without blocks (M = -inf)
+      const float sw = fast_exp2(mw[w] - Mall);                   // 0 for a wave without blocks, or times nothing
       lrun = __builtin_fmaf(part_ml[w][1], sw, lrun);
 #pragma unroll
       for (int e = 0; e < E; ++e) {

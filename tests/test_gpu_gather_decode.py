@@ -41,3 +41,24 @@ def test_decode_step_matches_the_oracle(B, H, T, n, tail, block, k, D, dtype):
                                                    n_buckets=128)    # 64 hold the window's group and 63 picked blocks
         assert torch.equal(idx[s].cpu(), want_idx)
         assert (out[s].float().cpu() - want.float()).abs().max() <= TOL
+
+
+@pytest.mark.parametrize("B,H,T,n,tail,block,D", [(1, 2, 1, 1, 5, 32, 64), (1, 3, 1, 3, 7, 64, 128), (1, 3, 1, 12, 7, 32, 64), (3, 11, 40, 1, 0, 64, 128),
+                                                  (1, 3, 40, 2, 0, 32, 64)])
+def test_a_first_block_behind_a_landmark_of_minus_infinity_weighs_nothing(B, H, T, n, tail, block, D):
+    """Every block is picked; the landmark of block 0, the first a wave takes, scores -infinity for every query.  Decode steps (a wave
+    for each block, for some of them) and chunks row by row (one row per wave, waves that share a row out)."""
+    from landmark_hip.retrieval import gather_attend
+    print(f"case {B} {H} {T} {n} {tail} block {block} D{D}", flush=True)
+    S = n * block + tail
+    g = torch.Generator().manual_seed(S + D)
+    make = lambda rows: (torch.randn(B, H, rows, D, generator=g) * 0.5).bfloat16()
+    q, kc, vc, kl, vl = (make(r) for r in (T, S, S, T, T))
+    q = q.abs()
+    kc[:, :, block - 1, 3] = -float("inf")                                  # both partners of its rotation by 0.5
+    cos, sin = (f(torch.full((S + T, D), 0.5)).bfloat16() for f in (torch.cos, torch.sin))
+    idx = torch.arange(n).expand(B, H, T, n).contiguous()
+    mem = ((torch.arange(T) + tail) % block == block - 1)[None].expand(B, T)
+    want, _ = oret.retrieve_and_attend(q, kc, vc, kl, vl, mem, cos, sin, block, n, idx=idx)
+    out = gather_attend(*(t.cuda() for t in (q, kc, vc, idx, kl, vl, cos, sin)), block, n)
+    assert (out.float().cpu() - want.float()).abs().max() <= TOL
