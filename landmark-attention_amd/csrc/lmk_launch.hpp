@@ -285,10 +285,17 @@ int launch_gather_decode(const RetrParams& p, int D, int dtype, hipStream_t stre
 // Gather by block (lmk_gather_blocks.hip): the rows of a (batch, head) whose picks the workspace holds at a time, or 0 where
 // the gather by row serves.  A rotation of a block's keys serves the picks of one rank, and a block is picked at about
 // sqrt(k) ranks, so what decides is picks per block and rank, times the block (a pick costs 1 KB of workspace traffic at head
-// dim 128 whatever its block); and the rows' reads must outweigh the second launch.  Whole steps by row and by block, us, 32
-// heads, 256 queries, top 4, D128: block 32, 8 picks a block 90.1 / 80.3, 4 picks 100.3 / 106.9; block 64, 8 picks 156 / 112,
-// 4 picks 172 / 159; block 128, 4 picks 400 / 292, top 1 of 256 blocks, 1 pick 153 / 199.  Fewer rows: 8 heads, 128 queries,
-// block 64, 8 picks, 134 MB 44.1 / 41.2; at D64, 67 MB 32.4 / 33.1; block 128 at D64, 134 MB 42.8 / 44.9 and 268 MB 67.4 / 62.3.
+// dim 128 whatever its block); and the rows' reads must outweigh the second launch.  Whole steps by row / by block, us, 256
+// queries of 32 heads, D128, picks spread evenly: block 32, 8 picks a rank 70.5 / 58.1, 4 picks 83.3 / 75.5; block 64, 4 picks
+// 143.6 / 107.3, 2.7 picks 150.2 / 131.8, 2 picks 159.1 / 163.9; block 128, 2.7 picks 133.3 / 102.6, 2 picks 133.1 / 129.8, 1.6
+// picks 140.7 / 154.2, 1.5 picks 138.6 / 159.7; D64, 512 queries, block 128, 2.7 picks 106.1 / 90.3, 2 picks 104.7 / 111.8.  (Block
+// 32 would gain from 128 on; the line is the one that holds for all blocks.)
+// Fewer rows, all picks 4 a rank or more: 8 heads, 128 queries, block 64, 134 MB 44.1 / 41.2; at D64, 67 MB 32.4 / 33.1; block 128 at
+// D64, 134 MB 42.8 / 44.9 and 268 MB 67.4 / 62.3.
+// Where all rows of a head pick the same blocks, few workgroups have all the work: with 32 heads that is made up for (block 64, 4
+// picks 106.0 / 66.6), with few heads and low k it is not: 8 heads, D128, block 64, 512 queries, top 1 47.6 / 31.8 spread evenly and
+// 40.5 / 57 all the same; 947 queries, top 3 106 / 75 and 97 / 121; 12 heads, D64, 789 queries, top 2 76 / 37 and 75 / 54.  How the
+// picks lie is not known when the launches are made.
 constexpr int64_t kGatherBlocksBytes = (int64_t)256 << 20;        // of workspace, at most
 inline int64_t gather_blocks_pick_bytes(int D) { return 4 * ((int64_t)D + 1); }
 inline int gather_blocks_rows(int B, int H, int T, int num_mems, int D, int block, int k, bool shared) {
@@ -297,7 +304,7 @@ inline int gather_blocks_rows(int B, int H, int T, int num_mems, int D, int bloc
   if (heads * rows * k * block * 4 * D < (int64_t)(block > 64 && D == 64 ? 256 : 128) << 20) return 0;
   // one selection for all rows of a head: k blocks, each at one rank
   const double picks = shared ? (double)rows : (double)rows * k / num_mems / std::sqrt((double)k);
-  return picks * block >= 192 ? (int)rows : 0;
+  return picks * block >= 192 && picks >= 2.25 ? (int)rows : 0;
 }
 int launch_gather_blocks(const RetrParams& p, int D, int BS, int rows, int dtype, hipStream_t stream);
 

@@ -429,3 +429,12 @@ def test_block_table_is_checked_on_the_host(lib):
     bwd = lib.lmk_attn_bwd_segments(t, t, t, t, t, 0x2000, 0x3000, t, t, t, 0x4000, 16, arr, 0x9000, 3, 6, 1, 1, 12, 12, 128,
                                     0.1, 0, 0, None)
     assert bwd == -8                                           # workspace too small: nothing is launched
+
+
+@pytest.mark.parametrize("T,n,D,block,k,shared,by_block", [
+    (256, 171, 128, 128, 1, 0, False), (256, 128, 128, 128, 1, 0, False),        # few picks of a block at a rank: by row
+    (256, 96, 128, 128, 1, 0, True), (512, 256, 64, 128, 1, 0, False), (512, 192, 64, 128, 1, 0, True),
+    (256, 256, 128, 64, 4, 0, False), (256, 128, 128, 64, 4, 0, True), (256, 2000, 128, 128, 1, 1, True)])
+def test_scratch_of_a_gather_by_block_says_where_it_serves(lib, T, n, D, block, k, shared, by_block):
+    need = lib.lmk_gather_blocks_workspace_bytes(1, 32, T, n, D, block, k, shared)
+    assert need == (-(-32 * T * k * (D + 1) * 4 // 256) * 256 if by_block else 0)
