@@ -159,3 +159,38 @@ def test_keys_that_are_not_finite(dtype):
     finite = by_row.isfinite()
     worst = (by_row - by_block)[finite].abs().max().item()
     assert worst <= (3e-2 if dtype == torch.bfloat16 else 4e-3)     # two roundings to 16 bits of values up to 4
+
+
+# The same kernels behind the flat cache's entry points: B, H, T, cached blocks, tokens behind them, block, top_k, D.  Rows that select by
+# slices, and others; chunks longer than a block, chunks behind a tail; every row stride of the window and its statistics counts.
+FLAT = [(1, 8, 128, 60, 0, 32, 8, 128), (1, 32, 256, 128, 0, 64, 4, 128), (1, 32, 64, 6, 40, 128, 4, 128), (3, 32, 24, 4, 8, 32, 4, 128),
+        (2, 37, 31, 4, 1, 32, 4, 128), (2, 32, 300, 20, 0, 64, 4, 64), (1, 12, 333, 70, 0, 128, 3, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,T,n,tail,block,k,D", FLAT)
+def test_flat_cache_by_block_matches_the_oracle(B, H, T, n, tail, block, k, D, dtype):
+    from landmark_hip import _lib
+    from landmark_hip.retrieval import gather_attend, retrieve_and_attend
+    from oracle import retrieval as oret
+    from oracle import rotary as orot
+    print(f"case {B} {H} {T} {n} {tail} block {block} top {k} D{D} {dtype}", flush=True)
+    assert _lib.lib().lmk_gather_blocks_workspace_bytes(B, H, T, n, D, block, k, 0) > 0
+    S = n * block + tail
+    g = torch.Generator().manual_seed(S + D + k)
+    make = lambda rows: (torch.randn(B, H, rows, D, generator=g) * 0.5).to(dtype)
+    q, kc, vc, kl, vl = (make(r) for r in (T, S, S, T, T))
+    cos, sin = orot.rotary_tables(S + T, D, dtype)
+    dev = [t.cuda() for t in (q, kc, vc, kl, vl, cos, sin)]
+    out, idx = retrieve_and_attend(dev[0], (dev[1], dev[2]), *dev[3:], block, k)
+    apart = gather_attend(*dev[:3], idx, *dev[3:], block, k)
+    assert torch.equal(apart, out)
+    rows = sorted({0, 1, T // 2, T - 2, T - 1, min(T - 1, block - 1), min(T - 1, block)})
+    for b, h in {(0, 0), (B - 1, H - 1)}:
+        s = (slice(b, b + 1), slice(h, h + 1))
+        want_idx = oret.select_topk(oret.landmark_scores(q[s], kc[s], cos, sin, block, k), k)
+        assert torch.equal(idx[s].cpu(), want_idx)
+        want = oret.retrieve_and_attend_s1(q[s], kc[s], vc[s], kl[s], vl[s], cos, sin, block, k, want_idx, tokens=rows)
+        for (_, _, t), o in want.items():
+            # 16-bit weights, output and (oracle) rotated keys, values up to about 2
+            assert (out[b, h, t].float().cpu() - o).abs().max() <= (2e-2 if dtype == torch.bfloat16 else 2.5e-3), (b, h, t)
