@@ -356,7 +356,8 @@ def test_baseline_config4_full_size(seed):
         assert (out[b, h, t] - o).abs().max().item() <= 2e-2, (b, h, t)
 
 
-@pytest.mark.parametrize("T,n_mems", [(8, 64), (520, 64), (40, 2500)])   # sliced, fused, segmented selection
+# sliced, a block per lane, several slices, exact tiles, brackets, brackets in segments
+@pytest.mark.parametrize("T,n_mems", [(8, 64), (520, 64), (40, 2500), (520, 200), (520, 300), (520, 1100)])
 def test_nan_queries_keep_indices_inside_the_cache(T, n_mems):
     # a NaN score wins no comparison, so a row of NaN scores picks nothing: the indices written must still
     # be block numbers of the cache (the gather follows them), and the output is NaN rather than a fault

@@ -29,6 +29,27 @@ def test_picks_match_the_oracle(n, T, k, D, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("n", [2, 100, 300])
+def test_quotients_of_every_value_rank_as_division_ranks_them(n, D, dtype):
+    """Two blocks score a finite 16-bit number and the next one, the others the lowest: the second is picked where the quotients by
+    sqrt(D), divided in fp32 and rounded, differ.  A quotient one place off would turn a tie into a difference, or the reverse."""
+    from landmark_hip.retrieval import retrieve_topk
+    block = 4
+    bits = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16)
+    x = bits.view(dtype)
+    x = x[x.isfinite()].float().sort().values.to(dtype)                 # -0 and +0 side by side
+    q = torch.zeros(1, 1, x.numel() - 1, D, dtype=dtype)
+    q[0, 0, :, 0], q[0, 0, :, 1], q[0, 0, :, 2] = x[:-1], x[1:], x[-1]
+    kc = torch.zeros(1, 1, n * block, D, dtype=dtype)
+    kc[0, 0, block - 1, 0], kc[0, 0, 2 * block - 1, 1], kc[0, 0, 3 * block - 1::block, 2] = 1, 1, -1
+    cos, sin = torch.ones((n + 2) * block, D, dtype=dtype), torch.zeros((n + 2) * block, D, dtype=dtype)
+    idx = retrieve_topk(q.cuda(), kc.cuda(), cos.cuda(), sin.cuda(), block, 1).cpu()[0, 0, :, 0]
+    c = (x.float() / torch.tensor(float(D)).sqrt()).to(dtype)
+    assert torch.equal(idx, (c[1:] > c[:-1]).long())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n", [50, 128, 200, 1024, 1100])
 def test_equal_scores_go_to_the_lowest_block(n, dtype):
     from landmark_hip.retrieval import retrieve_topk
