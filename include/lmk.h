@@ -286,8 +286,8 @@ int lmk_gather_attend(const lmk_tensor4* q, const lmk_tensor4* kcache, const lmk
                       int dtype, void* stream);
 
 /* Scratch of a gather by block: (row, picked block) pairs of a step in which a block is picked by several rows are worked on
- * block by block, on the matrix cores, and what each pair contributes is kept in fp32 until its row's are summed.  0 where the
- * gather by row serves.  n_blocks: complete blocks of the cache; shared: the queries of a head share one selection.
+ * block by block, on the matrix cores, and what each pair contributes is kept in fp32 until its row's are summed; at most 256 MiB,
+ * for as many rows at a time.  0 where the gather by row serves.  n_blocks: complete blocks of the cache; shared: the queries of a head share one selection.
  * lmk_attend and lmk_retrieve_and_attend work by block when their attend workspace is this much larger than
  * lmk_attend_workspace_bytes, lmk_ring_gather_attend_blocks when its workspace holds it; the results are the same
  * attention, summed in another order. */

@@ -233,8 +233,8 @@ __device__ __forceinline__ void store_tile_rows(const f32x16_t* acc, float scl, 
   const int rk = ln >> 2, rq = ln & 3;
   // 8-byte piece s of row r sits at piece s ^ (r / 4 & 7): four rows fill the banks' width, so the same piece of every fourth
   // row meets in one bank, and the writes of a tile took eight accesses each (eight waves' tiles at once are 16 K cycles of the
-  // compute unit's LDS): D128, B16 L512 H32 block 32 dQ 142.6 -> 137.5, forward 98.9 -> 94.7 us, B4 H12 L1000 block 100 dK/dV 62.5
-  // -> 60.5, B1 H8 L1024 block 32 30.2 -> 29.2; from 0 to 4 % over the attention kernels
+  // compute unit's LDS): D128, block 32, forward of B16 L512 H32 88.4 -> 84.6 us, dK/dV of B1 H8 L1024 30.0 -> 29.0; dQ and the
+  // kernels of B2 H32 L2048 or block 100 the same within 1 %
   const int wx = (ln >> 2) & 7, wr = xb + (ln & 31) * 64, rx = (rk >> 2) & 7;
   char* out[2];
 #pragma unroll

@@ -3,11 +3,11 @@
 // benchmark models' ring cache).
 //
 // Row by row, a block that 25 rows picked is read, rotated and multiplied 25 times, on the vector unit: 255 queries of 24
-// heads of 64 over a ring of 40 blocks of 51, top 4, took 54.7 us for 12 MB of cache; the two kernels here take 13.3 + 4.0.
+// heads of 64 over a ring of 40 blocks of 51, top 4, took 54.7 us for 12 MB of cache; the two kernels here take 15.0 + 4.0.
 // A workgroup owns up to four blocks of one (batch, head): it collects the rows that picked them, and attends for up to 32 of
 // them at a time on the matrix cores.
-// A pick is (row, rank), and a block's keys sit at positions that depend on the pick's rank in its row: a wave takes 32
-// picks of one rank, rotates the keys for that rank as it reads them -- fragment ks of a lane holds its key's head dims
+// A pick is (row, rank), and a block's keys sit at positions that depend on the pick's rank in its row: a wave takes up to 32
+// picks of one rank, rotates the keys for that rank, once for them, as it reads them -- fragment ks of a lane holds its key's head dims
 // 16 ks + 8 h .. + 7, whose rotary partners are fragment ks + KS / 2 of the same lane -- and multiplies the rotated key as
 // the sum of three 16-bit numbers, which keeps every bit of the fp32 rotation (KeyParts; with two, scores in the thousands
 // came out up to 1.6 times as far from float64 as row by row; the third costs the step 1 to 3 %).  The local softmax and the
@@ -368,9 +368,9 @@ static int launch_blocks_t(const RetrParams& p, int rows, hipStream_t stream) {
   static std::atomic<uint64_t> lds_ok{0};
   if (int rc = allow_dynamic_lds(kern, 2 * C::TILE * C::MAX_OWN + C::LIST_BYTES, lds_ok)) return rc;
   // Blocks per workgroup: its search of the picks and its first loads serve them all, and its waves even them out, as long
-  // as every compute unit has two workgroups (32 heads of 128, 256 queries, block 32, top 5 of 128 blocks: the step takes
-  // 102.9 us with one block, 92.8 with two, 86.8 with four; 12 heads of 64 x 2, 255 queries, top 4 of 40 blocks of 51: 50.5,
-  // 51.8 and 55.4)
+  // as every compute unit has two workgroups (256 queries of 32 heads of 128, top 4: 64 blocks of 32 take 63.4 us a step with one
+  // block, 59.9 with two, 58.1 with four, 128 blocks of 64 118.9 and 107.9; 512 queries of 12 heads of 64, 128 blocks of 64: 47.3,
+  // 45.1 and 48.7)
   int own = C::MAX_OWN;
   while (own > 1 && (int64_t)p.B * p.H * ((p.num_mems + own - 1) / own) < 2 * cu_count()) own >>= 1;
   for (int t = 0; t < p.T; t += rows) {                 // as many rows as the workspace holds the picks of

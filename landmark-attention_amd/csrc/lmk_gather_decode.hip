@@ -429,7 +429,9 @@ static int launch_decode_t(RetrParams p, hipStream_t stream) {
   // (head dim 64: four) of four waves, but one of five to eight where a SIMD takes three waves.  us a step by waves for the
   // blocks, D128: 512 rows, block 64, top 8: 8 46.8, 4 48.1, 3 43.1, 2 44.2; 1024 rows, top 5: 5 58.3, 3 55.6, 2 51.7 (with two, four
   // workgroups: all rows at once); block 128: 1024 rows, top 5: 5 110.6, 2 94.3, 1 85.3, 512 rows, top 4: 4 48.0, 2 43.5, 1 51.6;
-  // D64, 512 rows, block 64, top 8: 8 30.0, 4 27.3, 3 28.5, 1024 rows, top 5: 5 39.7, 4 33.2, 3 32.8.
+  // D64, 512 rows, block 64, top 8: 8 30.0, 4 27.3, 3 28.5, 1024 rows, top 5: 5 39.7, 4 33.2, 3 32.8.  Over 300 to 1024 rows and top 1,
+  // 2, 3, 4, 5 and 8 the lines below are within 1.3 % (geometric mean) of the best of one to four waves in every band, block and
+  // head dim, but for 3 % at D64, block 128, above 768 rows; against the kernels of longer chunks 0.84 of the time, 1.04 at worst.
   constexpr int most = std::min(kDecodeWaves, 131072 / C::REGION);
   const int64_t rows = (int64_t)p.B * p.H * p.T, cus = cu_count();
   int cap = most;

@@ -6,8 +6,9 @@
 // Selection must be reproducible bit for bit, so the score of (query, landmark) is defined
 // as: fp32 dot product accumulated sequentially over the head dim with one fma per element,
 // rounded to the model dtype, divided in fp32 by sqrt(hd), rounded again (the two roundings of
-// `matmul(...) / math.sqrt(head_dim)`, :367).  Up to 256 blocks every pair is evaluated that way (a block
-// per lane, or matrix-core tiles of the same chain); with more that would dominate the step, so the work is split:
+// `matmul(...) / math.sqrt(head_dim)`, :367).  Every pair is evaluated that way up to 64 blocks (a block per
+// lane), up to 256 where at most 16 are picked (matrix-core tiles of the same chain), and for few rows (slices); elsewhere
+// that would dominate the step, so the work is split:
 //   lk      rotate every cached landmark key at its slot position (:359-366), exactly as the
 //           model dtype would round it, into a dense side array, with its 2-norm
 //   score   MFMA product q . lk^T -> approximate fp32 scores
