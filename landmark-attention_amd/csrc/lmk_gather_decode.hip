@@ -431,8 +431,9 @@ static int launch_decode_t(RetrParams p, hipStream_t stream) {
   // workgroups: all rows at once); block 128: 1024 rows, top 5: 5 110.6, 2 94.3, 1 85.3, 512 rows, top 4: 4 48.0, 2 43.5, 1 51.6;
   // D64, 512 rows, block 64, top 8: 8 30.0, 4 27.3, 3 28.5, 1024 rows, top 5: 5 39.7, 4 33.2, 3 32.8.  Over 300 to 1024 rows and top 1,
   // 2, 3, 4, 5 and 8 the lines below are within 1.3 % (geometric mean) of the best of one to four waves in every band, block and
-  // head dim, but for 3 % at D64, block 128, above 768 rows; against the kernels of longer chunks 0.84 of the time, 1.04 at worst.
-  constexpr int most = std::min(kDecodeWaves, 131072 / C::REGION);
+  // head dim, but for 3 % at D64, block 128, above 768 rows; against the kernels of longer chunks 0.83 of the time, 1.04 at worst
+  // (block 128, D128, top 6, 8 rows: 25.8 for 24.8; top 5 takes five waves, all of a compute unit's LDS: 20.7, with three 24.8).
+  constexpr int most = std::min(kDecodeWaves, 163840 / C::REGION);
   const int64_t rows = (int64_t)p.B * p.H * p.T, cus = cu_count();
   int cap = most;
   if (rows > cus) {

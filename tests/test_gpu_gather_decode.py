@@ -17,7 +17,7 @@ CASES = [(1, 3, T, n, tail, block, k, D)
          for D in (64, 128)
          for block in (32, 64, 128)
          for T, n, tail, k in ((1, 1, 0, 1), (1, 9, block - 1, 9), (4, 5, block - 4, 3), (2, 17, 16, 17))]
-CASES += [(1, 2, 1, 70, 5, 32, 64, 64), (1, 2, 1, 66, 40, 64, 64, 128), (1, 2, 3, 300, 1, 32, 8, 128)]
+CASES += [(1, 2, 1, 70, 5, 32, 64, 64), (1, 2, 1, 66, 40, 64, 64, 128), (1, 2, 3, 300, 1, 32, 8, 128), (1, 2, 1, 9, 21, 128, 5, 128), (1, 2, 1, 11, 90, 128, 10, 128)]
 CASES += [(B, 32, 1, 9, 21, block, 5, D) for B in (9, 17, 25, 33) for block, D in ((32, 128), (64, 64), (128, 128))]
 CASES += [(33, 32, 2, 6, 3, 64, 4, 128), (33, 32, 2, 6, 3, 128, 4, 64)]
 
