@@ -1824,10 +1824,14 @@ static int launch_topk_shared_t(const RetrParams& p, hipStream_t stream) {
   const int64_t rows = (int64_t)p.B * p.H * p.T;
   if (p.num_mems <= kProbMems) {
     // rows per wave: a vector's rows in one workgroup where that is at most 8 each (the launch saved outweighs the rows in a
-    // row: 255 tokens over 40 blocks, maxima over 12 heads, 44.6 -> 42.1 us a step), else as many as leave the chip a few
-    // thousand waves
+    // row: 255 tokens over 40 blocks, maxima over 12 heads, 44.6 -> 42.1 us a step); over more than 256 blocks, where a row is 16 or
+    // 32 values a lane, at most 3 each or with other vectors to fill the chip; else as many as leave the chip a few thousand
+    // waves.  A selection of 8 heads, D128, 16 queries over 516 blocks: one row each 21.3 us, four 24.7; 32 queries 21.7, eight 33.1;
+    // over 2048 blocks 30.6 and 61.9.  Maxima over 12 heads, 500 blocks: one 26.6, three 26.1; over 32, 1000 blocks, 2 x 16 queries
+    // 31.4, eight 45.5, 2 x 500 150.7 and 137.6.
     const int group = p.agg_over_heads ? p.H : p.T;
-    const int rpw = group <= 32 ? (group + 3) / 4 : (int)std::max<int64_t>(1, std::min<int64_t>(8, rows / 4096));
+    const bool whole = group <= (p.num_mems <= 256 || rows >= 16384 ? 32 : 12);
+    const int rpw = whole ? (group + 3) / 4 : (int)std::max<int64_t>(1, std::min<int64_t>(8, rows / 4096));
     const int n_parts = (group + 4 * rpw - 1) / (4 * rpw);
     const dim3 grid((unsigned)(sel_rows * n_parts));
     auto launch = [&](auto prob, auto select) {

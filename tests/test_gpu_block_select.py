@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n,T,k", [(1, 1, 1), (64, 32, 64), (65, 33, 3), (256, 70, 8), (257, 31, 4), (1024, 129, 5), (1025, 5, 2),
-                                   (2048, 34, 64), (2049, 34, 7)])
+@pytest.mark.parametrize("n,T,k", [(1, 1, 1), (64, 32, 64), (65, 33, 3), (256, 70, 8), (257, 31, 4), (257, 12, 4), (300, 13, 5),
+                                   (1024, 129, 5), (1025, 5, 2), (2048, 34, 64), (2049, 34, 7)])
 def test_per_head_picks_match_the_oracle(n, T, k, dtype):
     from landmark_hip.retrieval import retrieve_topk
     print(f"case per head: {n} blocks T{T} top {k} {dtype}", flush=True)
@@ -27,7 +27,8 @@ def test_per_head_picks_match_the_oracle(n, T, k, dtype):
 
 
 @pytest.mark.parametrize("method,code", [("max_over_heads", 1), ("max_over_tokens", 2)])
-@pytest.mark.parametrize("n,oldest,H,T,k", [(1, 0, 3, 2, 1), (8, 3, 33, 5, 4), (64, 17, 12, 40, 4), (65, 64, 2, 33, 64), (300, 7, 32, 3, 5)])
+@pytest.mark.parametrize("n,oldest,H,T,k", [(1, 0, 3, 2, 1), (8, 3, 33, 5, 4), (64, 17, 12, 40, 4), (65, 64, 2, 33, 64), (300, 7, 32, 3, 5),
+                                                  (270, 7, 32, 260, 3)])
 def test_ring_picks_match_the_oracle(n, oldest, H, T, k, method, code):
     from landmark_hip import _lib
     print(f"case ring {method}: {n} blocks, oldest {oldest}, H{H} T{T} top {k}", flush=True)
